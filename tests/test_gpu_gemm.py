@@ -184,6 +184,17 @@ def test_f32_bf16_acts_and_group64(q, orc):
     assert orc.relerr(got, want) < TOL_F32
 
 
+@pytest.mark.parametrize("mode,K,N,rows,act", [
+    ("nn", 40, 3072, [2049], "f32"), ("tn", 128, 3080, [2047], "f32"), ("nt", 2048, 3072, [33], "f32"),      # 64x64 outputs per workgroup
+    ("nn", 136, 512, [1, 513, 31], "f32"), ("tn", 128, 264, [577], "bf16"), ("nt", 520, 512, [0, 129], "bf16"),  # 32x32, four along the contraction
+    ("nn", 392, 128, [9, 1, 33], "f32"), ("tn", 640, 72, [5], "f32"), ("nt", 40, 72, [300, 7], "f32"),        # 32x32, sixteen
+    ("nn", 37, 128, [50, 6], "f32"), ("tn", 128, 45, [66], "bf16"), ("nt", 45, 37, [101], "f32")])            # units put together element by element
+def test_f32_shapes_of_a_workgroup(q, orc, mode, K, N, rows, act):
+    got, want = run_case(q, orc, mode, len(rows), rows, K, N, pkg.ACT_F32 if act == "f32" else pkg.ACT_BF16, pkg.MATH_F32, seed=11,
+                         beta=1.0 if mode == "tn" else 0.0)
+    assert orc.relerr(got, want) < TOL_F32
+
+
 # ------------------------------------------------------------------ bf16 MFMA kernels
 @pytest.mark.parametrize("mode", ["nn", "tn", "nt"])
 def test_mfma_grouped_zipf_small(q, orc, mode):
