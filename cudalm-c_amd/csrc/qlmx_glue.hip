@@ -16,8 +16,8 @@
 #include "qlmx_dev.h"
 #include "qlmx_gemm.h"
 
-/* ---- router: one thread per token, experts visited in order so the softmax sum rounds exactly as
- * the reference's loop does. `logit` points at the token's E logits and `pr` at E floats for its
+/* ---- router, more than 64 experts: one thread per token, experts visited in order so the softmax sum rounds
+ * exactly as the reference's loop does. `logit` points at the token's E logits and `pr` at E floats for its
  * probabilities (the two may be the same place). ---- */
 __device__ __forceinline__ void route_token(const float *logit, float *pr, int n, int *assign, float *gate,
                                             int N, int E, int K, const float *bias, int bs){
@@ -84,138 +84,149 @@ __global__ void __launch_bounds__(RT_TOK) k_router_topk_lds(const float *rt, flo
     }
 }
 
-/* Expert count known at compile time (at most 64): the token's row lives in registers between the
- * staged load and the staged store, the chosen experts in a bit mask. Same operations in the same
- * order as route_token. */
-template<int EE>
-__global__ void __launch_bounds__(RT_TOK) k_router_topk_reg(const float *rt, float *rprobs, int *assign, float *gate,
-                                                            int N, int K, const float *bias, int bs){
-    __shared__ float rows[RT_TOK * (EE | 1)];
-    constexpr int ld = EE | 1;
-    const int n0 = blockIdx.x * RT_TOK, tid = threadIdx.x;
-    const int cnt = min(RT_TOK, N - n0) * EE;
-    const float *src = rt + (size_t)n0 * EE;
-    for(int i = tid; i < cnt; i += RT_TOK) rows[(i / EE) * ld + (i % EE)] = src[i];
+/* At most 64 experts: a token on G lanes, one expert each (G = 8, 16, 32 or 64, 64/G tokens per wavefront). A thread
+ * per token walked its experts one after the other, K + 3 times, each time a chain of dependent instructions: 6-10 us
+ * for one to sixteen tokens, 20 for a few hundred, 48 for 32768 x 64, against 2.4-4.6 and 22 with a lane per expert. What
+ * the contract fixes is the softmax sum: in expert order from 0. Every lane adds the G terms in that order, read
+ * from LDS four at a time (the lanes past E hold zeros, which change no sum). A pick is the largest score, ties to the
+ * lowest expert: the group's maximum, then the lowest lane that holds it; a score not above -1e30 (or NaN) is no
+ * candidate, and without a candidate the pick is expert k, as in the loop above. */
+template<int G> __device__ __forceinline__ float rt_group_max(float v){
+    v = fmaxf(v, qx_dpp<0xB1>(v));
+    v = fmaxf(v, qx_dpp<0x4E>(v));
+    v = fmaxf(v, qx_dpp<0x141>(v));
+    if(G >= 16) v = fmaxf(v, qx_dpp<0x140>(v));
+    if(G >= 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
+    if(G >= 64) v = fmaxf(v, __shfl_xor(v, 32, 64));
+    return v;
+}
+#define RT_WG 256
+template<int G>
+__global__ void __launch_bounds__(RT_WG) k_router_topk_lanes(const float *rt, float *rprobs, int *assign, float *gate,
+                                                            int N, int E, int K, const float *bias, int bs){
+    __shared__ __attribute__((aligned(16))) float terms[RT_WG];
+    const int tid = threadIdx.x, lane = tid & 63, e = tid & (G - 1), g0 = lane & ~(G - 1);
+    const int n = blockIdx.x * (RT_WG / G) + tid / G;
+    const bool on = n < N && e < E;
+    const size_t at = (size_t)n * E + e;
+    const float l = on ? rt[at] : -INFINITY;
+    const float mx = fmaxf(rt_group_max<G>(l), -1e30f);
+    float p = on ? qx_fexp(l - mx) : 0.0f;
+    terms[tid] = p;
     __syncthreads();
-    const int n = n0 + tid;
-    if(n < N){
-        float p[EE];
+    float sum = 0.0f;
+    const float4 *row = (const float4 *)(terms + (tid & ~(G - 1)));
 #pragma unroll
-        for(int e = 0; e < EE; e++) p[e] = rows[tid * ld + e];
-        float mx = -1e30f;
-#pragma unroll
-        for(int e = 0; e < EE; e++) if(p[e] > mx) mx = p[e];
-        float sum = 0.0f;
-#pragma unroll
-        for(int e = 0; e < EE; e++){ p[e] = qx_fexp(p[e] - mx); sum += p[e]; }
-        const float inv = 1.0f / sum;
-#pragma unroll
-        for(int e = 0; e < EE; e++){ p[e] *= inv; rows[tid * ld + e] = p[e]; }
-        unsigned long long taken = 0ULL;
-        for(int k = 0; k < K; k++){
-            int best = -1; float bestp = -1e30f;
-#pragma unroll
-            for(int e = 0; e < EE; e++){
-                const float sc = p[e] + (bias ? bias[k * bs + e] : 0.0f);
-                if(!((taken >> e) & 1ULL) && sc > bestp){ bestp = sc; best = e; }
-            }
-            if(best < 0) best = k;
-            taken |= 1ULL << best;
-            float gv = 0.0f;
-#pragma unroll
-            for(int e = 0; e < EE; e++) if(e == best) gv = p[e];
-            assign[(size_t)k * N + n] = best;
-            gate[(size_t)k * N + n] = gv;
-        }
+    for(int i = 0; i < G / 4; i++){ const float4 v = row[i]; sum += v.x; sum += v.y; sum += v.z; sum += v.w; }
+    p *= 1.0f / sum;
+    if(on) rprobs[at] = p;
+    bool open = on;                                       /* an expert of this token that is not picked yet */
+    for(int k = 0; k < K; k++){
+        const float sc = p + (bias && on ? bias[k * bs + e] : 0.0f);
+        const float v = (open && sc > -1e30f) ? sc : -INFINITY;
+        const float m = rt_group_max<G>(v);
+        unsigned long long hit = __ballot(v == m && v > -INFINITY) >> g0;
+        if(G < 64) hit &= (1ull << G) - 1;
+        const int best = hit ? __ffsll((long long)hit) - 1 : k;
+        const float gv = __shfl(p, g0 + best, 64);
+        if(e == 0 && n < N){ assign[(size_t)k * N + n] = best; gate[(size_t)k * N + n] = gv; }
+        open = open && e != best;
     }
-    __syncthreads();
-    float *dst = rprobs + (size_t)n0 * EE;
-    for(int i = tid; i < cnt; i += RT_TOK) dst[i] = rows[(i / EE) * ld + (i % EE)];
 }
 
 /* ---- grouping permutation of one pass: perm lists the tokens expert by expert, tokens of one
  * expert in ascending order; off[e] is the first row of expert e, off[E] = N.
- * Launches: clear, per-chunk histograms (which also add up the experts' totals), scan, stable placement. ---- */
-#define GP_CHUNK 256
-/* workspace: ch[K][NC][E] chunk histograms, then 4 ints (the first is the out-of-range flag), then
- * tot[K][E] per-expert totals */
-__global__ void __launch_bounds__(256) k_gp_clear(int *bad, int ntot){
-    for(int i = threadIdx.x; i < 4 + ntot; i += 256) bad[i] = 0;
-}
-__global__ void __launch_bounds__(GP_CHUNK) k_gp_hist(const int *asn, int N, int E, int NC, int *ch, int *bad){
-    extern __shared__ int hist[];
-    const int c = blockIdx.x, k = blockIdx.y, n = c * GP_CHUNK + threadIdx.x;
-    int *tot = bad + 4;
-    for(int e = threadIdx.x; e < E; e += GP_CHUNK) hist[e] = 0;
+ * A workgroup places the tokens of one chunk, its wavefronts one contiguous segment each, 64 tokens at a time: the
+ * lanes that share an expert are found with one ballot per bit of the expert's number, a token's row is the next free
+ * row of (wavefront, expert) plus the number of earlier lanes with its expert. Up to GP_ONE tokens are one chunk and
+ * one launch; more are cut into at most 64 chunks, whose histograms a first launch leaves in the workspace and every
+ * workgroup of the second adds up for itself. Kernel times for 386 tokens: 3.9 us (clear, histograms, scan and placement
+ * as four launches: 17); 16384: 11 us (20); 131072: 13 us (33). ---- */
+#define GP_ONE 4096
+static inline int gp_chunk(int N){ return N <= GP_ONE ? N : 2048 * ((N + 2048 * 64 - 1) / (2048 * 64)); }
+static inline int gp_threads(int E){ return E <= 896 ? 1024 : E <= 2600 ? 256 : 64; }   /* [wavefronts + 2][E] counters in 64 KB of LDS */
+/* workspace: hist[K][NC][E], then seen[K][NC] (0, or -1-e for an expert number e out of range) and, at the offset that
+ * qlmx_moe_perm_status reads, the flag for the whole call */
+__global__ void __launch_bounds__(1024) k_gp_hist(const int *asn, int N, int E, int chunk, int *hist, int *seen){
+    extern __shared__ int cnt[];                          /* [E], then the flag */
+    const int c = blockIdx.x, k = blockIdx.y, end = min(N, (c + 1) * chunk);
+    for(int e = threadIdx.x; e <= E; e += blockDim.x) cnt[e] = 0;
     __syncthreads();
-    if(n < N){
+    for(int n = c * chunk + threadIdx.x; n < end; n += blockDim.x){
         const int e = asn[(size_t)k * N + n];
-        if((unsigned)e >= (unsigned)E) atomicExch(bad, -1 - e); else atomicAdd(&hist[e], 1);
+        if((unsigned)e < (unsigned)E) atomicAdd(&cnt[e], 1); else cnt[E] = -1 - e;
     }
     __syncthreads();
-    for(int e = threadIdx.x; e < E; e += GP_CHUNK){
-        const int h = hist[e];
-        ch[((size_t)k * NC + c) * E + e] = h;
-        if(h) atomicAdd(&tot[(size_t)k * E + e], h);
-    }
+    const size_t at = (size_t)k * gridDim.x + c;
+    for(int e = threadIdx.x; e < E; e += blockDim.x) hist[at * E + e] = cnt[e];
+    if(threadIdx.x == 0) seen[at] = cnt[E];
 }
 __device__ __forceinline__ int wave_incl_scan(int v, int lane){
 #pragma unroll
     for(int d = 1; d < 64; d <<= 1){ const int u = __shfl_up(v, d, 64); if(lane >= d) v += u; }
     return v;
 }
-/* one wavefront per (pass, expert), and one more per pass for off[E]: the expert's first row is the
- * sum of the totals of the experts before it; ch[k][c][e] becomes the first output row of
- * (chunk c, expert e), 64 chunks per scan step */
-__global__ void __launch_bounds__(256) k_gp_scan(int *ch, const int *tot, int E, int NC, int *off){
-    const int k = blockIdx.y, lane = threadIdx.x & 63, e = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if(e > E) return;
-    int base = 0;
-    for(int j0 = 0; j0 < e; j0 += 64){
-        const int j = j0 + lane;
-        base += j < e ? tot[(size_t)k * E + j] : 0;
-    }
-#pragma unroll
-    for(int d = 32; d >= 1; d >>= 1) base += __shfl_xor(base, d, 64);
-    if(lane == 0) off[(size_t)k * (E + 1) + e] = base;
-    if(e == E) return;
-    int *col = ch + (size_t)k * NC * E + e;
-    int run = base;
-    for(int c0 = 0; c0 < NC; c0 += 64){
-        const int c = c0 + lane;
-        const int t = c < NC ? col[(size_t)c * E] : 0;
-        const int incl = wave_incl_scan(t, lane);
-        if(c < NC) col[(size_t)c * E] = run + incl - t;
-        run += __shfl(incl, 63, 64);
-    }
-}
-/* stable placement: a token's row = start of (its chunk, its expert) + the number of earlier
- * tokens of the chunk with the same expert. Inside a wavefront that number is a population count
- * over the lanes that share the expert; the four wavefronts add up in order through LDS. */
-__global__ void __launch_bounds__(GP_CHUNK) k_gp_scatter(const int *asn, int N, int E, int NC, const int *co, int *perm){
-    extern __shared__ int wcnt[];                       /* [4][E] */
-    const int c = blockIdx.x, k = blockIdx.y, n = c * GP_CHUNK + threadIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for(int i = threadIdx.x; i < 4 * E; i += GP_CHUNK) wcnt[i] = 0;
+__global__ void __launch_bounds__(1024) k_gp_place(const int *asn, int N, int E, int chunk, const int *hist, const int *seen,
+                                                   int *perm, int *off, int *bad){
+    extern __shared__ int lds[];                          /* next[waves][E], first[E + 1] (totals, then first rows), earlier[E], flag */
+    const int c = blockIdx.x, k = blockIdx.y, NC = gridDim.x, NT = blockDim.x, NW = NT >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int *next = lds, *mine = lds + wave * E, *first = lds + NW * E, *earlier = first + E + 1, *flag = earlier + E;
+    const int *a = asn + (size_t)k * N;
+    const int n0 = c * chunk, n1 = min(N, n0 + chunk);
+    const int seg = ((n1 - n0 + NW - 1) / NW + 63) & ~63, s0 = n0 + wave * seg, s1 = min(n1, s0 + seg);
+    for(int i = tid; i < (NW + 2) * E + 2; i += NT) lds[i] = 0;
     __syncthreads();
-    int e = -1;
-    if(n < N){ e = asn[(size_t)k * N + n]; if((unsigned)e >= (unsigned)E) e = -1; }
-    int rank = 0;
-    unsigned long long remaining = __ballot(e >= 0);
-    while(remaining){
-        const int leader = __ffsll((long long)remaining) - 1;
-        const int e0 = __shfl(e, leader, 64);
-        const unsigned long long m = __ballot(e == e0);
-        if(e == e0){
-            rank = __popcll(m & ((1ull << lane) - 1ull));
-            if(lane == leader) wcnt[wave * E + e0] = __popcll(m);
+    for(int n = s0 + lane; n < s1; n += 64){
+        const int e = a[n];
+        if((unsigned)e < (unsigned)E) atomicAdd(&mine[e], 1); else *flag = -1 - e;
+    }
+    __syncthreads();
+    /* an expert's tokens in the chunks before this one, and in all of them */
+    if(NC > 1){
+        for(int x = tid; x < NC * E; x += NT){
+            const int h = hist[(size_t)k * NC * E + x], i = x / E, e = x - i * E;
+            if(h){ atomicAdd(&first[e], h); if(i < c) atomicAdd(&earlier[e], h); }
         }
-        remaining &= ~m;
+        __syncthreads();
+    }
+    for(int e = tid; e < E; e += NT){
+        int row = earlier[e];
+        for(int w = 0; w < NW; w++){ const int h = next[w * E + e]; next[w * E + e] = row; row += h; }
+        if(NC == 1) first[e] = row;
     }
     __syncthreads();
-    if(e >= 0){
-        for(int w = 0; w < wave; w++) rank += wcnt[w * E + e];
-        perm[(size_t)k * N + co[((size_t)k * NC + c) * E + e] + rank] = n;
+    if(wave == 0){
+        int run = 0;
+        for(int e0 = 0; e0 < E; e0 += 64){
+            const int e = e0 + lane, t = e < E ? first[e] : 0, incl = wave_incl_scan(t, lane);
+            if(e < E) first[e] = run + incl - t;
+            run += __shfl(incl, 63, 64);
+        }
+        if(lane == 0) first[E] = run;
+    }
+    __syncthreads();
+    if(c == 0){
+        for(int e = tid; e <= E; e += NT) off[(size_t)k * (E + 1) + e] = first[e];
+        if(k == 0 && wave == 0){
+            int f = *flag;
+            if(seen) for(int i = lane; i < NC * (int)gridDim.y; i += 64) if(seen[i]) f = seen[i];
+            const unsigned long long any = __ballot(f != 0);
+            f = any ? __shfl(f, __ffsll((long long)any) - 1, 64) : 0;
+            if(lane == 0) *bad = f;
+        }
+    }
+    const int bits = 32 - __clz(E);
+    for(int n = s0 + lane; n - lane < s1; n += 64){
+        const int e = n < s1 ? a[n] : -1;
+        const bool ok = (unsigned)e < (unsigned)E;
+        unsigned long long same = __ballot(ok);
+        for(int b = 0; b < bits; b++){ const unsigned long long m = __ballot((e >> b) & 1); same &= ((e >> b) & 1) ? m : ~m; }
+        if(ok){
+            const int row = mine[e], rank = __popcll(same & ((1ull << lane) - 1));
+            perm[(size_t)k * N + first[e] + row + rank] = n;
+            if(rank == 0) mine[e] = row + __popcll(same);
+        }
     }
 }
 
@@ -301,6 +312,17 @@ __global__ void __launch_bounds__(256) k_moe_dgate(const float4 *dout, const flo
 /* ---- all K passes as ONE expert-grouped list of K*N rows (the reference's merged top-K, cudalm.cu:3532-3561,
  * 4022-4034): the grouping permutation of the K*N assignments names entries m = pass * N + token; row p of the
  * grouped buffers holds token perm[p] % N, and inv[m] is the row that holds entry m. ---- */
+/* one workgroup for all of it: the fill and what follows it need no launch of their own */
+#define MR_ONE 8192
+__global__ void __launch_bounds__(1024) k_merge_rows_one(const int *perm, int KN, int N, int *tok, int *inv){
+    for(int p = threadIdx.x; p < KN; p += 1024) inv[p] = -1;
+    __syncthreads();
+    for(int p = threadIdx.x; p < KN; p += 1024){
+        const int m = perm[p];
+        tok[p] = m < 0 ? -1 : m % N;
+        if(m >= 0) inv[m] = p;
+    }
+}
 __global__ void __launch_bounds__(256) k_merge_rows(const int *perm, int KN, int N, int *tok, int *inv){
     const int p = blockIdx.x * 256 + threadIdx.x;
     if(p >= KN) return;
@@ -372,13 +394,13 @@ extern "C" int qlmx_router_topk(const float *rt, float *rprobs, int *assign, flo
     QLMX_REQUIRE(rt && rprobs && assign && gate, "qlmx_router_topk: NULL buffer");
     QLMX_REQUIRE(N >= 0 && E > 0 && K > 0 && K <= 8 && K <= E, "qlmx_router_topk: N=%d E=%d K=%d (K at most 8 and at most E)", N, E, K);
     if(N == 0) return QLMX_OK;
-    const dim3 rgrid((N + RT_TOK - 1) / RT_TOK);
-#define ROUTE_REG(EE) hipLaunchKernelGGL(k_router_topk_reg<EE>, rgrid, dim3(RT_TOK), 0, (hipStream_t)stream, rt, rprobs, assign, gate, N, K, bias, bs)
-    if(E == 8) ROUTE_REG(8);
-    else if(E == 16) ROUTE_REG(16);
-    else if(E == 32) ROUTE_REG(32);
-    else if(E == 64) ROUTE_REG(64);
-#undef ROUTE_REG
+#define ROUTE_LANES(G) hipLaunchKernelGGL(k_router_topk_lanes<G>, dim3((N + RT_WG / G - 1) / (RT_WG / G)), dim3(RT_WG), 0, (hipStream_t)stream, \
+                                          rt, rprobs, assign, gate, N, E, K, bias, bs)
+    if(E <= 8) ROUTE_LANES(8);
+    else if(E <= 16) ROUTE_LANES(16);
+    else if(E <= 32) ROUTE_LANES(32);
+    else if(E <= 64) ROUTE_LANES(64);
+#undef ROUTE_LANES
     else if(E <= RT_MAXE)
         hipLaunchKernelGGL(k_router_topk_lds, dim3((N + RT_TOK - 1) / RT_TOK), dim3(RT_TOK), (size_t)RT_TOK * (E | 1) * sizeof(float),
                            (hipStream_t)stream, rt, rprobs, assign, gate, N, E, K, bias, bs);
@@ -388,9 +410,10 @@ extern "C" int qlmx_router_topk(const float *rt, float *rprobs, int *assign, flo
     return QLMX_OK;
 }
 
+#define GP_CHUNK 256          /* the workspace has room for a histogram per 256 tokens, more than gp_chunk cuts */
+static size_t gp_flag_at(int N, int E, int K){ return (size_t)K * ((size_t)(N + GP_CHUNK - 1) / GP_CHUNK) * E; }
 extern "C" size_t qlmx_moe_perm_workspace(int N, int E, int K){
-    const size_t NC = (size_t)(N + GP_CHUNK - 1) / GP_CHUNK;
-    return ((size_t)K * NC * E + 4 + (size_t)K * E) * sizeof(int);
+    return (gp_flag_at(N, E, K) + 4 + (size_t)K * E) * sizeof(int);
 }
 
 extern "C" int qlmx_moe_perm(const int *assign, int N, int E, int K, int *perm, int *off, void *workspace, void *stream){
@@ -398,16 +421,15 @@ extern "C" int qlmx_moe_perm(const int *assign, int N, int E, int K, int *perm, 
     hipStream_t st = (hipStream_t)stream;
     QLMX_REQUIRE(assign && perm && off && workspace, "qlmx_moe_perm: NULL buffer");
     QLMX_REQUIRE(N > 0 && E > 0 && E <= 4096 && K > 0, "qlmx_moe_perm: N=%d E=%d K=%d", N, E, K);
-    const int NC = (N + GP_CHUNK - 1) / GP_CHUNK;
-    int *ch = (int *)workspace, *bad = ch + (size_t)K * NC * E;
-    hipLaunchKernelGGL(k_gp_clear, dim3(1), dim3(256), 0, st, bad, K * E);       /* a kernel, not a memset: callers may capture this into a graph */
-    QLMX_LAUNCH_CHECK("perm flag clear");
-    hipLaunchKernelGGL(k_gp_hist, dim3(NC, K), dim3(GP_CHUNK), E * sizeof(int), st, assign, N, E, NC, ch, bad);
-    QLMX_LAUNCH_CHECK("perm histogram launch");
-    hipLaunchKernelGGL(k_gp_scan, dim3((E + 1 + 3) / 4, K), dim3(256), 0, st, ch, (const int *)(bad + 4), E, NC, off);
-    QLMX_LAUNCH_CHECK("perm scan launch");
-    hipLaunchKernelGGL(k_gp_scatter, dim3(NC, K), dim3(GP_CHUNK), 4 * E * sizeof(int), st, assign, N, E, NC, (const int *)ch, perm);
-    QLMX_LAUNCH_CHECK("perm scatter launch");
+    const int chunk = gp_chunk(N), NC = (N + chunk - 1) / chunk, NT = gp_threads(E);
+    int *hist = (int *)workspace, *seen = hist + (size_t)K * NC * E, *bad = hist + gp_flag_at(N, E, K);
+    if(NC > 1){
+        hipLaunchKernelGGL(k_gp_hist, dim3(NC, K), dim3(NT), (E + 1) * sizeof(int), st, assign, N, E, chunk, hist, seen);
+        QLMX_LAUNCH_CHECK("perm histogram launch");
+    }
+    hipLaunchKernelGGL(k_gp_place, dim3(NC, K), dim3(NT), ((size_t)(NT / 64 + 2) * E + 2) * sizeof(int), st, assign, N, E, chunk,
+                       (const int *)hist, (const int *)(NC > 1 ? seen : nullptr), perm, off, bad);
+    QLMX_LAUNCH_CHECK("perm placement launch");
     return QLMX_OK;
 }
 
@@ -416,9 +438,8 @@ extern "C" int qlmx_moe_perm(const int *assign, int N, int E, int K, int *perm, 
 extern "C" int qlmx_moe_perm_status(const void *workspace, int N, int E, int K, void *stream){
     int rc = qlmx_check_ready(); if(rc) return rc;
     QLMX_REQUIRE(workspace, "qlmx_moe_perm_status: NULL workspace");
-    const int NC = (N + GP_CHUNK - 1) / GP_CHUNK;
     int bad = 0;
-    QLMX_HIP(hipMemcpyAsync(&bad, (const int *)workspace + (size_t)K * NC * E, sizeof(int), hipMemcpyDeviceToHost, (hipStream_t)stream), "perm flag read");
+    QLMX_HIP(hipMemcpyAsync(&bad, (const int *)workspace + gp_flag_at(N, E, K), sizeof(int), hipMemcpyDeviceToHost, (hipStream_t)stream), "perm flag read");
     QLMX_HIP(hipStreamSynchronize((hipStream_t)stream), "perm flag sync");
     if(bad){ qlmx_set_error("qlmx_moe_perm: expert index %d out of range [0, %d)", -1 - bad, E); return QLMX_E_ARG; }
     return QLMX_OK;
@@ -482,6 +503,11 @@ extern "C" int qlmx_moe_merge_rows(const int *perm, int N, int K, int *tok, int 
     QLMX_REQUIRE(perm && tok && inv, "qlmx_moe_merge_rows: NULL buffer");
     QLMX_REQUIRE(N > 0 && K > 0 && (long long)N * K < (1LL << 31), "qlmx_moe_merge_rows: N=%d K=%d", N, K);
     const int KN = N * K;
+    if(KN <= MR_ONE){
+        hipLaunchKernelGGL(k_merge_rows_one, dim3(1), dim3(1024), 0, (hipStream_t)stream, perm, KN, N, tok, inv);
+        QLMX_LAUNCH_CHECK("merge rows launch");
+        return QLMX_OK;
+    }
     /* rows a caller dropped (perm < 0) leave no inverse: -1 everywhere first, by a kernel so that a capture holds no memset node */
     hipLaunchKernelGGL(k_fill_i32, dim3((KN + 255) / 256), dim3(256), 0, (hipStream_t)stream, inv, -1, KN);
     QLMX_LAUNCH_CHECK("merge rows: inverse fill");

@@ -130,6 +130,39 @@ def test_perm_vs_oracle(q, orc, N, E, K):
         assert np.array_equal(perm[k * N:(k + 1) * N], wp)
 
 
+@pytest.mark.parametrize("N,E,K", [(4096, 64, 1), (4097, 2, 2), (6145, 896, 1), (5000, 897, 2), (300, 2601, 1), (4500, 4096, 1), (131073, 64, 1), (64, 1, 3)])
+def test_perm_chunks_vs_oracle(q, orc, N, E, K):
+    """The last size that is one chunk, the first that is several, chunks that grow past 2048 tokens, a chunk of one
+    token, and the expert counts at which the workgroup gets fewer wavefronts."""
+    asn = np.random.default_rng(N + E).integers(0, E, K * N).astype(np.int32)
+    perm, off, _ = gpu_perm(q, asn, N, E, K)
+    for k in range(K):
+        wp = np.zeros(N, np.int32); wo = np.zeros(E + 1, np.int32)
+        assert orc.moe_perm(asn[k * N:(k + 1) * N], N, E, wp, wo) == 0
+        assert np.array_equal(off[k * (E + 1):(k + 1) * (E + 1)], wo)
+        assert np.array_equal(perm[k * N:(k + 1) * N], wp)
+
+
+@pytest.mark.parametrize("N,K", [(1, 2), (4096, 2), (4097, 2)])
+def test_merge_rows_with_dropped_entries(q, N, K):
+    import torch
+    perm = np.random.default_rng(N).permutation(N * K).astype(np.int32)
+    perm[::3] = -1
+    tok, inv = zeros(N * K, torch.int32), zeros(N * K, torch.int32)
+    q.moe_merge_rows(dev(perm), N, K, tok, inv)
+    torch.cuda.synchronize()
+    want = np.full(N * K, -1, np.int32)
+    want[perm[perm >= 0]] = np.nonzero(perm >= 0)[0]
+    assert np.array_equal(inv.cpu().numpy(), want)
+    assert np.array_equal(tok.cpu().numpy(), np.where(perm < 0, -1, perm % N))
+
+
+def test_perm_reports_bad_expert_of_any_chunk(q):
+    asn = np.zeros(9000, np.int32); asn[8999] = 77
+    with pytest.raises(pkg.QlmxError, match="index 77 out of range"):
+        gpu_perm(q, asn, 9000, 4, 1)
+
+
 def test_perm_workspace_reused(q, orc):
     """The same workspace serves one call after another (its counters are cleared by each call)."""
     import torch
