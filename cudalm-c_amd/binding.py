@@ -262,14 +262,15 @@ class Qlmx:
         """P: fp32 numpy array -> (uint8 numpy array in the wire format, number of raw groups)"""
         import numpy as np
         cap = int(self.lib.qlmx_q4n_bound(P.size, group))
-        out = np.zeros(max(cap, 1), np.uint8)
+        out = np.empty(max(cap, 1), np.uint8)            # the bound; given back down to the length in use
         n, raw = C.c_size_t(0), C.c_size_t(0)
         self.call("qlmx_q4n_quantize", P, P.size, group, out, cap, C.addressof(n), C.addressof(raw))
-        return out[:n.value].copy(), int(raw.value)
+        out.resize(n.value, refcheck=False)
+        return out, int(raw.value)
 
     def q4n_dequantize(self, buf, n, group):
         import numpy as np
-        P = np.zeros(n, np.float32)
+        P = np.empty(n, np.float32)
         used = C.c_size_t(0)
         self.call("qlmx_q4n_dequantize", buf, buf.size, P, n, group, C.addressof(used))
         return P, int(used.value)

@@ -69,6 +69,28 @@ def test_rendered_qlm_view_round_trips_without_raw_groups(lib, orc):
     assert oraw == 0 and np.array_equal(ob, buf)
 
 
+@pytest.mark.parametrize("n,group", [(1, 2), (15, 16), (17, 34), (8 * 128 + 9, 128), (262143, 64), (262145, 128), (700001, 96), (2300000, 128)])
+def test_sizes_around_the_vector_and_thread_shares(lib, orc, n, group):
+    """Tails of a vector and of a group, and value counts that are one, two and many threads' shares; groups that are
+    raw, zero, hold infinities and NaN, or take a later candidate."""
+    rng = np.random.default_rng(n)
+    P = (rng.integers(-7, 8, n) * f32(0.0173)).astype(f32)
+    ng = -(-n // group)
+    for k, q in enumerate(rng.permutation(ng)[:max(1, ng // 5)]):
+        v = P[q * group:(q + 1) * group]
+        if k % 5 == 0: v[:] = rng.normal(size=v.size)
+        elif k % 5 == 1: v[:] = 0.0
+        elif k % 5 == 2: v[-1] = np.inf
+        elif k % 5 == 3: v[0] = np.nan
+        else: v[:] = (rng.integers(-3, 4, v.size) * f32(3e-41)).astype(f32)
+    want, wraw = orc.q4n_quantize(P, group)
+    got, raw = lib.q4n_quantize(P, group)
+    assert raw == wraw and np.array_equal(got, want)
+    back, used = lib.q4n_dequantize(got, n, group)
+    ok, wback = orc.q4n_dequantize(want, n, group)
+    assert ok == 1 and used == want.size and np.array_equal(back.view(np.uint32), wback.view(np.uint32))
+
+
 def test_truncated_buffer_is_refused(lib, orc, golden):
     g = golden("q4n")
     n, group = (int(v) for v in g["dims"])
