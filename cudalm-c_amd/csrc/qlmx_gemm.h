@@ -40,6 +40,15 @@ int qlmx_upload_problems_split(const qlmx_gemm_prob *first, const qlmx_gemm_prob
                                int tile_rows, int tile_cols, const RowBytes *rb, hipStream_t stream, ProbUpload *out, int *slot);
 int qlmx_upload_done(int slot, hipStream_t stream);
 
+/* The kernels for problems of few rows (qlmx_gemm_small.hip), and whether a call is theirs */
+bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int N, int group);
+int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N,
+                              int io, const void *xsrc, float *out, const float *gate, hipStream_t st);
+int qlmx_gemm_nn_small_swiglu_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *gate, const qlmx_gemm_prob *up_, int nprob,
+                                     int K, int N, const void *xsrc, hipStream_t st);
+int qlmx_gemm_tn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, const qlmx_gemm_prob *second, int nprob,
+                              int K, int N, float *out, const float *gp, const float *up_, void *dg, void *du, hipStream_t st);
+
 /* Locate the problem owning flattened tile t: the last one whose tile0 <= t (tile0 ascending, empty
  * problems share the tile0 of their successor). Every lane reads the tile0 of one problem and the
  * wavefront counts the hits, so the lookup costs one memory round trip per 64 problems; a binary

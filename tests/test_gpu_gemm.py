@@ -209,6 +209,18 @@ def test_mfma_grouped_zipf_small(q, orc, mode):
     assert err < TOL_MFMA, err
 
 
+@pytest.mark.parametrize("mode,K,N,group", [("nn", 768, 256, 128), ("nn", 32, 128, 64), ("nn", 96, 384, 64), ("nn", 2048, 512, 256),
+                                            ("tn", 768, 256, 128), ("tn", 64, 128, 64), ("tn", 192, 384, 64), ("tn", 2048, 128, 256)])
+@pytest.mark.parametrize("rows", [[1], [16, 0, 9], [17, 32, 3, 31], [33, 64, 48]])
+def test_mfma_few_rows(q, orc, mode, K, N, group, rows):
+    """The kernels for experts of few rows: every row tile, contractions shorter than a step per wavefront, scale groups
+    that split a lane group's columns, both load widths of the input gradient; beta 0 and 1."""
+    for beta in ((0.0,) if mode == "nn" else (0.0, 1.0)):
+        got, want = run_case(q, orc, mode, len(rows), rows, K, N, pkg.ACT_BF16, pkg.MATH_MFMA_F16 if mode == "nn" else pkg.MATH_MFMA,
+                             seed=21, beta=beta, group=group)
+        assert orc.relerr(got, want) < (4e-4 if mode == "nn" else 3e-6)
+
+
 @pytest.mark.parametrize("mode,K,N", [("nn", 768, 2048), ("nn", 2048, 768), ("tn", 768, 2048), ("tn", 2048, 768),
                                       ("nt", 768, 2048), ("nt", 2048, 768)])
 def test_mfma_layer_shapes(q, orc, mode, K, N):
