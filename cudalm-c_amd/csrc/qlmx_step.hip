@@ -809,8 +809,8 @@ extern "C" int qlmx_step_touched(float *P, const float *Gc, signed char *d, sign
  * k_sqsum: 64 partial sums of squares; partial c covers G[n*c/64 .. n*(c+1)/64), is accumulated in
  * double and rounded to float once (the CPU path's definition; the reference's GPU kernel sums
  * strided in fp32 and differs from its own CPU kernel in the last bits). The 64 partials are the
- * contract, 64 workgroups are not: each chunk is cut into SQ_W pieces, one workgroup each (1024
- * workgroups for the 256 CUs), which sum in double -- lanes strided, then a fixed tree -- and leave
+ * contract, 64 workgroups are not: each chunk is shared by SQ_W workgroups (1024
+ * for the 256 CUs), which sum in double -- threads strided, then a fixed tree -- and leave
  * their sum in a device array; the workgroup that arrives last at a chunk (a counter) adds the SQ_W
  * sums in piece order, so the result does not depend on arrival order. The order of the double
  * additions is not the CPU's, which can move the double sum by a few units in its last place -- far
@@ -823,22 +823,35 @@ static __device__ unsigned g_sq_count[64];
 __global__ void __launch_bounds__(256) k_qlmx_sqsum(const float *G, unsigned long long n, float *part){
     __shared__ double red[256];
     const unsigned c = blockIdx.x / SQ_W, w = blockIdx.x % SQ_W;
-    const unsigned long long c0 = n * c / 64, c1 = n * (c + 1) / 64, len = c1 - c0;
-    const unsigned long long i0 = c0 + len * w / SQ_W, i1 = c0 + len * (w + 1) / SQ_W;
+    const unsigned long long i0 = n * c / 64, i1 = n * (c + 1) / 64, t0 = w * 256 + threadIdx.x, stride = SQ_W * 256;
     double s = 0.0;
     /* 16-byte loads over the aligned middle, single elements at both ends */
     unsigned long long a0 = (i0 + 3) & ~3ULL; if(a0 > i1) a0 = i1;
     const unsigned long long a1 = a0 + ((i1 - a0) & ~3ULL);
-    for(unsigned long long i = i0 + threadIdx.x; i < a0; i += 256){ const double g = (double)G[i]; s += g * g; }
+    for(unsigned long long i = i0 + t0; i < a0; i += stride){ const double g = (double)G[i]; s += g * g; }
     if((((uintptr_t)G) & 15) == 0){
-        for(unsigned long long i = a0 + 4ULL * threadIdx.x; i < a1; i += 1024){
-            const float4 v = *(const float4 *)(G + i);
-            s += (double)v.x * (double)v.x; s += (double)v.y * (double)v.y; s += (double)v.z * (double)v.z; s += (double)v.w * (double)v.w;
+        /* The chunk's workgroups side by side, four loads of a thread on their way and four sums: with a stretch of its
+         * own per workgroup, one load and one chain of additions HBM delivered 3.2 TB/s (125.8 M values: 157 us, now
+         * 127, the 4 TB/s that reading alone reaches; twice and four times the workgroups: 178 and 281). A square of
+         * a float is exact in double, so the fma adds what the product and the sum would. */
+        double u[4] = {0.0, 0.0, 0.0, 0.0};
+        auto add = [](double &t, const float4 &v){
+            t = fma((double)v.x, (double)v.x, t); t = fma((double)v.y, (double)v.y, t); t = fma((double)v.z, (double)v.z, t); t = fma((double)v.w, (double)v.w, t);
+        };
+        unsigned long long i = a0 + 4 * t0;
+        for(; i + 12 * stride < a1; i += 16 * stride){
+            float4 v[4];
+#pragma unroll
+            for(int q = 0; q < 4; q++) v[q] = *(const float4 *)(G + i + q * (4 * stride));
+#pragma unroll
+            for(int q = 0; q < 4; q++) add(u[q], v[q]);
         }
+        for(; i < a1; i += 4 * stride) add(u[0], *(const float4 *)(G + i));
+        s += (u[0] + u[1]) + (u[2] + u[3]);
     } else {
-        for(unsigned long long i = a0 + threadIdx.x; i < a1; i += 256){ const double g = (double)G[i]; s += g * g; }
+        for(unsigned long long i = a0 + t0; i < a1; i += stride){ const double g = (double)G[i]; s += g * g; }
     }
-    for(unsigned long long i = a1 + threadIdx.x; i < i1; i += 256){ const double g = (double)G[i]; s += g * g; }
+    for(unsigned long long i = a1 + t0; i < i1; i += stride){ const double g = (double)G[i]; s += g * g; }
     red[threadIdx.x] = s;
     __syncthreads();
     for(int o = 128; o > 0; o >>= 1){
@@ -859,11 +872,19 @@ __global__ void __launch_bounds__(256) k_qlmx_sqsum(const float *G, unsigned lon
 
 /* k_gnorm (cudalm.cu:2811-2816 = cpu_kern.h:541-546): part = G's 64 partials followed by nside more
  * slices of 64; gs[0] = clip multiplier (exactly 1 when the norm is <= 1), gs[1] = the norm; a
- * non-finite side sum makes the norm NaN. One thread, the reference's order of additions. */
-__global__ void k_qlmx_gnorm(const float *part, int nside, int clip_side, float *gs){
+ * non-finite side sum makes the norm NaN. One wavefront reads a slice, one thread adds in the reference's order. */
+__global__ void __launch_bounds__(64) k_qlmx_gnorm(const float *part, int nside, int clip_side, float *gs){
+    __shared__ double slice[64];
     double ss = 0.0, sd = 0.0;
-    for(int i = 0; i < 64; i++) ss += (double)part[i];
-    for(int i = 64; i < 64 * (1 + nside); i++) sd += (double)part[i];
+    for(int k = 0; k <= nside; k++){
+        slice[threadIdx.x] = (double)part[k * 64 + threadIdx.x];
+        __syncthreads();
+        double &t = k ? sd : ss;
+#pragma unroll
+        for(int i = 0; i < 64; i++) t += slice[i];
+        __syncthreads();
+    }
+    if(threadIdx.x != 0) return;
     float gn = (float)sqrt(clip_side ? ss + sd : ss);
     if(!isfinite(sd)) gn = __builtin_nanf("");
     gs[0] = gn > 1.0f ? 1.0f / gn : 1.0f;
@@ -881,7 +902,7 @@ extern "C" int qlmx_sqsum(const float *G, unsigned long long n, float *part64, v
 extern "C" int qlmx_gnorm(const float *part, int nside, int clip_side, float *gs, void *stream){
     int rc = qlmx_check_ready(); if(rc) return rc;
     QLMX_REQUIRE(part && gs && nside >= 0, "qlmx_gnorm: bad arguments");
-    hipLaunchKernelGGL(k_qlmx_gnorm, dim3(1), dim3(1), 0, (hipStream_t)stream, part, nside, clip_side, gs);
+    hipLaunchKernelGGL(k_qlmx_gnorm, dim3(1), dim3(64), 0, (hipStream_t)stream, part, nside, clip_side, gs);
     QLMX_LAUNCH_CHECK("qlmx_gnorm launch");
     return QLMX_OK;
 }
