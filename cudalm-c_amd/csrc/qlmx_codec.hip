@@ -114,43 +114,13 @@ __global__ void __launch_bounds__(256) k_qlmx_render(float *P, const signed char
     }
 }
 
-__global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char *r, float *s,
-                                                    const qlmx_span *sp, int nspan, int group, int dmax,
-                                                    float f_hi, float f_lo, int packed, int ngrp, int vec_ok){
-    const int lane16 = threadIdx.x & 15;
-    const int gi = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) >> 4);
-    if(gi >= ngrp) return;
-    const GroupLoc L = group_loc(sp, nspan, gi, group);
-    if(vec_ok && group == 128 && packed && L.n == 128 && (L.qi0 & 7ULL) == 0){
-        /* 8 consecutive elements per lane: one 32-bit word of digits, and 8 residual bytes only where the
-         * group is rescaled */
-        const uint64_t e0 = L.qi0 + (uint64_t)lane16 * 8;
-        const uint32_t dw = *(const uint32_t *)(d + (e0 >> 1));
-        int dv[8], railed = 0;
-#pragma unroll
-        for(int k = 0; k < 8; k++){ dv[k] = qx_nib(dw, k); railed += (dv[k] == dmax) | (dv[k] == -dmax); }
-        railed = qx_row16_sum(railed);
-        const float f = (float)railed / 128.0f, sg = s[gi];
-        float sn;
-        if(f > f_hi)      sn = sg * 1.09051f;
-        else if(f < f_lo) sn = sg / 1.09051f;
-        else return;
-        const float conv = sg / sn;
-        if(lane16 == 0) s[gi] = sn;
-        const uint2 rw = *(const uint2 *)(r + e0);
-        uint32_t dn = 0, r0 = 0, r1 = 0;
-#pragma unroll
-        for(int k = 0; k < 8; k++){
-            const int rb = (int)(signed char)(((k < 4 ? rw.x : rw.y) >> (8 * (k & 3))) & 0xFFu);
-            const float t = ((float)dv[k] + (float)rb * (1.0f / 128.0f)) * conv;
-            int dd, rr; quantize(t, dmax, dd, rr);
-            dn |= ((uint32_t)dd & 15u) << (4 * k);
-            if(k < 4) r0 |= ((uint32_t)rr & 0xFFu) << (8 * k); else r1 |= ((uint32_t)rr & 0xFFu) << (8 * (k - 4));
-        }
-        *(uint32_t *)(d + (e0 >> 1)) = dn;
-        *(uint2 *)(r + e0) = make_uint2(r0, r1);
-        return;
-    }
+/* the servo's new scale for a group with `railed` of n digits at their bound; the old one where it stays */
+__device__ __forceinline__ float servo_scale(float sg, int railed, int n, float f_hi, float f_lo){
+    const float f = (float)railed / (float)n;
+    return f > f_hi ? sg * 1.09051f : f < f_lo ? sg / 1.09051f : sg;          /* 2^(1/8) */
+}
+/* any group: a pair of elements per lane and step */
+__device__ void servo_pairs(const GroupLoc &L, int gi, int lane16, signed char *d, signed char *r, float *s, int dmax, float f_hi, float f_lo, int packed){
     int railed = 0;
     for(int jb = 2 * lane16; jb < L.n; jb += 32)
         for(int h = 0; h < 2; h++){
@@ -159,11 +129,8 @@ __global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char 
         }
     railed = qx_row16_sum(railed);
     const float f = (float)railed / (float)L.n, sg = s[gi];
-    float sn;
-    if(f > f_hi)      sn = sg * 1.09051f;          /* 2^(1/8) */
-    else if(f < f_lo) sn = sg / 1.09051f;
-    else return;                                   /* uniform over the row */
-    const float conv = sg / sn;
+    if(!(f > f_hi || f < f_lo)) return;             /* uniform over the row */
+    const float sn = servo_scale(sg, railed, L.n, f_hi, f_lo), conv = sg / sn;
     if(lane16 == 0) s[gi] = sn;
     for(int jb = 2 * lane16; jb < L.n; jb += 32){
         int dn[2] = {0, 0};
@@ -180,6 +147,82 @@ __global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char 
         }
         if(packed) d[(L.qi0 + jb) >> 1] = (signed char)(((dn[1] & 15) << 4) | (dn[0] & 15));
     }
+}
+/* how many of w's eight nibbles equal those of `of` */
+__device__ __forceinline__ int nibbles_equal(uint32_t w, uint32_t of){
+    uint32_t x = w ^ of;
+    x |= x >> 2; x |= x >> 1;
+    return 8 - __popc(x & 0x11111111u);
+}
+/* Full aligned groups of 128 go 8 consecutive elements per lane: one 32-bit word of digits, and 8 residual bytes only
+ * where the group is rescaled. What bounds the kernel is vector instructions, not HBM. A workgroup counts 64 groups, a
+ * row of 16 lanes SV_G of them with their loads side by side, and lists the few that move; its rows then share the list,
+ * so that re-encoding (160 instructions) runs for wavefronts full of moving groups instead of for every wavefront with
+ * one among its four. 151 M weights, 15 % of the groups moving: 119 us with one group per row from start to end, 77
+ * now. */
+#define SV_G 4
+__global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char *r, float *s,
+                                                    const qlmx_span *sp, int nspan, int group, int dmax,
+                                                    float f_hi, float f_lo, int packed, int ngrp, int vec_ok){
+    __shared__ uint64_t at[16 * SV_G];                     /* the moving groups: first element, old scale / new scale */
+    __shared__ float conv[16 * SV_G];
+    __shared__ int moving;
+    const int lane16 = threadIdx.x & 15, row = threadIdx.x >> 4, first = (int)blockIdx.x * (16 * SV_G) + row;
+    if(threadIdx.x == 0) moving = 0;
+    __syncthreads();
+    bool fast[SV_G];
+    if(first < ngrp){
+        qlmx_span S = sp[qx_span_of(sp, nspan, first)];
+        uint64_t q0[SV_G]; uint32_t dw[SV_G]; float sg[SV_G];
+#pragma unroll
+        for(int q = 0; q < SV_G; q++){
+            const int gi = first + q * 16;
+            fast[q] = false; dw[q] = 0; sg[q] = 0.0f; q0[q] = 0;
+            if(gi >= ngrp) continue;
+            if(gi >= S.gi0 + S.ngrp) S = sp[qx_span_of(sp, nspan, gi)];
+            const uint64_t j0 = (uint64_t)(gi - S.gi0) * (uint64_t)group;
+            fast[q] = vec_ok && group == 128 && packed && S.n - j0 >= 128 && ((S.qi0 + j0) & 7ULL) == 0;
+            if(!fast[q]) continue;
+            q0[q] = S.qi0 + j0;
+            dw[q] = *(const uint32_t *)(d + (q0[q] >> 1) + lane16 * 4);
+            sg[q] = s[gi];
+        }
+        const uint32_t up = 0x11111111u * (uint32_t)(dmax & 15), down = 0x11111111u * (uint32_t)(-dmax & 15);
+#pragma unroll
+        for(int q = 0; q < SV_G; q++){
+            const int railed = qx_row16_sum(nibbles_equal(dw[q], up) + nibbles_equal(dw[q], down));
+            const float f = (float)railed * (1.0f / 128.0f);
+            if(fast[q] && lane16 == 0 && (f > f_hi || f < f_lo)){
+                const float sn = servo_scale(sg[q], railed, 128, f_hi, f_lo);
+                const int k = atomicAdd(&moving, 1);
+                at[k] = q0[q]; conv[k] = sg[q] / sn;
+                s[first + q * 16] = sn;
+            }
+        }
+    }
+    __syncthreads();
+    for(int k = row; k < moving; k += 16){
+        const uint64_t e0 = at[k] + (uint64_t)lane16 * 8;
+        const uint32_t dw = *(const uint32_t *)(d + (e0 >> 1));
+        const uint2 rw = *(const uint2 *)(r + e0);
+        const float cv = conv[k];
+        uint32_t dn = 0, r0 = 0, r1 = 0;
+#pragma unroll
+        for(int k8 = 0; k8 < 8; k8++){
+            const int rb = (int)(signed char)(((k8 < 4 ? rw.x : rw.y) >> (8 * (k8 & 3))) & 0xFFu);
+            const float t = ((float)qx_nib(dw, k8) + (float)rb * (1.0f / 128.0f)) * cv;
+            int dd, rr; quantize(t, dmax, dd, rr);
+            dn |= ((uint32_t)dd & 15u) << (4 * k8);
+            if(k8 < 4) r0 |= ((uint32_t)rr & 0xFFu) << (8 * k8); else r1 |= ((uint32_t)rr & 0xFFu) << (8 * (k8 - 4));
+        }
+        *(uint32_t *)(d + (e0 >> 1)) = dn;
+        *(uint2 *)(r + e0) = make_uint2(r0, r1);
+    }
+    if(first < ngrp)
+        for(int q = 0; q < SV_G; q++){
+            const int gi = first + q * 16;
+            if(gi < ngrp && !fast[q]) servo_pairs(group_loc(sp, nspan, gi, group), gi, lane16, d, r, s, dmax, f_hi, f_lo, packed);
+        }
 }
 
 static int codec_args_ok(const char *who, int nspan, int group, int dmax, int packed){
@@ -227,7 +270,7 @@ extern "C" int qlmx_servo(signed char *d, signed char *r, float *s,
     rc = codec_args_ok("qlmx_servo", nspan, group, dmax, packed); if(rc) return rc;
     if(ngrp <= 0) return QLMX_OK;
     const int vec_ok = ((uintptr_t)r & 7) == 0 && ((uintptr_t)d & 3) == 0;
-    hipLaunchKernelGGL(k_qlmx_servo, dim3((unsigned)((ngrp + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_qlmx_servo, dim3((unsigned)((ngrp + 16 * SV_G - 1) / (16 * SV_G))), dim3(256), 0, (hipStream_t)stream,
                        d, r, s, sp, nspan, group, dmax, f_hi, f_lo, packed, ngrp, vec_ok);
     QLMX_LAUNCH_CHECK("qlmx_servo launch");
     return QLMX_OK;

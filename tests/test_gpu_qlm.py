@@ -97,6 +97,21 @@ def test_servo_vs_oracle_seeded(q, orc):
     assert up > 100 and down > 100 and ng - up - down > 100
 
 
+@pytest.mark.parametrize("sizes", [[128], [128 * 63], [128 * 64, 128], [128 * 64 + 8, 128 * 70 + 40, 128 * 3]])
+@pytest.mark.parametrize("f_hi,f_lo", [(2.0, -1.0), (-1.0, -2.0), (0.14, 0.13)])
+def test_servo_workgroup_shares_vs_oracle(q, orc, sizes, f_hi, f_lo):
+    """Group counts around the 64 of a workgroup, spans that begin inside one (aligned and not), with no group, every
+    group and nearly every group moving."""
+    group, dmax = 128, 7
+    tab, nq, ng = make_spans(sizes, group)
+    hd = orc.digits(nq, 9, 1); hr = orc.int8(nq, 9, 2, -64, 64)
+    hs = orc.uniform(ng, 9, 3, 0.5, 1.5) * f32(0.02 * 3 / 7)
+    d, r, s = dev(hd), dev(hr), dev(hs)
+    q.servo(d, r, s, dev(tab), len(tab), group, dmax, f_hi, f_lo, 1, ng)
+    orc.servo(hd, hr, hs, tab, group, dmax, f_hi, f_lo, 1, ng)
+    assert beq(d, hd) and beq(r, hr) and beq(s, hs)
+
+
 @pytest.mark.parametrize("nopview", [False, True])
 def test_step_vs_oracle_seeded_2m(q, orc, nopview):
     """Three consecutive steps over 2M weights in two spans (one with a short tail group and a
