@@ -41,7 +41,7 @@ int qlmx_upload_problems_split(const qlmx_gemm_prob *first, const qlmx_gemm_prob
 int qlmx_upload_done(int slot, hipStream_t stream);
 
 /* The kernels for problems of few rows (qlmx_gemm_small.hip), and whether a call is theirs */
-bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int N, int group);
+bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, int N, int nseg, int group);
 int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N,
                               int io, const void *xsrc, float *out, const float *gate, hipStream_t st);
 int qlmx_gemm_nn_small_swiglu_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *gate, const qlmx_gemm_prob *up_, int nprob,

@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_nn_h_swiglu(NhArgs a){
 int qlmx_gemm_nn_h_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob,
                           int K, int N, int io, const void *xsrc, float *out, const float *gate, hipStream_t st){
     QLMX_REQUIRE(io != NH_GATHER || (size_t)K * 2 <= NH_ZERO_BYTES, "grouped gemm nn with gather: K=%d exceeds %d", K, NH_ZERO_BYTES / 2);
-    if(qlmx_small_rows(probs, nprob, N, group)) return qlmx_gemm_nn_small_launch(d, s, group, probs, nprob, K, N, io, xsrc, out, gate, st);
+    if(qlmx_small_rows(probs, nprob, GEMM_NN, K, N, 1, group)) return qlmx_gemm_nn_small_launch(d, s, group, probs, nprob, K, N, io, xsrc, out, gate, st);
     ProbUpload up; int slot;
     const RowBytes rb = {io == NH_GATHER ? sizeof(int) : (size_t)K * 2, io == NH_SCATTER ? sizeof(int) : (size_t)N * 4, 0, 0, 0};
     int rc = qlmx_upload_problems_split(probs, nullptr, nprob, GEMM_NN, K, N, NH_BM, NH_BN, &rb, st, &up, &slot); if(rc) return rc;
@@ -363,7 +363,7 @@ int qlmx_gemm_nn_h_launch(const signed char *d, const float *s, int group, const
 int qlmx_gemm_nn_h_swiglu_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *gate, const qlmx_gemm_prob *up_,
                                  int nprob, int K, int N, const void *xsrc, hipStream_t st){
     QLMX_REQUIRE(!xsrc || (size_t)K * 2 <= NH_ZERO_BYTES, "grouped gemm nn + swiglu with gather: K=%d exceeds %d", K, NH_ZERO_BYTES / 2);
-    if(N % 128 == 0 && qlmx_small_rows(gate, nprob, N, group)) return qlmx_gemm_nn_small_swiglu_launch(d, s, group, gate, up_, nprob, K, N, xsrc, st);
+    if(N % 128 == 0 && qlmx_small_rows(gate, nprob, GEMM_NN, K, N, 1, group)) return qlmx_gemm_nn_small_swiglu_launch(d, s, group, gate, up_, nprob, K, N, xsrc, st);
     ProbUpload up; int slot;
     const RowBytes rb = {xsrc ? sizeof(int) : (size_t)K * 2, (size_t)N * 4, 0, (size_t)N * 2, (size_t)N * 4};
     int rc = qlmx_upload_problems_split(gate, up_, nprob, GEMM_NN, K, N, NH_BM, NH_BN / 2, &rb, st, &up, &slot); if(rc) return rc;

@@ -5,27 +5,29 @@
  * whole contraction, one LDS tile and one barrier per 32 of it. With a dozen rows a step is some 1000 cycles of
  * LDS, barrier and issue latency around four matrix products, and a call has too few strips to hide it: 36 us for the
  * down projection of 32 experts (2048 x 768, 12 rows each), whose 25 MB of weights take 5. Here nothing passes
- * through LDS on the way in, four (input gradient: eight) wavefronts split the contraction and add up at the end:
+ * meets a barrier on the way in, four wavefronts split the contraction and add up at the end:
  *
  * A wavefront owns 128 (64) columns and its share of the contraction. v_mfma_f32_16x16x32 wants eight consecutive k of one
  * column per lane (lane = column lane%16, k group lane/16). Weights of the forward lie along the columns: the lane
  * loads, for its eight k, the 4-byte word of eight neighbouring columns, and product j takes digit j of the eight words
- * -- the columns of a product are then eight apart, which only the store has to know. Weights of the input
- * gradient lie along k as they should; a lane loads 16 or 32 k of four columns sixteen apart. Activations come from
- * L2 straight as operands (16 bytes of a row per lane). All loads of a step are plain register loads, one to four steps
- * ahead, without a barrier in the loop.
+ * -- the columns of a product are then eight apart, which only the store has to know. Activations come from
+ * L2 straight as operands (16 bytes of a row per lane), all loads are plain register loads, one to four steps ahead. Weights
+ * of the input gradient lie along k as they should; they and the activations go through LDS, each wavefront its own stages.
  *
  * Arithmetic as in the tiled kernels: forward weights fp16(s * digit * 2^8), activations converted exactly; the input
  * gradient multiplies exact digits and applies the scale to the fp32 sums of each group of k.
  *
- * Which calls come here (qlmx_small_rows): all problems of at most 32 rows, or of at most 64 when the call has few column
- * strips. The rule looks at what the forms of a call that are documented to agree bit for bit have in common -- with and
- * without gather, SwiGLU, scatter, inside a pair or not -- so that they run the same arithmetic in the same order.
- * 32 experts, 768 x 2048, us per call at 4 / 30 rows each, tiled kernels -> these: gate|up + SwiGLU 37 / 33 -> 20 / 22, down
- * 27 / 26 -> 12 / 16, its input gradient + SwiGLU 20 / 22 -> 11 / 20, paired input gradient 56 / 58 -> 27 / 33. At 60 rows
- * (two row tiles of 32, the weights converted twice): 192 strips 27 -> 23 and 58 -> 49, 512 strips 35 -> 39 and 25 -> 36.
- * What bounds them now: the conversion of the weights (some 220 vector instructions for 32 x 128 of them) on as many
- * wavefronts as there are, and the round trips in front of and behind it.
+ * Which calls come here (qlmx_small_rows): all whose problems have at most 32 rows, and those that would leave the tiled
+ * kernels with few workgroups, each walking the whole contraction at 0.3 (64 rows) to 0.7 us (256) per 32 of it. Counted in
+ * tiles of 64 rows: forward, 128 columns, up to 256 tiles, 512 where the contraction is twice the width (a wide gate | up
+ * has tiles enough for the tiled kernel); input gradient, 64 columns, up to 512, 1024 where the contraction is twice the
+ * width. Around these lines both take about the same time. The forward's rule looks at what the forms of a call that are documented to agree bit for bit have in common -- with and without gather,
+ * SwiGLU, scatter -- so that they run the same arithmetic in the same order.
+ * us per call, tiled kernels -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
+ * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16
+ * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
+ * What bounds them now: the forward, the conversion of the weights (some 220 vector instructions for 32 x 128 of them); the input
+ * gradient, the 64 bytes per cycle of a CU's address unit; both, the round trips in front of and behind the loop.
  */
 #include "qlmx_gemm.h"
 #include <type_traits>
@@ -39,13 +41,11 @@ typedef float  f32x4 __attribute__((ext_vector_type(4)));
 typedef int    i32x2 __attribute__((ext_vector_type(2)));
 typedef int    i32x4 __attribute__((ext_vector_type(4)));
 
-#define SM_COLS 128
-#define SM_WAVES 4                              /* along the forward's contraction (eight: the same for 2048, 20 % slower for 768) */
-#define SM_TWAVES 8                             /* along the input gradient's */
+#define SM_COLS 128                             /* of a forward strip */
+#define SM_TCOLS 64                             /* of an input-gradient strip */
+#define SM_WAVES 4                              /* along the contraction (eight: the same for 2048, 20 % slower for 768) */
 #define SM_WSCALE 4096.0f                       /* 16 (digits come as digit/16) * 2^8, as NH_WSCALE */
 #define SM_UNSCALE (1.0f / 256.0f)
-#define SM_ROWS 32
-#define SM_STRIPS 256
 
 enum { SM_PLAIN = 0, SM_GATHER = 1, SM_SCATTER = 2, SM_SWIGLU_BWD = 3 };
 struct SmArgs { const DevProb *pr; int nprob, ntiles; const signed char *d; const float *s; int gshift; int K, N;
@@ -54,11 +54,21 @@ struct SmArgs { const DevProb *pr; int nprob, ntiles; const signed char *d; cons
 
 static __device__ __align__(16) unsigned char sm_zero_row[32768];       /* what a dropped row of a gather reads */
 
-bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int N, int group){
+/* see the head of this file */
+bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, int N, int nseg, int group){
     if(group < 64) return false;
-    int most = 0;
-    for(int i = 0; i < nprob; i++) if(probs[i].M > most) most = probs[i].M;
-    return most <= SM_ROWS || (most <= 2 * SM_ROWS && (long long)nprob * (N / SM_COLS) <= SM_STRIPS);
+    long long tiles = 0; int most = 0;
+    for(int i = 0; i < nprob; i++){
+        if(probs[i].M > most) most = probs[i].M;
+        tiles += (probs[i].M + 63) / 64;
+    }
+    if(most <= 32) return true;
+    if(mode == GEMM_NN){
+        tiles *= N / SM_COLS;
+        return (tiles <= 256 && K >= N) || (tiles <= 512 && K >= 2 * N);
+    }
+    tiles *= N / SM_TCOLS;
+    return tiles <= 512 || (tiles <= 1024 && (long long)K * nseg >= 2 * N);
 }
 
 __device__ __forceinline__ int sm_pk_f16(float lo, float hi){ f32x2 v = {lo, hi}; return __builtin_bit_cast(int, __builtin_convertvector(v, f16x2)); }
@@ -76,39 +86,40 @@ template<int I> __device__ __forceinline__ float sm_bcast_hi(float low, float v)
 }
 template<int I, int N, class F> __device__ __forceinline__ void sm_each(const F &f){ if constexpr(I < N){ f(std::integral_constant<int, I>()); sm_each<I + 1, N>(f); } }
 
-/* The sums of the SM_WAVES wavefronts from `first` on, of one 16-row tile, through LDS: `mine(e, j)` is a lane's sum of
- * row (lane/16)*4 + e, column j of its eight. total[u] belongs to place u * threads + thread of the tile's 16 x 32
- * places of four columns. */
-template<int NT, class F> __device__ __forceinline__ void sm_reduce(float *red, int first, const F &mine, f32x4 (&total)[512 / NT]){
-    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) - first, c = lane & 15, g = lane >> 4;
+/* The sums of the four wavefronts from `first` on, of one 16-row tile, through LDS: acc holds a lane's sums of rows
+ * (lane/16)*4 + e, columns (lane%16)*8 + j. */
+__device__ __forceinline__ void sm_put(float *red, int first, const f32x4 (&acc)[8]){
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) - first, c = lane & 15, g = lane >> 4;
     __syncthreads();                                      /* the tile before has been read */
     if(wave >= 0 && wave < SM_WAVES){
         float *w = red + wave * (16 * SM_COLS);
 #pragma unroll
         for(int e = 0; e < 4; e++){
-            *(f32x4 *)&w[(g * 4 + e) * SM_COLS + c * 8]     = (f32x4){mine(e, 0), mine(e, 1), mine(e, 2), mine(e, 3)};
-            *(f32x4 *)&w[(g * 4 + e) * SM_COLS + c * 8 + 4] = (f32x4){mine(e, 4), mine(e, 5), mine(e, 6), mine(e, 7)};
+            *(f32x4 *)&w[(g * 4 + e) * SM_COLS + c * 8]     = (f32x4){acc[0][e], acc[1][e], acc[2][e], acc[3][e]};
+            *(f32x4 *)&w[(g * 4 + e) * SM_COLS + c * 8 + 4] = (f32x4){acc[4][e], acc[5][e], acc[6][e], acc[7][e]};
         }
     }
     __syncthreads();
-    constexpr int U = 512 / NT;
+}
+/* four columns of a row */
+__device__ __forceinline__ f32x4 sm_get(const float *red, int row, int col){
+    f32x4 v = *(const f32x4 *)&red[row * SM_COLS + col];
 #pragma unroll
-    for(int u = 0; u < U; u++){
-        const int x = u * NT + tid;                       /* four columns of one row */
-        f32x4 v = *(const f32x4 *)&red[x * 4];
-#pragma unroll
-        for(int k = 1; k < SM_WAVES; k++) v += *(const f32x4 *)&red[k * (16 * SM_COLS) + x * 4];
-        total[u] = v * SM_UNSCALE;
-    }
+    for(int k = 1; k < SM_WAVES; k++) v += *(const f32x4 *)&red[k * (16 * SM_COLS) + row * SM_COLS + col];
+    return v * SM_UNSCALE;
 }
 
-/* ---- forward. DUAL: gate | up, as many wavefronts again on the second matrix (wq, wg of Q) ---- */
-template<int RT, int IO, bool DUAL, bool G64>
+/* ---- forward, and gate | up in one (the second matrix at wq, wg of Q): SM_BY_WAVE, four more wavefronts work on 128 columns
+ * of up; SM_BY_LANE, the strip is 64 columns of gate (lanes 0-7 of each 16) and 64 of up (lanes 8-15). By wave a row of
+ * weights is read in 64-byte pieces, which is what counts while the weights set the pace (32 experts of 12 rows, 768 x 2048:
+ * 20.6 against 26.3 us); by lane a workgroup is half as large and twice as many fit where 64 rows need 216 registers (8
+ * experts of 250 rows, 512 x 1536: 24.5 against 30.2). TWO: the halves of the strip have scales of their own. ---- */
+enum { SM_ONE = 0, SM_BY_WAVE = 1, SM_BY_LANE = 2 };
+template<int RT, int IO, int DUAL, bool TWO>
 __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, const DevProb &Q, int i0, int j0, float *red){
-    constexpr int PF = RT == 1 ? (DUAL ? 3 : 4) : (DUAL ? 1 : 2);        /* steps on their way */
+    constexpr int PF = RT == 1 ? (DUAL == SM_BY_WAVE ? 3 : 4) : RT == 2 ? (DUAL == SM_BY_WAVE ? 1 : 2) : 1;        /* steps on their way */
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int steps = a.K / 32, ks = wave & (SM_WAVES - 1), st0 = steps * ks / SM_WAVES, st1 = steps * (ks + 1) / SM_WAVES;
-    const bool second = DUAL && wave >= SM_WAVES;
     const char *pa[RT];
 #pragma unroll
     for(int r = 0; r < RT; r++){
@@ -120,8 +131,9 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
         pa[r] += g * 16;
     }
     const size_t gpr = (size_t)a.N >> a.gshift, rowb = (size_t)a.N >> 1;       /* scale groups and bytes per row of weights */
-    const signed char *pw = a.d + (((second ? Q.wq : P.wq) + (size_t)(g * 8) * a.N + j0 + c * 8) >> 1);
-    const float *ps = a.s + (second ? Q.wg : P.wg) + (size_t)(g * 8 + (c & 7)) * gpr + (j0 >> a.gshift) + (G64 ? c >> 3 : 0);
+    const bool second = DUAL == SM_BY_WAVE ? wave >= SM_WAVES : DUAL == SM_BY_LANE && c >= 8;
+    const signed char *pw = a.d + (((second ? Q.wq : P.wq) + (size_t)(g * 8) * a.N + j0 + (DUAL == SM_BY_LANE ? c & 7 : c) * 8) >> 1);
+    const float *ps = a.s + (second ? Q.wg : P.wg) + (size_t)(g * 8 + (c & 7)) * gpr + (j0 >> a.gshift) + (TWO && DUAL != SM_BY_LANE ? c >> 3 : 0);
     f32x4 acc[RT][8];
 #pragma unroll
     for(int r = 0; r < RT; r++)
@@ -151,7 +163,7 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
         sm_each<0, 8>([&](auto KC){
             constexpr int k = decltype(KC)::value;
             sk[k] = sm_bcast<k>(sv);
-            if(G64) sk[k] = sm_bcast_hi<k>(sk[k], sv);
+            if(TWO) sk[k] = sm_bcast_hi<k>(sk[k], sv);
             nb[k] = qx_nibs(w[I][k]);
         });
         load(I, st + PF);
@@ -174,157 +186,217 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
         sm_each<0, PF - 1>([&](auto IC){ if(st + decltype(IC)::value < st1) step(IC, st + decltype(IC)::value); });
     }
     /* ---- totals ---- */
-    constexpr int NT = 64 * SM_WAVES * (DUAL ? 2 : 1), U = 512 / NT;
+    auto swiglu = [&](int lr, int col, const f32x4 &y, const f32x4 &u){
+        if(lr >= P.M) return;
+        const size_t o = (size_t)lr * a.N + j0 + col;
+        if(P.C){ *(f32x4 *)(P.C + o) = y; *(f32x4 *)(Q.C + o) = u; }
+        ushort4 h;
+        h.x = qx_f32_to_bf16(y[0] * qx_fsig_hw(y[0]) * u[0]); h.y = qx_f32_to_bf16(y[1] * qx_fsig_hw(y[1]) * u[1]);
+        h.z = qx_f32_to_bf16(y[2] * qx_fsig_hw(y[2]) * u[2]); h.w = qx_f32_to_bf16(y[3] * qx_fsig_hw(y[3]) * u[3]);
+        *(ushort4 *)((unsigned short *)Q.B + o) = h;
+    };
 #pragma unroll
     for(int r = 0; r < RT; r++){
-        auto mine = [&](int e, int j){ return acc[r][j][e]; };
-        f32x4 ty[U], tu[U];
-        sm_reduce<NT>(red, 0, mine, ty);
-        if constexpr(DUAL) sm_reduce<NT>(red, SM_WAVES, mine, tu);
+        const int i = i0 + r * 16;
+        sm_put(red, 0, acc[r]);
+        if constexpr(DUAL == SM_BY_LANE){
+            const int row = tid >> 4, col = (tid & 15) * 4;
+            swiglu(i + row, col, sm_get(red, row, col), sm_get(red, row, 64 + col));
+        } else if constexpr(DUAL == SM_BY_WAVE){
+            const int row = tid >> 5, col = (tid & 31) * 4;
+            const f32x4 y = sm_get(red, row, col);
+            sm_put(red, SM_WAVES, acc[r]);
+            swiglu(i + row, col, y, sm_get(red, row, col));
+        } else {
 #pragma unroll
-        for(int v = 0; v < U; v++){
-            const int x = v * NT + tid, lr = i0 + r * 16 + (x >> 5);
-            if(lr >= P.M) continue;
-            const f32x4 y = ty[v];
-            const size_t o = (size_t)lr * a.N + j0 + (x & 31) * 4;
-            if constexpr(DUAL){
-                const f32x4 u = tu[v];
-                if(P.C){ *(f32x4 *)(P.C + o) = y; *(f32x4 *)(Q.C + o) = u; }
-                ushort4 h;
-                h.x = qx_f32_to_bf16(y[0] * qx_fsig_hw(y[0]) * u[0]); h.y = qx_f32_to_bf16(y[1] * qx_fsig_hw(y[1]) * u[1]);
-                h.z = qx_f32_to_bf16(y[2] * qx_fsig_hw(y[2]) * u[2]); h.w = qx_f32_to_bf16(y[3] * qx_fsig_hw(y[3]) * u[3]);
-                *(ushort4 *)((unsigned short *)Q.B + o) = h;
-            } else if constexpr(IO == SM_SCATTER){
-                const int tok = ((const int *)P.C)[lr];
-                if(tok >= 0){
-                    qx_gfloat *t = (qx_gfloat *)(a.out + (size_t)tok * a.N + j0 + (x & 31) * 4);
-                    const float gt = a.gate ? a.gate[tok] : 1.0f;
+            for(int v = 0; v < 2; v++){
+                const int row = v * 8 + (tid >> 5), col = (tid & 31) * 4, lr = i + row;
+                const f32x4 y = sm_get(red, row, col);
+                if(lr >= P.M) continue;
+                if constexpr(IO == SM_SCATTER){
+                    const int tok = ((const int *)P.C)[lr];
+                    if(tok >= 0){
+                        qx_gfloat *t = (qx_gfloat *)(a.out + (size_t)tok * a.N + j0 + col);
+                        const float gt = a.gate ? a.gate[tok] : 1.0f;
 #pragma unroll
-                    for(int q = 0; q < 4; q++) (void)__builtin_amdgcn_global_atomic_fadd_f32(t + q, a.gate ? gt * y[q] : y[q]);
-                }
-            } else *(f32x4 *)(P.C + o) = y;
+                        for(int q = 0; q < 4; q++) (void)__builtin_amdgcn_global_atomic_fadd_f32(t + q, a.gate ? gt * y[q] : y[q]);
+                    }
+                } else *(f32x4 *)(P.C + (size_t)lr * a.N + j0 + col) = y;
+            }
         }
     }
 }
 
-template<int RT, int IO, bool DUAL>
-__global__ void __launch_bounds__(64 * SM_WAVES * (DUAL ? 2 : 1), RT == 1 || DUAL ? 4 : 2) k_gemm_nn_small(SmArgs a){
+template<int RT, int IO, int DUAL>
+__global__ void __launch_bounds__(64 * SM_WAVES * (DUAL == SM_BY_WAVE ? 2 : 1), RT == 1 || DUAL == SM_BY_WAVE ? 4 : 2) k_gemm_nn_small(SmArgs a){
     __shared__ __attribute__((aligned(16))) float red[SM_WAVES * 16 * SM_COLS];
     const int t = qx_xcd_tile(blockIdx.x, gridDim.x);
     if(t >= a.ntiles) return;
     const int pi = qx_find_problem(a.pr, a.nprob, t);
     const DevProb P = a.pr[pi], Q = a.pr[DUAL ? pi + 1 : pi];
     const int lt = t - P.tile0, ti = lt / P.tiles_n, tj = lt - ti * P.tiles_n;
-    const int i0 = ti * (RT * 16), j0 = tj * SM_COLS, left = P.M - i0;
-    if(a.gshift == 6){
-        if(RT == 2 && left > 16) sm_nn_tile<RT, IO, DUAL, true>(a, P, Q, i0, j0, red);
-        else                     sm_nn_tile<1, IO, DUAL, true>(a, P, Q, i0, j0, red);
+    const int i0 = ti * (RT * 16), j0 = tj * (DUAL == SM_BY_LANE ? SM_COLS / 2 : SM_COLS), left = P.M - i0;
+    if(DUAL == SM_BY_LANE || a.gshift == 6){
+        if(RT == 4 && left > 32)      sm_nn_tile<RT, IO, DUAL, true>(a, P, Q, i0, j0, red);
+        else if(RT >= 2 && left > 16) sm_nn_tile<RT >= 2 ? 2 : 1, IO, DUAL, true>(a, P, Q, i0, j0, red);
+        else                          sm_nn_tile<1, IO, DUAL, true>(a, P, Q, i0, j0, red);
     } else {
-        if(RT == 2 && left > 16) sm_nn_tile<RT, IO, DUAL, false>(a, P, Q, i0, j0, red);
-        else                     sm_nn_tile<1, IO, DUAL, false>(a, P, Q, i0, j0, red);
+        if(RT == 4 && left > 32)      sm_nn_tile<RT, IO, DUAL, DUAL == SM_BY_LANE>(a, P, Q, i0, j0, red);
+        else if(RT >= 2 && left > 16) sm_nn_tile<RT >= 2 ? 2 : 1, IO, DUAL, DUAL == SM_BY_LANE>(a, P, Q, i0, j0, red);
+        else                          sm_nn_tile<1, IO, DUAL, DUAL == SM_BY_LANE>(a, P, Q, i0, j0, red);
     }
 }
 
-/* ---- input gradient: 64 columns per wavefront; nseg operand pairs (a continued problem's second pair comes from the
- * table entry behind it). A lane loads ND words of eight k from each of four rows of weights (16 bytes each where the scale
- * group is 128 or more: the 16 lanes of a k group must share a scale group, and the four k groups of a product too). ---- */
-#define SM_TCOLS 64
-template<int RT, int IO, int ND>
-__device__ __forceinline__ void sm_tn_tile(const SmArgs &a, const DevProb &P, const DevProb &Q, int nseg, int i0, int j0, float *red){
-    constexpr int PF = RT == 1 ? 2 : 1, KS = ND * 32;     /* steps on their way; contraction values of a step */
+/* ---- input gradient: 64 columns per workgroup; nseg operand pairs (a continued problem's second pair comes from the
+ * table entry behind it). A wavefront's step is 64 of the contraction: 16 RT rows of activations (128 bytes each) and 64
+ * rows of weights (32 bytes each) go straight into stages of LDS of its own, so there is no barrier in the loop, only the
+ * wavefront's own wait counts. Loaded as operands (lane = row lane%16) instead, sixteen bytes each from sixty-four places,
+ * a load kept the CU's address unit busy for 57 cycles instead of 16, and that unit set the pace. Piece q of row r of a stage
+ * lies at q ^ ((r >> 1) & 7): the sixteen rows of an operand read hit sixteen different units.
+ * LDS accesses are inline assembly: the compiler would wait for every load to LDS in front of them. ---- */
+#define SM_TSTAGE(RT) (2048 * ((RT) + 1) + 256)      /* activations, weights, scales */
+#define SM_TSTAGES(RT) ((RT) == 1 ? 4 : 3)            /* 70, 77, 126 KB: two workgroups per CU, for 64 rows one */
+#define SM_TLDS(RT) (SM_WAVES * SM_TSTAGES(RT) * SM_TSTAGE(RT))
+typedef __attribute__((address_space(3))) void lds_void;
+typedef const __attribute__((address_space(1))) void glb_void;
+template<int OFF> __device__ __forceinline__ i32x4 sm_rd128(uint32_t addr){
+    i32x4 v;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    return v;
+}
+template<int OFF> __device__ __forceinline__ i32x2 sm_rd64(uint32_t addr){
+    i32x2 v;
+    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    return v;
+}
+template<int OFF> __device__ __forceinline__ int sm_rd32(uint32_t addr){
+    int v;
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    return v;
+}
+template<int RT, int IO>
+__device__ __forceinline__ void sm_tn_tile(const SmArgs &a, const DevProb &P, const DevProb &Q, int nseg, int i0, int j0, unsigned char *lds){
+    constexpr int ST = SM_TSTAGES(RT), STAGE = SM_TSTAGE(RT), LOADS = 2 * RT + 3;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
-    /* the wavefronts take the steps in turn: a step reads 16 ND bytes of a weight row, the eight of them 128 ND side by side */
-    const int steps1 = a.K / KS, steps = steps1 * nseg, mine = (steps - wave + SM_TWAVES - 1) / SM_TWAVES;
+    /* the wavefronts take pairs of steps in turn: 128 of the contraction, which share a scale group where it is that long */
+    const int steps1 = a.K / 64, steps = steps1 * nseg, pairs = (steps + 1) / 2, mypairs = (pairs - wave + SM_WAVES - 1) / SM_WAVES;
+    const int mine = 2 * mypairs - ((steps & 1) && mypairs > 0 && (mypairs - 1) * SM_WAVES + wave == pairs - 1 ? 1 : 0);
     const int ngroups = a.K >> a.gshift;
     f32x4 acc[RT][4];
 #pragma unroll
     for(int r = 0; r < RT; r++)
 #pragma unroll
         for(int j = 0; j < 4; j++) acc[r][j] = (f32x4)(0.0f);
-    size_t ra[RT];                                        /* the lane's rows of A, in bytes */
+    /* what this lane loads: piece lane%8 of rows n*8 + lane/8 of the activations, half lane%2 of rows n*32 + lane/2 of the
+     * weights, the scale of column `lane` */
+    size_t ra[2 * RT];
 #pragma unroll
-    for(int r = 0; r < RT; r++) ra[r] = (size_t)min(i0 + r * 16 + c, P.M - 1) * a.K * 2 + g * (ND * 16);
-    int w[PF][4][ND]; float s[PF][4]; i32x4 x[PF][RT][ND];
-    auto load = [&](int set, int st){
-        const int t = wave + SM_TWAVES * min(st, mine - 1);
+    for(int n = 0; n < 2 * RT; n++){
+        const int r = n * 8 + (lane >> 3);
+        ra[n] = (size_t)min(i0 + r, P.M - 1) * a.K * 2 + ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    }
+    const size_t rw = (((size_t)(j0 + (lane >> 1)) * a.K) >> 1) + (lane & 1) * 16, rs = (size_t)(j0 + lane) * ngroups;
+    unsigned char *base = lds + wave * (ST * STAGE);
+    auto load = [&](auto SC, int n){
+        constexpr int S = decltype(SC)::value;
+        const int m = min(n, mine - 1), t = ((m >> 1) * SM_WAVES + wave) * 2 + (m & 1);   /* past the end: the last step again, never used */
         const bool two = t >= steps1;
         const int u = two ? t - steps1 : t;
-        const char *A = (const char *)(two ? Q.A : P.A) + (size_t)u * (KS * 2);
-        const signed char *W = a.d + (((two ? Q.wq : P.wq) + (size_t)(j0 + c) * a.K + (size_t)u * KS) >> 1) + g * (ND * 4);
-        const float *S = a.s + (two ? Q.wg : P.wg) + (size_t)(j0 + c) * ngroups + ((u * KS) >> a.gshift);
+        const char *A = (const char *)(two ? Q.A : P.A) + (size_t)u * 128;
+        const signed char *W = a.d + ((two ? Q.wq : P.wq) >> 1) + (size_t)u * 32 + rw;
 #pragma unroll
-        for(int j = 0; j < 4; j++){
-            if constexpr(ND == 4){ const i32x4 v = *(const i32x4 *)(W + (size_t)(j * 16) * a.K / 2); w[set][j][0] = v[0]; w[set][j][1] = v[1]; w[set][j][2] = v[2]; w[set][j][3] = v[3]; }
-            else                 { const i32x2 v = *(const i32x2 *)(W + (size_t)(j * 16) * a.K / 2); w[set][j][0] = v[0]; w[set][j][1] = v[1]; }
-            s[set][j] = S[(size_t)(j * 16) * ngroups];
-        }
+        for(int k = 0; k < 2 * RT; k++) __builtin_amdgcn_global_load_lds((glb_void *)(A + ra[k]), (lds_void *)(base + S * STAGE + k * 1024), 16, 0, 0);
 #pragma unroll
-        for(int r = 0; r < RT; r++)
-#pragma unroll
-            for(int i = 0; i < ND; i++) x[set][r][i] = *(const i32x4 *)(A + ra[r] + i * 16);
+        for(int k = 0; k < 2; k++) __builtin_amdgcn_global_load_lds((glb_void *)(W + (size_t)(k * 16) * a.K), (lds_void *)(base + S * STAGE + RT * 2048 + k * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((glb_void *)(a.s + (two ? Q.wg : P.wg) + rs + ((u * 64) >> a.gshift)), (lds_void *)(base + S * STAGE + RT * 2048 + 2048), 4, 0, 0);
+        asm volatile("" ::: "memory");                    /* the stages' loads stay in order: the waits count them */
     };
-    auto step = [&](auto IC, int st){
-        constexpr int I = decltype(IC)::value;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_void *)base;
+    uint32_t rdx[2];                                      /* activations of product i, row lane%16 of the first 16 */
+#pragma unroll
+    for(int i = 0; i < 2; i++) rdx[i] = lds_base + c * 128 + (((2 * g + i) ^ (c >> 1)) << 4);
+    const uint32_t rdw = lds_base + c * 32 + g * 8, rds = lds_base + c * 4;
+    auto step = [&](auto SC, int n){
+        constexpr int S = decltype(SC)::value;
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"((ST - 1) * LOADS) : "memory");
+        i32x4 x[RT][2]; i32x2 w[4]; int sc[4];
+        sm_each<0, 4>([&](auto JC){ constexpr int j = decltype(JC)::value; w[j] = sm_rd64<S * STAGE + RT * 2048 + j * 512>(rdw); });
+        sm_each<0, RT>([&](auto RC){
+            constexpr int r = decltype(RC)::value;
+            x[r][0] = sm_rd128<S * STAGE + r * 2048>(rdx[0]); x[r][1] = sm_rd128<S * STAGE + r * 2048>(rdx[1]);
+        });
+        sm_each<0, 4>([&](auto JC){ constexpr int j = decltype(JC)::value; sc[j] = sm_rd32<S * STAGE + RT * 2048 + 2048 + j * 64>(rds); });
+        /* everything is in registers before the stage is loaded again */
+#pragma unroll
+        for(int r = 0; r < RT; r++) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(x[r][0]), "+v"(x[r][1]) :: "memory");
+        asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(sc[0]), "+v"(sc[1]), "+v"(sc[2]), "+v"(sc[3]));
+        load(SC, n + ST);
 #pragma unroll
         for(int j = 0; j < 4; j++){
             f32x4 p[RT];
 #pragma unroll
             for(int r = 0; r < RT; r++) p[r] = (f32x4)(0.0f);
 #pragma unroll
-            for(int i = 0; i < ND; i++){
-                const QxNibs nb = qx_nibs((uint32_t)w[I][j][i]);
+            for(int i = 0; i < 2; i++){
+                const QxNibs nb = qx_nibs((uint32_t)w[j][i]);
                 i32x4 b;
 #pragma unroll
                 for(int q = 0; q < 4; q++) b[q] = sm_pk_bf16(qx_nib16(nb, 2 * q), qx_nib16(nb, 2 * q + 1));
 #pragma unroll
                 for(int r = 0; r < RT; r++)
-                    p[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[I][r][i]), __builtin_bit_cast(bf16x8, b), p[r], 0, 0, 0);
+                    p[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[r][i]), __builtin_bit_cast(bf16x8, b), p[r], 0, 0, 0);
             }
-            const float sc = s[I][j] * 16.0f;
+            const float f = __int_as_float(sc[j]) * 16.0f;
 #pragma unroll
             for(int r = 0; r < RT; r++)
 #pragma unroll
-                for(int e = 0; e < 4; e++) acc[r][j][e] = fmaf(sc, p[r][e], acc[r][j][e]);
+                for(int e = 0; e < 4; e++) acc[r][j][e] = fmaf(f, p[r][e], acc[r][j][e]);
         }
-        load(I, st + PF);
     };
     if(mine > 0){
-        sm_each<0, PF>([&](auto IC){ load(decltype(IC)::value, decltype(IC)::value); });
-        int st = 0;
-        for(; st + PF <= mine; st += PF) sm_each<0, PF>([&](auto IC){ step(IC, st + decltype(IC)::value); });
-        sm_each<0, PF - 1>([&](auto IC){ if(st + decltype(IC)::value < mine) step(IC, st + decltype(IC)::value); });
+        sm_each<0, ST>([&](auto IC){ load(IC, decltype(IC)::value); });
+        int n = 0;
+        for(; n + ST <= mine; n += ST) sm_each<0, ST>([&](auto IC){ step(IC, n + decltype(IC)::value); });
+        sm_each<0, ST - 1>([&](auto IC){ if(n + decltype(IC)::value < mine) step(IC, n + decltype(IC)::value); });
     }
-    /* ---- totals: the thread holds row tid/32, two columns ---- */
-    const int row = tid >> 5, col = (tid & 31) * 2;
+    __builtin_amdgcn_s_waitcnt(0x0F70);                   /* vmcnt(0): no load may land in a stage any more */
+    /* ---- totals: [row tile][wavefront][16 rows][64 columns]; the thread holds row tid/16, four columns ---- */
+    float *red = (float *)lds;
+    __syncthreads();
 #pragma unroll
-    for(int r = 0; r < RT; r++){
-        __syncthreads();                                  /* the tile before has been read */
+    for(int r = 0; r < RT; r++)
 #pragma unroll
         for(int e = 0; e < 4; e++)
 #pragma unroll
-            for(int j = 0; j < 4; j++) red[(wave * 16 + g * 4 + e) * SM_TCOLS + j * 16 + c] = acc[r][j][e];
-        __syncthreads();
-        f32x2 y = *(const f32x2 *)&red[tid * 2];
+            for(int j = 0; j < 4; j++) red[((r * SM_WAVES + wave) * 16 + g * 4 + e) * SM_TCOLS + j * 16 + c] = acc[r][j][e];
+    __syncthreads();
+    const int row = tid >> 4, col = (tid & 15) * 4;
 #pragma unroll
-        for(int k = 1; k < SM_TWAVES; k++) y += *(const f32x2 *)&red[k * (16 * SM_TCOLS) + tid * 2];
+    for(int r = 0; r < RT; r++){
         const int lr = i0 + r * 16 + row;
         if(lr >= P.M) continue;
+        f32x4 y = *(const f32x4 *)&red[(r * SM_WAVES * 16 + row) * SM_TCOLS + col];
+#pragma unroll
+        for(int k = 1; k < SM_WAVES; k++) y += *(const f32x4 *)&red[((r * SM_WAVES + k) * 16 + row) * SM_TCOLS + col];
         if constexpr(IO == SM_SCATTER){
             const int tok = ((const int *)P.C)[lr];
             if(tok >= 0){
                 qx_gfloat *t = (qx_gfloat *)(a.out + (size_t)tok * a.N + j0 + col);
-                (void)__builtin_amdgcn_global_atomic_fadd_f32(t, y[0]);
-                (void)__builtin_amdgcn_global_atomic_fadd_f32(t + 1, y[1]);
+#pragma unroll
+                for(int q = 0; q < 4; q++) (void)__builtin_amdgcn_global_atomic_fadd_f32(t + q, y[q]);
             }
         } else if constexpr(IO == SM_SWIGLU_BWD){
             const size_t o = (size_t)(P.C - a.gp) + (size_t)lr * a.N + j0 + col;      /* even: pairs of bf16 are 4-byte aligned */
-            float dg[2], du[2];
+            float dg[4], du[4];
 #pragma unroll
-            for(int q = 0; q < 2; q++) qx_swiglu_bwd1<true>(a.gp[o + q], a.up[o + q], y[q], dg[q], du[q]);
-            *(uint32_t *)(a.dg + o) = (uint32_t)qx_f32_to_bf16(dg[0]) | ((uint32_t)qx_f32_to_bf16(dg[1]) << 16);
-            *(uint32_t *)(a.du + o) = (uint32_t)qx_f32_to_bf16(du[0]) | ((uint32_t)qx_f32_to_bf16(du[1]) << 16);
+            for(int q = 0; q < 4; q++) qx_swiglu_bwd1<true>(a.gp[o + q], a.up[o + q], y[q], dg[q], du[q]);
+#pragma unroll
+            for(int q = 0; q < 4; q += 2){
+                *(uint32_t *)(a.dg + o + q) = (uint32_t)qx_f32_to_bf16(dg[q]) | ((uint32_t)qx_f32_to_bf16(dg[q + 1]) << 16);
+                *(uint32_t *)(a.du + o + q) = (uint32_t)qx_f32_to_bf16(du[q]) | ((uint32_t)qx_f32_to_bf16(du[q + 1]) << 16);
+            }
         } else {
-            f32x2 *o = (f32x2 *)(P.C + (size_t)lr * a.N + j0 + col);
+            f32x4 *o = (f32x4 *)(P.C + (size_t)lr * a.N + j0 + col);
             if(P.beta != 0.0f) y = *o + y;
             *o = y;
         }
@@ -332,8 +404,8 @@ __device__ __forceinline__ void sm_tn_tile(const SmArgs &a, const DevProb &P, co
 }
 
 template<int RT, int IO>
-__global__ void __launch_bounds__(64 * SM_TWAVES, 4) k_gemm_tn_small(SmArgs a){
-    __shared__ __attribute__((aligned(16))) float red[SM_TWAVES * 16 * SM_TCOLS];
+__global__ void __launch_bounds__(64 * SM_WAVES, 2) k_gemm_tn_small(SmArgs a){
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int t = qx_xcd_tile(blockIdx.x, gridDim.x);
     if(t >= a.ntiles) return;
     const int pi = qx_find_problem(a.pr, a.nprob, t);
@@ -341,19 +413,16 @@ __global__ void __launch_bounds__(64 * SM_TWAVES, 4) k_gemm_tn_small(SmArgs a){
     const DevProb Q = a.pr[P.chunk ? pi + 1 : pi];
     const int lt = t - P.tile0, ti = lt / P.tiles_n, tj = lt - ti * P.tiles_n;
     const int i0 = ti * (RT * 16), j0 = tj * SM_TCOLS, left = P.M - i0, nseg = P.chunk ? 2 : 1;
-    if(a.gshift >= 7 && a.K % 128 == 0){
-        if(RT == 2 && left > 16) sm_tn_tile<RT, IO, 4>(a, P, Q, nseg, i0, j0, red);
-        else                     sm_tn_tile<1, IO, 4>(a, P, Q, nseg, i0, j0, red);
-    } else {
-        if(RT == 2 && left > 16) sm_tn_tile<RT, IO, 2>(a, P, Q, nseg, i0, j0, red);
-        else                     sm_tn_tile<1, IO, 2>(a, P, Q, nseg, i0, j0, red);
-    }
+    if(RT == 4 && left > 32)      sm_tn_tile<RT, IO>(a, P, Q, nseg, i0, j0, lds);
+    else if(RT >= 2 && left > 16) sm_tn_tile<RT >= 2 ? 2 : 1, IO>(a, P, Q, nseg, i0, j0, lds);
+    else                          sm_tn_tile<1, IO>(a, P, Q, nseg, i0, j0, lds);
 }
 
 /* ---- launches ---- */
 static int sm_row_tiles(const qlmx_gemm_prob *probs, int nprob){
-    for(int i = 0; i < nprob; i++) if(probs[i].M > 16) return 2;
-    return 1;
+    int most = 0;
+    for(int i = 0; i < nprob; i++) if(probs[i].M > most) most = probs[i].M;
+    return most > 32 ? 4 : most > 16 ? 2 : 1;
 }
 static SmArgs sm_args(const signed char *d, const float *s, int group, int K, int N, const ProbUpload &up){
     SmArgs a = {};
@@ -361,7 +430,7 @@ static SmArgs sm_args(const signed char *d, const float *s, int group, int K, in
     while((1 << a.gshift) < group) a.gshift++;
     return a;
 }
-#define SM_LAUNCH(KERNEL, WAVES) hipLaunchKernelGGL(KERNEL, dim3((a.ntiles + 7) & ~7), dim3(64 * (WAVES)), 0, st, a)
+#define SM_LAUNCH(KERNEL, WAVES, LDS) hipLaunchKernelGGL(KERNEL, dim3((a.ntiles + 7) & ~7), dim3(64 * (WAVES)), LDS, st, a)
 
 /* N % 128 == 0, K % 32 == 0, group a power of two >= 64; io, xsrc, out, gate as in qlmx_gemm_nn_h_launch */
 int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N,
@@ -372,7 +441,8 @@ int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, c
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
     a.xsrc = (const char *)xsrc; a.out = out; a.gate = gate;
-#define SM_NN(IO) do{ if(rt == 1) SM_LAUNCH((k_gemm_nn_small<1, IO, false>), SM_WAVES); else SM_LAUNCH((k_gemm_nn_small<2, IO, false>), SM_WAVES); }while(0)
+#define SM_NN(IO) do{ if(rt == 1) SM_LAUNCH((k_gemm_nn_small<1, IO, SM_ONE>), SM_WAVES, 0); else if(rt == 2) SM_LAUNCH((k_gemm_nn_small<2, IO, SM_ONE>), SM_WAVES, 0); \
+                      else SM_LAUNCH((k_gemm_nn_small<4, IO, SM_ONE>), SM_WAVES, 0); }while(0)
     if(io == SM_GATHER) SM_NN(SM_GATHER); else if(io == SM_SCATTER) SM_NN(SM_SCATTER); else SM_NN(SM_PLAIN);
 #undef SM_NN
     QLMX_LAUNCH_CHECK("grouped gemm nn (few rows) launch");
@@ -383,11 +453,12 @@ int qlmx_gemm_nn_small_swiglu_launch(const signed char *d, const float *s, int g
                                      int K, int N, const void *xsrc, hipStream_t st){
     const int rt = sm_row_tiles(gate, nprob);
     ProbUpload up; int slot;
-    int rc = qlmx_upload_problem_pairs(gate, up_, nprob, GEMM_NN, K, N, rt * 16, SM_COLS, st, &up, &slot); if(rc) return rc;
+    int rc = qlmx_upload_problem_pairs(gate, up_, nprob, GEMM_NN, K, N, rt * 16, rt == 4 ? SM_COLS / 2 : SM_COLS, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
     a.xsrc = (const char *)xsrc;
-#define SM_DUAL(IO) do{ if(rt == 1) SM_LAUNCH((k_gemm_nn_small<1, IO, true>), 2 * SM_WAVES); else SM_LAUNCH((k_gemm_nn_small<2, IO, true>), 2 * SM_WAVES); }while(0)
+#define SM_DUAL(IO) do{ if(rt == 1) SM_LAUNCH((k_gemm_nn_small<1, IO, SM_BY_WAVE>), 2 * SM_WAVES, 0); else if(rt == 2) SM_LAUNCH((k_gemm_nn_small<2, IO, SM_BY_WAVE>), 2 * SM_WAVES, 0); \
+                        else SM_LAUNCH((k_gemm_nn_small<4, IO, SM_BY_LANE>), SM_WAVES, 0); }while(0)
     if(xsrc) SM_DUAL(SM_GATHER); else SM_DUAL(SM_PLAIN);
 #undef SM_DUAL
     QLMX_LAUNCH_CHECK("grouped gemm nn + swiglu (few rows) launch");
@@ -404,9 +475,14 @@ int qlmx_gemm_tn_small_launch(const signed char *d, const float *s, int group, c
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
     a.out = out; a.gp = gp; a.up = up_; a.dg = (unsigned short *)dg; a.du = (unsigned short *)du;
-#define SM_TN(IO) do{ if(rt == 1) SM_LAUNCH((k_gemm_tn_small<1, IO>), SM_TWAVES); else SM_LAUNCH((k_gemm_tn_small<2, IO>), SM_TWAVES); }while(0)
+#define SM_TN1(RT, IO) do{ \
+        static bool attr_set = false; \
+        if(!attr_set){ QLMX_HIP(hipFuncSetAttribute((const void *)k_gemm_tn_small<RT, IO>, hipFuncAttributeMaxDynamicSharedMemorySize, SM_TLDS(RT)), "tn (few rows) LDS size"); attr_set = true; } \
+        SM_LAUNCH((k_gemm_tn_small<RT, IO>), SM_WAVES, SM_TLDS(RT)); }while(0)
+#define SM_TN(IO) do{ if(rt == 1) SM_TN1(1, IO); else if(rt == 2) SM_TN1(2, IO); else SM_TN1(4, IO); }while(0)
     if(out) SM_TN(SM_SCATTER); else if(gp) SM_TN(SM_SWIGLU_BWD); else SM_TN(SM_PLAIN);
 #undef SM_TN
+#undef SM_TN1
     QLMX_LAUNCH_CHECK("grouped gemm tn (few rows) launch");
     return qlmx_upload_done(slot, st);
 }

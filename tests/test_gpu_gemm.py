@@ -221,6 +221,24 @@ def test_mfma_few_rows(q, orc, mode, K, N, group, rows):
         assert orc.relerr(got, want) < (4e-4 if mode == "nn" else 3e-6)
 
 
+@pytest.mark.parametrize("K,N,group", [(768, 256, 128), (128, 128, 64), (2048, 256, 256)])
+@pytest.mark.parametrize("rows", [[65, 1, 130, 34], [257]])
+def test_mfma_few_tiles(q, orc, K, N, group, rows):
+    """Calls with too few tiles for the tiled kernels take the kernels for few rows with 64-row tiles: last tiles of every
+    height behind whole ones, alone, paired and with the SwiGLU behind."""
+    for mode, tol in (("nn", 4e-4), ("tn", 3e-6)):
+        got, want = run_case(q, orc, mode, len(rows), rows, K, N, pkg.ACT_BF16, pkg.MATH_MFMA_F16 if mode == "nn" else pkg.MATH_MFMA, seed=23,
+                             beta=1.0 if mode == "tn" else 0.0, group=group)
+        assert orc.relerr(got, want) < tol
+    if group == 128:
+        got, want = _pair_case(q, orc, rows, K, N, pkg.ACT_BF16, pkg.MATH_MFMA, 1.0, seed=24)
+        assert orc.relerr(got, want) < 3e-6
+        (f, sep), want = _swiglu_case(q, orc, rows, K, N, pkg.ACT_BF16, pkg.MATH_MFMA_F16, seed=25)
+        assert orc.relerr(f[0], want) < 4e-4
+        for a, b in zip(f[:2], sep[:2]):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 @pytest.mark.parametrize("mode,K,N", [("nn", 768, 2048), ("nn", 2048, 768), ("tn", 768, 2048), ("tn", 2048, 768),
                                       ("nt", 768, 2048), ("nt", 2048, 768)])
 def test_mfma_layer_shapes(q, orc, mode, K, N):
