@@ -809,64 +809,77 @@ extern "C" int qlmx_step_touched(float *P, const float *Gc, signed char *d, sign
  * k_sqsum: 64 partial sums of squares; partial c covers G[n*c/64 .. n*(c+1)/64), is accumulated in
  * double and rounded to float once (the CPU path's definition; the reference's GPU kernel sums
  * strided in fp32 and differs from its own CPU kernel in the last bits). The 64 partials are the
- * contract, 64 workgroups are not: each chunk is shared by SQ_W workgroups (1024
- * for the 256 CUs), which sum in double -- threads strided, then a fixed tree -- and leave
- * their sum in a device array; the workgroup that arrives last at a chunk (a counter) adds the SQ_W
+ * contract, 64 workgroups are not: each chunk is shared by `pieces` workgroups, one stretch of it each (16, or fewer
+ * where a stretch would hold less than a load per thread and loop), which sum in double -- threads strided, then a fixed
+ * tree -- and leave their sum in a device array; the workgroup that arrives last at a chunk (a counter) adds the
  * sums in piece order, so the result does not depend on arrival order. The order of the double
  * additions is not the CPU's, which can move the double sum by a few units in its last place -- far
  * below half a float ulp except on an exact tie. The array and the counters are static device
  * memory (the last workgroup resets its counter): calls that overlap on different streams would
- * mix their pieces and are not supported. */
+ * mix their pieces and are not supported.
+ *
+ * The hand-over is device-scope accesses, which go past the caches, and a wait for the store in front of the count. As an
+ * acquire-release count it wrote back and invalidated an XCD's L2 once per workgroup, which cost more than the reading:
+ * 127 us for 125.8 M values, 18 for any small number. A stretch of its own per workgroup keeps what it reads in few DRAM
+ * pages: 6.1 TB/s at any grid of 1024 workgroups or more, side by side 4.9 to 5.8. */
 #define SQ_W 16
 static __device__ double   g_sq_piece[64 * SQ_W];
 static __device__ unsigned g_sq_count[64];
-__global__ void __launch_bounds__(256) k_qlmx_sqsum(const float *G, unsigned long long n, float *part){
-    __shared__ double red[256];
-    const unsigned c = blockIdx.x / SQ_W, w = blockIdx.x % SQ_W;
-    const unsigned long long i0 = n * c / 64, i1 = n * (c + 1) / 64, t0 = w * 256 + threadIdx.x, stride = SQ_W * 256;
+__global__ void __launch_bounds__(256) k_qlmx_sqsum(const float *G, unsigned long long n, float *part, int pieces){
+    __shared__ double red[128];
+    const unsigned c = blockIdx.x / pieces, w = blockIdx.x - c * pieces, tid = threadIdx.x;
+    const unsigned long long c0 = n * c / 64, cn = n * (c + 1) / 64 - c0;
+    const unsigned long long i0 = c0 + cn * w / pieces, i1 = c0 + cn * (w + 1) / pieces;
     double s = 0.0;
     /* 16-byte loads over the aligned middle, single elements at both ends */
     unsigned long long a0 = (i0 + 3) & ~3ULL; if(a0 > i1) a0 = i1;
     const unsigned long long a1 = a0 + ((i1 - a0) & ~3ULL);
-    for(unsigned long long i = i0 + t0; i < a0; i += stride){ const double g = (double)G[i]; s += g * g; }
+    for(unsigned long long i = i0 + tid; i < a0; i += 256){ const double g = (double)G[i]; s += g * g; }
     if((((uintptr_t)G) & 15) == 0){
-        /* The chunk's workgroups side by side, four loads of a thread on their way and four sums: with a stretch of its
-         * own per workgroup, one load and one chain of additions HBM delivered 3.2 TB/s (125.8 M values: 157 us, now
-         * 127, the 4 TB/s that reading alone reaches; twice and four times the workgroups: 178 and 281). A square of
-         * a float is exact in double, so the fma adds what the product and the sum would. */
+        /* four loads of a thread on their way and four sums; a square of a float is exact in double, so the fma adds
+         * what the product and the sum would */
         double u[4] = {0.0, 0.0, 0.0, 0.0};
         auto add = [](double &t, const float4 &v){
             t = fma((double)v.x, (double)v.x, t); t = fma((double)v.y, (double)v.y, t); t = fma((double)v.z, (double)v.z, t); t = fma((double)v.w, (double)v.w, t);
         };
-        unsigned long long i = a0 + 4 * t0;
-        for(; i + 12 * stride < a1; i += 16 * stride){
+        unsigned long long i = a0 + 4 * tid;
+        for(; i + 3072 < a1; i += 4096){
             float4 v[4];
 #pragma unroll
-            for(int q = 0; q < 4; q++) v[q] = *(const float4 *)(G + i + q * (4 * stride));
+            for(int q = 0; q < 4; q++) v[q] = *(const float4 *)(G + i + q * 1024);
 #pragma unroll
             for(int q = 0; q < 4; q++) add(u[q], v[q]);
         }
-        for(; i < a1; i += 4 * stride) add(u[0], *(const float4 *)(G + i));
+        for(; i < a1; i += 1024) add(u[0], *(const float4 *)(G + i));
         s += (u[0] + u[1]) + (u[2] + u[3]);
     } else {
-        for(unsigned long long i = a0 + t0; i < a1; i += stride){ const double g = (double)G[i]; s += g * g; }
+        for(unsigned long long i = a0 + tid; i < a1; i += 256){ const double g = (double)G[i]; s += g * g; }
     }
-    for(unsigned long long i = a1 + t0; i < i1; i += stride){ const double g = (double)G[i]; s += g * g; }
-    red[threadIdx.x] = s;
+    for(unsigned long long i = a1 + tid; i < i1; i += 256){ const double g = (double)G[i]; s += g * g; }
+    if(tid >= 128) red[tid - 128] = s;
     __syncthreads();
-    for(int o = 128; o > 0; o >>= 1){
-        if((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
+    if(tid < 128) s += red[tid];
+    __syncthreads();
+    if(tid >= 64 && tid < 128) red[tid - 64] = s;
+    __syncthreads();
+    if(tid >= 64) return;
+    s += red[tid];
+    for(int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+    if(pieces == 1){ if(tid == 0) part[c] = (float)s; return; }
+    unsigned before = 0;
+    if(tid == 0){
+        __hip_atomic_store(&g_sq_piece[c * SQ_W + w], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        before = __hip_atomic_fetch_add(&g_sq_count[c], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if(threadIdx.x == 0){
-        __hip_atomic_store(&g_sq_piece[c * SQ_W + w], red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned before = __hip_atomic_fetch_add(&g_sq_count[c], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if(before == SQ_W - 1){
-            double t = 0.0;
-            for(int k = 0; k < SQ_W; k++) t += __hip_atomic_load(&g_sq_piece[c * SQ_W + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            part[c] = (float)t;
-            __hip_atomic_store(&g_sq_count[c], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+    if(__builtin_amdgcn_readfirstlane(before) != (unsigned)pieces - 1) return;
+    asm volatile("" ::: "memory");
+    const double p = (int)tid < pieces ? __hip_atomic_load(&g_sq_piece[c * SQ_W + tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+    double t = 0.0;
+    for(int k = 0; k < pieces; k++) t += __shfl(p, k, 64);
+    if(tid == 0){
+        part[c] = (float)t;
+        __hip_atomic_store(&g_sq_count[c], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -894,7 +907,10 @@ __global__ void __launch_bounds__(64) k_qlmx_gnorm(const float *part, int nside,
 extern "C" int qlmx_sqsum(const float *G, unsigned long long n, float *part64, void *stream){
     int rc = qlmx_check_ready(); if(rc) return rc;
     QLMX_REQUIRE(G && part64, "qlmx_sqsum: NULL buffer");
-    hipLaunchKernelGGL(k_qlmx_sqsum, dim3(64 * SQ_W), dim3(256), 0, (hipStream_t)stream, G, n, part64);
+    /* a stretch holds at least the 4096 values of one round of its workgroup */
+    const unsigned long long most = n / (64 * 4096);
+    const int pieces = most < 1 ? 1 : most > SQ_W ? SQ_W : (int)most;
+    hipLaunchKernelGGL(k_qlmx_sqsum, dim3(64 * pieces), dim3(256), 0, (hipStream_t)stream, G, n, part64, pieces);
     QLMX_LAUNCH_CHECK("qlmx_sqsum launch");
     return QLMX_OK;
 }

@@ -395,6 +395,17 @@ def test_step_eight_groups_per_wavefront_equals_one_per_row(q, orc, v4, render):
         assert np.array_equal(results[0][i].view(np.uint8), np.asarray(want[i]).view(np.uint8)), nm
 
 
+@pytest.mark.parametrize("n", [1, 63, 64 * 4096 + 5, 64 * 4096 * 3 + 2, 64 * 4096 * 17 + 1])
+def test_sqsum_pieces(q, orc, n):
+    """One, three and sixteen workgroups per partial sum, chunk ends that are not aligned, twice in a row (the counters)."""
+    hG = orc.normal(n, 18, 1, 1e-3)
+    want = np.array([np.float32((hG[n * c // 64:n * (c + 1) // 64].astype(np.float64) ** 2).sum()) for c in range(64)], f32)
+    G, part = dev(hG), dev(np.zeros(64, f32))
+    for _ in range(2):
+        q.sqsum(G, n, part)
+        assert np.allclose(host(part), want, rtol=1e-7, atol=0.0)
+
+
 def test_argument_errors(q):
     import torch
     x = torch.zeros(256, device="cuda")
