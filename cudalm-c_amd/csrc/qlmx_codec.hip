@@ -5,17 +5,17 @@
  * qi0+i; packed digits sit two per byte, even element in the low nibble, two's complement; one
  * fp32 scale per group of `group` consecutive elements of a span, the last group may be short.
  *
- * As in the optimizer kernel a group belongs to one DPP row of 16 lanes. With group 128, full and
- * 8-element aligned, each lane handles 8 consecutive elements through 128/64/32-bit accesses;
- * everything else goes pair-per-lane so that a lane always owns whole bytes of packed digits.
+ * As in the optimizer kernel a group belongs to a team of W lanes: a DPP row of 16, or half of one for groups
+ * of 64. With groups of 8 W, full and 8-element aligned, each lane handles 8 consecutive elements through
+ * 128/64/32-bit accesses; everything else goes pair-per-lane so that a lane always owns whole bytes of packed digits
+ * (which took 535 us for encode + servo + render of 64 M weights in groups of 64, against 152 in groups of 128).
  * All three are streaming kernels bound by HBM (encode: read 4 B, write 1.5 B per weight; render:
  * read 0.5 B, write 4 B; servo: read 1.5 B, write at most 1.5 B).
  */
 #include "qlmx_dev.h"
 
 struct GroupLoc { int n; uint64_t pof, qi0; };
-__device__ __forceinline__ GroupLoc group_loc(const qlmx_span *sp, int nspan, int gi, int group){
-    const int si = qx_span_of(sp, nspan, gi);
+__device__ __forceinline__ GroupLoc group_loc(const qlmx_span *sp, int si, int gi, int group){
     const qlmx_span S = sp[si];
     const uint64_t j0 = (uint64_t)(gi - S.gi0) * (uint64_t)group;
     const uint64_t left = S.n - j0;
@@ -36,28 +36,31 @@ __device__ __forceinline__ void quantize(float t, int dmax, int &dd, int &rr){
     rr = qx_clamp((int)rintf((t - (float)dd) * 128.0f), -64, 64);
 }
 
+template<int W>
 __global__ void __launch_bounds__(256) k_qlmx_encode(const float *P, signed char *d, signed char *r, float *s,
                                                      const qlmx_span *sp, int nspan, int group, int dmax,
                                                      int packed, int ngrp, int vec_ok){
-    const int lane16 = threadIdx.x & 15;
-    const int gi = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) >> 4);
+    const int tl = threadIdx.x & (W - 1);
+    const int gi = (int)((blockIdx.x * 256u + threadIdx.x) / W);
+    const int si = qx_span_of_teams<64 / W>(sp, nspan, __builtin_amdgcn_readfirstlane(gi), (threadIdx.x & 63) / W);
     if(gi >= ngrp) return;
-    const GroupLoc L = group_loc(sp, nspan, gi, group);
-    const bool fast = vec_ok && group == 128 && packed && L.n == 128 && ((L.pof | L.qi0) & 7ULL) == 0;
+    const GroupLoc L = group_loc(sp, si, gi, group);
+    const bool fast = vec_ok && group == 8 * W && packed && L.n == 8 * W && ((L.pof | L.qi0) & 7ULL) == 0;
     if(fast){
-        const uint64_t e0 = (uint64_t)lane16 * 8;
+        const uint64_t e0 = (uint64_t)tl * 8;
         const float4 p0 = *(const float4 *)(P + L.pof + e0), p1 = *(const float4 *)(P + L.pof + e0 + 4);
         const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
         float amax = 0.0f;
 #pragma unroll
         for(int k = 0; k < 8; k++) amax = fmaxf(amax, fabsf(pv[k]));
-        amax = qx_row16_max(amax);
+        amax = qx_team_max<W>(amax);
         float sg = amax / (float)dmax; if(!(sg > 0.0f)) sg = 1e-8f;
-        if(lane16 == 0) s[gi] = sg;
+        if(tl == 0) s[gi] = sg;
+        const GroupDiv div = qx_mkdiv(sg);                 /* 151 M weights, encode + servo + render: 333 -> 322 us */
         uint32_t dw = 0, r0 = 0, r1 = 0;
 #pragma unroll
         for(int k = 0; k < 8; k++){
-            int dd, rr; quantize(pv[k] / sg, dmax, dd, rr);
+            int dd, rr; quantize(qx_gdiv(pv[k], div), dmax, dd, rr);
             dw |= ((uint32_t)dd & 15u) << (4 * k);
             if(k < 4) r0 |= ((uint32_t)rr & 0xFFu) << (8 * k); else r1 |= ((uint32_t)rr & 0xFFu) << (8 * (k - 4));
         }
@@ -65,11 +68,11 @@ __global__ void __launch_bounds__(256) k_qlmx_encode(const float *P, signed char
         *(uint2 *)(r + L.qi0 + e0) = make_uint2(r0, r1);
     } else {
         float amax = 0.0f;
-        for(int j = lane16; j < L.n; j += 16) amax = fmaxf(amax, fabsf(P[L.pof + j]));
-        amax = qx_row16_max(amax);
+        for(int j = tl; j < L.n; j += W) amax = fmaxf(amax, fabsf(P[L.pof + j]));
+        amax = qx_team_max<W>(amax);
         float sg = amax / (float)dmax; if(!(sg > 0.0f)) sg = 1e-8f;
-        if(lane16 == 0) s[gi] = sg;
-        for(int jb = 2 * lane16; jb < L.n; jb += 32){
+        if(tl == 0) s[gi] = sg;
+        for(int jb = 2 * tl; jb < L.n; jb += 2 * W){
             int dn[2] = {0, 0};
 #pragma unroll
             for(int h = 0; h < 2; h++){
@@ -85,32 +88,33 @@ __global__ void __launch_bounds__(256) k_qlmx_encode(const float *P, signed char
     }
 }
 
+template<int W>
 __global__ void __launch_bounds__(256) k_qlmx_render(float *P, const signed char *d, const float *s,
                                                      const qlmx_span *sp, int nspan, int group, int packed,
                                                      int gi_base, int ng, int vec_ok){
-    const int lane16 = threadIdx.x & 15;
-    const int w = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) >> 4);
+    const int tl = threadIdx.x & (W - 1);
+    const int w = (int)((blockIdx.x * 256u + threadIdx.x) / W), gi = gi_base + w;
+    const int si = qx_span_of_teams<64 / W>(sp, nspan, __builtin_amdgcn_readfirstlane(gi), (threadIdx.x & 63) / W);
     if(w >= ng) return;
-    const int gi = gi_base + w;
-    const GroupLoc L = group_loc(sp, nspan, gi, group);
+    const GroupLoc L = group_loc(sp, si, gi, group);
     const float sg = s[gi];
-    const bool fast = vec_ok && group == 128 && packed && L.n == 128 && ((L.pof | L.qi0) & 7ULL) == 0;
+    const bool fast = vec_ok && group == 8 * W && packed && L.n == 8 * W && ((L.pof | L.qi0) & 7ULL) == 0;
     if(fast){
-        /* a lane renders elements 4*lane16 .. +3 and the same 64 further on: each of the two stores of
-         * a 16-lane row covers 256 contiguous bytes of P, written past the caches */
+        /* a lane renders elements 4*tl .. +3 and the same half a group further on: each of the two stores of
+         * a team covers 16 W contiguous bytes of P, written past the caches */
         typedef float f4 __attribute__((ext_vector_type(4)));
-        const uint64_t e0 = (uint64_t)lane16 * 4;
+        const uint64_t e0 = (uint64_t)tl * 4;
         const unsigned short *dh = (const unsigned short *)(d + (L.qi0 >> 1));
-        const uint32_t w0 = dh[lane16], w1 = dh[16 + lane16];
+        const uint32_t w0 = dh[tl], w1 = dh[W + tl];
         f4 o0, o1;
         o0.x = sg * (float)qx_nib(w0, 0); o0.y = sg * (float)qx_nib(w0, 1);
         o0.z = sg * (float)qx_nib(w0, 2); o0.w = sg * (float)qx_nib(w0, 3);
         o1.x = sg * (float)qx_nib(w1, 0); o1.y = sg * (float)qx_nib(w1, 1);
         o1.z = sg * (float)qx_nib(w1, 2); o1.w = sg * (float)qx_nib(w1, 3);
         __builtin_nontemporal_store(o0, (f4 *)(P + L.pof + e0));
-        __builtin_nontemporal_store(o1, (f4 *)(P + L.pof + e0 + 64));
+        __builtin_nontemporal_store(o1, (f4 *)(P + L.pof + e0 + 4 * W));
     } else {
-        for(int j = lane16; j < L.n; j += 16) P[L.pof + j] = sg * (float)load_digit(d, L.qi0 + j, packed);
+        for(int j = tl; j < L.n; j += W) P[L.pof + j] = sg * (float)load_digit(d, L.qi0 + j, packed);
     }
 }
 
@@ -120,19 +124,20 @@ __device__ __forceinline__ float servo_scale(float sg, int railed, int n, float 
     return f > f_hi ? sg * 1.09051f : f < f_lo ? sg / 1.09051f : sg;          /* 2^(1/8) */
 }
 /* any group: a pair of elements per lane and step */
-__device__ void servo_pairs(const GroupLoc &L, int gi, int lane16, signed char *d, signed char *r, float *s, int dmax, float f_hi, float f_lo, int packed){
+template<int W>
+__device__ void servo_pairs(const GroupLoc &L, int gi, int tl, signed char *d, signed char *r, float *s, int dmax, float f_hi, float f_lo, int packed){
     int railed = 0;
-    for(int jb = 2 * lane16; jb < L.n; jb += 32)
+    for(int jb = 2 * tl; jb < L.n; jb += 2 * W)
         for(int h = 0; h < 2; h++){
             const int j = jb + h;
             if(j < L.n){ const int dd = load_digit(d, L.qi0 + j, packed); railed += (dd == dmax) | (dd == -dmax); }
         }
-    railed = qx_row16_sum(railed);
+    railed = qx_team_sum<W>(railed);
     const float f = (float)railed / (float)L.n, sg = s[gi];
-    if(!(f > f_hi || f < f_lo)) return;             /* uniform over the row */
+    if(!(f > f_hi || f < f_lo)) return;             /* uniform over the team */
     const float sn = servo_scale(sg, railed, L.n, f_hi, f_lo), conv = sg / sn;
-    if(lane16 == 0) s[gi] = sn;
-    for(int jb = 2 * lane16; jb < L.n; jb += 32){
+    if(tl == 0) s[gi] = sn;
+    for(int jb = 2 * tl; jb < L.n; jb += 2 * W){
         int dn[2] = {0, 0};
 #pragma unroll
         for(int h = 0; h < 2; h++){
@@ -154,55 +159,57 @@ __device__ __forceinline__ int nibbles_equal(uint32_t w, uint32_t of){
     x |= x >> 2; x |= x >> 1;
     return 8 - __popc(x & 0x11111111u);
 }
-/* Full aligned groups of 128 go 8 consecutive elements per lane: one 32-bit word of digits, and 8 residual bytes only
- * where the group is rescaled. What bounds the kernel is vector instructions, not HBM. A workgroup counts 64 groups, a
- * row of 16 lanes SV_G of them with their loads side by side, and lists the few that move; its rows then share the list,
+/* Full aligned groups of 8 W go 8 consecutive elements per lane: one 32-bit word of digits, and 8 residual bytes only
+ * where the group is rescaled. What bounds the kernel is vector instructions, not HBM. A workgroup counts G groups per
+ * team, their loads side by side, and lists the few that move; its teams then share the list,
  * so that re-encoding (160 instructions) runs for wavefronts full of moving groups instead of for every wavefront with
  * one among its four. 151 M weights, 15 % of the groups moving: 119 us with one group per row from start to end, 77
- * now. */
-#define SV_G 4
+ * with four. Few groups leave most CUs empty at four per team, and there only the chain counts: one per team. */
+template<int W, int G>
 __global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char *r, float *s,
                                                     const qlmx_span *sp, int nspan, int group, int dmax,
                                                     float f_hi, float f_lo, int packed, int ngrp, int vec_ok){
-    __shared__ uint64_t at[16 * SV_G];                     /* the moving groups: first element, old scale / new scale */
-    __shared__ float conv[16 * SV_G];
+    constexpr int TEAMS = 256 / W;
+    __shared__ uint64_t at[TEAMS * G];                     /* the moving groups: first element, old scale / new scale */
+    __shared__ float conv[TEAMS * G];
     __shared__ int moving;
-    const int lane16 = threadIdx.x & 15, row = threadIdx.x >> 4, first = (int)blockIdx.x * (16 * SV_G) + row;
+    const int tl = threadIdx.x & (W - 1), team = threadIdx.x / W, first = (int)blockIdx.x * (TEAMS * G) + team;
     if(threadIdx.x == 0) moving = 0;
+    const int s0 = qx_span_of_teams<64 / W>(sp, nspan, __builtin_amdgcn_readfirstlane(first), (threadIdx.x & 63) / W);
     __syncthreads();
-    bool fast[SV_G];
+    bool fast[G];
     if(first < ngrp){
-        qlmx_span S = sp[qx_span_of(sp, nspan, first)];
-        uint64_t q0[SV_G]; uint32_t dw[SV_G]; float sg[SV_G];
+        qlmx_span S = sp[s0];
+        uint64_t q0[G]; uint32_t dw[G]; float sg[G];
 #pragma unroll
-        for(int q = 0; q < SV_G; q++){
-            const int gi = first + q * 16;
+        for(int q = 0; q < G; q++){
+            const int gi = first + q * TEAMS;
             fast[q] = false; dw[q] = 0; sg[q] = 0.0f; q0[q] = 0;
             if(gi >= ngrp) continue;
             if(gi >= S.gi0 + S.ngrp) S = sp[qx_span_of(sp, nspan, gi)];
             const uint64_t j0 = (uint64_t)(gi - S.gi0) * (uint64_t)group;
-            fast[q] = vec_ok && group == 128 && packed && S.n - j0 >= 128 && ((S.qi0 + j0) & 7ULL) == 0;
+            fast[q] = vec_ok && group == 8 * W && packed && S.n - j0 >= 8 * W && ((S.qi0 + j0) & 7ULL) == 0;
             if(!fast[q]) continue;
             q0[q] = S.qi0 + j0;
-            dw[q] = *(const uint32_t *)(d + (q0[q] >> 1) + lane16 * 4);
+            dw[q] = *(const uint32_t *)(d + (q0[q] >> 1) + tl * 4);
             sg[q] = s[gi];
         }
         const uint32_t up = 0x11111111u * (uint32_t)(dmax & 15), down = 0x11111111u * (uint32_t)(-dmax & 15);
 #pragma unroll
-        for(int q = 0; q < SV_G; q++){
-            const int railed = qx_row16_sum(nibbles_equal(dw[q], up) + nibbles_equal(dw[q], down));
-            const float f = (float)railed * (1.0f / 128.0f);
-            if(fast[q] && lane16 == 0 && (f > f_hi || f < f_lo)){
-                const float sn = servo_scale(sg[q], railed, 128, f_hi, f_lo);
+        for(int q = 0; q < G; q++){
+            const int railed = qx_team_sum<W>(nibbles_equal(dw[q], up) + nibbles_equal(dw[q], down));
+            const float f = (float)railed * (1.0f / (8 * W));
+            if(fast[q] && tl == 0 && (f > f_hi || f < f_lo)){
+                const float sn = servo_scale(sg[q], railed, 8 * W, f_hi, f_lo);
                 const int k = atomicAdd(&moving, 1);
                 at[k] = q0[q]; conv[k] = sg[q] / sn;
-                s[first + q * 16] = sn;
+                s[first + q * TEAMS] = sn;
             }
         }
     }
     __syncthreads();
-    for(int k = row; k < moving; k += 16){
-        const uint64_t e0 = at[k] + (uint64_t)lane16 * 8;
+    for(int k = team; k < moving; k += TEAMS){
+        const uint64_t e0 = at[k] + (uint64_t)tl * 8;
         const uint32_t dw = *(const uint32_t *)(d + (e0 >> 1));
         const uint2 rw = *(const uint2 *)(r + e0);
         const float cv = conv[k];
@@ -219,9 +226,9 @@ __global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char 
         *(uint2 *)(r + e0) = make_uint2(r0, r1);
     }
     if(first < ngrp)
-        for(int q = 0; q < SV_G; q++){
-            const int gi = first + q * 16;
-            if(gi < ngrp && !fast[q]) servo_pairs(group_loc(sp, nspan, gi, group), gi, lane16, d, r, s, dmax, f_hi, f_lo, packed);
+        for(int q = 0; q < G; q++){
+            const int gi = first + q * TEAMS;
+            if(gi < ngrp && !fast[q]) servo_pairs<W>(group_loc(sp, qx_span_of(sp, nspan, gi), gi, group), gi, tl, d, r, s, dmax, f_hi, f_lo, packed);
         }
 }
 
@@ -241,8 +248,10 @@ extern "C" int qlmx_encode(const float *P, signed char *d, signed char *r, float
     rc = codec_args_ok("qlmx_encode", nspan, group, dmax, packed); if(rc) return rc;
     if(ngrp <= 0) return QLMX_OK;
     const int vec_ok = ((uintptr_t)P & 15) == 0 && ((uintptr_t)r & 7) == 0 && ((uintptr_t)d & 3) == 0;
-    hipLaunchKernelGGL(k_qlmx_encode, dim3((unsigned)((ngrp + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
-                       P, d, r, s, sp, nspan, group, dmax, packed, ngrp, vec_ok);
+    if(group == 64) hipLaunchKernelGGL(k_qlmx_encode<8>, dim3((unsigned)((ngrp + 31) / 32)), dim3(256), 0, (hipStream_t)stream,
+                                       P, d, r, s, sp, nspan, group, dmax, packed, ngrp, vec_ok);
+    else hipLaunchKernelGGL(k_qlmx_encode<16>, dim3((unsigned)((ngrp + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
+                            P, d, r, s, sp, nspan, group, dmax, packed, ngrp, vec_ok);
     QLMX_LAUNCH_CHECK("qlmx_encode launch");
     return QLMX_OK;
 }
@@ -256,8 +265,10 @@ extern "C" int qlmx_render(float *P, const signed char *d, const float *s,
     QLMX_REQUIRE(gi_base >= 0, "qlmx_render: gi_base %d", gi_base);
     if(ng <= 0) return QLMX_OK;
     const int vec_ok = ((uintptr_t)P & 15) == 0 && ((uintptr_t)d & 3) == 0;
-    hipLaunchKernelGGL(k_qlmx_render, dim3((unsigned)((ng + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
-                       P, d, s, sp, nspan, group, packed, gi_base, ng, vec_ok);
+    if(group == 64) hipLaunchKernelGGL(k_qlmx_render<8>, dim3((unsigned)((ng + 31) / 32)), dim3(256), 0, (hipStream_t)stream,
+                                       P, d, s, sp, nspan, group, packed, gi_base, ng, vec_ok);
+    else hipLaunchKernelGGL(k_qlmx_render<16>, dim3((unsigned)((ng + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
+                            P, d, s, sp, nspan, group, packed, gi_base, ng, vec_ok);
     QLMX_LAUNCH_CHECK("qlmx_render launch");
     return QLMX_OK;
 }
@@ -270,8 +281,12 @@ extern "C" int qlmx_servo(signed char *d, signed char *r, float *s,
     rc = codec_args_ok("qlmx_servo", nspan, group, dmax, packed); if(rc) return rc;
     if(ngrp <= 0) return QLMX_OK;
     const int vec_ok = ((uintptr_t)r & 7) == 0 && ((uintptr_t)d & 3) == 0;
-    hipLaunchKernelGGL(k_qlmx_servo, dim3((unsigned)((ngrp + 16 * SV_G - 1) / (16 * SV_G))), dim3(256), 0, (hipStream_t)stream,
-                       d, r, s, sp, nspan, group, dmax, f_hi, f_lo, packed, ngrp, vec_ok);
+    const bool few = ngrp < (group == 64 ? 65536 : 32768);                 /* at four groups per team: less than two workgroups per CU */
+#define SERVO(W, G) hipLaunchKernelGGL((k_qlmx_servo<W, G>), dim3((unsigned)((ngrp + 256 / W * G - 1) / (256 / W * G))), dim3(256), 0, (hipStream_t)stream, \
+                                       d, r, s, sp, nspan, group, dmax, f_hi, f_lo, packed, ngrp, vec_ok)
+    if(group == 64){ if(few) SERVO(8, 1); else SERVO(8, 4); }
+    else           { if(few) SERVO(16, 1); else SERVO(16, 4); }
+#undef SERVO
     QLMX_LAUNCH_CHECK("qlmx_servo launch");
     return QLMX_OK;
 }

@@ -59,6 +59,21 @@ __device__ __forceinline__ float qx_nib16(const QxNibs &n, int k){
     return __builtin_amdgcn_cvt_off_f32_i4((int)((src >> (8 * (k >> 1))) & 0xFFu));
 }
 
+/* Division of many values by one per-group divisor (encoding, qlm.cuh:155-162; the requantisation of the moments, 261-278).
+ * With y = 1/b correctly rounded (one real division per group), q = a*y, r = fma(-q, b, a) exact and
+ * q' = fma(r, y, q), q' is the correctly rounded a/b (Markstein's final-step theorem) as long as nothing
+ * leaves the normal range; checked against a/b on 4e9 pairs on the CPU. The short form is used only
+ * when b is in [2^-60, 2^60] (|a| is at most 255 b here); quotients so small that r is subnormal are
+ * far below 2^-24 and round (stochastically, or to nearest after times 128) to the same integer either way. Anything else divides. */
+struct GroupDiv { float b, y; bool fast; };
+__device__ __forceinline__ GroupDiv qx_mkdiv(float b){
+    GroupDiv d; d.b = b; d.fast = b >= 0x1p-60f && b <= 0x1p60f; d.y = 1.0f / b; return d;
+}
+__device__ __forceinline__ float qx_gdiv(float a, const GroupDiv &d){
+    if(d.fast){ const float q = a * d.y; const float r = fmaf(-q, d.b, a); return fmaf(r, d.y, q); }
+    return a / d.b;
+}
+
 /* ---- span lookup: the owner of group gi. The table is ascending in gi0, so a binary search
  * returns what the reference's first-match linear scan returns (qlm.cuh:114-117). ---- */
 __device__ __forceinline__ int qx_span_of(const qlmx_span *sp, int nspan, int gi){
@@ -70,35 +85,47 @@ __device__ __forceinline__ int qx_span_of(const qlmx_span *sp, int nspan, int gi
     return lo;
 }
 
-/* ---- DPP reductions over a row of 16 lanes ----
+/* The same for a wavefront whose TEAMS teams of 64 / TEAMS lanes own consecutive groups: the owner of group g0 + team,
+ * g0 the same in all lanes, every lane active. Up to 64 spans a lane reads one entry and the wavefront counts: one
+ * round trip instead of one per halving, which is what a launch over a few groups spends its time on. */
+template<int TEAMS> __device__ __forceinline__ int qx_span_of_teams(const qlmx_span *sp, int nspan, int g0, int team){
+    if(nspan > 64) return qx_span_of(sp, nspan, g0 + team);
+    const int lane = threadIdx.x & 63, at = lane < nspan ? sp[lane].gi0 : 0x7FFFFFFF;
+    int si = 0;
+#pragma unroll
+    for(int k = 0; k < TEAMS; k++){
+        const int n = __popcll(__ballot(at <= g0 + k)) - 1;
+        si = team == k ? n : si;
+    }
+    return si < 0 ? 0 : si;
+}
+
+/* ---- DPP reductions over teams of W = 16 lanes (a row) or 8 (half a row) ----
  * quad_perm [1,0,3,2] = 0xB1, [2,3,0,1] = 0x4E, row_half_mirror = 0x141, row_mirror = 0x140.
- * After the four steps every lane of the row holds the row's maximum. */
+ * After the steps every lane of the team holds the result. */
 template<int CTRL> __device__ __forceinline__ float qx_dpp(float v){
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 template<int CTRL> __device__ __forceinline__ int qx_dpp_i(int v){
     return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, true);
 }
-__device__ __forceinline__ float qx_row16_max(float v){
+template<int W> __device__ __forceinline__ float qx_team_max(float v){
     v = fmaxf(v, qx_dpp<0xB1>(v));
     v = fmaxf(v, qx_dpp<0x4E>(v));
     v = fmaxf(v, qx_dpp<0x141>(v));
-    v = fmaxf(v, qx_dpp<0x140>(v));
-    return v;
+    return W == 16 ? fmaxf(v, qx_dpp<0x140>(v)) : v;
 }
-__device__ __forceinline__ int qx_row16_maxi(int v){
+template<int W> __device__ __forceinline__ int qx_team_maxi(int v){
     v = max(v, qx_dpp_i<0xB1>(v));
     v = max(v, qx_dpp_i<0x4E>(v));
     v = max(v, qx_dpp_i<0x141>(v));
-    v = max(v, qx_dpp_i<0x140>(v));
-    return v;
+    return W == 16 ? max(v, qx_dpp_i<0x140>(v)) : v;
 }
-__device__ __forceinline__ int qx_row16_sum(int v){
+template<int W> __device__ __forceinline__ int qx_team_sum(int v){
     v += qx_dpp_i<0xB1>(v);
     v += qx_dpp_i<0x4E>(v);
     v += qx_dpp_i<0x141>(v);
-    v += qx_dpp_i<0x140>(v);
-    return v;
+    return W == 16 ? v + qx_dpp_i<0x140>(v) : v;
 }
 /* full 64-lane sum / max built from the row step plus two cross-row exchanges */
 __device__ __forceinline__ float qx_wave_sum(float v){

@@ -6,7 +6,7 @@
  * integer state. Divisions and square roots are the correctly rounded ones.
  *
  * Mapping. The reference gives a CUDA block (or a 32-lane warp) to each group. Here a group
- * belongs to one DPP row (16 lanes) of a 64-lane wavefront, so a wave carries four groups and a
+ * belongs to one DPP row (16 lanes; half a row for groups of 64) of a 64-lane wavefront, so a wave carries four groups and a
  * 256-thread workgroup sixteen. With the headline group of 128 each lane owns 8 consecutive
  * elements: one 32-bit word of packed digits, one 64-bit word each of residuals and of both
  * moments, two 128-bit words of gradient. A lane therefore writes whole bytes it alone owns, and
@@ -42,21 +42,6 @@ struct GroupCtx {           /* per-group constants, uniform over the row */
 };
 
 struct ElemRes { float mn, rv; int dd, rr, idl, carry; };
-
-/* Division of many values by one per-group divisor (the requantisation of the moments, qlm.cuh:261-278).
- * With y = 1/b correctly rounded (one real division per group), q = a*y, r = fma(-q, b, a) exact and
- * q' = fma(r, y, q), q' is the correctly rounded a/b (Markstein's final-step theorem) as long as nothing
- * leaves the normal range; checked against a/b on 4e9 pairs on the CPU. The short form is used only
- * when b is in [2^-60, 2^60] (|a| is at most 255 b here); quotients so small that r is subnormal are
- * far below 2^-24 and round stochastically to the same integer either way. Anything else divides. */
-struct GroupDiv { float b, y; bool fast; };
-__device__ __forceinline__ GroupDiv qx_mkdiv(float b){
-    GroupDiv d; d.b = b; d.fast = b >= 0x1p-60f && b <= 0x1p60f; d.y = 1.0f / b; return d;
-}
-__device__ __forceinline__ float qx_gdiv(float a, const GroupDiv &d){
-    if(d.fast){ const float q = a * d.y; const float r = fmaf(-q, d.b, a); return fmaf(r, d.y, q); }
-    return a / d.b;
-}
 
 /* Correctly rounded square root for a whole row of values at a lower price. sqrtf() as the compiler expands it
  * is v_sqrt_f32 (good to one unit in the last place) followed by a test of both neighbours through exact
@@ -181,8 +166,8 @@ __device__ __forceinline__ ElemRes step_elem(const GroupCtx &c, float graw, int 
  * changes a result): second moments >= 2^-96 with roots <= 2^25, |m * inv_bc1| in [2^-40, 2^40] (zero excluded, so
  * that the quotient's residuals cannot underflow), the lane's largest |m| in [2^-32, 2^40], eps <= 2^20; the launch
  * checks 0 <= inv_sqrt_bc2 <= 2^10 on the host (a.mid_ok). */
-template<bool HASP, bool V4>
-__device__ __forceinline__ bool step_row8_mid(const StepParams &a, const GroupCtx &c, int gi, int lane16, uint64_t q, uint64_t pofe,
+template<bool HASP, bool V4, int W>
+__device__ __forceinline__ bool step_row8_mid(const StepParams &a, const GroupCtx &c, int gi, int tl, uint64_t q, uint64_t pofe,
                                               const float (&gv)[8], uint32_t dw, uint2 rw, uint2 mw, uint2 vw,
                                               uint64_t kt, uint64_t ktm, uint64_t ktv){
     float mn[8], vv[8], rv[8], uu[8];
@@ -255,10 +240,11 @@ __device__ __forceinline__ bool step_row8_mid(const StepParams &a, const GroupCt
         __builtin_nontemporal_store(p1, (f4 *)(a.P + pofe + 4));
     }
     /* ---- fresh scales and the re-quantised moments (qlm.cuh:244-278); both maxima are positive here ---- */
-    am = qx_row16_max_nonneg(am); vm = qx_row16_max_nonneg(vm);
+    if(W == 16){ am = qx_row16_max_nonneg(am); vm = qx_row16_max_nonneg(vm); }
+    else       { am = qx_row8_max_nonneg(am);  vm = qx_row8_max_nonneg(vm); }
     const float ms = qx_div_mid(am, 127.0f), vs = qx_div_mid(vm, 255.0f);
     const float ym = qx_div_mid(1.0f, ms), yv = qx_div_mid(1.0f, vs);      /* ms, vs in [2^-40, 2^34]: qx_gdiv's reciprocal form holds */
-    if(lane16 == 0){ a.m8s[gi] = ms; a.v8s[gi] = vs; }
+    if(tl == 0){ a.m8s[gi] = ms; a.v8s[gi] = vs; }
     uint32_t mo0 = 0, mo1 = 0, vo0 = 0, vo1 = 0;
     uint64_t keym = key0 + ktm, keyv = key0 + ktv;
 #pragma unroll
@@ -420,12 +406,15 @@ __device__ __forceinline__ bool step_row16_mid(const StepParams &a, const GroupC
 /* STAT: the four counters are kept; HASP: the fp32 view is written; V4: the second moment is stored as its
  * fourth root (a.v4). All are fixed per launch, so they are template parameters and the usual launch (none of
  * them) carries no trace of them: as a run-time flag, v4 made the compiler compute the second square root of
- * every element and select (18 of 186 vector instructions per weight). */
-template<bool ADAM, bool STAT, bool HASP, bool V4>
-__device__ __forceinline__ void step_team(const StepParams &a, const int team, const int lane16){
-    if(team >= a.ng) return;                       /* whole rows leave together */
+ * every element and select (18 of 186 vector instructions per weight). W lanes form the team of a group, eight weights
+ * each where the group is 8 W long: W = 8 for groups of 64 (a pair per lane and step: 480 us for 64 M weights, 250 so),
+ * 16 for all others. The teams of a wavefront own consecutive groups and it calls with all its lanes. */
+template<bool ADAM, bool STAT, bool HASP, bool V4, int W>
+__device__ __forceinline__ void step_team(const StepParams &a, const int team, const int tl, const bool skip = false){
+    const int k0 = (threadIdx.x & 63) / W, si = a.touched ? 0 : qx_span_of_teams<64 / W>(a.sp, a.nspan, a.gi_base + __builtin_amdgcn_readfirstlane(team), k0);
+    if(team >= a.ng || skip) return;               /* whole teams leave together */
     const int gi = a.touched ? a.touched[team] : a.gi_base + team;
-    const qlmx_span S = a.touched ? a.one : a.sp[qx_span_of(a.sp, a.nspan, gi)];
+    const qlmx_span S = a.touched ? a.one : a.sp[si];
     const uint64_t j0 = (uint64_t)(gi - S.gi0) * (uint64_t)a.group;
     const uint64_t left = S.n - j0;
     const int n = (int)((uint64_t)a.group < left ? (uint64_t)a.group : left);
@@ -451,15 +440,15 @@ __device__ __forceinline__ void step_team(const StepParams &a, const int team, c
     unsigned long long st_carry = 0, st_rail = 0, st_zero = 0, st_idl = 0;
     const bool want_stat = STAT;
 
-    const bool fast = a.vec_ok && a.group == 128 && a.packed && n == 128 && ((pof | qi0 | gof) & 7ULL) == 0;
+    const bool fast = a.vec_ok && a.group == 8 * W && a.packed && n == 8 * W && ((pof | qi0 | gof) & 7ULL) == 0;
     if(fast){
-        const uint64_t e0 = (uint64_t)lane16 * 8;
+        const uint64_t e0 = (uint64_t)tl * 8;
         const uint64_t q = qi0 + e0;
         if(ADAM && !STAT && a.mid_ok){
             const float4 h0 = *(const float4 *)(a.G + gof + e0);
             const float4 h1 = *(const float4 *)(a.G + gof + e0 + 4);
             const float hv[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-            if(step_row8_mid<HASP, V4>(a, c, gi, lane16, q, pof + e0, hv, *(const uint32_t *)(a.d + (q >> 1)), *(const uint2 *)(a.r + q),
+            if(step_row8_mid<HASP, V4, W>(a, c, gi, tl, q, pof + e0, hv, *(const uint32_t *)(a.d + (q >> 1)), *(const uint2 *)(a.r + q),
                                        *(const uint2 *)(a.m8 + q), *(const uint2 *)(a.v8 + q), kt, ktm, ktv)) return;
             /* nothing was stored; the general code loads its operands again rather than keep them in registers
              * across the attempt (the barrier keeps the compiler from merging the two sets of loads) */
@@ -560,12 +549,12 @@ __device__ __forceinline__ void step_team(const StepParams &a, const int team, c
             __builtin_nontemporal_store(p1, (f4 *)(a.P + pof + e0 + 4));
         }
         /* ---- fresh scales and the re-quantised moments (qlm.cuh:244-278) ---- */
-        am = qx_row16_max(am); vm = qx_row16_max(vm);
+        am = qx_team_max<W>(am); vm = qx_team_max<W>(vm);
         const float ms = am > 0.0f ? am / 127.0f : 1e-12f;
         const float vs = vm > 0.0f ? vm / 255.0f : 1e-12f;
         const GroupDiv dms = qx_mkdiv(ms), dvs = qx_mkdiv(vs);
-        if(lane16 == 0){ a.m8s[gi] = ms; if(ADAM) a.v8s[gi] = vs; }
-        /* one choice for the wavefront: the reciprocal form when all four groups allow it (the usual case) */
+        if(tl == 0){ a.m8s[gi] = ms; if(ADAM) a.v8s[gi] = vs; }
+        /* one choice for the wavefront: the reciprocal form when all groups allow it (the usual case) */
         const bool recip = __builtin_amdgcn_ballot_w64(!(dms.fast && (!ADAM || dvs.fast))) == 0;
         uint32_t mo0 = 0, mo1 = 0, vo0 = 0, vo1 = 0;
         uint64_t keym = key0 + ktm, keyv = key0 + ktv;
@@ -597,12 +586,12 @@ __device__ __forceinline__ void step_team(const StepParams &a, const int team, c
         *(uint2 *)(a.m8 + q) = make_uint2(mo0, mo1);
         if(ADAM) *(uint2 *)(a.v8 + q) = make_uint2(vo0, vo1);
     } else {
-        /* pair-per-lane path: lane owns elements {2*lane16, 2*lane16+1} + 32*k, i.e. whole bytes
+        /* pair-per-lane path: lane owns elements {2*tl, 2*tl+1} + 2*W*k, i.e. whole bytes
          * of packed digits. Sweep one updates digits, residuals and P; sweep two recomputes the
          * moments from m8/v8/G, which sweep one does not write (same operations, hence the same
          * bits), and requantises them. Nothing is held in registers across the reduction. */
         float am = 0.0f, vm = 0.0f;
-        for(int jb = 2 * lane16; jb < n; jb += 32){
+        for(int jb = 2 * tl; jb < n; jb += 2 * W){
             int ddn[2] = {0, 0};
             unsigned oldb = 0;
             if(a.packed) oldb = (unsigned char)a.d[(qi0 + jb) >> 1];
@@ -632,10 +621,10 @@ __device__ __forceinline__ void step_team(const StepParams &a, const int team, c
             }
             if(a.packed) a.d[(qi0 + jb) >> 1] = (signed char)(((ddn[1] & 15) << 4) | (ddn[0] & 15));
         }
-        am = qx_row16_max(am); vm = qx_row16_max(vm);
+        am = qx_team_max<W>(am); vm = qx_team_max<W>(vm);
         const float ms = am > 0.0f ? am / 127.0f : 1e-12f;
         const float vs = vm > 0.0f ? vm / 255.0f : 1e-12f;
-        for(int jb = 2 * lane16; jb < n; jb += 32){
+        for(int jb = 2 * tl; jb < n; jb += 2 * W){
 #pragma unroll
             for(int h = 0; h < 2; h++){
                 const int j = jb + h;
@@ -653,15 +642,15 @@ __device__ __forceinline__ void step_team(const StepParams &a, const int team, c
             }
         }
         /* written last: the recomputation above reads the old per-group moment scales via `c` */
-        if(lane16 == 0){ a.m8s[gi] = ms; if(ADAM) a.v8s[gi] = vs; }
+        if(tl == 0){ a.m8s[gi] = ms; if(ADAM) a.v8s[gi] = vs; }
     }
 
     if(want_stat){
-        /* row totals, then one lane per group updates the four counters */
-        unsigned sc = (unsigned)qx_row16_sum((int)st_carry), sr = (unsigned)qx_row16_sum((int)st_rail),
-                 sz = (unsigned)qx_row16_sum((int)st_zero);
-        unsigned mi = (unsigned)qx_row16_maxi((int)st_idl);
-        if(lane16 == 0){
+        /* team totals, then one lane per group updates the four counters */
+        unsigned sc = (unsigned)qx_team_sum<W>((int)st_carry), sr = (unsigned)qx_team_sum<W>((int)st_rail),
+                 sz = (unsigned)qx_team_sum<W>((int)st_zero);
+        unsigned mi = (unsigned)qx_team_maxi<W>((int)st_idl);
+        if(tl == 0){
             atomicAdd(&a.stat[0], (unsigned long long)sc);
             atomicAdd(&a.stat[1], (unsigned long long)sr);
             atomicAdd(&a.stat[2], (unsigned long long)sz);
@@ -670,27 +659,28 @@ __device__ __forceinline__ void step_team(const StepParams &a, const int team, c
     }
 }
 
-/* one group per row of 16 lanes: every shape, every option */
-template<bool ADAM, bool STAT, bool HASP, bool V4>
+/* one group per W lanes: every shape, every option */
+template<bool ADAM, bool STAT, bool HASP, bool V4, int W>
 __global__ void __launch_bounds__(256) k_qlmx_step(StepParams a){
-    step_team<ADAM, STAT, HASP, V4>(a, (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) >> 4), threadIdx.x & 15);
+    step_team<ADAM, STAT, HASP, V4, W>(a, (int)((blockIdx.x * 256u + threadIdx.x) / W), threadIdx.x & (W - 1));
 }
 /* Adam on packed groups of 128 without statistics (what a training step launches): one group per 8 lanes, eight
- * groups per wavefront, through step_row16_mid when all eight are whole, aligned groups with operands in the middle
- * of the range -- a choice per wavefront, made before anything is stored; otherwise the wavefront's groups go through
- * the code above, four at a time. */
+ * groups per wavefront. Whole, aligned groups go through step_row16_mid when all of the wavefront's have operands in the
+ * middle of the range -- a choice made before anything is stored; the others, and all where it is not so, go
+ * through the code above, four at a time. */
 template<bool HASP, bool V4>
 __global__ void __launch_bounds__(256) k_qlmx_step_wide(StepParams a){
     const int lane = threadIdx.x & 63;
     const int g0 = (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) >> 6) * 8;       /* first group of the wavefront */
     if(g0 >= a.ng) return;
-    if(g0 + 8 <= a.ng){
-        const int gi = a.gi_base + g0 + (lane >> 3);
-        const qlmx_span S = a.sp[qx_span_of(a.sp, a.nspan, gi)];
+    const int team = g0 + (lane >> 3), gi = a.gi_base + team;
+    const int si = qx_span_of_teams<8>(a.sp, a.nspan, a.gi_base + __builtin_amdgcn_readfirstlane(g0), lane >> 3);
+    bool done = false;
+    if(team < a.ng){
+        const qlmx_span S = a.sp[si];
         const uint64_t j0 = (uint64_t)(gi - S.gi0) * 128u;
         const uint64_t pof = S.pof + j0, qi0 = S.qi0 + j0, gof = S.gof + j0;
-        const bool whole = S.n - j0 >= 128u && ((pof | qi0 | gof) & 7ULL) == 0;
-        if(__builtin_amdgcn_ballot_w64(!whole) == 0){
+        if(S.n - j0 >= 128u && ((pof | qi0 | gof) & 7ULL) == 0){
             GroupCtx c;
             c.gs = a.gsp ? *a.gsp : a.gscale;
             c.sg = a.s[gi];
@@ -703,28 +693,41 @@ __global__ void __launch_bounds__(256) k_qlmx_step_wide(StepParams a){
             c.inv_bc1 = a.inv_bc1; c.inv_sqrt_bc2 = a.inv_sqrt_bc2;
             c.dmax = a.dmax; c.v4 = V4;
             const uint64_t kt = a.t * QLMX_KT;
-            if(step_row16_mid<HASP, V4>(a, c, gi, lane & 7, qi0, pof, gof, kt, kt + 0x5EEDULL * QLMX_KT, kt + 0xBEEFULL * QLMX_KT)) return;
-            asm volatile("" ::: "memory");         /* nothing was stored; the general code loads its operands itself */
+            done = step_row16_mid<HASP, V4>(a, c, gi, lane & 7, qi0, pof, gof, kt, kt + 0x5EEDULL * QLMX_KT, kt + 0xBEEFULL * QLMX_KT);
         }
     }
+    const uint64_t did = __builtin_amdgcn_ballot_w64(done);
+    if(did == ~0ULL) return;
+    asm volatile("" ::: "memory");                 /* nothing was stored for the others; the general code loads its operands itself */
 #pragma unroll 1
-    for(int p = 0; p < 2; p++) step_team<true, false, HASP, V4>(a, g0 + 4 * p + (lane >> 4), lane & 15);
+    for(int p = 0; p < 2; p++){
+        const int k = 4 * p + (lane >> 4);
+        step_team<true, false, HASP, V4, 16>(a, g0 + k, lane & 15, ((did >> (8 * k)) & 1) != 0);
+    }
 }
 
-template<bool ADAM, bool V4> static void step_launch_opt(const StepParams &a, unsigned blocks, hipStream_t st){
+template<bool ADAM, bool V4, int W> static void step_launch_opt(const StepParams &a, hipStream_t st){
     const bool stat = a.stat != nullptr, hasp = a.P != nullptr;
-    if(stat && hasp)  hipLaunchKernelGGL((k_qlmx_step<ADAM, true, true, V4>),   dim3(blocks), dim3(256), 0, st, a);
-    else if(stat)     hipLaunchKernelGGL((k_qlmx_step<ADAM, true, false, V4>),  dim3(blocks), dim3(256), 0, st, a);
-    else if(hasp)     hipLaunchKernelGGL((k_qlmx_step<ADAM, false, true, V4>),  dim3(blocks), dim3(256), 0, st, a);
-    else              hipLaunchKernelGGL((k_qlmx_step<ADAM, false, false, V4>), dim3(blocks), dim3(256), 0, st, a);
+    const dim3 grid((unsigned)(((long long)a.ng * W + 255) / 256)), block(256);
+    if(stat && hasp)  hipLaunchKernelGGL((k_qlmx_step<ADAM, true, true, V4, W>),   grid, block, 0, st, a);
+    else if(stat)     hipLaunchKernelGGL((k_qlmx_step<ADAM, true, false, V4, W>),  grid, block, 0, st, a);
+    else if(hasp)     hipLaunchKernelGGL((k_qlmx_step<ADAM, false, true, V4, W>),  grid, block, 0, st, a);
+    else              hipLaunchKernelGGL((k_qlmx_step<ADAM, false, false, V4, W>), grid, block, 0, st, a);
 }
-static void step_launch(const StepParams &a, bool adam, unsigned blocks, hipStream_t st){
+template<bool ADAM, bool V4> static void step_launch_width(const StepParams &a, hipStream_t st){
+    if(a.group == 64) step_launch_opt<ADAM, V4, 8>(a, st); else step_launch_opt<ADAM, V4, 16>(a, st);
+}
+static void step_launch(const StepParams &a, bool adam, hipStream_t st){
     /* v4 only exists for Adam's second moment (Lion keeps none) */
-    if(adam){ if(a.v4) step_launch_opt<true, true>(a, blocks, st); else step_launch_opt<true, false>(a, blocks, st); }
-    else step_launch_opt<false, false>(a, blocks, st);
+    if(adam){ if(a.v4) step_launch_width<true, true>(a, st); else step_launch_width<true, false>(a, st); }
+    else step_launch_width<false, false>(a, st);
 }
 
-static bool g_step_wide = true;
+/* Launches below this many groups take the one-group-per-row kernel: with eight groups to a wavefront there are too few of
+ * them to hide a wavefront's own chain, twice as long (16 M weights 83 against 80 us, 24 M 121 against 126, 126 M 538
+ * against 557, norm included). */
+#define STEP_WIDE_GROUPS 160000
+static int g_step_wide_min = STEP_WIDE_GROUPS;
 /* qlm_step_launch (qlm.cuh:377-397) */
 extern "C" int qlmx_step(float *P, const float *G, signed char *d, signed char *r, const float *s,
               signed char *m8, float *m8s, unsigned char *v8, float *v8s,
@@ -752,7 +755,7 @@ extern "C" int qlmx_step(float *P, const float *G, signed char *d, signed char *
     a.vec_ok = (((uintptr_t)P | (uintptr_t)G) & 15) == 0 && (((uintptr_t)r | (uintptr_t)m8 | (uintptr_t)v8) & 7) == 0
                && ((uintptr_t)d & 3) == 0;
     hipStream_t st = (hipStream_t)stream;
-    if(adam && !stat && packed && group == 128 && a.mid_ok && a.vec_ok && g_step_wide){
+    if(adam && !stat && packed && group == 128 && a.mid_ok && a.vec_ok && ng >= g_step_wide_min){
         /* a training step's launch: eight groups per wavefront (k_qlmx_step_wide) */
         const unsigned wblocks = (unsigned)((ng + 31) / 32);
         if(v4){ if(P) hipLaunchKernelGGL((k_qlmx_step_wide<true, true>), dim3(wblocks), dim3(256), 0, st, a);
@@ -760,15 +763,14 @@ extern "C" int qlmx_step(float *P, const float *G, signed char *d, signed char *
         else  { if(P) hipLaunchKernelGGL((k_qlmx_step_wide<true, false>), dim3(wblocks), dim3(256), 0, st, a);
                 else  hipLaunchKernelGGL((k_qlmx_step_wide<false, false>), dim3(wblocks), dim3(256), 0, st, a); }
     } else {
-        const unsigned blocks = (unsigned)((ng + 15) / 16);
-        step_launch(a, adam != 0, blocks, st);
+        step_launch(a, adam != 0, st);
     }
     QLMX_LAUNCH_CHECK("qlmx_step launch");
     return QLMX_OK;
 }
 /* Test hook: 0 sends every launch through the one-group-per-16-lanes kernel (the two kernels must agree byte for
- * byte), 1 (the default) lets training-shaped launches take the eight-groups-per-wavefront kernel. */
-extern "C" int qlmx_test_step_wide(int on){ g_step_wide = on != 0; return QLMX_OK; }
+ * byte), 1 every training-shaped launch through the eight-groups-per-wavefront kernel, 2 (the default) those with many groups. */
+extern "C" int qlmx_test_step_wide(int on){ g_step_wide_min = on == 0 ? 0x7FFFFFFF : on == 1 ? 0 : STEP_WIDE_GROUPS; return QLMX_OK; }
 
 /* k_ng_q4_step (cudalm.cu:4472-4520; CPU twin cpu_kern.h:620-648): the step restricted to a list of
  * touched groups of ONE packed 4-bit span that starts at element 0 of d/r/m8/v8/P (the n-gram
@@ -799,8 +801,7 @@ extern "C" int qlmx_step_touched(float *P, const float *Gc, signed char *d, sign
     a.mid_ok = inv_sqrt_bc2 >= 0.0f && inv_sqrt_bc2 <= 1024.0f;
     a.one.pof = 0; a.one.gof = 0; a.one.qi0 = 0; a.one.n = nt; a.one.gi0 = 0;
     a.one.ngrp = (int)((nt + (unsigned long long)group - 1) / (unsigned long long)group); a.one.sref = sref;
-    const unsigned blocks = (unsigned)((ntouched + 15) / 16);
-    step_launch(a, true, blocks, (hipStream_t)stream);
+    step_launch(a, true, (hipStream_t)stream);
     QLMX_LAUNCH_CHECK("qlmx_step_touched launch");
     return QLMX_OK;
 }

@@ -395,6 +395,52 @@ def test_step_eight_groups_per_wavefront_equals_one_per_row(q, orc, v4, render):
         assert np.array_equal(results[0][i].view(np.uint8), np.asarray(want[i]).view(np.uint8)), nm
 
 
+@pytest.mark.parametrize("group", [64, 128])
+@pytest.mark.parametrize("nspan", [3, 70])
+def test_teams_of_half_and_whole_rows_vs_oracle(q, orc, group, nspan):
+    """Encode, servo, render and the step with the groups of a wavefront spread over spans: short last groups and unaligned
+    spans among whole ones, more spans than a wavefront has lanes, groups with nothing but zeros among ordinary ones, a
+    count of groups that fills no wavefront; Adam (each of its kernels, with and without statistics and view) and Lion."""
+    import torch
+    dmax, rng = 7, np.random.default_rng(nspan)
+    sizes = [int(n) for n in rng.integers(1, 700, nspan) * 2] if nspan > 3 else [group * 37 + 8, group * 29, group * 3 + 2]
+    tab, nq, ng = make_spans(sizes, group)
+    tab["sref"] = 0.0086
+    hP = orc.normal(nq, 17, 1, 0.02)
+    d, r, s, P = dev(np.zeros(nq // 2 + 1, np.int8)), dev(np.zeros(nq, np.int8)), dev(np.zeros(ng, f32)), dev(hP)
+    hd, hr, hs = np.zeros(nq // 2 + 1, np.int8), np.zeros(nq, np.int8), np.zeros(ng, f32)
+    q.encode(P, d, r, s, dev(tab), nspan, group, dmax, 1, ng); orc.encode(hP.copy(), hd, hr, hs, tab, group, dmax, 1, ng)
+    assert beq(d, hd) and beq(r, hr) and beq(s, hs)
+    q.servo(d, r, s, dev(tab), nspan, group, dmax, 0.02, 0.012, 1, ng); orc.servo(hd, hr, hs, tab, group, dmax, 0.02, 0.012, 1, ng)
+    assert beq(d, hd) and beq(r, hr) and beq(s, hs)
+    base, hPv = ng // 3, np.zeros(nq, f32)
+    view = dev(hPv)
+    q.render(view, d, s, dev(tab), nspan, group, 1, base, ng - base); orc.render(hPv, hd, hs, tab, group, 1, base, ng - base)
+    assert beq(view, hPv)
+    hG = orc.normal(nq, 17, 2, 1e-3)
+    hG[group * 5:group * 6] = 0.0
+    for adam, wide, stat, render in ((1, 2, False, False), (1, 1, False, True), (1, 2, True, False), (0, 2, False, True)):
+        h = dict(d=hd.copy(), r=hr.copy(), m8=orc.int8(nq, 17, 3, -127, 127), m8s=orc.uniform(ng, 17, 4, 0.5, 1.5) * f32(3e-3 / 127),
+                 v8=orc.u8(nq, 17, 5, 0, 255), v8s=orc.uniform(ng, 17, 6, 0.5, 1.5) * f32(3e-3 / 255))
+        h["v8"][group * 5:group * 6] = 0; h["m8"][group * 5:group * 6] = 0
+        g = {k: dev(v.copy()) for k, v in h.items()}
+        hstat, gstat = (np.zeros(4, np.int64), torch.zeros(4, dtype=torch.int64, device="cuda")) if stat else (None, None)
+        hv, gv = (np.zeros(nq, f32), torch.zeros(nq, device="cuda")) if render else (None, None)
+        hp = (3e-4, 0.9, 0.95, 0.1, 1.0, None, 10.0, 4.4721, 0, 1, adam)
+        q.call("qlmx_test_step_wide", wide)
+        try:
+            q.step(gv, dev(hG), g["d"], g["r"], s, g["m8"], g["m8s"], g["v8"], g["v8s"], dev(tab), nspan, group, dmax, *hp, gstat, 1, 0, ng)
+        finally:
+            q.call("qlmx_test_step_wide", 2)
+        orc.step(hv, hG, h["d"], h["r"], hs, h["m8"], h["m8s"], h["v8"], h["v8s"], tab, group, dmax, *hp, hstat, 1, 0, ng)
+        for k in h:
+            assert beq(g[k], h[k]), (adam, wide, k)
+        if render:
+            assert beq(gv, hv)
+        if stat:
+            assert np.array_equal(host(gstat), hstat)
+
+
 @pytest.mark.parametrize("n", [1, 63, 64 * 4096 + 5, 64 * 4096 * 3 + 2, 64 * 4096 * 17 + 1])
 def test_sqsum_pieces(q, orc, n):
     """One, three and sixteen workgroups per partial sum, chunk ends that are not aligned, twice in a row (the counters)."""
