@@ -1,9 +1,15 @@
-"""ctypes view of libqlmx.so. Pointers may be given as ints, torch tensors (data_ptr), numpy arrays
-(host pointers, only where the C function takes host memory) or None."""
+"""Python view of libqlmx.so: the calls of a program's inner loop through the compiled module _qlmx_call, the others through
+ctypes. Pointers may be given as ints, torch tensors (data_ptr), numpy arrays (host pointers, only where the C function
+takes host memory) or None."""
 import ctypes as C
 import os
 
 import numpy as np
+
+try:
+    from . import _qlmx_call
+except ImportError:                          # not built: every call goes through ctypes
+    _qlmx_call = None
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
@@ -127,6 +133,7 @@ class Qlmx:
         for name, (res, args) in SIGNATURES.items():
             f = getattr(self.lib, name)
             f.restype, f.argtypes = res, args
+        self._direct = {name: _qlmx_call.bind(name, C.cast(getattr(self.lib, name), c_vp).value) for name in (_qlmx_call.names() if _qlmx_call else ())}
         if init:
             self.check(self.lib.qlmx_init(device))
 
@@ -138,6 +145,12 @@ class Qlmx:
             raise QlmxError("libqlmx error %d: %s" % (rc, self.last_error()))
 
     def call(self, name, *args):
+        direct = self._direct.get(name)
+        if direct is not None:
+            rc = direct(*args)
+            if rc:
+                self.check(rc)
+            return rc
         conv = []
         for a, t in zip(args, SIGNATURES[name][1]):
             conv.append(_ptr(a) if t is c_vp else a)

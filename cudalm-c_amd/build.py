@@ -17,12 +17,14 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libqlmx.so")
 HOST_LIB = os.path.join(HERE, "libqlmx_host.so")
+CALL_LIB = os.path.join(HERE, "_qlmx_call.so")
 ARCH = "gfx950"
 
 HIP_SOURCES = ["qlmx_runtime.hip", "qlmx_step.hip", "qlmx_codec.hip", "qlmx_gemm_common.hip",
@@ -124,6 +126,8 @@ def build_all(jobs=8):
         _run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(HERE, "..", "include"),
               os.path.join(HERE, "host", "selftest.cpp"), "-o", os.path.join(HERE, "qlm_selftest"),
               "-L", HERE, "-lqlmx_host", "-lqlmx", "-Wl,-rpath,$ORIGIN"])
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-I", os.path.join(HERE, "..", "include"), "-I", sysconfig.get_paths()["include"],
+          os.path.join(HERE, "host", "qlmx_call.cpp"), "-o", CALL_LIB])
     return LIB
 
 
