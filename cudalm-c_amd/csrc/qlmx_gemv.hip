@@ -299,15 +299,15 @@ int qlmx_gemv_nn_dispatch(const signed char *d, const float *s, int group, const
  * the same problem table from `assign` in LDS (stable counting sort by expert, the order of the
  * reference's host permutation, cudalm.cu:3586-3599).
  *
- * Task kernel (a template over two multiply loops). fp32 loop, the default: 256 threads cover 16 rows x 256
- * columns per step (a lane owns 16 columns = 8 bytes of digits of one row; 16 lanes cover the 128 contiguous
- * bytes of a row's chunk). fp16-input loop (qlmx_decode_math(1)): 32 rows per step, a lane owns the same columns
- * of two consecutive rows and multiplies both at once (see df_task). Either way a task is two halves of
- * DF_BATCH 8-byte loads per lane, both in flight (the next task's halves are requested as soon as this task has
- * consumed them). The input rows are staged in LDS already multiplied by the row's group scales, so the loop
- * loads digits only. Tasks of one (problem, matrix) are given to workgroups of one XCD so that the 64-byte scale
- * sectors shared by neighbouring chunks are fetched into one L2 only (the groups left over after a full round of
- * 8 XCDs are cut into pieces, see the kernel).
+ * Task kernel (a template over two multiply loops): up to 256 rows x 256 columns, a lane owns 16 columns = 8 bytes of
+ * digits of the rows it loads, 16 lanes cover the 128 contiguous bytes of a row's chunk. Matrix-core loop, the default:
+ * exact digits times inputs in four bytes each (df_task_i8); a wavefront has a quarter of the rows to itself. fp16-input
+ * loop (qlmx_decode_math(1)): 32 rows per step, a lane owns the same columns of two consecutive rows and multiplies both
+ * at once (df_task_h). Either way a task is two halves of DF_BATCH 8-byte loads per lane, both in flight (the next task's
+ * halves are requested as soon as this task has consumed them). The input rows are staged in LDS already multiplied by
+ * the row's group scales, so the loop loads digits only. Tasks of one (problem, matrix) are given to workgroups of one XCD
+ * so that the 64-byte scale sectors shared by neighbouring chunks are fetched into one L2 only (the groups left over after
+ * a full round of 8 XCDs are cut into pieces, see the kernel).
  * ---------------------------------------------------------------------------------------- */
 #define DEC_MAXPAIR 64
 #define DF_THREADS 256
@@ -317,8 +317,8 @@ int qlmx_gemv_nn_dispatch(const signed char *d, const float *s, int group, const
 #define DF_CW 256             /* columns per task */
 #define DF_NG 2               /* scale groups per task row: group 128, or one when the group is a multiple of 256 */
 #define DF_RMAX 256           /* rows per task at most */
-#define DF_BATCH 8            /* 8-byte digit loads per lane and half task (fp32 loop: 8 steps of 16 rows; fp16-input loop: 4 steps of
-                                 32 rows, a lane's two rows each): a task is two halves of at most 128 rows */
+#define DF_BATCH 8            /* 8-byte digit loads per lane and half task (matrix-core loop: 8 steps of 16 rows; fp16-input loop: 4
+                                 steps of 32 rows, a lane's two rows each): a task is two halves of at most 128 rows */
 #define DF_SPIN_LIMIT (1 << 17)
 #define DF_MAXTASKS 128        /* tasks of one workgroup at most (both lists); the host refuses shapes that would need more */
 typedef unsigned long long u64;
@@ -355,10 +355,10 @@ struct DfArgs {
 };
 
 struct DfMeta {
-    int nprob;
-    int p_e[DEC_MAXPAIR], p_M[DEC_MAXPAIR], p_row0[DEC_MAXPAIR];
-    int rowpair[DEC_MAXPAIR], rowtok[DEC_MAXPAIR], pair_prob[DEC_MAXPAIR], pair_m[DEC_MAXPAIR];
-    int se[DEC_MAXPAIR], sj[DEC_MAXPAIR], ein[DEC_MAXPAIR], rk[4][DEC_MAXPAIR];
+    int ntasks;
+    bool full;                                                            /* list 1 gives most workgroups a task */
+    int p_e[DEC_MAXPAIR], p_M[DEC_MAXPAIR], p_tok[DEC_MAXPAIR][DF_MB];    /* a problem's expert, pairs, their tokens */
+    int pair_prob[DEC_MAXPAIR], pair_m[DEC_MAXPAIR];                      /* a pair's problem (-1: no such expert) and place in it */
 };
 
 /* a / b for 0 <= a < 2^22, b > 0, rb = 1/b as a float: the quotient of the floats is off by at most one,
@@ -480,15 +480,36 @@ __device__ __forceinline__ float df_stage(const float (&v)[DF_NG][DF_MB], bool l
     return inv;
 }
 
-/* The same for the fp32 loop: the values as they are, xs[g][row][m]; nothing to undo (returns 1). */
-__device__ __forceinline__ float df_stage_f32(const float (&v)[DF_NG][DF_MB], bool live, float (*xs)[DF_RMAX][DF_MB]){
-    __syncthreads();                                 /* the previous task is done with xs */
-    if(live){
+/* Staging for the matrix-core loop, wavefront by wavefront: a lane holds one row of its wavefront's share of the task
+ * (zeros past its end), v[g][m] as above. Each input row m is brought to a 31-bit fixed point at the largest magnitude
+ * among the wavefront's rows, k[m] = the power of two, and stored as four signed bytes whose sum times 1, 2^8, 2^16, 2^24 it
+ * is (q + 0x80808080 has the bytes plus 128): a value less than 2^7 below the largest keeps all its 24 bits, and what a smaller
+ * one loses lies below what the fp32 sums of the row would round away. bad[m]: a value is infinite or not a number.
+ * xs: [plane g * DF_MB + m][lane group of the loop][row of the group]; written and read by one wavefront, so no barrier. */
+#define DF_XPLANE 68          /* 64 rows, and 4 words so that the 16 (plane, lane group) pairs of a read start in different banks */
+__device__ __forceinline__ unsigned df_wave_max(unsigned v){
+    v = max(v, (unsigned)qx_dpp_i<0xB1>((int)v)); v = max(v, (unsigned)qx_dpp_i<0x4E>((int)v));
+    v = max(v, (unsigned)qx_dpp_i<0x141>((int)v)); v = max(v, (unsigned)qx_dpp_i<0x140>((int)v));
+    const unsigned a = max((unsigned)__builtin_amdgcn_readlane((int)v, 0), (unsigned)__builtin_amdgcn_readlane((int)v, 16));
+    const unsigned b = max((unsigned)__builtin_amdgcn_readlane((int)v, 32), (unsigned)__builtin_amdgcn_readlane((int)v, 48));
+    return max(a, b);
+}
+__device__ __forceinline__ void df_stage_i8(const float (&v)[DF_NG][DF_MB], uint32_t *xs, int (&k)[DF_MB], bool (&bad)[DF_MB]){
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-        for(int gg = 0; gg < DF_NG; gg++) *(float2 *)&xs[gg][threadIdx.x][0] = make_float2(v[gg][0], v[gg][1]);
+    for(int m = 0; m < DF_MB; m++){
+        unsigned mx = 0;
+#pragma unroll
+        for(int gg = 0; gg < DF_NG; gg++) mx = max(mx, __float_as_uint(v[gg][m]) & 0x7FFFFFFFu);
+        const int ex = (int)(df_wave_max(mx) >> 23);
+        bad[m] = ex == 255;
+        k[m] = 156 - ex;                                  /* the largest comes to [2^29, 2^30) */
+#pragma unroll
+        for(int gg = 0; gg < DF_NG; gg++){
+            const uint32_t q = (uint32_t)(int)rintf(__builtin_amdgcn_ldexpf(v[gg][m], k[m]));
+            xs[(gg * DF_MB + m) * DF_XPLANE + (lane & 3) * 16 + (lane >> 2)] = (q + 0x80808080u) ^ 0x80808080u;
+        }
     }
-    __syncthreads();
-    return 1.0f;
 }
 
 /* One task: which slice of which matrix, for which problem. list 0 = none. */
@@ -499,16 +520,16 @@ struct DfT { u64 wq, wg; int list, N, k0, rows, chunk, M, prob, mat, sl, ngl; };
 template<bool H>
 __device__ __forceinline__ const signed char *df_digits(const DfArgs &a, const DfT &t){
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int cl = lane & 15, rp = wave * 4 + (lane >> 4);
+    const int cl = lane & 15, rp = lane >> 4;
     const int col0 = t.chunk * DF_CW + cl * 16;
-    return a.d + ((t.wq + (size_t)(t.k0 + (H ? 2 * rp : rp)) * t.N + (col0 < t.N ? col0 : 0)) >> 1);
+    return a.d + ((t.wq + (size_t)(t.k0 + (H ? 2 * (wave * 4 + rp) : wave * (t.rows >> 2) + rp)) * t.N + (col0 < t.N ? col0 : 0)) >> 1);
 }
 /* Requests half h of a task's digits into W. fp16 loop (H): a step is 32 rows, the 16 row pairs of the
- * workgroup's 16 lane groups, and W[2 s + par] holds row `par` of the lane's pair in step s of the half; fp32
- * loop: a step is 16 rows, W[s] the lane's row in step s. rows is a multiple of 32, so a step is live or not
- * for the whole workgroup. Every load is issued unconditionally (a dead step re-reads step 0): loads under a
- * branch make the compiler wait for each one where the branches join, which turns a batch into a chain of
- * memory round trips. */
+ * workgroup's 16 lane groups, and W[2 s + par] holds row `par` of the lane's pair in step s of the half; matrix-core
+ * loop: a wavefront owns a quarter of the rows, a step is four of them, one per lane group, and a half eight steps.
+ * rows is a multiple of 32, so a step is live or not for the whole workgroup. Every load is issued unconditionally (a
+ * dead step re-reads step 0): loads under a branch make the compiler wait for each one where the branches join, which
+ * turns a batch into a chain of memory round trips. */
 template<bool H>
 __device__ __forceinline__ void df_load(uint2 (&W)[DF_BATCH], const signed char *dp, size_t rowb, int rows, int hsteps, int h){
 #pragma unroll
@@ -518,12 +539,21 @@ __device__ __forceinline__ void df_load(uint2 (&W)[DF_BATCH], const signed char 
             const int sc = ((b >> 1) < hsteps && st * 32 < rows) ? st : 0;
             W[b] = *(const uint2 *)(dp + (size_t)(sc * 32 + (b & 1)) * rowb);
         } else {
-            const int st = h * hsteps + b;
-            const int sc = (b < hsteps && st * 16 < rows) ? st : 0;
-            W[b] = *(const uint2 *)(dp + (size_t)sc * 16 * rowb);
+            const int st = h * DF_BATCH + b;
+            W[b] = *(const uint2 *)(dp + (size_t)(st * 16 < rows ? st * 4 : 0) * rowb);
         }
     }
 }
+
+/* the four bytes q of four words as one word each: t[q] = byte q of w0, w1, w2, w3 */
+__device__ __forceinline__ void df_bytes(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t (&t)[4]){
+    const uint32_t a = __builtin_amdgcn_perm(w1, w0, 0x05010400u), b = __builtin_amdgcn_perm(w3, w2, 0x05010400u);
+    const uint32_t c = __builtin_amdgcn_perm(w1, w0, 0x07030602u), d = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
+    t[0] = __builtin_amdgcn_perm(b, a, 0x05040100u); t[1] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    t[2] = __builtin_amdgcn_perm(d, c, 0x05040100u); t[3] = __builtin_amdgcn_perm(d, c, 0x07060302u);
+}
+typedef int df_i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ long df_pair(uint32_t lo, uint32_t hi){ return (long)(((u64)hi << 32) | (u64)lo); }
 
 /* dst[m*mstride + chunk*256 + c] = sum_{r<rows} x[m][r] * s * digit(k0+r, chunk*256+c), m < M, stored
  * tagged. w0, w1 hold the digits of the task's two halves, requested earlier. `prep` stages the inputs
@@ -531,17 +561,96 @@ __device__ __forceinline__ void df_load(uint2 (&W)[DF_BATCH], const signed char 
  * task's halves into w0 and w1 as soon as this task has consumed them, so the reduction, the stores and the
  * next task's staging overlap that trip from HBM.
  *
- * The multiply-adds are v_dot2_f32_f16: two products per instruction, exact, summed in fp32. One operand is the
+ * Matrix-core loop (the default). v_mfma_i32_16x16x32_i8 multiplies 16 rows of eight bytes per lane group with 16 columns of
+ * eight. A lane holds 16 neighbouring columns of every row it loads, so for column j of each lane its eight bytes are the
+ * digits of eight of its own rows: no value crosses lanes on its way in, a 4x4 byte transposition per four rows (8
+ * permutes) and three masks and shifts per word of eight digits make all 16 operands, 0.6 vector instructions per
+ * digit for one input row or two, against 2.6 and 3.6 for conversions and fp32 multiply-adds. The other operand's 16 rows
+ * are the four bytes of two inputs in two scale groups (df_stage_i8); the products are exact, a lane's four sums are the
+ * bytes of one input and are put together in fp32 at the end. Half of the lanes hold an input times the columns of
+ * the other scale group, which nobody reads. 11 sequences, 64 experts top-4, 2048 x 1408: 61 -> 45 us per layer.
+ *
+ * The fp16-input loop's multiply-adds are v_dot2_f32_f16: two products per instruction, exact, summed in fp32. One operand is the
  * pair of digits of a lane's two rows as fp16, built without a conversion: with u = digit + 8 (two's complement
  * nibble xor 8), 0x6400 | u is the fp16 number 1024 + u (even columns, low nibble) and 0x6400 | u << 4 is
  * 1024 + 16 u (odd columns, the nibble stays where it is), so one byte permute puts two bytes of both rows side
  * by side and one and-or per column does the rest: 14 instructions per 16 digits. The other operand is the pair
  * of staged inputs (divided by 16 for the odd columns). What the offsets add -- (1024 + 8) and (64 + 8) times
  * the sum of the staged inputs -- is taken out at the end. The inputs thus carry 11 significant bits. */
-template<bool H, int MT, class PREP, class NEXT0, class NEXT1>
-__device__ __forceinline__ void df_task(const DfArgs &a, const DfT &t, uint2 (&w0)[DF_BATCH], uint2 (&w1)[DF_BATCH], int hsteps,
-                                        const uint32_t *xs_raw, float *red, u64 *dst, size_t mstride,
-                                        PREP prep, NEXT0 next0, NEXT1 next1 DF_TRACE_PARAM){
+template<class PREP, class NEXT0, class NEXT1>
+__device__ __forceinline__ void df_task_i8(const DfArgs &a, const DfT &t, uint2 (&w0)[DF_BATCH], uint2 (&w1)[DF_BATCH], const uint32_t *xs,
+                                           float *red, u64 *dst, size_t mstride, PREP prep, NEXT0 next0, NEXT1 next1 DF_TRACE_PARAM){
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+    const int N = t.N, M = t.M, chunk = t.chunk;
+    DF_STAMP(10 + 16 * t.list);
+    int k[DF_MB]; bool bad[DF_MB];
+    prep(k, bad);
+    DF_STAMP(11);
+    __builtin_amdgcn_s_setprio(0);
+    df_i32x4 acc[16];
+#pragma unroll
+    for(int j = 0; j < 16; j++) acc[j] = (df_i32x4)(0);
+    const uint32_t p = c & 3, s01 = p | (p + 4) << 8 | 0x0C0C0000u, s23 = p << 16 | (p + 4) << 24 | 0x0C0Cu;
+    const uint4 *xr = (const uint4 *)(xs + (c >> 2) * DF_XPLANE + g * 16);
+    auto half = [&](const uint2 (&W)[DF_BATCH], int h){
+        uint32_t xb[2];
+#pragma unroll
+        for(int q = 0; q < 2; q++){
+            const uint4 r = xr[h * 2 + q];
+            xb[q] = __builtin_amdgcn_perm(r.y, r.x, s01) | __builtin_amdgcn_perm(r.w, r.z, s23);
+        }
+        const long x = df_pair(xb[0], xb[1]);
+#pragma unroll
+        for(int xy = 0; xy < 2; xy++){
+            uint32_t t0[4], t1[4];
+            if(xy == 0){ df_bytes(W[0].x, W[1].x, W[2].x, W[3].x, t0); df_bytes(W[4].x, W[5].x, W[6].x, W[7].x, t1); }
+            else       { df_bytes(W[0].y, W[1].y, W[2].y, W[3].y, t0); df_bytes(W[4].y, W[5].y, W[6].y, W[7].y, t1); }
+#pragma unroll
+            for(int q = 0; q < 4; q++){
+                /* a digit as a signed byte, times 16 */
+                const int j = xy * 8 + 2 * q;
+                acc[j]     = __builtin_amdgcn_mfma_i32_16x16x32_i8(x, df_pair((t0[q] << 4) & 0xF0F0F0F0u, (t1[q] << 4) & 0xF0F0F0F0u), acc[j], 0, 0, 0);
+                acc[j + 1] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x, df_pair(t0[q] & 0xF0F0F0F0u, t1[q] & 0xF0F0F0F0u), acc[j + 1], 0, 0, 0);
+            }
+        }
+    };
+    half(w0, 0);
+    next0();
+    DF_STAMP(12);
+    if(t.rows > 16 * DF_BATCH) half(w1, 1);
+    next1();
+    __builtin_amdgcn_s_setprio(3);
+    DF_STAMP(13);
+    __syncthreads();                                      /* the sums of the task before have been read */
+    const int m = g & 1;
+    if((c >= 8) == (g >= 2) && m < M){
+        const int e = -4 - (m ? k[1] : k[0]);
+        const float up = (m ? bad[1] : bad[0]) ? __builtin_nanf("") : 65536.0f;
+        float y[16];
+#pragma unroll
+        for(int j = 0; j < 16; j++){
+            const int hi = (acc[j][3] << 8) + acc[j][2], lo = (acc[j][1] << 8) + acc[j][0];
+            y[j] = __builtin_amdgcn_ldexpf(fmaf((float)hi, up, (float)lo), e);
+        }
+        float4 *o = (float4 *)&red[(wave * DF_MB + m) * DF_CW + c * 16];
+#pragma unroll
+        for(int q = 0; q < 4; q++) o[q] = make_float4(y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]);
+    }
+    __syncthreads();
+    const int col = chunk * DF_CW + tid;
+    if(col < N){
+        for(int m = 0; m < M; m++){
+            const float v = ((red[(0 * DF_MB + m) * DF_CW + tid] + red[(1 * DF_MB + m) * DF_CW + tid])
+                           + red[(2 * DF_MB + m) * DF_CW + tid]) + red[(3 * DF_MB + m) * DF_CW + tid];
+            df_st(dst + (size_t)m * mstride + col, v, a.epoch);
+        }
+    }
+    DF_STAMP(14);
+}
+template<int MT, class PREP, class NEXT0, class NEXT1>
+__device__ __forceinline__ void df_task_h(const DfArgs &a, const DfT &t, uint2 (&w0)[DF_BATCH], uint2 (&w1)[DF_BATCH], int hsteps,
+                                          const uint32_t *xs_raw, float *red, u64 *dst, size_t mstride,
+                                          PREP prep, NEXT0 next0, NEXT1 next1 DF_TRACE_PARAM){
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int cl = lane & 15, rp = wave * 4 + (lane >> 4);
     const int N = t.N, rows = t.rows, M = t.M, chunk = t.chunk;
@@ -553,7 +662,6 @@ __device__ __forceinline__ void df_task(const DfArgs &a, const DfT &t, uint2 (&w
         for(int j = 0; j < 16; j++) acc[m][j] = 0.0f; }
     const uint32_t magic = 0x64006400u;
     const uint32_t (*xs)[DF_RMAX / 2][2 * DF_MB] = (const uint32_t (*)[DF_RMAX / 2][2 * DF_MB])xs_raw;
-    const float (*xf)[DF_RMAX][DF_MB] = (const float (*)[DF_RMAX][DF_MB])xs_raw;
 #define DF_COMPUTE_H(W, h)                                                          \
     _Pragma("unroll")                                                              \
     for(int s_ = 0; s_ < DF_BATCH / 2; s_++){                                      \
@@ -585,31 +693,6 @@ __device__ __forceinline__ void df_task(const DfArgs &a, const DfT &t, uint2 (&w
             }                                                                      \
         }                                                                          \
     }
-    /* The fp32 loop: one row per lane and step, digits to fp32 one by one (v_cvt_f32_ubyteN; the nibble masks go
-     * through df_and so that those converts survive: seen through, the compiler rewrites mask + byte select into
-     * a bit-field extract per digit and doubles the instruction count), 16 fp32 multiply-adds per input row. */
-#define DF_COMPUTE_S(W, h)                                                        \
-    _Pragma("unroll")                                                              \
-    for(int b = 0; b < DF_BATCH; b++){                                             \
-        if(b < hsteps && ((h) * hsteps + b) * 16 < rows){                          \
-            const int r = ((h) * hsteps + b) * 16 + rp;                            \
-            const float2 x2 = *(const float2 *)&xf[gl][r][0];                      \
-            const float xm[DF_MB] = {x2.x, x2.y};                                  \
-            float f[16];                                                           \
-            const uint32_t u0 = W[b].x ^ 0x88888888u, u1 = W[b].y ^ 0x88888888u;   \
-            const uint32_t l0 = df_and(u0), h0 = df_and(u0 >> 4);                  \
-            const uint32_t l1 = df_and(u1), h1 = df_and(u1 >> 4);                  \
-            _Pragma("unroll")                                                      \
-            for(int k = 0; k < 4; k++){ f[2 * k] = ub(l0, k); f[2 * k + 1] = ub(h0, k); f[8 + 2 * k] = ub(l1, k); f[9 + 2 * k] = ub(h1, k); } \
-            _Pragma("unroll")                                                      \
-            for(int m = 0; m < MT; m++){                                           \
-                const float xv = xm[m];                                            \
-                corr[m] += xv;                                                     \
-                _Pragma("unroll")                                                  \
-                for(int j = 0; j < 16; j++) acc[m][j] = fmaf(xv, f[j], acc[m][j]); \
-            }                                                                      \
-        }                                                                          \
-    }
     DF_STAMP(10 + 16 * t.list);
     const float unscale = prep();
     DF_STAMP(11);
@@ -619,15 +702,14 @@ __device__ __forceinline__ void df_task(const DfArgs &a, const DfT &t, uint2 (&w
      * task is not starved by its neighbours' loops (the fourth workgroup of a CU otherwise reached its first task
      * 8 us after the first). */
     __builtin_amdgcn_s_setprio(0);
-    if(H){ DF_COMPUTE_H(w0, 0) } else { DF_COMPUTE_S(w0, 0) }
+    DF_COMPUTE_H(w0, 0)
     next0();
     DF_STAMP(12);
-    if(H){ DF_COMPUTE_H(w1, 1) } else { DF_COMPUTE_S(w1, 1) }
+    DF_COMPUTE_H(w1, 1)
     next1();
     __builtin_amdgcn_s_setprio(3);
     DF_STAMP(13);
 #undef DF_COMPUTE_H
-#undef DF_COMPUTE_S
     /* four row phases of a wave: reduce-scatter over lane bits 5 and 4, then the four waves via LDS */
     const bool hi32 = lane & 32, hi16 = lane & 16;
     __syncthreads();
@@ -635,7 +717,7 @@ __device__ __forceinline__ void df_task(const DfArgs &a, const DfT &t, uint2 (&w
     for(int m = 0; m < MT; m++){
         if(m < M){
             float k8[8], k4[4];
-            const float off_even = (H ? 1032.0f : 8.0f) * corr[m], off_odd = (H ? 72.0f : 8.0f) * corr[m];
+            const float off_even = 1032.0f * corr[m], off_odd = 72.0f * corr[m];
 #pragma unroll
             for(int j = 0; j < 8; j++){
                 const float off = (j & 1) ? off_odd : off_even;
@@ -666,10 +748,9 @@ __device__ __forceinline__ void df_task(const DfArgs &a, const DfT &t, uint2 (&w
 template<bool H>
 __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
     __shared__ DfMeta mt;
-    __shared__ __align__(16) uint32_t xs_raw[DF_NG * DF_RMAX * DF_MB];   /* staged inputs: df_stage (fp16 pairs) or df_stage_f32 */
+    __shared__ __align__(16) uint32_t xs_raw[4 * DF_NG * DF_MB * DF_XPLANE];   /* staged inputs: df_stage (fp16 pairs) or, a quarter per wavefront, df_stage_i8 */
     __shared__ float wmax[4];
     __shared__ DfT tasks[DF_MAXTASKS];
-    __shared__ int wcount[4];
     __shared__ float red[4 * DF_MB * DF_CW];
     __shared__ int giveup;
     const int tid = threadIdx.x;
@@ -693,137 +774,109 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
     const unsigned last = __hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if(tid == 0) giveup = 0;
 
-    /* ---- problem table (identical in every workgroup): rank of pair j among (expert, j) ---- */
-    if(tid < DEC_MAXPAIR){
-        int e = tid < npair ? e_in : 0x7FFFFFFF;
-        if(tid < npair && (unsigned)e >= (unsigned)a.E) e = 0x7FFFFFFE;   /* invalid: sorts after every valid expert */
-        mt.ein[tid] = e;
-    }
-    __syncthreads();
-    {
-        const int j = tid & 63, part = tid >> 6, e = mt.ein[j];
-        int rank = 0;
-        for(int i = part * 16; i < min(npair, part * 16 + 16); i++){
-            const int ei = mt.ein[i];
-            rank += (ei < e) || (ei == e && i < j);
-        }
-        mt.rk[part][j] = rank;
-    }
-    __syncthreads();
-    if(tid < 64){
-        const bool live = tid < npair;
-        const int e = mt.ein[tid];
-        const bool bad = live && e == 0x7FFFFFFE;
-        const int rank = mt.rk[0][tid] + mt.rk[1][tid] + mt.rk[2][tid] + mt.rk[3][tid];
-        if(live){ mt.se[rank] = e; mt.sj[rank] = tid; }
-        if(bad){ mt.pair_prob[tid] = -1; mt.pair_m[tid] = 0; }
-    }
-    __syncthreads();
-    if(tid < 64){
-        const bool live = tid < npair;
-        const int nvalid = __popcll(__ballot(live && mt.ein[tid] != 0x7FFFFFFE));
-        const int r = tid; const bool valid = r < nvalid;
-        const int er = valid ? mt.se[r] : -1;
-        const bool head = valid && (r == 0 || mt.se[r - 1] != er);
-        const u64 upto = r == 63 ? ~0ull : ((2ull << r) - 1ull);
-        const u64 hm = __ballot(head);
-        const int hidx = 63 - __clzll((long long)((hm & upto) | 1ull));
-        const u64 after = hm & ~upto;
-        const int nidx = after ? __ffsll((long long)after) - 1 : nvalid;
-        const int pos = r - hidx, cnt = nidx - hidx;
-        const bool start = valid && (pos % DF_MB == 0);
-        const u64 sm = __ballot(start);
-        const int prob = __popcll(sm & upto) - 1;
-        if(valid){
-            const int j = mt.sj[r];
-            mt.rowpair[r] = j; mt.rowtok[r] = j % a.T; mt.pair_prob[j] = prob; mt.pair_m[j] = pos % DF_MB;
-            if(start){ mt.p_e[prob] = er; mt.p_M[prob] = min(DF_MB, cnt - pos); mt.p_row0[prob] = r; }
-        }
-        if(tid == 0) mt.nprob = __popcll(sm);
-    }
-    __syncthreads();
-    const int nprob = mt.nprob;
-    DF_STAMP(2);
+    /* ---- The problem table (identical in every workgroup) and this workgroup's tasks, by the first wavefront alone, lane =
+     * pair, then candidate: nothing of it meets a barrier before it is all there. (Ranks counted through LDS by four wavefronts,
+     * a sort and a second pass over it, then the list by all threads, with seven barriers between them, stood 4.3 us in
+     * front of the first request with a full grid and 2.5 for a single token; so 2.7 and 2.0.) ---- */
     const int G = gridDim.x, xcd = blockIdx.x & 7, slot0 = blockIdx.x >> 3, nslot = G >> 3;
     const u64 DF = (u64)a.D * a.F;
-
-    /* ---- this workgroup's tasks, list 1 (gate|up) then list 2 (down), in one stream so that the
-     * first digits of a task are already on their way while the task before it finishes ---- */
-    /* Groups -- (problem, matrix) in list 1, problems in list 2 -- go to the XCDs round robin, whole, so that the
-     * scale sectors that a group's column chunks share meet in one L2. The groups left over after the last full
-     * round of 8 would give some XCDs a whole group more than others (a second task for a sixth of their
-     * workgroups while others have none; with a single token: 4 groups, half the device idle), so the chunks of
-     * each of those are cut into `parts` pieces that go to different XCDs (host table by the number left over). */
-    const int ngrp1 = 2 * nprob;
-    const int rem1 = ngrp1 & 7, rem2 = nprob & 7, full1 = ngrp1 - rem1, full2 = nprob - rem2;
-    const int parts1 = (int)((a.parts1 >> (8 * rem1)) & 0xFFu), parts2 = (int)((a.parts2 >> (8 * rem2)) & 0xFFu);
-    const int cpp1 = df_div(a.NC1, parts1, 1.0f / (float)parts1), cpp2 = df_div(a.NC2, parts2, 1.0f / (float)parts2);   /* chunks per piece */
-    const int tpw1 = a.NC1 * a.S1, tpw2 = a.NC2 * a.S2;               /* tasks of a whole group */
-    const int tpg1 = cpp1 * a.S1, tpg2 = cpp2 * a.S2;                 /* tasks of a piece */
-    const int nw1 = (full1 >> 3) * tpw1, nw2 = (full2 >> 3) * tpw2;   /* tasks that whole groups give each XCD */
-    const int nvg1 = rem1 * parts1, nvg2 = rem2 * parts2;             /* pieces */
-    const int lim1 = nw1 + ((nvg1 + 7) >> 3) * tpg1, lim2 = nw2 + ((nvg2 + 7) >> 3) * tpg2;
-    const float rtpw1 = 1.0f / (float)tpw1, rtpw2 = 1.0f / (float)tpw2;
-    const float rtpg1 = 1.0f / (float)tpg1, rtpg2 = 1.0f / (float)tpg2, rS1 = 1.0f / (float)a.S1, rS2 = 1.0f / (float)a.S2;
-    const float rparts1 = 1.0f / (float)parts1, rparts2 = 1.0f / (float)parts2;
-    /* The task list of this workgroup is worked out once, one candidate per thread, and kept in LDS: candidate k
-     * of list 1 is slot slot0 + k * nslot of this XCD's tasks, list 2's follow; candidates that fall behind the
-     * last group of the XCD are dropped and the rest keeps its order. (Worked out one after the other by every
-     * wavefront in front of each task, this arithmetic -- a microsecond of dependent instructions -- stood between
-     * any two tasks.) */
-    const int nc1 = nslot > 0 ? (lim1 - slot0 + nslot - 1) / nslot : 0, nc2 = nslot > 0 ? (lim2 - slot0 + nslot - 1) / nslot : 0;
-    const int c1 = nc1 > 0 ? nc1 : 0, c2 = nc2 > 0 ? nc2 : 0;           /* candidates of the two lists */
-    {
-        DfT t; t.list = 0; t.wq = 0; t.wg = 0; t.N = t.k0 = t.rows = t.chunk = t.M = t.prob = t.mat = t.sl = t.ngl = 0;
-        if(tid < c1){
-            const int q = slot0 + tid * nslot;
-            /* slot q of this XCD: first its whole groups, then its pieces of the groups left over */
-            const bool whole = q < nw1;
-            const int qq = whole ? q : q - nw1, tp = whole ? tpw1 : tpg1;
-            const int qd = df_div(qq, tp, whole ? rtpw1 : rtpg1), vg = qd * 8 + xcd, sub = qq - qd * tp;
-            if(whole || vg < nvg1){
-                const int gp = df_div(vg, parts1, rparts1);
-                const int g = whole ? vg : full1 + gp, part = whole ? 0 : vg - gp * parts1, cl = df_div(sub, a.S1, rS1);
-                t.list = 1; t.prob = g >> 1; t.mat = g & 1; t.chunk = part * cpp1 + cl; t.sl = sub - cl * a.S1;
-                t.N = a.F; t.k0 = t.sl * a.R1; t.rows = min(a.R1, a.D - t.k0); t.M = mt.p_M[t.prob];
-                t.ngl = (ng == 2 && t.N - t.chunk * DF_CW > a.group) ? 2 : 1;
-                const int ex = mt.p_e[t.prob];
-                t.wq = (t.mat ? a.w3q : a.w1q) + (u64)ex * DF;
-                t.wg = (t.mat ? a.w3g : a.w1g) + (u64)ex * a.dfg;
-            }
-        } else if(tid < c1 + c2){
-            const int q = slot0 + (tid - c1) * nslot;
-            const bool whole = q < nw2;
-            const int qq = whole ? q : q - nw2, tp = whole ? tpw2 : tpg2;
-            const int qd = df_div(qq, tp, whole ? rtpw2 : rtpg2), vg = qd * 8 + xcd, sub = qq - qd * tp;
-            if(whole || vg < nvg2){
-                const int gp = df_div(vg, parts2, rparts2);
-                const int prob = whole ? vg : full2 + gp, part = whole ? 0 : vg - gp * parts2, cl = df_div(sub, a.S2, rS2);
-                t.list = 2; t.prob = prob; t.mat = 0; t.chunk = part * cpp2 + cl; t.sl = sub - cl * a.S2;
-                t.N = a.D; t.k0 = t.sl * a.R2; t.rows = min(a.R2, a.F - t.k0); t.M = mt.p_M[prob];
-                t.ngl = (ng == 2 && t.N - t.chunk * DF_CW > a.group) ? 2 : 1;
-                const int ex = mt.p_e[prob];
-                t.wq = a.w2q + (u64)ex * DF;
-                t.wg = a.w2g + (u64)ex * a.dfg;
-            }
+    if(tid < 64){
+        const bool live = tid < npair, valid = live && (unsigned)e_in < (unsigned)a.E;
+        /* the valid pairs of the same expert: equal in every bit of the expert's number */
+        u64 peers = __ballot(valid);
+        for(int b = 0; (a.E - 1) >> b; b++){
+            const bool bit = (e_in >> b) & 1;
+            const u64 set = __ballot(bit);
+            peers &= bit ? set : ~set;
         }
-        /* keep the live ones, in order: rank inside the wavefront by a ballot, wavefronts added up through LDS */
-        const u64 bal = __ballot(t.list != 0);
-        const int lane = tid & 63, wv = tid >> 6;
-        if(lane == 0) wcount[wv] = __popcll(bal);
-        __syncthreads();
-        int base = 0;
-        for(int w = 0; w < wv; w++) base += wcount[w];
-        if(t.list != 0){
-            const int pos = base + __popcll(bal & ((1ull << lane) - 1ull));
-            if(pos < DF_MAXTASKS) tasks[pos] = t;
+        const u64 before = peers & ((1ull << tid) - 1ull);
+        const int pos = __popcll(before), m = pos % DF_MB;
+        const u64 starts = __ballot(valid && m == 0);
+        /* problems are numbered by their first pair; a second pair follows the pair of its expert before it */
+        const int first = m == 0 ? tid : 63 - __clzll((long long)(before | 1ull));
+        const int prob = __popcll(starts & ((1ull << first) - 1ull));
+        if(valid){
+            mt.p_tok[prob][m] = tid - df_div(tid, a.T, 1.0f / (float)a.T) * a.T;
+            if(m == 0){ mt.p_e[prob] = e_in; mt.p_M[prob] = min(DF_MB, __popcll(peers) - pos); }
         }
-        __syncthreads();
+        if(live){ mt.pair_prob[tid] = valid ? prob : -1; mt.pair_m[tid] = valid ? m : 0; }
+        const int nprob = __popcll(starts);
+        /* ---- this workgroup's tasks, list 1 (gate|up) then list 2 (down), in one stream so that the
+         * first digits of a task are already on their way while the task before it finishes ---- */
+        /* Groups -- (problem, matrix) in list 1, problems in list 2 -- go to the XCDs round robin, whole, so that the
+         * scale sectors that a group's column chunks share meet in one L2. The groups left over after the last full
+         * round of 8 would give some XCDs a whole group more than others (a second task for a sixth of their
+         * workgroups while others have none; with a single token: 4 groups, half the device idle), so the chunks of
+         * each of those are cut into `parts` pieces that go to different XCDs (host table by the number left over). */
+        const int ngrp1 = 2 * nprob;
+        const int rem1 = ngrp1 & 7, rem2 = nprob & 7, full1 = ngrp1 - rem1, full2 = nprob - rem2;
+        const int parts1 = (int)((a.parts1 >> (8 * rem1)) & 0xFFu), parts2 = (int)((a.parts2 >> (8 * rem2)) & 0xFFu);
+        const int cpp1 = df_div(a.NC1, parts1, 1.0f / (float)parts1), cpp2 = df_div(a.NC2, parts2, 1.0f / (float)parts2);   /* chunks per piece */
+        const int tpw1 = a.NC1 * a.S1, tpw2 = a.NC2 * a.S2;               /* tasks of a whole group */
+        const int tpg1 = cpp1 * a.S1, tpg2 = cpp2 * a.S2;                 /* tasks of a piece */
+        const int nw1 = (full1 >> 3) * tpw1, nw2 = (full2 >> 3) * tpw2;   /* tasks that whole groups give each XCD */
+        const int nvg1 = rem1 * parts1, nvg2 = rem2 * parts2;             /* pieces */
+        const int lim1 = nw1 + ((nvg1 + 7) >> 3) * tpg1, lim2 = nw2 + ((nvg2 + 7) >> 3) * tpg2;
+        const float rtpw1 = 1.0f / (float)tpw1, rtpw2 = 1.0f / (float)tpw2;
+        const float rtpg1 = 1.0f / (float)tpg1, rtpg2 = 1.0f / (float)tpg2, rS1 = 1.0f / (float)a.S1, rS2 = 1.0f / (float)a.S2;
+        const float rparts1 = 1.0f / (float)parts1, rparts2 = 1.0f / (float)parts2;
+        /* The task list of this workgroup is worked out once, one candidate per lane, and kept in LDS: candidate k
+         * of list 1 is slot slot0 + k * nslot of this XCD's tasks, list 2's follow; candidates that fall behind the
+         * last group of the XCD are dropped and the rest keeps its order. (Worked out one after the other by every
+         * wavefront in front of each task, this arithmetic -- a microsecond of dependent instructions -- stood between
+         * any two tasks.) */
+        const float rnslot = 1.0f / (float)nslot;                         /* the grid is a multiple of 8 and at least 8; slot0 < nslot */
+        const int c1 = df_div(lim1 - slot0 + nslot - 1, nslot, rnslot), c2 = df_div(lim2 - slot0 + nslot - 1, nslot, rnslot);   /* candidates of the two lists */
+        int n = 0;
+        for(int base = 0; base < c1 + c2; base += 64){
+            const int k = base + tid;
+            DfT t; t.list = 0; t.wq = 0; t.wg = 0; t.N = t.k0 = t.rows = t.chunk = t.M = t.prob = t.mat = t.sl = t.ngl = 0;
+            if(k < c1){
+                const int q = slot0 + k * nslot;
+                /* slot q of this XCD: first its whole groups, then its pieces of the groups left over */
+                const bool whole = q < nw1;
+                const int qq = whole ? q : q - nw1, tp = whole ? tpw1 : tpg1;
+                const int qd = df_div(qq, tp, whole ? rtpw1 : rtpg1), vg = qd * 8 + xcd, sub = qq - qd * tp;
+                if(whole || vg < nvg1){
+                    const int gp = df_div(vg, parts1, rparts1);
+                    const int g = whole ? vg : full1 + gp, part = whole ? 0 : vg - gp * parts1, cl = df_div(sub, a.S1, rS1);
+                    t.list = 1; t.prob = g >> 1; t.mat = g & 1; t.chunk = part * cpp1 + cl; t.sl = sub - cl * a.S1;
+                    t.N = a.F; t.k0 = t.sl * a.R1; t.rows = min(a.R1, a.D - t.k0); t.M = mt.p_M[t.prob];
+                    t.ngl = (ng == 2 && t.N - t.chunk * DF_CW > a.group) ? 2 : 1;
+                    const int ex = mt.p_e[t.prob];
+                    t.wq = (t.mat ? a.w3q : a.w1q) + (u64)ex * DF;
+                    t.wg = (t.mat ? a.w3g : a.w1g) + (u64)ex * a.dfg;
+                }
+            } else if(k < c1 + c2){
+                const int q = slot0 + (k - c1) * nslot;
+                const bool whole = q < nw2;
+                const int qq = whole ? q : q - nw2, tp = whole ? tpw2 : tpg2;
+                const int qd = df_div(qq, tp, whole ? rtpw2 : rtpg2), vg = qd * 8 + xcd, sub = qq - qd * tp;
+                if(whole || vg < nvg2){
+                    const int gp = df_div(vg, parts2, rparts2);
+                    const int prob = whole ? vg : full2 + gp, part = whole ? 0 : vg - gp * parts2, cl = df_div(sub, a.S2, rS2);
+                    t.list = 2; t.prob = prob; t.mat = 0; t.chunk = part * cpp2 + cl; t.sl = sub - cl * a.S2;
+                    t.N = a.D; t.k0 = t.sl * a.R2; t.rows = min(a.R2, a.F - t.k0); t.M = mt.p_M[prob];
+                    t.ngl = (ng == 2 && t.N - t.chunk * DF_CW > a.group) ? 2 : 1;
+                    const int ex = mt.p_e[prob];
+                    t.wq = a.w2q + (u64)ex * DF;
+                    t.wg = a.w2g + (u64)ex * a.dfg;
+                }
+            }
+            /* keep the live ones, in order */
+            const u64 bal = __ballot(t.list != 0);
+            const int at = n + __popcll(bal & ((1ull << tid) - 1ull));
+            if(t.list != 0 && at < DF_MAXTASKS) tasks[at] = t;
+            n += __popcll(bal);
+        }
+        if(tid == 0){ mt.ntasks = min(DF_MAXTASKS, n); mt.full = lim1 * 2 > nslot; }
     }
+    __syncthreads();
+    DF_STAMP(2);
     /* the tag is first needed when a partial sum is stored: its load (past the caches) has had the table and the
      * task list to come back */
     a.epoch = __builtin_amdgcn_readfirstlane(last == 0xFFFFFFFFu ? 1u : last + 1u);
-    const int ntasks = min(DF_MAXTASKS, wcount[0] + wcount[1] + wcount[2] + wcount[3]);
+    const int ntasks = mt.ntasks;
     int ti = 0;
     auto fetch = [&]() -> DfT {
         DfT t; t.list = 0; t.wq = 0; t.wg = 0; t.N = t.k0 = t.rows = t.chunk = t.M = t.prob = t.mat = t.sl = t.ngl = 0;
@@ -837,7 +890,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
         return t;
     };
     uint2 w0[DF_BATCH], w1[DF_BATCH];
-    const int hs1 = a.R1 >> (H ? 6 : 5), hs2 = a.R2 >> (H ? 6 : 5);   /* steps (of 32 rows, fp32 loop: 16) per half task */
+    const int hs1 = a.R1 >> 6, hs2 = a.R2 >> 6;              /* fp16-input loop: steps of 32 rows per half task */
     const int gprF = a.F / a.group, gprD = a.D / a.group;     /* scale groups per row of w1|w3 and of w2 */
     const int cpg = a.group >= DF_CW ? a.group / DF_CW : 1;   /* chunks per scale group when the group is wider than a chunk */
     /* first scale of a task: its first row, its chunk's first group */
@@ -845,11 +898,15 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
         const int cg = a.group >= DF_CW ? t.chunk / cpg : t.chunk * (DF_CW / a.group);
         return a.s + t.wg + (size_t)t.k0 * (t.list == 1 ? gprF : gprD) + cg;
     };
-    /* The group scales of row `tid` of a task, requested together with the task's digits -- a task ahead -- so
+    /* the row of a task that this thread stages (the last one for threads beyond them) */
+    auto row_of = [&](const DfT &t) -> int {
+        return H ? min(tid, t.rows - 1) : (tid >> 6) * (t.rows >> 2) + min(tid & 63, (t.rows >> 2) - 1);
+    };
+    /* The group scales of that row, requested together with the task's digits -- a task ahead -- so
      * that the staging finds them in registers instead of waiting for HBM. Requested without conditions (a
      * dead position re-reads a live one); the staging zeroes what lies outside the matrix. */
     auto scales_ahead = [&](const DfT &t, float (&sc)[DF_NG]){
-        const float *sp = scales_of(t) + (size_t)min(tid, t.rows - 1) * (t.list == 1 ? gprF : gprD);
+        const float *sp = scales_of(t) + (size_t)row_of(t) * (t.list == 1 ? gprF : gprD);
 #pragma unroll
         for(int gg = 0; gg < DF_NG; gg++) sc[gg] = sp[gg < t.ngl ? gg : 0];   /* a group past the row's end re-reads the first */
     };
@@ -881,18 +938,18 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
         u64 *dst; size_t mstride;
         if(cur.list == 1){ dst = a.part1 + ((((size_t)prob * 2 + cur.mat) * a.S1 + cur.sl) * DF_MB) * a.F; mstride = (size_t)a.F; }
         else             { dst = a.part2 + (((size_t)prob * a.S2 + cur.sl) * DF_MB) * a.D;                  mstride = (size_t)a.D; }
-        auto prep = [&]() -> float {
+        /* one scale group per chunk: the matrix-core loop wants it in both halves (csc[1] is the first then) */
+        auto inputs = [&](float (&v)[DF_NG][DF_MB]) -> bool {
             /* thread = row of the task (rows <= DF_RMAX = the threads) */
-            const int r = tid; const bool live = r < rows;
-            float v[DF_NG][DF_MB];
+            const int r = row_of(cur); const bool live = H ? tid < rows : (tid & 63) < (rows >> 2);
             if(cur.list == 1){
                 float xv[DF_MB];
 #pragma unroll
                 for(int m = 0; m < DF_MB; m++)
-                    xv[m] = (live && m < M) ? a.x[(size_t)mt.rowtok[mt.p_row0[prob] + m] * a.D + k0 + r] : 0.0f;
+                    xv[m] = (live && m < M) ? a.x[(size_t)mt.p_tok[prob][m] * a.D + k0 + r] : 0.0f;
 #pragma unroll
                 for(int gg = 0; gg < DF_NG; gg++){
-                    const float sc = (gg < ng && chunk * DF_CW + gg * a.group < a.F) ? csc[gg] : 0.0f;
+                    const float sc = (gg < ng ? chunk * DF_CW + gg * a.group < a.F : !H) ? csc[gg] : 0.0f;
 #pragma unroll
                     for(int m = 0; m < DF_MB; m++) v[gg][m] = xv[m] * sc;
                 }
@@ -902,7 +959,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                 /* with a full grid, one polling thread per producer first (everybody re-reading its sums until they
                  * are there slows the producers down: T=16 +0.6 us per layer); with few workgroups the poll and its
                  * barrier only add to the chain (T=1, 4: -0.3 us without) */
-                if(lim1 * 2 > nslot) df_wait_first(2 * a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, [=](int i){ return p1 + (size_t)i * sstride; });
+                if(mt.full) df_wait_first(2 * a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, [=](int i){ return p1 + (size_t)i * sstride; });
                 float hv[DF_MB];
 #pragma unroll
                 for(int m = 0; m < DF_MB; m++) hv[m] = 0.0f;
@@ -925,17 +982,23 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                 }
 #pragma unroll
                 for(int gg = 0; gg < DF_NG; gg++){
-                    const float sc = (gg < ng && chunk * DF_CW + gg * a.group < a.D) ? csc[gg] : 0.0f;
+                    const float sc = (gg < ng ? chunk * DF_CW + gg * a.group < a.D : !H) ? csc[gg] : 0.0f;
 #pragma unroll
                     for(int m = 0; m < DF_MB; m++) v[gg][m] = hv[m] * sc;
                 }
             }
-            if(H) return df_stage(v, live, (uint32_t (*)[DF_RMAX / 2][2 * DF_MB])xs_raw, wmax);
-            return df_stage_f32(v, live, (float (*)[DF_RMAX][DF_MB])xs_raw);
+            return live;
         };
-        /* the inner loop is compiled for 1 and 2 input rows */
-        if(M == 1) df_task<H, 1>(a, cur, w0, w1, hs, xs_raw, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
-        else       df_task<H, 2>(a, cur, w0, w1, hs, xs_raw, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
+        if constexpr(H){
+            auto prep = [&]() -> float { float v[DF_NG][DF_MB]; const bool live = inputs(v); return df_stage(v, live, (uint32_t (*)[DF_RMAX / 2][2 * DF_MB])xs_raw, wmax); };
+            /* the inner loop is compiled for 1 and 2 input rows */
+            if(M == 1) df_task_h<1>(a, cur, w0, w1, hs, xs_raw, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
+            else       df_task_h<2>(a, cur, w0, w1, hs, xs_raw, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
+        } else {
+            uint32_t *xs = xs_raw + (tid >> 6) * (DF_NG * DF_MB * DF_XPLANE);
+            auto prep = [&](int (&k)[DF_MB], bool (&bad)[DF_MB]){ float v[DF_NG][DF_MB]; inputs(v); df_stage_i8(v, xs, k, bad); };
+            df_task_i8(a, cur, w0, w1, xs, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
+        }
         cur = nxt;
 #pragma unroll
         for(int gg = 0; gg < DF_NG; gg++) csc[gg] = nsc[gg];
@@ -1074,19 +1137,18 @@ static int df_rows_down(int Kdim, double tasks_per_slice, int grid){
     return R;
 }
 
-/* Which multiply loop the decode layer runs. fp32 (the default): inputs as they are, 2.6 / 3.6 vector
- * instructions per digit for one / two input rows, 4e-7 relative L2 on a layer's output against the fp32 oracle.
- * fp16 inputs: the staged inputs as fp16 pairs and v_dot2_f32_f16, 1.4 / 2.0 instructions per digit, inputs
- * rounded to 11 bits (3.7e-4), 1-4 % faster per layer (the layer is bound by its chain of hand-overs and by HBM,
- * not by this loop). QLMX_DECODE_MATH=fp16 in the environment (read at the first call) or qlmx_decode_math(1)
- * selects the fp16 loop, qlmx_decode_math(0) the fp32 one. */
+/* Which multiply loop the decode layer runs. The matrix-core loop (the default): inputs in 31-bit fixed point, exact
+ * products, as close to the fp32 oracle as fp32 multiply-adds are. fp16 inputs: the staged inputs as fp16 pairs and
+ * v_dot2_f32_f16, 1.4 / 2.0 instructions per digit for one / two input rows, inputs rounded to 11 bits (3.7e-4); it was
+ * the faster one beside the fp32 loop of before and is kept for callers that select it. QLMX_DECODE_MATH=fp16 in the
+ * environment (read at the first call) or qlmx_decode_math(1) selects the fp16 loop, qlmx_decode_math(0) the default. */
 static int g_df_math = -1;
 static bool df_math_fp16(){
     if(g_df_math < 0){ const char *e = getenv("QLMX_DECODE_MATH"); g_df_math = (e && !strcmp(e, "fp16")) ? 1 : 0; }
     return g_df_math != 0;
 }
 extern "C" int qlmx_decode_math(int fp16_inputs){
-    QLMX_REQUIRE(fp16_inputs == 0 || fp16_inputs == 1, "qlmx_decode_math: 0 (fp32 loop) or 1 (fp16 inputs), not %d", fp16_inputs);
+    QLMX_REQUIRE(fp16_inputs == 0 || fp16_inputs == 1, "qlmx_decode_math: 0 (fp32 inputs) or 1 (fp16 inputs), not %d", fp16_inputs);
     g_df_math = fp16_inputs;
     return QLMX_OK;
 }

@@ -393,11 +393,11 @@ int qlmx_test_force_wait_timeout(int which);
  * from outside the process. */
 int qlmx_nt_tile(int tile);
 /* Math mode of the decode layer (no counterpart in the reference, whose decode path multiplies in fp32; the same
- * kind of choice as QLMX_MATH_MFMA_F16 for the training forward). fp16_inputs = 0, the default: the fp32 loop,
- * 4e-7 relative L2 on a layer's output against the fp32 reference. fp16_inputs = 1: a task's inputs (x times the
+ * kind of choice as QLMX_MATH_MFMA_F16 for the training forward). fp16_inputs = 0, the default: inputs to fp32
+ * precision, 4e-7 relative L2 on a layer's output against the fp32 reference. fp16_inputs = 1: a task's inputs (x times the
  * group scale, or silu(gate) * up times the group scale) are rounded to fp16 -- 11 significant bits, scaled per
  * task so that nothing underflows -- and multiplied with the exact digits by v_dot2_f32_f16 into fp32 sums:
- * 3.7e-4, and 1-4 % faster per layer. Applies to both decode entry points from the next call on;
+ * 3.7e-4. Applies to both decode entry points from the next call on;
  * QLMX_DECODE_MATH=fp16 in the environment is the same switch from outside the process. */
 int qlmx_decode_math(int fp16_inputs);
 /* Test hook. qlmx_step takes the square roots of the second moment with a short form of the correctly rounded

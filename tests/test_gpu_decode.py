@@ -263,3 +263,29 @@ def test_decode_limits(q):
         q.decode_forward(z, zi, z, z, z, z, 128, 0, 0, 0, 64, 2, 4, 128, 128)
     with pytest.raises(pkg.QlmxError, match="multiples of 32"):
         q.decode_forward(z, zi, z, z, z, z, 128, 0, 0, 0, 2, 2, 4, 100, 128)
+
+
+@pytest.mark.parametrize("D,F,group", [(128, 128, 128), (384, 640, 128), (256, 768, 256), (896, 512, 128)])
+def test_decode_inputs_of_very_different_size(q, orc, D, F, group):
+    """The default loop brings a task's inputs to a common fixed point: tokens that are tiny or huge, one value far above the
+    rest, all zeros, or not a number share experts (and problems of two) with ordinary ones, and each is held to the bound by
+    itself; widths that end inside a task's rows and columns."""
+    import torch
+    q.call("qlmx_decode_math", 0)
+    T, E, K = 7, 2, 2
+    d, s, P, n = encode_layer(orc, 31, E, D, F, group)
+    x = orc.normal(T * D, 31, 2).reshape(T, D)
+    x[1] *= f32(1e-18); x[2] *= f32(1e12); x[3, D // 3] = 3e4; x[4] = 0.0
+    asn = np.array([0, 0, 0, 1, 1, 1, 0] + [1, 1, 1, 0, 0, 0, 1], np.int32)
+    gate = np.full(K * T, 0.5, f32)
+    want = np.zeros(T * D, f32)
+    rc, ws = orc.moe_forward(x.reshape(-1), P[:n], P[n:2 * n], P[2 * n:], asn, gate, want, T, D, F, E, K)
+    orc.moe_ws_free(ws)
+    want = want.reshape(T, D)
+    x[6, 5] = np.nan
+    out = torch.zeros(T, D, device="cuda")
+    q.decode_forward(dev(x), dev(asn), dev(gate), out, dev(d), dev(s), group, 0, n, 2 * n, T, K, E, D, F)
+    got = out.cpu().numpy()
+    for t in (0, 1, 2, 3, 5):
+        assert orc.relerr(got[t], want[t]) < 2e-5, t
+    assert not got[4].any() and np.isnan(got[6]).all()
