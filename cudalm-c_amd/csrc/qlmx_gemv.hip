@@ -350,13 +350,14 @@ struct DfArgs {
     u64 *part1, *part2; unsigned epoch; unsigned *status;
     unsigned wait_xor; int spin_limit;   /* waits look for epoch ^ wait_xor (0) for at most spin_limit polls; the time-out test changes both */
     unsigned *ctl;            /* device words: [0] tag of the last finished call, [1] workgroups of this call that are done */
+    int full_at;              /* tasks per XCD */
     u64 parts1, parts2;       /* byte n: pieces a group's chunks are cut into when n groups are left over after the last round of 8 (a table in a
                                  word: indexing an array inside the kernel arguments would move them all to scratch memory) */
 };
 
 struct DfMeta {
     int ntasks;
-    bool full;                                                            /* list 1 gives most workgroups a task */
+    bool full;                                                            /* list 1 has tasks for half of the workgroups that fit */
     int p_e[DEC_MAXPAIR], p_M[DEC_MAXPAIR], p_tok[DEC_MAXPAIR][DF_MB];    /* a problem's expert, pairs, their tokens */
     int pair_prob[DEC_MAXPAIR], pair_m[DEC_MAXPAIR];                      /* a pair's problem (-1: no such expert) and place in it */
 };
@@ -869,7 +870,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
             if(t.list != 0 && at < DF_MAXTASKS) tasks[at] = t;
             n += __popcll(bal);
         }
-        if(tid == 0){ mt.ntasks = min(DF_MAXTASKS, n); mt.full = lim1 * 2 > nslot; }
+        if(tid == 0){ mt.ntasks = min(DF_MAXTASKS, n); mt.full = lim1 > a.full_at; }
     }
     __syncthreads();
     DF_STAMP(2);
@@ -957,8 +958,8 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                 const u64 *p1 = a.part1 + (((size_t)prob * 2) * a.S1 * DF_MB) * a.F + k0;
                 const size_t sstride = (size_t)DF_MB * a.F;
                 /* with a full grid, one polling thread per producer first (everybody re-reading its sums until they
-                 * are there slows the producers down: T=16 +0.6 us per layer); with few workgroups the poll and its
-                 * barrier only add to the chain (T=1, 4: -0.3 us without) */
+                 * are there slows the producers down: without it sixteen tokens take 31 us per layer instead of 28);
+                 * with few workgroups the poll and its barrier only add to the chain (two tokens 15.9 us against 15.2) */
                 if(mt.full) df_wait_first(2 * a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, [=](int i){ return p1 + (size_t)i * sstride; });
                 float hv[DF_MB];
 #pragma unroll
@@ -975,7 +976,8 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                     }
                     float gu[2 * DF_MB];
                     if(a.S1 <= 3) df_sum_wait<2 * DF_MB, 3>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
-                    else          df_sum_wait<2 * DF_MB, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                    else if(a.S1 == 5 || a.S1 == 6) df_sum_wait<2 * DF_MB, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                    else          df_sum_wait<2 * DF_MB, 4>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
 #pragma unroll
                     for(int m = 0; m < DF_MB; m++)
                         if(m < M) hv[m] = (gu[2 * m] / (1.0f + expf(-gu[2 * m]))) * gu[2 * m + 1];
@@ -1022,7 +1024,8 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                     const u64 *const src[2] = { a.part2 + (((size_t)mt.pair_prob[ja] * a.S2) * DF_MB + mt.pair_m[ja]) * a.D + col,
                                                 a.part2 + (((size_t)mt.pair_prob[jb] * a.S2) * DF_MB + mt.pair_m[jb]) * a.D + col };
                     float y[2];
-                    df_sum_wait<2, 12>(src, (size_t)DF_MB * a.D, a.S2, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, y);
+                    if(a.S2 <= 4) df_sum_wait<2, 4>(src, (size_t)DF_MB * a.D, a.S2, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, y);
+                    else          df_sum_wait<2, 8>(src, (size_t)DF_MB * a.D, a.S2, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, y);
                     if(prob0 >= 0) o = o + a.gate[j0] * y[0];
                     if(prob1 >= 0) o = o + a.gate[j1] * y[1];
                 }
@@ -1123,13 +1126,14 @@ static int df_rows(int Kdim, double tasks_per_slice, int grid){
     while((Kdim + R - 1) / R > 32 && R < DF_RMAX) R <<= 1;
     return R;
 }
-/* Rows per task of list 2 (a multiple of 64, two halves of whole 32-row steps): as many slices of the contraction as still leave one task per
- * resident workgroup -- a second round of tasks would double the list's time -- but at most 12, which is what
- * the combine reads in one round trip, and none shorter than 64 rows. */
+/* Rows per task of list 2 (a multiple of 64): four slices of the contraction where 256 rows a slice would be fewer, but no
+ * more than still leave one task per resident workgroup, and none shorter than 64 rows. Every slice is one more sum for the
+ * combine to wait for and one more task of the fixed costs; with up to 12 (one task per workgroup at T=16) 8 tokens, 16
+ * experts top-4, 1920 x 768 took 31.9 us per layer, with four 26.5; 16 tokens, 32 experts top-2, 768 x 2048 29.2 and 28.2. */
 static int df_rows_down(int Kdim, double tasks_per_slice, int grid){
     int S = tasks_per_slice > 0.0 ? (int)(0.95 * grid / tasks_per_slice) : 1;
     const int smin = (Kdim + DF_RMAX - 1) / DF_RMAX, smax = Kdim >= 64 ? Kdim / 64 : 1;
-    if(S > 12) S = 12;
+    if(S > 4) S = 4;
     if(S > smax) S = smax;
     if(S < smin) S = smin;
     int R = ((Kdim + S - 1) / S + 63) & ~63;
@@ -1208,6 +1212,7 @@ static int df_forward(bool fixed, const char *who, const float *x, const int *as
             return best; };
         a.parts1 |= (u64)pieces(a.NC1) << (8 * n); a.parts2 |= (u64)pieces(a.NC2) << (8 * n);
     }
+    a.full_at = dv.grid / 16;
     a.status = dv.status; a.epoch = 0;
     a.wait_xor = 0; a.spin_limit = DF_SPIN_LIMIT;
     if(qlmx_test_take_forced_timeout(1)){ a.wait_xor = 0x40000000u; a.spin_limit = 0; }
