@@ -4,8 +4,8 @@
  * The tiled kernels (qlmx_gemm_nn_h.hip, qlmx_gemm_tn_body.h) give a workgroup a column strip of an expert and the
  * whole contraction, one LDS tile and one barrier per 32 of it. With a dozen rows a step is some 1000 cycles of
  * LDS, barrier and issue latency around four matrix products, and a call has too few strips to hide it: 36 us for the
- * down projection of 32 experts (2048 x 768, 12 rows each), whose 25 MB of weights take 5. Here nothing passes
- * meets a barrier on the way in, four wavefronts split the contraction and add up at the end:
+ * down projection of 32 experts (2048 x 768, 12 rows each), whose 25 MB of weights take 5. Here nothing meets
+ * a barrier on the way in, four wavefronts split the contraction and add up at the end:
  *
  * A wavefront owns 128 (64) columns and its share of the contraction. v_mfma_f32_16x16x32 wants eight consecutive k of one
  * column per lane (lane = column lane%16, k group lane/16). Weights of the forward lie along the columns: the lane
@@ -19,10 +19,12 @@
  *
  * Which calls come here (qlmx_small_rows): all whose problems have at most 32 rows, and those that would leave the tiled
  * kernels with few workgroups, each walking the whole contraction at 0.3 (64 rows) to 0.7 us (256) per 32 of it. Counted in
- * tiles of 64 rows: forward, 128 columns, up to 256 tiles, 512 where the contraction is twice the width (a wide gate | up
- * has tiles enough for the tiled kernel); input gradient, 64 columns, up to 512, 1024 where the contraction is twice the
- * width. Around these lines both take about the same time. The forward's rule looks at what the forms of a call that are documented to agree bit for bit have in common -- with and without gather,
- * SwiGLU, scatter -- so that they run the same arithmetic in the same order.
+ * tiles of 64 rows: forward, 128 columns, up to 256 tiles where the contraction is not shorter than the width and up to 512
+ * where it is twice as long (a wide gate | up has tiles enough for the tiled kernel), and any number where one row tile
+ * holds every problem and the contraction is long (64 experts of 40 rows, 2048 x 1408: 102 -> 82 us and 48 -> 41); input
+ * gradient, 64 columns, up to 512, 1024 where the contraction is twice the width. Around these lines both take about the
+ * same time. The forward's rule looks at what the forms of a call that are documented to agree bit for bit have in common
+ * -- with and without gather, SwiGLU, scatter -- so that they run the same arithmetic in the same order.
  * us per call, tiled kernels -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16
  * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
@@ -65,7 +67,7 @@ bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, in
     if(most <= 32) return true;
     if(mode == GEMM_NN){
         tiles *= N / SM_COLS;
-        return (tiles <= 256 && K >= N) || (tiles <= 512 && K >= 2 * N);
+        return (most <= 64 && K > 1024) || (tiles <= 256 && K >= N) || (tiles <= 512 && K >= 2 * N);
     }
     tiles *= N / SM_TCOLS;
     return tiles <= 512 || (tiles <= 1024 && (long long)K * nseg >= 2 * N);
