@@ -153,61 +153,72 @@ __device__ void servo_pairs(const GroupLoc &L, int gi, int tl, signed char *d, s
         if(packed) d[(L.qi0 + jb) >> 1] = (signed char)(((dn[1] & 15) << 4) | (dn[0] & 15));
     }
 }
-/* how many of w's eight nibbles equal those of `of` */
-__device__ __forceinline__ int nibbles_equal(uint32_t w, uint32_t of){
-    uint32_t x = w ^ of;
-    x |= x >> 2; x |= x >> 1;
-    return 8 - __popc(x & 0x11111111u);
+/* adds to n how many of w's eight nibbles equal those of `up` or of `down` (which differ) */
+__device__ __forceinline__ int nibbles_equal(uint32_t w, uint32_t up, uint32_t down, int n){
+    uint32_t x = w ^ up, y = w ^ down;
+    x |= x >> 2; y |= y >> 2;
+    x |= x >> 1; y |= y >> 1;
+    return n + __popc(~(x & y) & 0x11111111u);
 }
-/* Full aligned groups of 8 W go 8 consecutive elements per lane: one 32-bit word of digits, and 8 residual bytes only
- * where the group is rescaled. What bounds the kernel is vector instructions, not HBM. A workgroup counts G groups per
- * team, their loads side by side, and lists the few that move; its teams then share the list,
- * so that re-encoding (160 instructions) runs for wavefronts full of moving groups instead of for every wavefront with
- * one among its four. 151 M weights, 15 % of the groups moving: 119 us with one group per row from start to end, 77
- * with four. Few groups leave most CUs empty at four per team, and there only the chain counts: one per team. */
-template<int W, int G>
+/* Full aligned groups of 8 W are counted by Q lanes with one load of digits each, G groups per team with their loads side
+ * by side. A workgroup lists the few groups that move; teams of W lanes then share the list and re-encode 8
+ * consecutive elements per lane (160 instructions), in wavefronts full of moving groups, and take the groups of any other
+ * shape a pair per lane. What bounds the kernel is the two round trips of a workgroup, not HBM. 151 M weights, 15 % of the
+ * groups moving: 119 us with one group per row of 16 lanes from start to end, 77 with the list and four groups per row,
+ * 44 with 16-byte loads (Q = W / 4) and two groups per team; below a million groups one (64 K groups, all three codec calls 24.5
+ * against 26.4 us). Few groups leave most CUs empty that way, and there only the chain counts: Q = W and one group per team
+ * (20 K groups 6.8 us, 7.5 to 8.7 the other way). */
+template<int W, int Q, int G>
 __global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char *r, float *s,
                                                     const qlmx_span *sp, int nspan, int group, int dmax,
                                                     float f_hi, float f_lo, int packed, int ngrp, int vec_ok){
-    constexpr int TEAMS = 256 / W;
-    __shared__ uint64_t at[TEAMS * G];                     /* the moving groups: first element, old scale / new scale */
-    __shared__ float conv[TEAMS * G];
-    __shared__ int moving;
-    const int tl = threadIdx.x & (W - 1), team = threadIdx.x / W, first = (int)blockIdx.x * (TEAMS * G) + team;
-    if(threadIdx.x == 0) moving = 0;
-    const int s0 = qx_span_of_teams<64 / W>(sp, nspan, __builtin_amdgcn_readfirstlane(first), (threadIdx.x & 63) / W);
+    constexpr int NW = W / Q, COUNTERS = 256 / Q, TEAMS = 256 / W;
+    struct __attribute__((packed, aligned(4))) Words { uint32_t w[NW]; };
+    __shared__ uint64_t at[COUNTERS * G];                  /* the moving groups: first element, old scale / new scale */
+    __shared__ float conv[COUNTERS * G];
+    __shared__ int other[COUNTERS * G];                    /* the groups of other shapes */
+    __shared__ int moving, others;
+    const int ql = threadIdx.x & (Q - 1), first = (int)blockIdx.x * (COUNTERS * G) + (int)threadIdx.x / Q;
+    if(threadIdx.x == 0) moving = others = 0;
+    const int s0 = qx_span_of_teams<64 / Q>(sp, nspan, __builtin_amdgcn_readfirstlane(first), (threadIdx.x & 63) / Q);
     __syncthreads();
-    bool fast[G];
     if(first < ngrp){
         qlmx_span S = sp[s0];
-        uint64_t q0[G]; uint32_t dw[G]; float sg[G];
+        uint64_t q0[G]; Words dw[G]; float sg[G]; bool fast[G];
 #pragma unroll
         for(int q = 0; q < G; q++){
-            const int gi = first + q * TEAMS;
-            fast[q] = false; dw[q] = 0; sg[q] = 0.0f; q0[q] = 0;
+            const int gi = first + q * COUNTERS;
+            fast[q] = false; dw[q] = Words{}; sg[q] = 0.0f; q0[q] = 0;
             if(gi >= ngrp) continue;
             if(gi >= S.gi0 + S.ngrp) S = sp[qx_span_of(sp, nspan, gi)];
             const uint64_t j0 = (uint64_t)(gi - S.gi0) * (uint64_t)group;
             fast[q] = vec_ok && group == 8 * W && packed && S.n - j0 >= 8 * W && ((S.qi0 + j0) & 7ULL) == 0;
-            if(!fast[q]) continue;
+            if(!fast[q]){ if(ql == 0) other[atomicAdd(&others, 1)] = gi; continue; }
             q0[q] = S.qi0 + j0;
-            dw[q] = *(const uint32_t *)(d + (q0[q] >> 1) + tl * 4);
+            dw[q] = *(const Words *)(d + (q0[q] >> 1) + ql * (4 * NW));
             sg[q] = s[gi];
         }
         const uint32_t up = 0x11111111u * (uint32_t)(dmax & 15), down = 0x11111111u * (uint32_t)(-dmax & 15);
 #pragma unroll
         for(int q = 0; q < G; q++){
-            const int railed = qx_team_sum<W>(nibbles_equal(dw[q], up) + nibbles_equal(dw[q], down));
+            int railed = 0;
+#pragma unroll
+            for(int k = 0; k < NW; k++) railed = nibbles_equal(dw[q].w[k], up, down, railed);
+            railed += qx_dpp_i<0xB1>(railed);
+            if(Q >= 4) railed += qx_dpp_i<0x4E>(railed);
+            if(Q >= 8) railed += qx_dpp_i<0x141>(railed);
+            if(Q >= 16) railed += qx_dpp_i<0x140>(railed);
             const float f = (float)railed * (1.0f / (8 * W));
-            if(fast[q] && tl == 0 && (f > f_hi || f < f_lo)){
+            if(fast[q] && ql == 0 && (f > f_hi || f < f_lo)){
                 const float sn = servo_scale(sg[q], railed, 8 * W, f_hi, f_lo);
                 const int k = atomicAdd(&moving, 1);
                 at[k] = q0[q]; conv[k] = sg[q] / sn;
-                s[first + q * TEAMS] = sn;
+                s[first + q * COUNTERS] = sn;
             }
         }
     }
     __syncthreads();
+    const int tl = threadIdx.x & (W - 1), team = threadIdx.x / W;
     for(int k = team; k < moving; k += TEAMS){
         const uint64_t e0 = at[k] + (uint64_t)tl * 8;
         const uint32_t dw = *(const uint32_t *)(d + (e0 >> 1));
@@ -225,11 +236,10 @@ __global__ void __launch_bounds__(256) k_qlmx_servo(signed char *d, signed char 
         *(uint32_t *)(d + (e0 >> 1)) = dn;
         *(uint2 *)(r + e0) = make_uint2(r0, r1);
     }
-    if(first < ngrp)
-        for(int q = 0; q < G; q++){
-            const int gi = first + q * TEAMS;
-            if(gi < ngrp && !fast[q]) servo_pairs<W>(group_loc(sp, qx_span_of(sp, nspan, gi), gi, group), gi, tl, d, r, s, dmax, f_hi, f_lo, packed);
-        }
+    for(int k = team; k < others; k += TEAMS){
+        const int gi = other[k];
+        servo_pairs<W>(group_loc(sp, qx_span_of(sp, nspan, gi), gi, group), gi, tl, d, r, s, dmax, f_hi, f_lo, packed);
+    }
 }
 
 static int codec_args_ok(const char *who, int nspan, int group, int dmax, int packed){
@@ -281,11 +291,11 @@ extern "C" int qlmx_servo(signed char *d, signed char *r, float *s,
     rc = codec_args_ok("qlmx_servo", nspan, group, dmax, packed); if(rc) return rc;
     if(ngrp <= 0) return QLMX_OK;
     const int vec_ok = ((uintptr_t)r & 7) == 0 && ((uintptr_t)d & 3) == 0;
-    const bool few = ngrp < (group == 64 ? 65536 : 32768);                 /* at four groups per team: less than two workgroups per CU */
-#define SERVO(W, G) hipLaunchKernelGGL((k_qlmx_servo<W, G>), dim3((unsigned)((ngrp + 256 / W * G - 1) / (256 / W * G))), dim3(256), 0, (hipStream_t)stream, \
-                                       d, r, s, sp, nspan, group, dmax, f_hi, f_lo, packed, ngrp, vec_ok)
-    if(group == 64){ if(few) SERVO(8, 1); else SERVO(8, 4); }
-    else           { if(few) SERVO(16, 1); else SERVO(16, 4); }
+    const bool few = ngrp < 49152, many = ngrp >= 1000000;
+#define SERVO(W, Q, G) hipLaunchKernelGGL((k_qlmx_servo<W, Q, G>), dim3((unsigned)((ngrp + 256 / Q * G - 1) / (256 / Q * G))), dim3(256), 0, (hipStream_t)stream, \
+                                          d, r, s, sp, nspan, group, dmax, f_hi, f_lo, packed, ngrp, vec_ok)
+    if(group == 64){ if(few) SERVO(8, 8, 1); else if(many) SERVO(8, 2, 2); else SERVO(8, 2, 1); }
+    else           { if(few) SERVO(16, 16, 1); else if(many) SERVO(16, 4, 2); else SERVO(16, 4, 1); }
 #undef SERVO
     QLMX_LAUNCH_CHECK("qlmx_servo launch");
     return QLMX_OK;

@@ -91,12 +91,12 @@ __device__ __forceinline__ int qx_span_of(const qlmx_span *sp, int nspan, int gi
 template<int TEAMS> __device__ __forceinline__ int qx_span_of_teams(const qlmx_span *sp, int nspan, int g0, int team){
     if(nspan > 64) return qx_span_of(sp, nspan, g0 + team);
     const int lane = threadIdx.x & 63, at = lane < nspan ? sp[lane].gi0 : 0x7FFFFFFF;
-    int si = 0;
-#pragma unroll
-    for(int k = 0; k < TEAMS; k++){
-        const int n = __popcll(__ballot(at <= g0 + k)) - 1;
-        si = team == k ? n : si;
-    }
+    int si = __popcll(__ballot(at <= g0)) - 1;
+    if(__popcll(__ballot(at <= g0 + TEAMS - 1)) - 1 != si)                /* not all in one span */
+        for(int k = 1; k < TEAMS; k++){
+            const int n = __popcll(__ballot(at <= g0 + k)) - 1;
+            si = team >= k ? n : si;
+        }
     return si < 0 ? 0 : si;
 }
 

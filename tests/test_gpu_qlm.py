@@ -441,6 +441,18 @@ def test_teams_of_half_and_whole_rows_vs_oracle(q, orc, group, nspan):
             assert np.array_equal(host(gstat), hstat)
 
 
+@pytest.mark.parametrize("group,ngroups", [(64, 49151), (64, 49152), (128, 49160), (128, 1000001)])
+def test_servo_launch_shapes_vs_oracle(q, orc, group, ngroups):
+    """Both sides of the lines between the servo's three shapes, an unaligned span and a short last group among the others."""
+    tab, nq, ng = make_spans([group * 70 + 4, group * (ngroups - 100) + 8, group * 28], group)
+    hd = orc.digits(nq, 19, 1); hr = orc.int8(nq, 19, 2, -64, 64)
+    hs = orc.uniform(ng, 19, 3, 0.5, 1.5) * f32(0.02 * 3 / 7)
+    d, r, s = dev(hd), dev(hr), dev(hs)
+    q.servo(d, r, s, dev(tab), len(tab), group, 7, 0.2, 0.08, 1, ng)
+    orc.servo(hd, hr, hs, tab, group, 7, 0.2, 0.08, 1, ng)
+    assert beq(d, hd) and beq(r, hr) and beq(s, hs)
+
+
 @pytest.mark.parametrize("n", [1, 63, 64 * 4096 + 5, 64 * 4096 * 3 + 2, 64 * 4096 * 17 + 1])
 def test_sqsum_pieces(q, orc, n):
     """One, three and sixteen workgroups per partial sum, chunk ends that are not aligned, twice in a row (the counters)."""
