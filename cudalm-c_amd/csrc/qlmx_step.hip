@@ -822,10 +822,20 @@ extern "C" int qlmx_step_touched(float *P, const float *Gc, signed char *d, sign
  * The hand-over is device-scope accesses, which go past the caches, and a wait for the store in front of the count. As an
  * acquire-release count it wrote back and invalidated an XCD's L2 once per workgroup, which cost more than the reading:
  * 127 us for 125.8 M values, 18 for any small number. A stretch of its own per workgroup keeps what it reads in few DRAM
- * pages: 6.1 TB/s at any grid of 1024 workgroups or more, side by side 4.9 to 5.8. */
+ * pages: 6.1 TB/s at any grid of 1024 workgroups or more, side by side 4.9 to 5.8. A gradient larger than the last-level
+ * cache (256 MB) is read past the caches (NT): norm and step of 125.8 M weights 551 -> 530 us. Of a smaller one the step
+ * finds a part there, and the plain loads stay (40 M weights: 169 us, 172 with NT). */
 #define SQ_W 16
+#define SQ_PAST_CACHE (64ull << 20)                    /* values */
 static __device__ double   g_sq_piece[64 * SQ_W];
 static __device__ unsigned g_sq_count[64];
+template<bool NT> __device__ __forceinline__ float4 load16(const float *p){
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    if(!NT) return *(const float4 *)p;
+    const f4 v = __builtin_nontemporal_load((const f4 *)p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+template<bool NT>
 __global__ void __launch_bounds__(256) k_qlmx_sqsum(const float *G, unsigned long long n, float *part, int pieces){
     __shared__ double red[128];
     const unsigned c = blockIdx.x / pieces, w = blockIdx.x - c * pieces, tid = threadIdx.x;
@@ -847,7 +857,7 @@ __global__ void __launch_bounds__(256) k_qlmx_sqsum(const float *G, unsigned lon
         for(; i + 3072 < a1; i += 4096){
             float4 v[4];
 #pragma unroll
-            for(int q = 0; q < 4; q++) v[q] = *(const float4 *)(G + i + q * 1024);
+            for(int q = 0; q < 4; q++) v[q] = load16<NT>(G + i + q * 1024);
 #pragma unroll
             for(int q = 0; q < 4; q++) add(u[q], v[q]);
         }
@@ -911,7 +921,7 @@ extern "C" int qlmx_sqsum(const float *G, unsigned long long n, float *part64, v
     /* a stretch holds at least the 4096 values of one round of its workgroup */
     const unsigned long long most = n / (64 * 4096);
     const int pieces = most < 1 ? 1 : most > SQ_W ? SQ_W : (int)most;
-    hipLaunchKernelGGL(k_qlmx_sqsum, dim3(64 * pieces), dim3(256), 0, (hipStream_t)stream, G, n, part64, pieces);
+    hipLaunchKernelGGL((n >= SQ_PAST_CACHE ? k_qlmx_sqsum<true> : k_qlmx_sqsum<false>), dim3(64 * pieces), dim3(256), 0, (hipStream_t)stream, G, n, part64, pieces);
     QLMX_LAUNCH_CHECK("qlmx_sqsum launch");
     return QLMX_OK;
 }
