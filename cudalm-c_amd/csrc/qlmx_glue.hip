@@ -235,20 +235,38 @@ __global__ void __launch_bounds__(256) k_fill_i32(int *p, int v, int n){
     if(i < n) p[i] = v;
 }
 
-/* ---- row movers. One workgroup per row; D % 4 == 0. ---- */
-template<bool OUT_BF16>
+/* ---- row movers. One workgroup per row; D % 4 == 0. Bound by HBM. What a launch touches once goes past the caches (NT)
+ * where it is more than the last-level cache holds: it would only push out the rows that the K experts of a token read
+ * again, and plain loads of such a stream reach 5.2 TB/s, these 6.6. 131072 rows of 2048: combine 314 -> 242 us, gate
+ * gradient 449 -> 357, gather 228 -> 218. Smaller buffers are partly in the cache, left there by the GEMM before or kept for
+ * the one after (16384 rows of 768 again and again: gate gradient 19.1 us, 20.3 with NT). ---- */
+#define PAST_CACHE (256ull << 20)                      /* bytes of the launch's rows in fp32 */
+typedef float gl_f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t gl_u2 __attribute__((ext_vector_type(2)));
+template<bool NT> __device__ __forceinline__ float4 row_load(const float4 *p){
+    if(!NT) return *p;
+    const gl_f4 v = __builtin_nontemporal_load((const gl_f4 *)p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+/* v as unit i of four values of a row buffer of either type */
+template<bool OUT_BF16, bool NT> __device__ __forceinline__ void row_store(void *rows, size_t i, float4 v){
+    if(OUT_BF16){
+        const gl_u2 o = {(uint32_t)qx_f32_to_bf16(v.x) | ((uint32_t)qx_f32_to_bf16(v.y) << 16),
+                         (uint32_t)qx_f32_to_bf16(v.z) | ((uint32_t)qx_f32_to_bf16(v.w) << 16)};
+        if(NT) __builtin_nontemporal_store(o, (gl_u2 *)rows + i); else ((gl_u2 *)rows)[i] = o;
+    } else {
+        const gl_f4 o = {v.x, v.y, v.z, v.w};
+        if(NT) __builtin_nontemporal_store(o, (gl_f4 *)rows + i); else ((gl_f4 *)rows)[i] = o;
+    }
+}
+template<bool OUT_BF16, bool NT>
 __global__ void __launch_bounds__(256) k_gather_rows(const float4 *src, const int *perm, void *Xp, int D4){
     const int j = blockIdx.x, n = perm[j];
     const float4 *s = src + (size_t)(n < 0 ? 0 : n) * D4;
     for(int d = threadIdx.x; d < D4; d += 256){
         float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if(n >= 0) v = s[d];
-        if(OUT_BF16){
-            uint2 o;
-            o.x = (uint32_t)qx_f32_to_bf16(v.x) | ((uint32_t)qx_f32_to_bf16(v.y) << 16);
-            o.y = (uint32_t)qx_f32_to_bf16(v.z) | ((uint32_t)qx_f32_to_bf16(v.w) << 16);
-            ((uint2 *)Xp)[(size_t)j * D4 + d] = o;
-        } else ((float4 *)Xp)[(size_t)j * D4 + d] = v;
+        row_store<OUT_BF16, NT>(Xp, (size_t)j * D4 + d, v);
     }
 }
 /* out[perm[j],:] = out[perm[j],:] + gate[perm[j]] * yp[j,:] (multiply, then add); a pass names every
@@ -275,7 +293,7 @@ __global__ void __launch_bounds__(256) k_scatter_add(const float4 *dXp, const in
     }
 }
 /* d_gate[n] = dout[n,:] . yp[j,:];  dyp[j,:] = gate[n] * dout[n,:] */
-template<bool OUT_BF16>
+template<bool OUT_BF16, bool NT>
 __global__ void __launch_bounds__(256) k_moe_dgate(const float4 *dout, const float4 *yp, const int *perm, const float *gate,
                                                    float *d_gate, void *dyp, int D4, int tokens){
     __shared__ float red[4];
@@ -283,25 +301,16 @@ __global__ void __launch_bounds__(256) k_moe_dgate(const float4 *dout, const flo
      * list: perm names pass * tokens + token, which indexes gate and d_gate, and the token is the remainder */
     const int j = blockIdx.x, m = perm[j], n = (tokens && m >= 0) ? m % tokens : m;
     if(n < 0){
-        for(int d = threadIdx.x; d < D4; d += 256){
-            if(OUT_BF16) ((uint2 *)dyp)[(size_t)j * D4 + d] = make_uint2(0u, 0u);
-            else ((float4 *)dyp)[(size_t)j * D4 + d] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
+        for(int d = threadIdx.x; d < D4; d += 256) row_store<OUT_BF16, NT>(dyp, (size_t)j * D4 + d, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
         return;
     }
     const float4 *dr = dout + (size_t)n * D4, *y = yp + (size_t)j * D4;
     const float g = gate[m];
     float acc = 0.0f;
     for(int d = threadIdx.x; d < D4; d += 256){
-        const float4 a = dr[d], b = y[d];
+        const float4 a = dr[d], b = row_load<NT>(&y[d]);
         acc += a.x * b.x; acc += a.y * b.y; acc += a.z * b.z; acc += a.w * b.w;
-        const float4 v = make_float4(g * a.x, g * a.y, g * a.z, g * a.w);
-        if(OUT_BF16){
-            uint2 o;
-            o.x = (uint32_t)qx_f32_to_bf16(v.x) | ((uint32_t)qx_f32_to_bf16(v.y) << 16);
-            o.y = (uint32_t)qx_f32_to_bf16(v.z) | ((uint32_t)qx_f32_to_bf16(v.w) << 16);
-            ((uint2 *)dyp)[(size_t)j * D4 + d] = o;
-        } else ((float4 *)dyp)[(size_t)j * D4 + d] = v;
+        row_store<OUT_BF16, NT>(dyp, (size_t)j * D4 + d, make_float4(g * a.x, g * a.y, g * a.z, g * a.w));
     }
     acc = qx_wave_sum(acc);
     if((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
@@ -312,16 +321,30 @@ __global__ void __launch_bounds__(256) k_moe_dgate(const float4 *dout, const flo
 /* ---- all K passes as ONE expert-grouped list of K*N rows (the reference's merged top-K, cudalm.cu:3532-3561,
  * 4022-4034): the grouping permutation of the K*N assignments names entries m = pass * N + token; row p of the
  * grouped buffers holds token perm[p] % N, and inv[m] is the row that holds entry m. ---- */
-/* one workgroup for all of it: the fill and what follows it need no launch of their own */
-#define MR_ONE 8192
-__global__ void __launch_bounds__(1024) k_merge_rows_one(const int *perm, int KN, int N, int *tok, int *inv){
-    for(int p = threadIdx.x; p < KN; p += 1024) inv[p] = -1;
+/* A workgroup reads the whole permutation and keeps the inverse of its own MR_WINDOW entries in LDS: one launch, where a fill
+ * and the kernel that overwrites it are two. The reading grows with the square of the rows; beyond MR_WHOLE of them two
+ * launches are the faster (12004 rows 5.7 -> 3.4 us, 32768 5.8 -> 5.5, 131072 5.4 and 16.5). */
+#define MR_WINDOW 1024
+#define MR_WHOLE 32768
+__global__ void __launch_bounds__(MR_WINDOW) k_merge_rows_windows(const int *perm, int KN, int N, int *tok, int *inv){
+    __shared__ int at[MR_WINDOW];
+    const int first = (int)blockIdx.x * MR_WINDOW, own = first + (int)threadIdx.x;
+    at[threadIdx.x] = -1;
     __syncthreads();
-    for(int p = threadIdx.x; p < KN; p += 1024){
-        const int m = perm[p];
-        tok[p] = m < 0 ? -1 : m % N;
-        if(m >= 0) inv[m] = p;
+    for(int p0 = 0; p0 < KN; p0 += 8 * MR_WINDOW){
+        int m[8];
+#pragma unroll
+        for(int k = 0; k < 8; k++) m[k] = perm[min(p0 + k * MR_WINDOW + (int)threadIdx.x, KN - 1)];
+#pragma unroll
+        for(int k = 0; k < 8; k++){
+            const int p = p0 + k * MR_WINDOW + (int)threadIdx.x;
+            if(p >= KN) continue;
+            if(m[k] >= first && m[k] - first < MR_WINDOW) at[m[k] - first] = p;
+            if(p == own) tok[p] = m[k] < 0 ? -1 : m[k] % N;
+        }
     }
+    __syncthreads();
+    if(own < KN) inv[own] = at[threadIdx.x];
 }
 __global__ void __launch_bounds__(256) k_merge_rows(const int *perm, int KN, int N, int *tok, int *inv){
     const int p = blockIdx.x * 256 + threadIdx.x;
@@ -332,6 +355,7 @@ __global__ void __launch_bounds__(256) k_merge_rows(const int *perm, int KN, int
 }
 /* out[n,:] = (..(out[n,:] + g[0*N+n] * y[inv[0*N+n],:]) + ..) + g[(K-1)*N+n] * y[inv[(K-1)*N+n],:], pass after pass:
  * the sums the per-pass scatters build, in their order (g NULL: plain additions; inv < 0: the pass dropped the token) */
+template<bool NT>
 __global__ void __launch_bounds__(256) k_combine(const float4 *y, const int *inv, const float *g, float4 *out, int N, int K, int D4){
     const int n = blockIdx.x;
     float4 *o = out + (size_t)n * D4;
@@ -341,7 +365,7 @@ __global__ void __launch_bounds__(256) k_combine(const float4 *y, const int *inv
             const size_t i = (size_t)k * N + n;
             const int p = inv[i];
             if(p < 0) continue;
-            const float4 b = y[(size_t)p * D4 + d];
+            const float4 b = row_load<NT>(&y[(size_t)p * D4 + d]);
             if(g){ const float w = g[i]; a.x = a.x + w * b.x; a.y = a.y + w * b.y; a.z = a.z + w * b.z; a.w = a.w + w * b.w; }
             else { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
         }
@@ -455,8 +479,9 @@ extern "C" int qlmx_moe_gather(const float *src, const int *perm, void *Xp, int 
     QLMX_REQUIRE(GLUE_ALIGN16(src) && GLUE_ALIGN16(Xp), "qlmx_moe_gather: buffers must be 16-byte aligned");
     QLMX_REQUIRE(out_dtype == QLMX_ACT_F32 || out_dtype == QLMX_ACT_BF16, "qlmx_moe_gather: unknown output type %d", out_dtype);
     if(N <= 0) return QLMX_OK;
-    if(out_dtype == QLMX_ACT_BF16) hipLaunchKernelGGL(k_gather_rows<true>, dim3(N), dim3(256), 0, (hipStream_t)stream, (const float4 *)src, perm, Xp, D / 4);
-    else                           hipLaunchKernelGGL(k_gather_rows<false>, dim3(N), dim3(256), 0, (hipStream_t)stream, (const float4 *)src, perm, Xp, D / 4);
+    const bool bf = out_dtype == QLMX_ACT_BF16, nt = (unsigned long long)N * D * 4 >= PAST_CACHE;
+    hipLaunchKernelGGL((bf ? nt ? k_gather_rows<true, true> : k_gather_rows<true, false> : nt ? k_gather_rows<false, true> : k_gather_rows<false, false>),
+                       dim3(N), dim3(256), 0, (hipStream_t)stream, (const float4 *)src, perm, Xp, D / 4);
     QLMX_LAUNCH_CHECK("gather launch");
     return QLMX_OK;
 }
@@ -483,6 +508,13 @@ extern "C" int qlmx_moe_scatter_add(const float *dXp, const int *perm, float *ds
     return QLMX_OK;
 }
 
+static void dgate_launch(const float *dout, const float *yp, const int *perm, const float *gate, float *d_gate, void *dyp, int rows, int D, int out_dtype,
+                         int tokens, hipStream_t stream){
+    const bool bf = out_dtype == QLMX_ACT_BF16, nt = (unsigned long long)rows * D * 4 >= PAST_CACHE;
+    hipLaunchKernelGGL((bf ? nt ? k_moe_dgate<true, true> : k_moe_dgate<true, false> : nt ? k_moe_dgate<false, true> : k_moe_dgate<false, false>),
+                       dim3(rows), dim3(256), 0, stream, (const float4 *)dout, (const float4 *)yp, perm, gate, d_gate, dyp, D / 4, tokens);
+}
+
 extern "C" int qlmx_moe_dgate(const float *dout, const float *yp, const int *perm, const float *gate,
                               float *d_gate, void *dyp, int N, int D, int out_dtype, void *stream){
     int rc = qlmx_check_ready(); if(rc) return rc;
@@ -491,8 +523,7 @@ extern "C" int qlmx_moe_dgate(const float *dout, const float *yp, const int *per
     QLMX_REQUIRE(GLUE_ALIGN16(dout) && GLUE_ALIGN16(yp) && GLUE_ALIGN16(dyp), "qlmx_moe_dgate: buffers must be 16-byte aligned");
     QLMX_REQUIRE(out_dtype == QLMX_ACT_F32 || out_dtype == QLMX_ACT_BF16, "qlmx_moe_dgate: unknown output type %d", out_dtype);
     if(N <= 0) return QLMX_OK;
-    if(out_dtype == QLMX_ACT_BF16) hipLaunchKernelGGL(k_moe_dgate<true>, dim3(N), dim3(256), 0, (hipStream_t)stream, (const float4 *)dout, (const float4 *)yp, perm, gate, d_gate, dyp, D / 4, 0);
-    else                           hipLaunchKernelGGL(k_moe_dgate<false>, dim3(N), dim3(256), 0, (hipStream_t)stream, (const float4 *)dout, (const float4 *)yp, perm, gate, d_gate, dyp, D / 4, 0);
+    dgate_launch(dout, yp, perm, gate, d_gate, dyp, N, D, out_dtype, 0, (hipStream_t)stream);
     QLMX_LAUNCH_CHECK("dgate launch");
     return QLMX_OK;
 }
@@ -503,8 +534,8 @@ extern "C" int qlmx_moe_merge_rows(const int *perm, int N, int K, int *tok, int 
     QLMX_REQUIRE(perm && tok && inv, "qlmx_moe_merge_rows: NULL buffer");
     QLMX_REQUIRE(N > 0 && K > 0 && (long long)N * K < (1LL << 31), "qlmx_moe_merge_rows: N=%d K=%d", N, K);
     const int KN = N * K;
-    if(KN <= MR_ONE){
-        hipLaunchKernelGGL(k_merge_rows_one, dim3(1), dim3(1024), 0, (hipStream_t)stream, perm, KN, N, tok, inv);
+    if(KN <= MR_WHOLE){
+        hipLaunchKernelGGL(k_merge_rows_windows, dim3((KN + MR_WINDOW - 1) / MR_WINDOW), dim3(MR_WINDOW), 0, (hipStream_t)stream, perm, KN, N, tok, inv);
         QLMX_LAUNCH_CHECK("merge rows launch");
         return QLMX_OK;
     }
@@ -522,7 +553,7 @@ extern "C" int qlmx_moe_combine(const float *y, const int *inv, const float *gat
     GLUE_ROWS_CHECK("qlmx_moe_combine", D);
     QLMX_REQUIRE(K > 0 && GLUE_ALIGN16(y) && GLUE_ALIGN16(out), "qlmx_moe_combine: K=%d, buffers must be 16-byte aligned", K);
     if(N <= 0) return QLMX_OK;
-    hipLaunchKernelGGL(k_combine, dim3(N), dim3(256), 0, (hipStream_t)stream, (const float4 *)y, inv, gate, (float4 *)out, N, K, D / 4);
+    hipLaunchKernelGGL(((unsigned long long)N * K * D * 4 >= PAST_CACHE ? k_combine<true> : k_combine<false>), dim3(N), dim3(256), 0, (hipStream_t)stream, (const float4 *)y, inv, gate, (float4 *)out, N, K, D / 4);
     QLMX_LAUNCH_CHECK("combine launch");
     return QLMX_OK;
 }
@@ -537,8 +568,7 @@ extern "C" int qlmx_moe_dgate_merged(const float *dout, const float *yp, const i
     QLMX_REQUIRE(K > 0 && (long long)N * K < (1LL << 31), "qlmx_moe_dgate_merged: N=%d K=%d", N, K);
     if(N <= 0) return QLMX_OK;
     const int KN = N * K;
-    if(out_dtype == QLMX_ACT_BF16) hipLaunchKernelGGL(k_moe_dgate<true>, dim3(KN), dim3(256), 0, (hipStream_t)stream, (const float4 *)dout, (const float4 *)yp, perm, gate, d_gate, dyp, D / 4, N);
-    else                           hipLaunchKernelGGL(k_moe_dgate<false>, dim3(KN), dim3(256), 0, (hipStream_t)stream, (const float4 *)dout, (const float4 *)yp, perm, gate, d_gate, dyp, D / 4, N);
+    dgate_launch(dout, yp, perm, gate, d_gate, dyp, KN, D, out_dtype, N, (hipStream_t)stream);
     QLMX_LAUNCH_CHECK("merged dgate launch");
     return QLMX_OK;
 }

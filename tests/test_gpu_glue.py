@@ -143,7 +143,7 @@ def test_perm_chunks_vs_oracle(q, orc, N, E, K):
         assert np.array_equal(perm[k * N:(k + 1) * N], wp)
 
 
-@pytest.mark.parametrize("N,K", [(1, 2), (4096, 2), (4097, 2)])
+@pytest.mark.parametrize("N,K", [(1, 2), (4096, 2), (4097, 2), (512, 2), (1025, 1), (16384, 2), (32769, 1)])
 def test_merge_rows_with_dropped_entries(q, N, K):
     import torch
     perm = np.random.default_rng(N).permutation(N * K).astype(np.int32)
@@ -155,6 +155,40 @@ def test_merge_rows_with_dropped_entries(q, N, K):
     want[perm[perm >= 0]] = np.nonzero(perm >= 0)[0]
     assert np.array_equal(inv.cpu().numpy(), want)
     assert np.array_equal(tok.cpu().numpy(), np.where(perm < 0, -1, perm % N))
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_row_moves_larger_than_the_last_level_cache(q, bf16):
+    """The rows as one launch of 256 MiB, and a few rows at a time."""
+    import torch
+    N, K, D, step = 517, 2, 65544, 94
+    g = torch.Generator(device="cuda"); g.manual_seed(5)
+    x = torch.randn(N, D, device="cuda", generator=g); y = torch.randn(N * K, D, device="cuda", generator=g)
+    perm = torch.randperm(N * K, device="cuda", generator=g).to(torch.int32); perm[::7] = -1
+    tok, inv = zeros(N * K, torch.int32), zeros(N * K, torch.int32)
+    gate = torch.rand(N * K, device="cuda", generator=g)
+    q.moe_merge_rows(perm, N, K, tok, inv)
+    dt, out_dtype = (torch.bfloat16, pkg.ACT_BF16) if bf16 else (torch.float32, pkg.ACT_F32)
+    got = [torch.empty(N * K, D, device="cuda", dtype=dt) for _ in range(4)]
+    dg = [torch.zeros(N * K, device="cuda") for _ in range(2)]
+    q.moe_gather(x, tok, got[0], N * K, D, out_dtype)
+    q.moe_dgate_merged(x, y, perm, gate, dg[0], got[1], N, K, D, out_dtype)
+    for r in range(0, N * K, step):
+        n = min(step, N * K - r)
+        q.moe_gather(x, tok[r:], got[2][r:], n, D, out_dtype)
+        for j in range(r, r + n):
+            m = int(perm[j])
+            if m < 0: got[3][j].zero_()
+            else: q.moe_dgate(x[m % N], y[j], zeros(1, torch.int32), gate[m:], dg[1][m:], got[3][j], 1, D, out_dtype)
+    assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3]) and torch.equal(dg[0], dg[1])
+    for w in (gate, None):
+        out = torch.ones(N, D, device="cuda"); want = out.clone()
+        q.moe_combine(y, inv, w, out, N, K, D)
+        for k in range(K):
+            p = inv[k * N:(k + 1) * N].long(); on = (p >= 0)[:, None]
+            b = y[p.clamp(min=0)]
+            want = torch.where(on, want + (b if w is None else gate[k * N:(k + 1) * N, None] * b), want)
+        assert torch.equal(out, want)
 
 
 def test_perm_reports_bad_expert_of_any_chunk(q):
