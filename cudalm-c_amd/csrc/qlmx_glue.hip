@@ -146,7 +146,8 @@ __global__ void __launch_bounds__(RT_WG) k_router_topk_lanes(const float *rt, fl
 static inline int gp_chunk(int N){ return N <= GP_ONE ? N : 2048 * ((N + 2048 * 64 - 1) / (2048 * 64)); }
 static inline int gp_threads(int E){ return E <= 896 ? 1024 : E <= 2600 ? 256 : 64; }   /* [wavefronts + 2][E] counters in 64 KB of LDS */
 /* workspace: hist[K][NC][E], then seen[K][NC] (0, or -1-e for an expert number e out of range) and, at the offset that
- * qlmx_moe_perm_status reads, the flag for the whole call */
+ * qlmx_moe_perm_status reads, bad[K], the same for each whole pass: every pass has a workgroup of its own that writes its
+ * word, so no word has to be cleared first and none is written by two */
 __global__ void __launch_bounds__(1024) k_gp_hist(const int *asn, int N, int E, int chunk, int *hist, int *seen){
     extern __shared__ int cnt[];                          /* [E], then the flag */
     const int c = blockIdx.x, k = blockIdx.y, end = min(N, (c + 1) * chunk);
@@ -208,12 +209,12 @@ __global__ void __launch_bounds__(1024) k_gp_place(const int *asn, int N, int E,
     __syncthreads();
     if(c == 0){
         for(int e = tid; e <= E; e += NT) off[(size_t)k * (E + 1) + e] = first[e];
-        if(k == 0 && wave == 0){
+        if(wave == 0){
             int f = *flag;
-            if(seen) for(int i = lane; i < NC * (int)gridDim.y; i += 64) if(seen[i]) f = seen[i];
+            if(seen) for(int i = lane; i < NC; i += 64) if(seen[(size_t)k * NC + i]) f = seen[(size_t)k * NC + i];
             const unsigned long long any = __ballot(f != 0);
             f = any ? __shfl(f, __ffsll((long long)any) - 1, 64) : 0;
-            if(lane == 0) *bad = f;
+            if(lane == 0) bad[k] = f;
         }
     }
     const int bits = 32 - __clz(E);
@@ -437,7 +438,7 @@ extern "C" int qlmx_router_topk(const float *rt, float *rprobs, int *assign, flo
 #define GP_CHUNK 256          /* the workspace has room for a histogram per 256 tokens, more than gp_chunk cuts */
 static size_t gp_flag_at(int N, int E, int K){ return (size_t)K * ((size_t)(N + GP_CHUNK - 1) / GP_CHUNK) * E; }
 extern "C" size_t qlmx_moe_perm_workspace(int N, int E, int K){
-    return (gp_flag_at(N, E, K) + 4 + (size_t)K * E) * sizeof(int);
+    return (gp_flag_at(N, E, K) + 4 + (size_t)K * E) * sizeof(int);       /* the flags are the first K of the words behind the histograms */
 }
 
 extern "C" int qlmx_moe_perm(const int *assign, int N, int E, int K, int *perm, int *off, void *workspace, void *stream){
@@ -462,10 +463,15 @@ extern "C" int qlmx_moe_perm(const int *assign, int N, int E, int K, int *perm, 
 extern "C" int qlmx_moe_perm_status(const void *workspace, int N, int E, int K, void *stream){
     int rc = qlmx_check_ready(); if(rc) return rc;
     QLMX_REQUIRE(workspace, "qlmx_moe_perm_status: NULL workspace");
-    int bad = 0;
-    QLMX_HIP(hipMemcpyAsync(&bad, (const int *)workspace + gp_flag_at(N, E, K), sizeof(int), hipMemcpyDeviceToHost, (hipStream_t)stream), "perm flag read");
-    QLMX_HIP(hipStreamSynchronize((hipStream_t)stream), "perm flag sync");
-    if(bad){ qlmx_set_error("qlmx_moe_perm: expert index %d out of range [0, %d)", -1 - bad, E); return QLMX_E_ARG; }
+    enum { AT_ONCE = 64 };                                 /* more passes than any caller has */
+    int bad[AT_ONCE];
+    for(int k0 = 0; k0 < K; k0 += AT_ONCE){
+        const int n = K - k0 < AT_ONCE ? K - k0 : AT_ONCE;
+        QLMX_HIP(hipMemcpyAsync(bad, (const int *)workspace + gp_flag_at(N, E, K) + k0, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, (hipStream_t)stream), "perm flag read");
+        QLMX_HIP(hipStreamSynchronize((hipStream_t)stream), "perm flag sync");
+        for(int k = 0; k < n; k++)
+            if(bad[k]){ qlmx_set_error("qlmx_moe_perm: expert index %d out of range [0, %d)", -1 - bad[k], E); return QLMX_E_ARG; }
+    }
     return QLMX_OK;
 }
 

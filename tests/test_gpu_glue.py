@@ -220,6 +220,27 @@ def test_perm_reports_bad_expert(q):
         gpu_perm(q, asn, 4, 4, 1)
 
 
+@pytest.mark.parametrize("N", [4, 4096, 4097, 9000])
+@pytest.mark.parametrize("K,k", [(2, 0), (2, 1), (3, 1), (300, 299)])
+def test_perm_reports_bad_expert_of_any_pass(q, N, K, k):
+    """One chunk and several: the flag is the whole call's, whichever pass holds the index, and a later call on the same
+    workspace clears it. Every other pass is grouped as usual."""
+    import torch
+    E = 4
+    asn = np.random.default_rng(N + k).integers(0, E, K * N).astype(np.int32)
+    ok = dev(asn)
+    asn[(k + 1) * N - 1] = 77
+    ws = torch.zeros(q.moe_perm_workspace(N, E, K), dtype=torch.uint8, device="cuda")
+    perm, off = zeros(K * N, torch.int32), zeros(K * (E + 1), torch.int32)
+    q.moe_perm(dev(asn), N, E, K, perm, off, ws)
+    with pytest.raises(pkg.QlmxError, match="index 77 out of range"):
+        q.moe_perm_status(ws, N, E, K)
+    j = (k + 1) % K
+    assert np.array_equal(perm.cpu().numpy()[j * N:(j + 1) * N], np.argsort(asn[j * N:(j + 1) * N], kind="stable"))
+    q.moe_perm(ok, N, E, K, perm, off, ws)
+    q.moe_perm_status(ws, N, E, K)
+
+
 # ------------------------------------------------------------------ row movers, dgate, swiglu
 def test_glue_vs_reference_fixture(q, golden):
     import torch
