@@ -482,12 +482,14 @@ __device__ __forceinline__ float df_stage(const float (&v)[DF_NG][DF_MB], bool l
 }
 
 /* Staging for the matrix-core loop, wavefront by wavefront: a lane holds one row of its wavefront's share of the task
- * (zeros past its end), v[g][m] as above. Each input row m is brought to a 31-bit fixed point at the largest magnitude
- * among the wavefront's rows, k[m] = the power of two, and stored as four signed bytes whose sum times 1, 2^8, 2^16, 2^24 it
- * is (q + 0x80808080 has the bytes plus 128): a value less than 2^7 below the largest keeps all its 24 bits, and what a smaller
- * one loses lies below what the fp32 sums of the row would round away. bad[m]: a value is infinite or not a number.
- * xs: [plane g * DF_MB + m][lane group of the loop][row of the group]; written and read by one wavefront, so no barrier. */
+ * (zeros past its end), v[g][m] as above. The rows of one (scale group, input row) pair, and no others -- a column adds up values
+ * of one group only --, are brought to a 31-bit fixed point at the largest magnitude among them and stored as four signed bytes
+ * whose sum times 1, 2^8, 2^16, 2^24 it is (q + 0x80808080 has the bytes plus 128): a value less than 2^7 below the largest keeps
+ * all its 24 bits, and what a smaller one loses is at most 2^-31 of the largest.
+ * xs: [plane g * DF_MB + m][lane group of the loop][row of the group], behind the rows the biased exponent of the largest (255: a
+ * value is infinite or not a number); written and read by one wavefront, so no barrier. */
 #define DF_XPLANE 68          /* 64 rows, and 4 words so that the 16 (plane, lane group) pairs of a read start in different banks */
+#define DF_XEXP 64            /* the first of these words */
 __device__ __forceinline__ unsigned df_wave_max(unsigned v){
     v = max(v, (unsigned)qx_dpp_i<0xB1>((int)v)); v = max(v, (unsigned)qx_dpp_i<0x4E>((int)v));
     v = max(v, (unsigned)qx_dpp_i<0x141>((int)v)); v = max(v, (unsigned)qx_dpp_i<0x140>((int)v));
@@ -495,21 +497,15 @@ __device__ __forceinline__ unsigned df_wave_max(unsigned v){
     const unsigned b = max((unsigned)__builtin_amdgcn_readlane((int)v, 32), (unsigned)__builtin_amdgcn_readlane((int)v, 48));
     return max(a, b);
 }
-__device__ __forceinline__ void df_stage_i8(const float (&v)[DF_NG][DF_MB], uint32_t *xs, int (&k)[DF_MB], bool (&bad)[DF_MB]){
+__device__ __forceinline__ void df_stage_i8(const float (&v)[DF_NG][DF_MB], uint32_t *xs){
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for(int m = 0; m < DF_MB; m++){
-        unsigned mx = 0;
-#pragma unroll
-        for(int gg = 0; gg < DF_NG; gg++) mx = max(mx, __float_as_uint(v[gg][m]) & 0x7FFFFFFFu);
-        const int ex = (int)(df_wave_max(mx) >> 23);
-        bad[m] = ex == 255;
-        k[m] = 156 - ex;                                  /* the largest comes to [2^29, 2^30) */
-#pragma unroll
-        for(int gg = 0; gg < DF_NG; gg++){
-            const uint32_t q = (uint32_t)(int)rintf(__builtin_amdgcn_ldexpf(v[gg][m], k[m]));
-            xs[(gg * DF_MB + m) * DF_XPLANE + (lane & 3) * 16 + (lane >> 2)] = (q + 0x80808080u) ^ 0x80808080u;
-        }
+    for(int p = 0; p < DF_NG * DF_MB; p++){
+        const float x = v[p / DF_MB][p % DF_MB];
+        const int ex = (int)(df_wave_max(__float_as_uint(x) & 0x7FFFFFFFu) >> 23);
+        const uint32_t q = (uint32_t)(int)rintf(__builtin_amdgcn_ldexpf(x, 156 - ex));       /* the largest comes to [2^29, 2^30) */
+        xs[p * DF_XPLANE + (lane & 3) * 16 + (lane >> 2)] = (q + 0x80808080u) ^ 0x80808080u;
+        if(lane == 0) xs[p * DF_XPLANE + DF_XEXP] = (uint32_t)ex;
     }
 }
 
@@ -584,8 +580,7 @@ __device__ __forceinline__ void df_task_i8(const DfArgs &a, const DfT &t, uint2 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
     const int N = t.N, M = t.M, chunk = t.chunk;
     DF_STAMP(10 + 16 * t.list);
-    int k[DF_MB]; bool bad[DF_MB];
-    prep(k, bad);
+    prep();
     DF_STAMP(11);
     __builtin_amdgcn_s_setprio(0);
     df_i32x4 acc[16];
@@ -625,8 +620,8 @@ __device__ __forceinline__ void df_task_i8(const DfArgs &a, const DfT &t, uint2 
     __syncthreads();                                      /* the sums of the task before have been read */
     const int m = g & 1;
     if((c >= 8) == (g >= 2) && m < M){
-        const int e = -4 - (m ? k[1] : k[0]);
-        const float up = (m ? bad[1] : bad[0]) ? __builtin_nanf("") : 65536.0f;
+        const int ex = (int)xs[(g >> 1) * DF_MB * DF_XPLANE + m * DF_XPLANE + DF_XEXP], e = ex - 160;
+        const float up = ex == 255 ? __builtin_nanf("") : 65536.0f;
         float y[16];
 #pragma unroll
         for(int j = 0; j < 16; j++){
@@ -998,7 +993,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
             else       df_task_h<2>(a, cur, w0, w1, hs, xs_raw, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
         } else {
             uint32_t *xs = xs_raw + (tid >> 6) * (DF_NG * DF_MB * DF_XPLANE);
-            auto prep = [&](int (&k)[DF_MB], bool (&bad)[DF_MB]){ float v[DF_NG][DF_MB]; inputs(v); df_stage_i8(v, xs, k, bad); };
+            auto prep = [&](){ float v[DF_NG][DF_MB]; inputs(v); df_stage_i8(v, xs); };
             df_task_i8(a, cur, w0, w1, xs, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
         }
         cur = nxt;

@@ -289,3 +289,65 @@ def test_decode_inputs_of_very_different_size(q, orc, D, F, group):
     for t in (0, 1, 2, 3, 5):
         assert orc.relerr(got[t], want[t]) < 2e-5, t
     assert not got[4].any() and np.isnan(got[6]).all()
+
+
+class Layer64:
+    """A decode layer whose digits and scales a test changes before it runs: d1, d3 [E, D, F], d2 [E, F, D], s1, s3
+    [E, D, F / group], s2 [E, F, D / group], and the layer's output in 64 bits from those digits and scales."""
+    T, E, K, D, F, group = 3, 2, 2, 384, 640, 128
+
+    def __init__(self, orc, seed):
+        T, E, K, D, F = self.T, self.E, self.K, self.D, self.F
+        rng = np.random.default_rng(seed)
+        self.d1, self.d3 = (rng.integers(-7, 8, (E, D, F)) for _ in range(2))
+        self.d2 = rng.integers(-7, 8, (E, F, D))
+        self.s1, self.s3 = (f32(0.01) * (f32(0.5) + rng.random((E, D, F // self.group), dtype=f32)) for _ in range(2))
+        self.s2 = f32(0.01) * (f32(0.5) + rng.random((E, F, D // self.group), dtype=f32))
+        self.x = rng.standard_normal((T, D), dtype=f32)
+        self.asn = np.array([0, 0, 0, 1, 1, 1], np.int32)             # an expert's three tokens: a problem of two rows, one of one
+        self.gate = (f32(0.2) + rng.random(K * T, dtype=f32)).astype(f32)
+
+    def want(self):
+        y = np.zeros((self.T, self.D))
+        w = lambda d, s: d * np.repeat(s.astype(np.float64), self.group, axis=2)
+        w1, w3, w2 = w(self.d1, self.s1), w(self.d3, self.s3), w(self.d2, self.s2)
+        for j, e in enumerate(self.asn):
+            x = self.x[j % self.T].astype(np.float64)
+            g, u = x @ w1[e], x @ w3[e]
+            with np.errstate(over="ignore"):
+                y[j % self.T] += self.gate[j].astype(np.float64) * ((g / (1.0 + np.exp(-g)) * u) @ w2[e])
+        return y
+
+    def run(self, q):
+        import torch
+        q.call("qlmx_decode_math", 0)
+        digits = np.concatenate([m.reshape(-1) for m in (self.d1, self.d3, self.d2)]).astype(np.int64) & 15
+        scales = np.concatenate([m.reshape(-1) for m in (self.s1, self.s3, self.s2)]).astype(f32)
+        out = torch.zeros(self.T, self.D, device="cuda")
+        n = self.E * self.D * self.F
+        q.decode_forward(dev(self.x), dev(self.asn), dev(self.gate), out, dev((digits[0::2] | digits[1::2] << 4).astype(np.uint8)), dev(scales),
+                         self.group, 0, n, 2 * n, self.T, self.K, self.E, self.D, self.F)
+        return out.cpu().numpy()
+
+
+def rel64(got, want):
+    return float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("n", [0, 10, 14, 22, 30, 40])
+def test_decode_neighbouring_scale_groups_of_different_size(q, orc, n):
+    """A column's sum holds nothing of the scale group beside it, so the size of that group's scales must not show in it: every
+    second group of the down projection 2^-n of its neighbours, and every second group of gate and up with the down
+    projection's rows behind them as much larger, so that the output shows those columns' own error. Bound: three fp32 sums,
+    one after the other, of some hundred rounded products."""
+    a = Layer64(orc, 100 + n)
+    a.s2[:, :, 1::2] *= f32(2.0 ** -n)
+    got, want = a.run(q), a.want()
+    for c in range(0, a.D, a.group):
+        assert rel64(got[:, c:c + a.group], want[:, c:c + a.group]) < 1e-6, c
+    b = Layer64(orc, 200 + n)
+    b.s1[:, :, 1::2] *= f32(2.0 ** -n); b.s3[:, :, 1::2] *= f32(2.0 ** -n)
+    for f in range(b.group, b.F, 2 * b.group):
+        b.s2[:, f:f + b.group] *= f32(2.0 ** min(2 * n, 100))
+    got, want = b.run(q), b.want()
+    assert rel64(got, want) < 1e-6
