@@ -484,10 +484,16 @@ __device__ __forceinline__ float df_stage(const float (&v)[DF_NG][DF_MB], bool l
 /* Staging for the matrix-core loop, wavefront by wavefront: a lane holds one row of its wavefront's share of the task
  * (zeros past its end), v[g][m] as above. The rows of one (scale group, input row) pair, and no others -- a column adds up values
  * of one group only --, are brought to a 31-bit fixed point at the largest magnitude among them and stored as four signed bytes
- * whose sum times 1, 2^8, 2^16, 2^24 it is (q + 0x80808080 has the bytes plus 128): a value less than 2^7 below the largest keeps
- * all its 24 bits, and what a smaller one loses is at most 2^-31 of the largest.
- * xs: [plane g * DF_MB + m][lane group of the loop][row of the group], behind the rows the biased exponent of the largest (255: a
- * value is infinite or not a number); written and read by one wavefront, so no barrier. */
+ * whose sum times 1, 2^8, 2^16, 2^24 it is (q + 0x80808080 has the bytes plus 128). A value less than 2^7 below the largest
+ * keeps all its 24 bits; every value is held to 2^-31 of the largest. That is less than an fp32 sum with the largest in it
+ * rounds away, but a column whose digits are zero where the large values are is a sum of the small ones alone. Returns true where
+ * such a column could be the worse for it: where most of a pair's nonzero values lie more than 2^8 below the largest, or a value
+ * is infinite or not a number. The wavefront then multiplies in fp32 (df_fma_task). Otherwise the
+ * larger half of the values keep 21 bits at least (rounding 1.4e-7 of the value, as much as an fp32 sum's). Most of them: of
+ * normally distributed inputs 0.6 % lie there and of silu(gate) * up 2 to 5 %, so that ordinary layers keep to the fixed point
+ * (with a quarter as the line one wavefront in a thousand would not, and a layer waits for each).
+ * xs: [plane g * DF_MB + m][lane group of the loop][row of the group], behind the rows the biased exponent of the largest; written
+ * and read by one wavefront, so no barrier. */
 #define DF_XPLANE 68          /* 64 rows, and 4 words so that the 16 (plane, lane group) pairs of a read start in different banks */
 #define DF_XEXP 64            /* the first of these words */
 __device__ __forceinline__ unsigned df_wave_max(unsigned v){
@@ -497,16 +503,25 @@ __device__ __forceinline__ unsigned df_wave_max(unsigned v){
     const unsigned b = max((unsigned)__builtin_amdgcn_readlane((int)v, 32), (unsigned)__builtin_amdgcn_readlane((int)v, 48));
     return max(a, b);
 }
-__device__ __forceinline__ void df_stage_i8(const float (&v)[DF_NG][DF_MB], uint32_t *xs){
+__device__ __forceinline__ bool df_stage_i8(const float (&v)[DF_NG][DF_MB], int M, uint32_t *xs){
     const int lane = threadIdx.x & 63;
+    int plain = 0;
 #pragma unroll
-    for(int p = 0; p < DF_NG * DF_MB; p++){
-        const float x = v[p / DF_MB][p % DF_MB];
-        const int ex = (int)(df_wave_max(__float_as_uint(x) & 0x7FFFFFFFu) >> 23);
-        const uint32_t q = (uint32_t)(int)rintf(__builtin_amdgcn_ldexpf(x, 156 - ex));       /* the largest comes to [2^29, 2^30) */
-        xs[p * DF_XPLANE + (lane & 3) * 16 + (lane >> 2)] = (q + 0x80808080u) ^ 0x80808080u;
-        if(lane == 0) xs[p * DF_XPLANE + DF_XEXP] = (uint32_t)ex;
+    for(int m = 0; m < DF_MB; m++){
+        if(m >= M) break;                                 /* the sums of a row that is not there are not read */
+#pragma unroll
+        for(int gg = 0; gg < DF_NG; gg++){
+            const float x = v[gg][m];
+            uint32_t *plane = xs + (gg * DF_MB + m) * DF_XPLANE;
+            const unsigned mag = __float_as_uint(x) & 0x7FFFFFFFu, ex = df_wave_max(mag) >> 23;
+            const uint32_t q = (uint32_t)(int)rintf(__builtin_amdgcn_ldexpf(x, 156 - (int)ex));      /* the largest comes to [2^29, 2^30) */
+            plane[(lane & 3) * 16 + (lane >> 2)] = (q + 0x80808080u) ^ 0x80808080u;
+            plane[DF_XEXP] = ex;
+            const int low = __popcll(__ballot(mag - 1u < (max(ex, 8u) << 23) - 0x4000001u));         /* 0 < mag < 2^-8 of the largest's power of two */
+            plain |= (int)(2 * low > __popcll(__ballot(mag != 0u))) | (int)(ex == 255u);
+        }
     }
+    return __builtin_amdgcn_readfirstlane(plain) != 0;
 }
 
 /* One task: which slice of which matrix, for which problem. list 0 = none. */
@@ -552,6 +567,39 @@ __device__ __forceinline__ void df_bytes(uint32_t w0, uint32_t w1, uint32_t w2, 
 typedef int df_i32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ long df_pair(uint32_t lo, uint32_t hi){ return (long)(((u64)hi << 32) | (u64)lo); }
 
+/* A wavefront's share of a task in fp32 multiply-adds. v as df_stage_i8 takes it, and laid out in xs as that does. The lane's 16
+ * columns are summed over the four lane groups into sums[input][256 columns]. Two columns at a time in a loop: unrolled, it is
+ * 8 KB of instructions between the staging and the matrix-core loop. */
+__device__ __forceinline__ void df_fma_task(const uint2 (&w0)[DF_BATCH], const uint2 (&w1)[DF_BATCH], const float (&v)[DF_NG][DF_MB], uint32_t *xs, float *sums){
+    int lane4 = (threadIdx.x & 63) << 2; asm("" : "+v"(lane4));
+#pragma unroll
+    for(int p = 0; p < DF_NG * DF_MB; p++) xs[p * DF_XPLANE + (lane4 & 12) * 4 + (lane4 >> 4)] = __float_as_uint(v[p / DF_MB][p % DF_MB]);
+    const uint32_t *xf = xs + ((lane4 >> 5) & 1) * DF_MB * DF_XPLANE + (lane4 >> 6) * 16;
+    auto from = [&](int flip, float v){ return __int_as_float(__builtin_amdgcn_ds_bpermute(lane4 ^ (flip << 2), __float_as_int(v))); };
+    const bool hi32 = lane4 & 128;
+    float *mine = sums + ((lane4 >> 2) & 15) * 16 + (hi32 ? 8 : 0);
+#pragma unroll 1
+    for(int j = 0; j < 8; j++){
+        float fx[DF_MB] = {}, fy[DF_MB] = {};             /* columns j and 8 + j */
+#pragma unroll
+        for(int b = 0; b < 2 * DF_BATCH; b++){
+            const uint2 w = b < DF_BATCH ? w0[b % DF_BATCH] : w1[b % DF_BATCH];
+            const float dx = (float)(int)__builtin_amdgcn_sbfe(w.x, 4 * j, 4), dy = (float)(int)__builtin_amdgcn_sbfe(w.y, 4 * j, 4);
+#pragma unroll
+            for(int m = 0; m < DF_MB; m++){
+                const float x = __uint_as_float(xf[m * DF_XPLANE + b]);
+                fx[m] = fmaf(x, dx, fx[m]);
+                fy[m] = fmaf(x, dy, fy[m]);
+            }
+        }
+#pragma unroll
+        for(int m = 0; m < DF_MB; m++){
+            const float half = (hi32 ? fy[m] : fx[m]) + from(32, hi32 ? fx[m] : fy[m]);
+            mine[m * DF_CW + j] = half + from(16, half);  /* the same word from two lanes */
+        }
+    }
+}
+
 /* dst[m*mstride + chunk*256 + c] = sum_{r<rows} x[m][r] * s * digit(k0+r, chunk*256+c), m < M, stored
  * tagged. w0, w1 hold the digits of the task's two halves, requested earlier. `prep` stages the inputs
  * (df_stage) and returns the power of two to apply to the sums. `next0` and `next1` request the following
@@ -566,6 +614,7 @@ __device__ __forceinline__ long df_pair(uint32_t lo, uint32_t hi){ return (long)
  * are the four bytes of two inputs in two scale groups (df_stage_i8); the products are exact, a lane's four sums are the
  * bytes of one input and are put together in fp32 at the end. Half of the lanes hold an input times the columns of
  * the other scale group, which nobody reads. 11 sequences, 64 experts top-4, 2048 x 1408: 61 -> 45 us per layer.
+ * A wavefront whose inputs the fixed point does not hold (df_stage_i8) takes fp32 multiply-adds instead (df_fma_task).
  *
  * The fp16-input loop's multiply-adds are v_dot2_f32_f16: two products per instruction, exact, summed in fp32. One operand is the
  * pair of digits of a lane's two rows as fp16, built without a conversion: with u = digit + 8 (two's complement
@@ -575,12 +624,17 @@ __device__ __forceinline__ long df_pair(uint32_t lo, uint32_t hi){ return (long)
  * of staged inputs (divided by 16 for the odd columns). What the offsets add -- (1024 + 8) and (64 + 8) times
  * the sum of the staged inputs -- is taken out at the end. The inputs thus carry 11 significant bits. */
 template<class PREP, class NEXT0, class NEXT1>
-__device__ __forceinline__ void df_task_i8(const DfArgs &a, const DfT &t, uint2 (&w0)[DF_BATCH], uint2 (&w1)[DF_BATCH], const uint32_t *xs,
+__device__ __forceinline__ void df_task_i8(const DfArgs &a, const DfT &t, uint2 (&w0)[DF_BATCH], uint2 (&w1)[DF_BATCH], uint32_t *xs,
                                            float *red, u64 *dst, size_t mstride, PREP prep, NEXT0 next0, NEXT1 next1 DF_TRACE_PARAM){
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
     const int N = t.N, M = t.M, chunk = t.chunk;
     DF_STAMP(10 + 16 * t.list);
-    prep();
+    float v[DF_NG][DF_MB];
+    prep(v);
+    const bool plain = df_stage_i8(v, M, xs);
+    /* such a wavefront then goes through the loop below with the others and drops what comes out: branches around its halves would
+     * stand between the multiplications and the requests that are interleaved with them (sixteen tokens 28.9 -> 29.6 us) */
+    if(plain) df_fma_task(w0, w1, v, xs, red + wave * DF_MB * DF_CW);
     DF_STAMP(11);
     __builtin_amdgcn_s_setprio(0);
     df_i32x4 acc[16];
@@ -617,18 +671,18 @@ __device__ __forceinline__ void df_task_i8(const DfArgs &a, const DfT &t, uint2 
     next1();
     __builtin_amdgcn_s_setprio(3);
     DF_STAMP(13);
-    __syncthreads();                                      /* the sums of the task before have been read */
-    const int m = g & 1;
-    if((c >= 8) == (g >= 2) && m < M){
-        const int ex = (int)xs[(g >> 1) * DF_MB * DF_XPLANE + m * DF_XPLANE + DF_XEXP], e = ex - 160;
-        const float up = ex == 255 ? __builtin_nanf("") : 65536.0f;
+    /* the places from here on are worked out anew: kept from the loop's start they would be the registers too many */
+    int here = tid; asm("" : "+v"(here));
+    const int ec = here & 15, eg = (here >> 4) & 3, ew = here >> 6;
+    if(!plain && (ec >= 8) == (eg >= 2) && (eg & 1) < M){
+        const int e = (int)xs[eg * DF_XPLANE + DF_XEXP] - 160;          /* lane group = plane: scale group * DF_MB + input */
         float y[16];
 #pragma unroll
         for(int j = 0; j < 16; j++){
             const int hi = (acc[j][3] << 8) + acc[j][2], lo = (acc[j][1] << 8) + acc[j][0];
-            y[j] = __builtin_amdgcn_ldexpf(fmaf((float)hi, up, (float)lo), e);
+            y[j] = __builtin_amdgcn_ldexpf(fmaf((float)hi, 65536.0f, (float)lo), e);
         }
-        float4 *o = (float4 *)&red[(wave * DF_MB + m) * DF_CW + c * 16];
+        float4 *o = (float4 *)&red[(ew * DF_MB + (eg & 1)) * DF_CW + ec * 16];
 #pragma unroll
         for(int q = 0; q < 4; q++) o[q] = make_float4(y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]);
     }
@@ -747,7 +801,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
     __shared__ __align__(16) uint32_t xs_raw[4 * DF_NG * DF_MB * DF_XPLANE];   /* staged inputs: df_stage (fp16 pairs) or, a quarter per wavefront, df_stage_i8 */
     __shared__ float wmax[4];
     __shared__ DfT tasks[DF_MAXTASKS];
-    __shared__ float red[4 * DF_MB * DF_CW];
+    __shared__ float red[(H ? 1 : 2) * 4 * DF_MB * DF_CW];    /* matrix-core loop: two, of which a task writes one while the task before it is read in the other */
     __shared__ int giveup;
     const int tid = threadIdx.x;
     __builtin_amdgcn_s_setprio(3);
@@ -886,6 +940,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
         return t;
     };
     uint2 w0[DF_BATCH], w1[DF_BATCH];
+    int flip = 0;
     const int hs1 = a.R1 >> 6, hs2 = a.R2 >> 6;              /* fp16-input loop: steps of 32 rows per half task */
     const int gprF = a.F / a.group, gprD = a.D / a.group;     /* scale groups per row of w1|w3 and of w2 */
     const int cpg = a.group >= DF_CW ? a.group / DF_CW : 1;   /* chunks per scale group when the group is wider than a chunk */
@@ -947,7 +1002,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                 for(int gg = 0; gg < DF_NG; gg++){
                     const float sc = (gg < ng ? chunk * DF_CW + gg * a.group < a.F : !H) ? csc[gg] : 0.0f;
 #pragma unroll
-                    for(int m = 0; m < DF_MB; m++) v[gg][m] = xv[m] * sc;
+                    for(int m = 0; m < DF_MB; m++){ const float x = xv[m] * sc; v[gg][m] = live ? x : 0.0f; }   /* the last row's scale may be no finite number */
                 }
             } else {
                 const u64 *p1 = a.part1 + (((size_t)prob * 2) * a.S1 * DF_MB) * a.F + k0;
@@ -981,7 +1036,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                 for(int gg = 0; gg < DF_NG; gg++){
                     const float sc = (gg < ng ? chunk * DF_CW + gg * a.group < a.D : !H) ? csc[gg] : 0.0f;
 #pragma unroll
-                    for(int m = 0; m < DF_MB; m++) v[gg][m] = hv[m] * sc;
+                    for(int m = 0; m < DF_MB; m++){ const float x = hv[m] * sc; v[gg][m] = live ? x : 0.0f; }   /* the last row's scale may be no finite number */
                 }
             }
             return live;
@@ -993,10 +1048,10 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
             else       df_task_h<2>(a, cur, w0, w1, hs, xs_raw, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
         } else {
             uint32_t *xs = xs_raw + (tid >> 6) * (DF_NG * DF_MB * DF_XPLANE);
-            auto prep = [&](){ float v[DF_NG][DF_MB]; inputs(v); df_stage_i8(v, xs); };
-            df_task_i8(a, cur, w0, w1, xs, red, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
+            auto prep = [&](float (&v)[DF_NG][DF_MB]){ inputs(v); };
+            df_task_i8(a, cur, w0, w1, xs, red + flip, dst, mstride, prep, next0, next1 DF_TRACE_ARG);
         }
-        cur = nxt;
+        cur = nxt; flip ^= 4 * DF_MB * DF_CW;
 #pragma unroll
         for(int gg = 0; gg < DF_NG; gg++) csc[gg] = nsc[gg];
     }

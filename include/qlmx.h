@@ -393,8 +393,11 @@ int qlmx_test_force_wait_timeout(int which);
  * from outside the process. */
 int qlmx_nt_tile(int tile);
 /* Math mode of the decode layer (no counterpart in the reference, whose decode path multiplies in fp32; the same
- * kind of choice as QLMX_MATH_MFMA_F16 for the training forward). fp16_inputs = 0, the default: inputs to fp32
- * precision, 4e-7 relative L2 on a layer's output against the fp32 reference. fp16_inputs = 1: a task's inputs (x times the
+ * kind of choice as QLMX_MATH_MFMA_F16 for the training forward). fp16_inputs = 0, the default: exact products of the
+ * digits with inputs of 31 bits under one power of two for the (at most 64) rows of a wavefront, scale group by scale group --
+ * an input down to 2^-7 of the largest of them keeps all its bits, every one is held to 2^-31 of the largest -- or, where most
+ * of these inputs lie below 2^-8 of the largest or one is infinite or NaN, fp32 multiply-adds; 4e-7 relative L2 on a layer's
+ * output against the fp32 reference. fp16_inputs = 1: a task's inputs (x times the
  * group scale, or silu(gate) * up times the group scale) are rounded to fp16 -- 11 significant bits, scaled per
  * task so that nothing underflows -- and multiplied with the exact digits by v_dot2_f32_f16 into fp32 sums:
  * 3.7e-4. Applies to both decode entry points from the next call on;

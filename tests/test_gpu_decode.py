@@ -351,3 +351,33 @@ def test_decode_neighbouring_scale_groups_of_different_size(q, orc, n):
         b.s2[:, f:f + b.group] *= f32(2.0 ** min(2 * n, 100))
     got, want = b.run(q), b.want()
     assert rel64(got, want) < 1e-6
+
+
+@pytest.mark.parametrize("n", [4, 9, 12, 20, 30])
+def test_decode_columns_that_take_nothing_of_the_largest_input(q, orc, n):
+    """One input 2^n times the others, whose digits are zero in most columns: those columns are sums of the small inputs alone.
+    The few columns that do hold it have down rows of zeros, so the output is of the small ones alone too."""
+    a = Layer64(orc, 300 + n)
+    a.x[:, 5] *= f32(2.0 ** n); a.x[1, 200] *= f32(2.0 ** n)
+    for d in (a.d1, a.d3):
+        d[:, (5, 200), 8:] = 0
+    a.d2[:, :8] = 0
+    got, want = a.run(q), a.want()
+    for t in range(a.T):
+        assert rel64(got[t], want[t]) < 1e-6, t
+
+
+@pytest.mark.parametrize("v", [np.nan, np.inf])
+def test_decode_nan_and_infinite_scales_stay_in_their_columns(q, orc, v):
+    """A scale of the down projection that is no finite number reaches the columns of its group as fp32 multiply-adds take it
+    there (an infinity times the digit 0 is NaN), and no others."""
+    a = Layer64(orc, 400)
+    want = a.want()
+    a.s2[1, 77, 1] = v
+    got = a.run(q)
+    there = slice(a.group, 2 * a.group)
+    nan = np.isnan(v) | (a.d2[1, 77, there] == 0)
+    assert np.array_equal(np.isnan(got[:, there]), np.broadcast_to(nan, (a.T, a.group)))
+    assert np.array_equal(np.isinf(got[:, there]), np.broadcast_to(~nan, (a.T, a.group)))
+    for c in (0, 2 * a.group):
+        assert rel64(got[:, c:c + a.group], want[:, c:c + a.group]) < 1e-6, c
