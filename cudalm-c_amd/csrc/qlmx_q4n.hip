@@ -17,7 +17,8 @@
 #include <string.h>
 #include <algorithm>
 #include <atomic>
-#include <system_error>
+#include <new>
+#include <stdexcept>
 #include <thread>
 #include <vector>
 
@@ -31,10 +32,11 @@
 #define Q4N_WRITE_SHARE (128 * 1024)
 #define Q4N_READ_SHARE (256 * 1024)
 #define Q4N_MAX_THREADS 8
-static int q4n_parts(size_t n, size_t share){
+static int q4n_parts(size_t n, size_t ngroups, size_t share){
     const unsigned hw = std::thread::hardware_concurrency();
-    return (int)std::max<size_t>(1, std::min<size_t>(n / share, std::min<unsigned>(Q4N_MAX_THREADS, hw)));
+    return (int)std::max<size_t>(1, std::min({n / share, ngroups, (size_t)std::min<unsigned>(Q4N_MAX_THREADS, hw)}));
 }
+static size_t q4n_groups(size_t n, int group){ return n / (size_t)group + (n % (size_t)group != 0); }
 /* first(part) for every part, and once all are done, second(part) */
 template<class F, class S> static void q4n_run(int parts, const F &first, const S &second){
     std::atomic<int> done(0);
@@ -43,17 +45,16 @@ template<class F, class S> static void q4n_run(int parts, const F &first, const 
         while(done.load(std::memory_order_acquire) < parts) std::this_thread::yield();
         for(int p = p0; p < p1; p++) second(p);
     };
-    std::vector<std::thread> th;
-    th.reserve((size_t)parts);
+    std::thread th[Q4N_MAX_THREADS];
     int own = 0;                                           /* parts from here on are this thread's */
     for(; own + 1 < parts; own++){
         const int p = own;
-        try { th.emplace_back([&, p]{ first(p); finish(p, p + 1); }); }
-        catch(const std::system_error &){ break; }         /* no more threads to be had */
+        try { th[p] = std::thread([&, p]{ first(p); finish(p, p + 1); }); }
+        catch(const std::exception &){ break; }            /* no more threads, or no memory for one, to be had */
     }
     for(int p = own; p < parts; p++) first(p);
     finish(own, parts);
-    for(auto &t : th) t.join();
+    for(int p = 0; p < own; p++) th[p].join();
 }
 static bool q4n_avx2(){ static const bool yes = __builtin_cpu_supports("avx2"); return yes; }
 
@@ -152,15 +153,11 @@ extern "C" size_t qlmx_q4n_bound(size_t n, int group){
     return 4 * ((n + (size_t)group - 1) / (size_t)group) + 4 * n;
 }
 
-extern "C" int qlmx_q4n_quantize(const float *P, size_t n, int group, unsigned char *out, size_t cap,
-                                 size_t *out_len, size_t *nraw){
-    QLMX_REQUIRE(P && out && out_len, "qlmx_q4n_quantize: NULL buffer");
-    QLMX_REQUIRE(group > 0 && group % 2 == 0, "qlmx_q4n_quantize: group %d must be positive and even", group);
-    QLMX_REQUIRE(cap >= qlmx_q4n_bound(n, group), "qlmx_q4n_quantize: output buffer smaller than qlmx_q4n_bound()");
-    const size_t ngroups = (n + (size_t)group - 1) / (size_t)group;
-    const int parts = q4n_parts(n, Q4N_WRITE_SHARE);
+static int q4n_write(const float *P, size_t n, int group, unsigned char *out, size_t *out_len, size_t *nraw){
+    const size_t ngroups = q4n_groups(n, group);
+    const int parts = q4n_parts(n, ngroups, Q4N_WRITE_SHARE);
     std::vector<float> scales(ngroups);
-    const size_t stride = (size_t)group + 256;             /* a part's digits share no cache line with another's */
+    const size_t stride = std::min((size_t)group, n) + 256;     /* a part's digits share no cache line with another's */
     std::vector<signed char> digits((size_t)parts * stride);
     size_t len[Q4N_MAX_THREADS] = {}, raw[Q4N_MAX_THREADS] = {};
     auto begin = [&](int p){ return ngroups * (size_t)p / (size_t)parts; };
@@ -197,27 +194,26 @@ extern "C" int qlmx_q4n_quantize(const float *P, size_t n, int group, unsigned c
     return QLMX_OK;
 }
 
-extern "C" int qlmx_q4n_dequantize(const unsigned char *buf, size_t len, float *P, size_t n, int group, size_t *used){
-    QLMX_REQUIRE(buf && P, "qlmx_q4n_dequantize: NULL buffer");
-    QLMX_REQUIRE(group > 0, "qlmx_q4n_dequantize: group %d", group);
-    const size_t ngroups = (n + (size_t)group - 1) / (size_t)group;
-    std::vector<size_t> at(ngroups + 1);                   /* where a group starts */
+static int q4n_read(const unsigned char *buf, size_t len, float *P, size_t n, int group, size_t *used){
+    const size_t ngroups = q4n_groups(n, group);
+    /* where a group starts: for as many as the buffer can hold at most (all but the last are whole), not as n names */
+    std::vector<size_t> at(std::min(ngroups, len / (4 + ((size_t)group + 1) / 2) + 1));
     size_t o = 0;
     for(size_t q = 0; q < ngroups; q++){
         const size_t g = std::min((size_t)group, n - q * (size_t)group);
         float scale;
-        QLMX_REQUIRE(o + 4 <= len, "qlmx_q4n_dequantize: buffer ends inside group %zu", q);
+        QLMX_REQUIRE(len - o >= 4, "qlmx_q4n_dequantize: buffer ends inside group %zu", q);
         memcpy(&scale, buf + o, 4);
         at[q] = o; o += 4;
         if(scale != scale){
-            QLMX_REQUIRE(o + 4 * g <= len, "qlmx_q4n_dequantize: buffer ends inside raw group %zu", q);
+            QLMX_REQUIRE((len - o) / 4 >= g, "qlmx_q4n_dequantize: buffer ends inside raw group %zu", q);
             o += 4 * g;
         } else {
-            QLMX_REQUIRE(o + (g + 1) / 2 <= len, "qlmx_q4n_dequantize: buffer ends inside group %zu", q);
+            QLMX_REQUIRE(len - o >= (g + 1) / 2, "qlmx_q4n_dequantize: buffer ends inside group %zu", q);
             o += (g + 1) / 2;
         }
     }
-    const int parts = q4n_parts(n, Q4N_READ_SHARE);
+    const int parts = q4n_parts(n, ngroups, Q4N_READ_SHARE);
     q4n_run(parts, [&](int p){
         for(size_t q = ngroups * (size_t)p / (size_t)parts; q < ngroups * (size_t)(p + 1) / (size_t)parts; q++){
             const size_t i = q * (size_t)group;
@@ -230,4 +226,26 @@ extern "C" int qlmx_q4n_dequantize(const unsigned char *buf, size_t len, float *
     }, [](int){});
     if(used) *used = o;
     return QLMX_OK;
+}
+
+/* What a call does, with an allocation that fails as an error of the call: no exception passes a C entry point. */
+template<class F> static int q4n_guarded(const char *who, const F &body){
+    try { return body(); }
+    catch(const std::bad_alloc &){}
+    catch(const std::length_error &){}                     /* more than a vector can name */
+    qlmx_set_error("%s: out of memory for the scratch", who);
+    return QLMX_E_LIMIT;
+}
+extern "C" int qlmx_q4n_quantize(const float *P, size_t n, int group, unsigned char *out, size_t cap,
+                                 size_t *out_len, size_t *nraw){
+    QLMX_REQUIRE(P && out && out_len, "qlmx_q4n_quantize: NULL buffer");
+    QLMX_REQUIRE(group > 0 && group % 2 == 0, "qlmx_q4n_quantize: group %d must be positive and even", group);
+    QLMX_REQUIRE(cap >= qlmx_q4n_bound(n, group), "qlmx_q4n_quantize: output buffer smaller than qlmx_q4n_bound()");
+    return q4n_guarded("qlmx_q4n_quantize", [&]{ return q4n_write(P, n, group, out, out_len, nraw); });
+}
+
+extern "C" int qlmx_q4n_dequantize(const unsigned char *buf, size_t len, float *P, size_t n, int group, size_t *used){
+    QLMX_REQUIRE(buf && P, "qlmx_q4n_dequantize: NULL buffer");
+    QLMX_REQUIRE(group > 0, "qlmx_q4n_dequantize: group %d", group);
+    return q4n_guarded("qlmx_q4n_dequantize", [&]{ return q4n_read(buf, len, P, n, group, used); });
 }

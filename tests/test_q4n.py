@@ -1,6 +1,10 @@
 """q4n wire format (quantize_params / dequantize_params qtype 3, cudalm.cu:638-656, 688-696): the
 oracle's restatement and the library's host functions against the bytes the compiled reference wrote
 (tests/golden/q4n.npz). Host code only, so these run without a GPU; byte-exact both ways."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -8,6 +12,7 @@ from __graft_entry__ import load_package
 
 pkg = load_package()
 f32 = np.float32
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.fixture(scope="module")
@@ -99,6 +104,54 @@ def test_truncated_buffer_is_refused(lib, orc, golden):
             lib.q4n_dequantize(g["buf"][:cut].copy(), n, group)
         ok, _ = orc.q4n_dequantize(g["buf"][:cut].copy(), n, group)
         assert ok == 0
+
+
+@pytest.mark.parametrize("n", [2 ** 31, 2 ** 50, 2 ** 64 - 1, 2 ** 64 - 200])
+def test_count_larger_than_the_buffer_is_refused(lib, n):
+    """A count that the buffer cannot hold (a damaged file names any) ends at the group where the buffer does, whatever the
+    scratch for that many groups would have been."""
+    import ctypes
+    group = 128
+    whole, _ = lib.q4n_quantize(np.zeros(3 * group, f32), group)
+    for buf, at in ((whole[:8].copy(), 0), (whole, 3)):
+        P, used = np.zeros(4 * group, f32), ctypes.c_size_t(0)
+        with pytest.raises(pkg.QlmxError, match="buffer ends inside group %d$" % at):
+            lib.call("qlmx_q4n_dequantize", buf, buf.size, P, n, group, ctypes.addressof(used))
+
+
+def limited(code, spare):
+    """Runs `code` in a process that may take `spare` bytes of memory more than it holds when the library is loaded."""
+    head = ("import resource, numpy as np\nfrom __graft_entry__ import load_package\n"
+            "pkg = load_package(); lib = pkg.Qlmx(init=False); f32 = np.float32\n"
+            "def limit():\n"
+            "    now = int(open('/proc/self/statm').read().split()[0]) * resource.getpagesize()\n"
+            "    resource.setrlimit(resource.RLIMIT_AS, (now + %d, now + %d))\n" % (spare, spare))
+    return subprocess.run([sys.executable, "-c", head + code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+
+
+def test_scratch_is_bounded_by_the_values():
+    """A group far longer than the values is one group of all of them: no scratch for what is not there."""
+    r = limited("P = (np.arange(300000) %% 15 - 7).astype(f32) * f32(0.25)\n"
+                "want, _ = lib.q4n_quantize(P, 300000)\nlimit()\n"
+                "for group in (300002, 2 ** 31 - 2):\n"
+                "    got, raw = lib.q4n_quantize(P, group)\n"
+                "    assert raw == 0 and np.array_equal(got, want)\n"
+                "    back, used = lib.q4n_dequantize(got, P.size, group)\n"
+                "    assert used == got.size and np.array_equal(back, P)\n".replace("%%", "%"), 256 << 20)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
+def test_allocation_failure_is_an_error_code():
+    """Scratch that cannot be had is reported as an error of the call; the process goes on and a smaller call works."""
+    r = limited("n = 24 << 20\nbuf = np.zeros(5 * n, np.uint8); P = np.zeros(n, f32); out = np.zeros(8 * n, np.uint8)\nlimit()\n"
+                "import ctypes; u = ctypes.c_size_t(0)\n"
+                "for name, args in (('qlmx_q4n_dequantize', (buf, buf.size, P, n, 1, ctypes.addressof(u))),\n"
+                "                   ('qlmx_q4n_quantize', (P, n, 2, out, out.size, ctypes.addressof(u), None))):\n"
+                "    try:\n        lib.call(name, *args)\n"
+                "    except pkg.QlmxError as e:\n        assert 'memory' in str(e), e\n"
+                "    else:\n        raise AssertionError(name)\n"
+                "back, used = lib.q4n_dequantize(buf[:50], 10, 1)\nassert used == 50 and not back.any()\n", 40 << 20)
+    assert r.returncode == 0, r.stderr[-2000:]
 
 
 def test_against_reference_library_when_present(lib, orc, ref):
