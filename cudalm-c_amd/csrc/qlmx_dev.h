@@ -137,6 +137,14 @@ __device__ __forceinline__ float qx_wave_max(float v){
     return v;
 }
 
+/* Between LDS writes and the reads of them by other lanes of the same wavefront: nothing the hardware has to do (a wavefront's LDS
+ * accesses are carried out in order), but the compiler may neither move accesses across nor take them for another thread's. */
+__device__ __forceinline__ void qx_wave_sync(){
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 /* cpu_kern.h:29-34: clamp, Cody-Waite split of ln 2, degree-6 Horner polynomial, exponent built
  * with integer bit arithmetic */
 __device__ __forceinline__ float qx_fexp(float x){

@@ -493,7 +493,7 @@ __device__ __forceinline__ float df_stage(const float (&v)[DF_NG][DF_MB], bool l
  * normally distributed inputs 0.6 % lie there and of silu(gate) * up 2 to 5 %, so that ordinary layers keep to the fixed point
  * (with a quarter as the line one wavefront in a thousand would not, and a layer waits for each).
  * xs: [plane g * DF_MB + m][lane group of the loop][row of the group], behind the rows the biased exponent of the largest; written
- * and read by one wavefront, so no barrier. */
+ * and read by one wavefront, so no workgroup barrier. */
 #define DF_XPLANE 68          /* 64 rows, and 4 words so that the 16 (plane, lane group) pairs of a read start in different banks */
 #define DF_XEXP 64            /* the first of these words */
 __device__ __forceinline__ unsigned df_wave_max(unsigned v){
@@ -521,6 +521,7 @@ __device__ __forceinline__ bool df_stage_i8(const float (&v)[DF_NG][DF_MB], int 
             plain |= (int)(2 * low > __popcll(__ballot(mag != 0u))) | (int)(ex == 255u);
         }
     }
+    qx_wave_sync();
     return __builtin_amdgcn_readfirstlane(plain) != 0;
 }
 
@@ -574,6 +575,7 @@ __device__ __forceinline__ void df_fma_task(const uint2 (&w0)[DF_BATCH], const u
     int lane4 = (threadIdx.x & 63) << 2; asm("" : "+v"(lane4));
 #pragma unroll
     for(int p = 0; p < DF_NG * DF_MB; p++) xs[p * DF_XPLANE + (lane4 & 12) * 4 + (lane4 >> 4)] = __float_as_uint(v[p / DF_MB][p % DF_MB]);
+    qx_wave_sync();
     const uint32_t *xf = xs + ((lane4 >> 5) & 1) * DF_MB * DF_XPLANE + (lane4 >> 6) * 16;
     auto from = [&](int flip, float v){ return __int_as_float(__builtin_amdgcn_ds_bpermute(lane4 ^ (flip << 2), __float_as_int(v))); };
     const bool hi32 = lane4 & 128;
@@ -850,6 +852,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
             if(m == 0){ mt.p_e[prob] = e_in; mt.p_M[prob] = min(DF_MB, __popcll(peers) - pos); }
         }
         if(live){ mt.pair_prob[tid] = valid ? prob : -1; mt.pair_m[tid] = valid ? m : 0; }
+        qx_wave_sync();
         const int nprob = __popcll(starts);
         /* ---- this workgroup's tasks, list 1 (gate|up) then list 2 (down), in one stream so that the
          * first digits of a task are already on their way while the task before it finishes ---- */

@@ -228,6 +228,7 @@ __global__ void __launch_bounds__(1024) k_gp_place(const int *asn, int N, int E,
             perm[(size_t)k * N + first[e] + row + rank] = n;
             if(rank == 0) mine[e] = row + __popcll(same);
         }
+        qx_wave_sync();
     }
 }
 
