@@ -819,9 +819,12 @@ extern "C" int qlmx_step_touched(float *P, const float *Gc, signed char *d, sign
  * memory (the last workgroup resets its counter): calls that overlap on different streams would
  * mix their pieces and are not supported.
  *
- * The hand-over is device-scope accesses, which go past the caches, and a wait for the store in front of the count. As an
- * acquire-release count it wrote back and invalidated an XCD's L2 once per workgroup, which cost more than the reading:
- * 127 us for 125.8 M values, 18 for any small number. A stretch of its own per workgroup keeps what it reads in few DRAM
+ * The hand-over is device-scope accesses and a wait for the store in front of the count. What it rests on: a device-scope store is
+ * written through the XCD's L2 to the memory behind it that all XCDs share (it leaves no dirty line there, so there is nothing a
+ * release would have to write back), vmcnt counts it until that memory has acknowledged it, and a device-scope load reads from
+ * there; the count is carried out there too, so whoever sees it complete reads every sum. As an acquire-release count it wrote
+ * back and invalidated an XCD's L2 once per workgroup, which cost more than the reading: 127 us for 125.8 M values, 18 for any
+ * small number. A stretch of its own per workgroup keeps what it reads in few DRAM
  * pages: 6.1 TB/s at any grid of 1024 workgroups or more, side by side 4.9 to 5.8. A gradient larger than the last-level
  * cache (256 MB) is read past the caches (NT): norm and step of 125.8 M weights 551 -> 530 us. Of a smaller one the step
  * finds a part there, and the plain loads stay (40 M weights: 169 us, 172 with NT). */
