@@ -24,7 +24,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libqlmx.so")
 HOST_LIB = os.path.join(HERE, "libqlmx_host.so")
-CALL_LIB = os.path.join(HERE, "_qlmx_call.so")
+CALL_LIB = os.path.join(HERE, "_qlmx_call" + sysconfig.get_config_var("EXT_SUFFIX"))     # the ABI tag: no other interpreter loads it
 ARCH = "gfx950"
 
 HIP_SOURCES = ["qlmx_runtime.hip", "qlmx_step.hip", "qlmx_codec.hip", "qlmx_gemm_common.hip",
@@ -126,9 +126,23 @@ def build_all(jobs=8):
         _run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(HERE, "..", "include"),
               os.path.join(HERE, "host", "selftest.cpp"), "-o", os.path.join(HERE, "qlm_selftest"),
               "-L", HERE, "-lqlmx_host", "-lqlmx", "-Wl,-rpath,$ORIGIN"])
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-I", os.path.join(HERE, "..", "include"), "-I", sysconfig.get_paths()["include"],
-          os.path.join(HERE, "host", "qlmx_call.cpp"), "-o", CALL_LIB])
+    build_call_module()
     return LIB
+
+
+def build_call_module(out=CALL_LIB, include=None):
+    """Python's way into the inner loop's calls, for the interpreter that runs this. Without its C headers there is none, and
+    binding.py makes every call through ctypes. What an earlier build left is removed first."""
+    include = include or sysconfig.get_paths()["include"]
+    for f in (out, os.path.join(os.path.dirname(out), "_qlmx_call.so")):
+        if os.path.exists(f):
+            os.remove(f)
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print("no Python.h in %s: calls go through ctypes" % include, flush=True)
+        return None
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-I", os.path.join(HERE, "..", "include"), "-I", include,
+          os.path.join(HERE, "host", "qlmx_call.cpp"), "-o", out])
+    return out
 
 
 def _drain(procs):

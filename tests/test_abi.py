@@ -65,3 +65,19 @@ def test_compute_refuses_without_device(lib):
     buf = np.zeros(256, np.float32)
     rc = lib.lib.qlmx_render(buf.ctypes.data, buf.ctypes.data, buf.ctypes.data, buf.ctypes.data, 1, 128, 1, 0, 1, None)
     assert rc == -3 and "qlmx_init" in lib.last_error()
+
+
+def test_call_module_belongs_to_one_interpreter_and_may_be_missing(tmp_path):
+    """The compiled call module carries the interpreter's ABI tag, so that no other interpreter takes it for its own; where
+    Python's C headers are not installed the build goes on without it (every call then goes through ctypes)."""
+    import importlib.util
+    import sysconfig
+    spec = importlib.util.spec_from_file_location("qlmx_build", os.path.join(ROOT, "cudalm-c_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec); spec.loader.exec_module(build)
+    assert build.CALL_LIB.endswith("_qlmx_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+    stale = tmp_path / "_qlmx_call.so"; stale.write_bytes(b"")
+    out = tmp_path / os.path.basename(build.CALL_LIB); out.write_bytes(b"")
+    assert build.build_call_module(str(out), include=str(tmp_path)) is None
+    assert not out.exists() and not stale.exists()             # nothing of another build is left to be loaded
+    from cudalm_c_amd import binding
+    assert binding._qlmx_call is None or binding._qlmx_call.__file__ == build.CALL_LIB
