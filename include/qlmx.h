@@ -174,10 +174,15 @@ int qlmx_servo(signed char *d, signed char *r, float *s,
  * call takes the whole queue: an array of problems that share K and N. Results equal the
  * reference's P = s*digit -> fp32 SGEMM semantics to rounding (fp32 math) or to bf16-MFMA
  * accumulation order (MFMA math); C is always fp32.
+ * Which kernel a call runs -- tiles of 256 rows or of 64 and fewer, the contraction in one piece or shared by several
+ * wavefronts or workgroups and added up -- depends on the row counts of all its problems, on K, N and the group. Calls of the
+ * same sizes give the same bits, and so do the forms below that are said to. A problem's rows beside other problems than
+ * before (a sequence served in another batch) may differ in the last bits: by the order of K fp32 additions, about 1e-6 of
+ * the result and never by the precision of a product. A caller that needs bits that do not depend on the batch keeps the sizes.
  * ===================================================================================== */
 #define QLMX_ACT_F32   0     /* activation operands are fp32                         */
 #define QLMX_ACT_BF16  1     /* activation operands are bf16 (high half of an fp32)  */
-#define QLMX_MATH_F32  0     /* fp32 FMA on the vector ALU                           */
+#define QLMX_MATH_F32  0     /* fp32 products and sums (fp32 matrix core)            */
 #define QLMX_MATH_MFMA 1     /* bf16 MFMA, fp32 accumulate                           */
 #define QLMX_MATH_MFMA_F16 2 /* as QLMX_MATH_MFMA, except that qlmx_moe_gemm_nn on bf16 activations runs on the fp16
                               * matrix core: the activations are converted exactly (|x| in [2^-14, 65504]; smaller ones
@@ -291,6 +296,8 @@ int qlmx_moe_gemm_nt(const qlmx_gemm_prob *probs_host, int nprob, int K, int N,
  *   w1q/w3q/w2q: element offsets of expert 0's matrices in d; expert e adds e*D*F. All multiples of
  *   `group`; w1, w3 are [D,F] row-major and w2 is [F,D] row-major (cudalm.cu:263-265). The scale of
  *   element q is s[q / group] (every span a multiple of the group, true of all reference presets).
+ * The contractions are split by T, K, E, D and F, and two tokens on one expert share the choice between the two ways of
+ * multiplying (qlmx_decode_math): equal calls give equal bits, a token served beside others the last bits of another order.
  * Limits: K*T <= 64 pairs, D and F multiples of 32 and <= 8192 (QLMX_E_LIMIT for the few shapes in that range
  * whose task lists a workgroup cannot hold). Uses a library-owned workspace that
  * is (re)allocated on first use or growth; calls on different streams must not overlap. The tag that

@@ -195,6 +195,21 @@ def test_f32_shapes_of_a_workgroup(q, orc, mode, K, N, rows, act):
     assert orc.relerr(got, want) < TOL_F32
 
 
+@pytest.mark.parametrize("mode,K,N,math,company", [("nn", 768, 2048, "f16", [600]), ("tn", 768, 2048, "mfma", [3000]), ("nn", 768, 512, "f32", [3000]),
+                                                   ("nn", 768, 512, "f32", [13000]), ("tn", 768, 512, "f32", [3000])])
+@pytest.mark.parametrize("M", [3, 16])
+def test_rows_alone_and_in_company(q, orc, mode, K, N, math, company, M):
+    """The kernel, and with it the order of the sums, is chosen by the sizes of the whole call: a problem's rows come out with the
+    same bits in every call of the same sizes, and beside other problems within what two orders of K fp32 additions differ by
+    (each within sqrt(K) * 2^-24 of the exact sum: 3.3e-6 for both)."""
+    act, m = (pkg.ACT_F32, pkg.MATH_F32) if math == "f32" else (pkg.ACT_BF16, pkg.MATH_MFMA_F16 if math == "f16" else pkg.MATH_MFMA)
+    alone, _ = run_case(q, orc, mode, 1, [M], K, N, act, m, seed=31)
+    again, _ = run_case(q, orc, mode, 1, [M], K, N, act, m, seed=31)
+    beside, _ = run_case(q, orc, mode, 2, [M] + company, K, N, act, m, seed=31)
+    assert np.array_equal(alone.view(np.uint32), again.view(np.uint32))
+    assert orc.relerr(beside[:M * N], alone) < 3.3e-6
+
+
 # ------------------------------------------------------------------ bf16 MFMA kernels
 @pytest.mark.parametrize("mode", ["nn", "tn", "nt"])
 def test_mfma_grouped_zipf_small(q, orc, mode):
