@@ -5,7 +5,6 @@
 #include <stdint.h>
 #include "../../include/qlmx.h"
 
-#define QLMX_WAVE 64
 
 /* ---- error plumbing (host) ---- */
 void qlmx_set_error(const char *fmt, ...);
@@ -127,13 +126,9 @@ template<int W> __device__ __forceinline__ int qx_team_sum(int v){
     v += qx_dpp_i<0x141>(v);
     return W == 16 ? v + qx_dpp_i<0x140>(v) : v;
 }
-/* full 64-lane sum / max built from the row step plus two cross-row exchanges */
+/* full 64-lane sum */
 __device__ __forceinline__ float qx_wave_sum(float v){
     for(int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-__device__ __forceinline__ float qx_wave_max(float v){
-    for(int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
     return v;
 }
 

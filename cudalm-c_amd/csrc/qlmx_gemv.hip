@@ -427,10 +427,6 @@ __device__ __forceinline__ void df_wait_first(int n, unsigned epoch, int limit, 
     __syncthreads();
 }
 
-__device__ __forceinline__ uint32_t df_and(uint32_t v){
-    uint32_t r; asm("v_and_b32 %0, %1, %2" : "=v"(r) : "s"(0x0F0F0F0Fu), "v"(v)); return r;
-}
-
 /* (v & mask) | magic in one instruction; written out because the compiler emits an and and an or */
 __device__ __forceinline__ uint32_t df_and_or(uint32_t v, uint32_t mask, uint32_t magic){
     uint32_t r; asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(magic)); return r;
