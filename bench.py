@@ -571,7 +571,7 @@ def bench_decode(torch, q, args, E=32, D=768, F=2048, topk=2, layers=8):
         res = {"ms_8_layers": tm["event_ms_avg"], "distinct_expert_hits": hits, "bytes": hits * per_expert,
                "gbs": hits * per_expert / (tm["event_ms_avg"] * 1e-3) / 1e9}
         # beside it: the same sequence with the layer's inputs taken as fp16 pairs (qlmx_decode_math(1); 3.7e-4
-        # against the fp32 reference instead of 4e-7); the figures of the line are the default fp32 loop's
+        # against the fp32 reference instead of 4e-7); the figures of the line are the default loop's
         q.call("qlmx_decode_math", 1)
         try:
             th = timed(torch, step, args.steps, args.warmup)
@@ -898,12 +898,12 @@ def cpu_decode(args, E=32, D=768, F=2048, topk=2, T=16, layers=2):
 # HBM bytes from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (scaled by the 1 GiB copy calibration); the runs,
 # counter values and scale factors are in profiles/*.txt. adamw: per launch. train: per step, i.e. summed over
 # the step's 4 launches (1035.9 MiB read + 1086.2 MiB written). c5: per step over the 32 GEMM launches of the 8
-# layers (104.4 GiB read + 49.0 GiB written). decode: per launch = per layer at T=16 (64.1 MiB read + 5.1 MiB
+# layers (104.4 GiB read + 49.0 GiB written). decode: per launch = per layer at T=16 (77.0 MiB read + 4.6 MiB
 # written). layer: per step of the merged layer, all its kernels (2442.1 MiB read + 1393.2 MiB written). train and c5
 # are those of the default --bwd pair. The figures are constants of the code state they
 # were measured at; that state is named in the JSON line so that a reader can tell a stale one.
-PROFILED_TRAFFIC = {"adamw": 1.405e9, "train": 2.225e9, "layer": 4.022e9, "c5": 1.648e11, "decode": 7.39e7}
-PROFILED_AT = "git bd3f2f6 (train, layer, c5), ef06021 (decode), 497f628 (adamw)"
+PROFILED_TRAFFIC = {"adamw": 1.405e9, "train": 2.225e9, "layer": 4.022e9, "c5": 1.648e11, "decode": 8.56e7}
+PROFILED_AT = "git bd3f2f6 (train, layer, c5), e0aff96 (decode; adamw, train and layer measured again there), 497f628 (adamw)"
 
 
 def main():

@@ -1,5 +1,5 @@
 /* qlmx_gemm_api.hip -- C entry points of the grouped expert GEMMs: argument checks and the choice
- * between the fp32 vector-ALU kernels and the bf16 MFMA kernels. */
+ * between the fp32 kernels, the few-row GEMV and the bf16 and fp16 matrix-core kernels. */
 #include "qlmx_gemm.h"
 #include <stdlib.h>
 

@@ -28,8 +28,9 @@
  * us per call, tiled kernels -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16
  * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
- * What bounds them now: the forward, the conversion of the weights (some 220 vector instructions for 32 x 128 of them); the input
- * gradient, the 64 bytes per cycle of a CU's address unit; both, the round trips in front of and behind the loop.
+ * What bounds them now: a wavefront's chain -- the round trip in front of its loop, the steps one behind the other, the sum over
+ * the wavefronts behind it. Vector issue is at 36-38 % in the forward (231 to 261 vector instructions for 32 x 128 weights,
+ * everything included) and 15-29 % in the input gradient, the address units at 24-51 %, the matrix cores at 4-14 %.
  */
 #include "qlmx_gemm.h"
 #include <type_traits>
@@ -252,8 +253,8 @@ __global__ void __launch_bounds__(64 * SM_WAVES * (DUAL == SM_BY_WAVE ? 2 : 1), 
 /* ---- input gradient: 64 columns per workgroup; nseg operand pairs (a continued problem's second pair comes from the
  * table entry behind it). A wavefront's step is 64 of the contraction: 16 RT rows of activations (128 bytes each) and 64
  * rows of weights (32 bytes each) go straight into stages of LDS of its own, so there is no barrier in the loop, only the
- * wavefront's own wait counts. Loaded as operands (lane = row lane%16) instead, sixteen bytes each from sixty-four places,
- * a load kept the CU's address unit busy for 57 cycles instead of 16, and that unit set the pace. Piece q of row r of a stage
+ * wavefront's own wait counts. Loaded as operands (lane = row lane%16) instead, sixteen bytes each with neighbouring lanes in
+ * different rows, a load takes 66 cycles of a CU where four lanes per row of 64 bytes take 17.5, and that set the pace. Piece q of row r of a stage
  * lies at q ^ ((r >> 1) & 7): the sixteen rows of an operand read hit sixteen different units.
  * LDS accesses are inline assembly: the compiler would wait for every load to LDS in front of them. ---- */
 #define SM_TSTAGE(RT) (2048 * ((RT) + 1) + 256)      /* activations, weights, scales */

@@ -607,7 +607,7 @@ __device__ __forceinline__ void df_fma_task(const uint2 (&w0)[DF_BATCH], const u
  * Matrix-core loop (the default). v_mfma_i32_16x16x32_i8 multiplies 16 rows of eight bytes per lane group with 16 columns of
  * eight. A lane holds 16 neighbouring columns of every row it loads, so for column j of each lane its eight bytes are the
  * digits of eight of its own rows: no value crosses lanes on its way in, a 4x4 byte transposition per four rows (8
- * permutes) and three masks and shifts per word of eight digits make all 16 operands, 0.6 vector instructions per
+ * permutes) and three masks and shifts per word of eight digits make all 16 operands, 0.67 vector instructions per
  * digit for one input row or two, against 2.6 and 3.6 for conversions and fp32 multiply-adds. The other operand's 16 rows
  * are the four bytes of two inputs in two scale groups (df_stage_i8); the products are exact, a lane's four sums are the
  * bytes of one input and are put together in fp32 at the end. Half of the lanes hold an input times the columns of
@@ -1201,7 +1201,7 @@ static bool df_math_fp16(){
     return g_df_math != 0;
 }
 extern "C" int qlmx_decode_math(int fp16_inputs){
-    QLMX_REQUIRE(fp16_inputs == 0 || fp16_inputs == 1, "qlmx_decode_math: 0 (fp32 inputs) or 1 (fp16 inputs), not %d", fp16_inputs);
+    QLMX_REQUIRE(fp16_inputs == 0 || fp16_inputs == 1, "qlmx_decode_math: 0 (the default loop) or 1 (fp16 inputs), not %d", fp16_inputs);
     g_df_math = fp16_inputs;
     return QLMX_OK;
 }

@@ -239,8 +239,8 @@ __global__ void __launch_bounds__(256) k_fill_i32(int *p, int v, int n){
 
 /* ---- row movers. One workgroup per row; D % 4 == 0. Bound by HBM. What a launch touches once goes past the caches (NT)
  * where it is more than the last-level cache holds: it would only push out the rows that the K experts of a token read
- * again, and plain loads of such a stream reach 5.2 TB/s, these 6.6. 131072 rows of 2048: combine 314 -> 242 us, gate
- * gradient 449 -> 357, gather 228 -> 218. Smaller buffers are partly in the cache, left there by the GEMM before or kept for
+ * again, and plain loads of such a stream reach 5.1 TB/s, these 6.1. 131072 rows of 2048: combine 316 -> 263 us, gate
+ * gradient 437 -> 355, gather 222 -> 219. Smaller buffers are partly in the cache, left there by the GEMM before or kept for
  * the one after (16384 rows of 768 again and again: gate gradient 19.1 us, 20.3 with NT). ---- */
 #define PAST_CACHE (256ull << 20)                      /* bytes of the launch's rows in fp32 */
 typedef float gl_f4 __attribute__((ext_vector_type(4)));

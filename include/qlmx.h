@@ -324,9 +324,11 @@ int qlmx_decode_status(void);
  * QLMX_DECODE_SCRATCH_BYTES that is part of the library image (each GPU the library runs on holds it
  * until the process ends), and the call makes no hipMalloc, hipFree or other allocating call.
  * qlmx_init must have run for the current device. A shape whose partial sums
- *   8 * K*T * 2 * (2 * ceil(D/R1) * F + ceil(F/R2) * D)  bytes, R1, R2 = 64..256 rows per gate|up / down slice
+ *   8 * K*T * 2 * (2 * S1 * F + S2 * D)  bytes
  * exceed the array fails with QLMX_E_LIMIT (the 32-expert D=768 F=2048 layer at 16 tokens top-2
- * needs 10.6 MB). Every call on a GPU shares that GPU's array: calls that overlap on one GPU,
+ * needs 9.4 MB). S1 = ceil(D/R1) slices of gate|up, R1 = 256 rows, halved down to 64 while h * 2 * ceil(F/256) * S1 is below
+ * 0.15 of the workgroups the device holds, h = the expected number of experts hit; S2 = ceil(F/R2) slices of down: four, or as few
+ * as leave a task per workgroup, at least ceil(F/256), R2 rounded up to a multiple of 64. Every call on a GPU shares that GPU's array: calls that overlap on one GPU,
  * whatever their streams, race. */
 #define QLMX_DECODE_SCRATCH_BYTES (32u << 20)
 int qlmx_moe_decode_forward_noalloc(const float *x, const int *assign, const float *gate, float *out,

@@ -102,7 +102,7 @@ def run_case(q, orc, mode, E, rowsM, K, N, act, math, seed=0, beta=0.0, group=12
     return dC.cpu().numpy(), want
 
 
-# ------------------------------------------------------------------ fp32 vector-ALU kernels
+# ------------------------------------------------------------------ fp32 kernels
 @pytest.mark.parametrize("mode", ["nn", "tn", "nt"])
 def test_f32_ragged_small(q, orc, mode):
     """Ragged shapes incl. an empty expert and rows not a multiple of any tile (cudalm.cu:9919-9946 style)."""
