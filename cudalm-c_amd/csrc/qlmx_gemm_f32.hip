@@ -157,11 +157,10 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) k_gemm_f32(F32Args a){
             if constexpr(WEIGHT){
                 float e[8];
                 if constexpr(FAST){
-                    /* (16 s) * (digit / 16): both factors exact, so the product is fl(s * digit) */
+                    /* fl(s * digit); with the 16 on s it would be infinite from s = 2^124 on */
                     const QxNibs nb = qx_nibs(wb[u]);
-                    const float sc = sb[u] * 16.0f;
 #pragma unroll
-                    for(int q = 0; q < 8; q++) e[q] = sc * qx_nib16(nb, q);
+                    for(int q = 0; q < 8; q++) e[q] = sb[u] * (16.0f * qx_nib16(nb, q));
                 } else {
 #pragma unroll
                     for(int q = 0; q < 8; q++) e[q] = eb[u * 8 + q];

@@ -195,6 +195,27 @@ def test_f32_shapes_of_a_workgroup(q, orc, mode, K, N, rows, act):
     assert orc.relerr(got, want) < TOL_F32
 
 
+@pytest.mark.parametrize("mode", ["nn", "tn"])
+@pytest.mark.parametrize("lo,hi,x", [(120, 127.9, -40), (-149, -127, 60), (-60, -40, -86)])
+def test_f32_scales_and_inputs_at_the_ends_of_the_range(q, mode, lo, hi, x):
+    """A weight is the product s * digit, finite where that is: scales above 2^124, whose sixteenfold is not; subnormal scales;
+    subnormal products."""
+    import torch
+    M, K, N, group = 40, 64, 64, 32
+    rng = np.random.default_rng(5)
+    d = rng.integers(-1, 2, K * N)
+    s = (2.0 ** rng.uniform(lo, hi, K * N // group)).astype(f32)
+    W = (np.repeat(s, group) * d.astype(f32)).astype(np.float64).reshape((K, N) if mode == "nn" else (N, K))
+    A = (rng.standard_normal((M, K)) * 2.0 ** x).astype(f32)
+    want = A.astype(np.float64) @ (W if mode == "nn" else W.T)
+    C = torch.zeros(M, N, device="cuda")
+    packed = (d[0::2] & 15 | (d[1::2] & 15) << 4).astype(np.uint8)
+    (q.gemm_nn if mode == "nn" else q.gemm_tn)(dev(packed), dev(s), group, q.problems([(dev(A), None, C, 0, 0, M, 0.0)]), 1, K, N, pkg.ACT_F32, pkg.MATH_F32)
+    got = C.cpu().numpy().astype(np.float64)
+    assert np.isfinite(got).all()
+    assert np.linalg.norm(got - want) < TOL_F32 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("mode,K,N,math,company", [("nn", 768, 2048, "f16", [600]), ("tn", 768, 2048, "mfma", [3000]), ("nn", 768, 512, "f32", [3000]),
                                                    ("nn", 768, 512, "f32", [13000]), ("tn", 768, 512, "f32", [3000])])
 @pytest.mark.parametrize("M", [3, 16])
