@@ -541,7 +541,7 @@ extern "C" int qlmx_moe_merge_rows(const int *perm, int N, int K, int *tok, int 
     QLMX_REQUIRE(perm && tok && inv, "qlmx_moe_merge_rows: NULL buffer");
     QLMX_REQUIRE(N > 0 && K > 0 && (long long)N * K < (1LL << 31), "qlmx_moe_merge_rows: N=%d K=%d", N, K);
     const int KN = N * K;
-    if(KN <= MR_WHOLE){
+    if(KN <= MR_WHOLE && tok != perm){                     /* over the permutation: a workgroup there reads what another may have overwritten */
         hipLaunchKernelGGL(k_merge_rows_windows, dim3((KN + MR_WINDOW - 1) / MR_WINDOW), dim3(MR_WINDOW), 0, (hipStream_t)stream, perm, KN, N, tok, inv);
         QLMX_LAUNCH_CHECK("merge rows launch");
         return QLMX_OK;

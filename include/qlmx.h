@@ -374,7 +374,7 @@ int qlmx_moe_dgate(const float *dout, const float *yp, const int *perm, const fl
  * runs once per layer on K times the rows instead of once per pass. The grouping itself is qlmx_moe_perm over the
  * K*N assignments as a single pass (N' = K*N, K' = 1): its perm names entries m = pass * N + token.
  *   qlmx_moe_merge_rows: tok[p] = perm[p] % N (the token row p holds; what a gather or a gathering GEMM takes as
- *     its index list) and inv[m] = the row that holds entry m (-1 if none), both int32 [K*N].
+ *     its index list) and inv[m] = the row that holds entry m (-1 if none), both int32 [K*N]; tok may be perm.
  *   qlmx_moe_combine: out[n,:] = (..(out[n,:] + gate[0*N+n] * y[inv[0*N+n],:]) ..) + gate[(K-1)*N+n] * y[inv[(K-1)*N+n],:]
  *     -- the sums that K calls of qlmx_moe_scatter_gate build, in their order and to their bits; gate NULL adds
  *     the rows themselves (K calls of qlmx_moe_scatter_add). y fp32 [K*N, D].

@@ -157,6 +157,21 @@ def test_merge_rows_with_dropped_entries(q, N, K):
     assert np.array_equal(tok.cpu().numpy(), np.where(perm < 0, -1, perm % N))
 
 
+@pytest.mark.parametrize("N,K", [(700, 3), (16385, 2)])
+def test_merge_rows_may_write_the_tokens_over_the_permutation(q, N, K):
+    """tok in place of perm, on both sides of the one-launch form."""
+    import torch
+    perm = np.random.default_rng(N).permutation(N * K).astype(np.int32)
+    perm[::5] = -1
+    for _ in range(5):
+        p, inv = dev(perm), zeros(N * K, torch.int32)
+        q.moe_merge_rows(p, N, K, p, inv)
+        want = np.full(N * K, -1, np.int32)
+        want[perm[perm >= 0]] = np.nonzero(perm >= 0)[0]
+        assert np.array_equal(inv.cpu().numpy(), want)
+        assert np.array_equal(p.cpu().numpy(), np.where(perm < 0, -1, perm % N))
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_row_moves_larger_than_the_last_level_cache(q, bf16):
     """The rows as one launch of 256 MiB, and a few rows at a time."""
