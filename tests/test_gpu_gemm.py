@@ -257,6 +257,27 @@ def test_mfma_few_rows(q, orc, mode, K, N, group, rows):
         assert orc.relerr(got, want) < (4e-4 if mode == "nn" else 3e-6)
 
 
+@pytest.mark.parametrize("mode,math", [("nn", "f16"), ("tn", "mfma"), ("nn", "f32"), ("tn", "f32")])
+@pytest.mark.parametrize("M", [5, 40, 100])
+def test_few_rows_outputs_at_any_float(q, orc, mode, math, M):
+    """An output that begins four bytes behind a 16-byte boundary, as a view into a larger buffer may: the same bits as on the
+    boundary, and nothing written before or behind."""
+    import torch
+    K, N = 256, 128
+    act, m = (pkg.ACT_F32, pkg.MATH_F32) if math == "f32" else (pkg.ACT_BF16, pkg.MATH_MFMA_F16 if math == "f16" else pkg.MATH_MFMA)
+    d, s, _ = make_weights(orc, 41, 1, *((K, N) if mode == "nn" else (N, K)))
+    A = dev(orc.bf16_round(orc.normal(M * K, 41, 1))); a = A if math == "f32" else to_bf16_bits(A)
+    dd, ds = dev(d), dev(s)
+    outs = []
+    for at in (4, 5):
+        buf = torch.full((M * N + 9,), 3.0, device="cuda")
+        (q.gemm_nn if mode == "nn" else q.gemm_tn)(dd, ds, 128, q.problems([(a, None, buf.data_ptr() + 4 * at, 0, 0, M, 1.0 if mode == "tn" else 0.0)]),
+                                                   1, K, N, act, m)
+        outs.append(buf[at:at + M * N].clone())
+        assert bool((buf[:at] == 3.0).all()) and bool((buf[at + M * N:] == 3.0).all())
+    assert torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("K,N,group", [(768, 256, 128), (128, 128, 64), (2048, 256, 256)])
 @pytest.mark.parametrize("rows", [[65, 1, 130, 34], [257]])
 def test_mfma_few_tiles(q, orc, K, N, group, rows):
