@@ -3,7 +3,7 @@ qlmx_moe_gemm_nn and the fused qlmx_moe_decode_forward, against the CPU oracle's
 fp32 layer (moe_forward call order, cudalm.cu:4193-4228). Tolerance 1e-3 relative L2 as stated for
 matmul outputs. The fused layer has two multiply loops and every layer test runs with both: the default
 one (exact digits, inputs of 31 bits under a common power of two, or fp32 multiply-adds) is as close to the oracle as two
-orders of fp32 sums and the libm exp are (observed 4e-7, held to 2e-5; against 64 bits further down, held to 1e-6),
+orders of fp32 sums and the libm exp are (observed 4e-7, held to 2e-5; against 64 bits further down, held to 6e-7),
 the other (qlmx_decode_math(1)) takes its inputs as fp16 pairs (11 significant bits; observed 2.4e-4 ..
 4.9e-4 on a layer's output, held to 7e-4 here). Routing indices come from the oracle's router and are consumed as
 given."""
@@ -268,7 +268,7 @@ def test_decode_limits(q):
 
 @pytest.mark.parametrize("D,F,group", [(128, 128, 128), (384, 640, 128), (256, 768, 256), (896, 512, 128)])
 def test_decode_inputs_of_very_different_size(q, orc, D, F, group):
-    """The default loop brings a task's inputs to a common fixed point: tokens that are tiny or huge, one value far above the
+    """The default loop brings the inputs of a wavefront's rows to a common fixed point: tokens that are tiny or huge, one value far above the
     rest, all zeros, or not a number share experts (and problems of two) with ordinary ones, and each is held to the bound by
     itself; widths that end inside a task's rows and columns."""
     import torch
@@ -331,6 +331,11 @@ class Layer64:
         return out.cpu().numpy()
 
 
+# A value of the output passes some ten fp32 roundings after the products: staging, the four wavefronts' and the slices' sums, SwiGLU,
+# the gated sum over the passes, 2^-24 each: 6e-7 if all of them added up. 1.7e-7 at most is what the cases below show.
+REL64 = 6e-7
+
+
 def rel64(got, want):
     return float(np.linalg.norm(got - want) / np.linalg.norm(want))
 
@@ -339,19 +344,18 @@ def rel64(got, want):
 def test_decode_neighbouring_scale_groups_of_different_size(q, orc, n):
     """A column's sum holds nothing of the scale group beside it, so the size of that group's scales must not show in it: every
     second group of the down projection 2^-n of its neighbours, and every second group of gate and up with the down
-    projection's rows behind them as much larger, so that the output shows those columns' own error. Bound: three fp32 sums,
-    one after the other, of some hundred rounded products."""
+    projection's rows behind them as much larger, so that the output shows those columns' own error."""
     a = Layer64(orc, 100 + n)
     a.s2[:, :, 1::2] *= f32(2.0 ** -n)
     got, want = a.run(q), a.want()
     for c in range(0, a.D, a.group):
-        assert rel64(got[:, c:c + a.group], want[:, c:c + a.group]) < 1e-6, c
+        assert rel64(got[:, c:c + a.group], want[:, c:c + a.group]) < REL64, c
     b = Layer64(orc, 200 + n)
     b.s1[:, :, 1::2] *= f32(2.0 ** -n); b.s3[:, :, 1::2] *= f32(2.0 ** -n)
     for f in range(b.group, b.F, 2 * b.group):
         b.s2[:, f:f + b.group] *= f32(2.0 ** min(2 * n, 100))
     got, want = b.run(q), b.want()
-    assert rel64(got, want) < 1e-6
+    assert rel64(got, want) < REL64
 
 
 @pytest.mark.parametrize("n", [4, 9, 12, 20, 30])
@@ -365,7 +369,7 @@ def test_decode_columns_that_take_nothing_of_the_largest_input(q, orc, n):
     a.d2[:, :8] = 0
     got, want = a.run(q), a.want()
     for t in range(a.T):
-        assert rel64(got[t], want[t]) < 1e-6, t
+        assert rel64(got[t], want[t]) < REL64, t
 
 
 @pytest.mark.parametrize("v", [np.nan, np.inf])
@@ -381,4 +385,4 @@ def test_decode_nan_and_infinite_scales_stay_in_their_columns(q, orc, v):
     assert np.array_equal(np.isnan(got[:, there]), np.broadcast_to(nan, (a.T, a.group)))
     assert np.array_equal(np.isinf(got[:, there]), np.broadcast_to(~nan, (a.T, a.group)))
     for c in (0, 2 * a.group):
-        assert rel64(got[:, c:c + a.group], want[:, c:c + a.group]) < 1e-6, c
+        assert rel64(got[:, c:c + a.group], want[:, c:c + a.group]) < REL64, c
