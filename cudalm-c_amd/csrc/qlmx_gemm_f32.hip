@@ -5,7 +5,9 @@
  * formed as the single fp32 product s*digit (exactly the value the reference renders into P,
  * qlm.cuh:177) and every multiply-accumulate is an fp32 FMA (v_mfma_f32_32x32x2_f32 multiplies and adds
  * fp32 values), as in the reference's 6x16 micro-kernel (cpu_rt.h:196-208); only the summation order
- * differs. It serves activations of any shape under QLMX_MATH_F32, the default of the host mirror's mg_bind.
+ * differs. Under QLMX_MATH_F32 (the default of the host mirror's mg_bind) it serves what the kernels of
+ * qlmx_gemm_f32s.hip, twice as fast, do not take: bf16 activations, groups below 64, odd sizes and addresses, and
+ * weight gradients of a few rows and tiles.
  *
  *   nn: out[m,n] = sum_k A[m,k] * W[k,n]      W row-major [K,N], groups along n
  *   tn: out[m,n] = sum_k A[m,k] * W[n,k]      W row-major [N,K], groups along k   (+ beta*out)
@@ -274,8 +276,13 @@ static int launch_mode(const F32Args &a, const qlmx_gemm_prob *probs, int nprob,
     return          b ? launch_f32<MODE, true, false>(a, probs, nprob, st) : launch_f32<MODE, false, false>(a, probs, nprob, st);
 }
 
+bool qlmx_gemm_f32s_takes(int mode, const signed char *d, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N);
+int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N, hipStream_t st);
+
 int qlmx_gemm_f32_dispatch(int mode, const signed char *d, const float *s, int group,
                            const qlmx_gemm_prob *probs, int nprob, int K, int N, int act_dtype, hipStream_t st){
+    if(act_dtype == QLMX_ACT_F32 && qlmx_gemm_f32s_takes(mode, d, group, probs, nprob, K, N))
+        return qlmx_gemm_f32s_launch(mode, d, s, group, probs, nprob, K, N, st);
     F32Args a; a.pr = nullptr; a.nprob = a.ntiles = 0; a.d = d; a.s = s; a.group = group; a.K = K; a.N = N;
     if(mode == GEMM_NN) return launch_mode<GEMM_NN>(a, probs, nprob, act_dtype, st);
     if(mode == GEMM_TN) return launch_mode<GEMM_TN>(a, probs, nprob, act_dtype, st);

@@ -216,6 +216,78 @@ def test_f32_scales_and_inputs_at_the_ends_of_the_range(q, mode, lo, hi, x):
     assert np.linalg.norm(got - want) < TOL_F32 * np.linalg.norm(want)
 
 
+def f32_call(q, mode, A, X, digits, s, group, rows, K, N, beta=0.0):
+    """One fp32 call over the problems of `rows`; A [rows, K] and X the old output or, for nt, dY [rows, N]. Returns the output and what
+    64 bits give for it, the weight the fp32 product s * digit."""
+    import torch
+    E, off = len(rows), np.concatenate([[0], np.cumsum(rows)])
+    if mode == "nt":
+        C = torch.zeros(E * K * N, device="cuda")
+        a, b = dev(A), dev(X)
+        probs = [(a.data_ptr() + off[e] * K * 4, b.data_ptr() + off[e] * N * 4, C.data_ptr() + e * K * N * 4, 0, 0, rows[e], 0.0) for e in range(E)]
+        q.gemm_nt(q.problems(probs), E, K, N, pkg.ACT_F32, pkg.MATH_F32)
+        with np.errstate(all="ignore"):
+            want = np.concatenate([(A[off[e]:off[e + 1]].astype(np.float64).T @ X[off[e]:off[e + 1]].astype(np.float64)).ravel() for e in range(E)])
+        return C.cpu().numpy().astype(np.float64), want
+    with np.errstate(all="ignore"):
+        W = (np.repeat(s, group) * digits.astype(f32)).astype(np.float64).reshape((E, K, N) if mode == "nn" else (E, N, K))
+        want = np.concatenate([A[off[e]:off[e + 1]].astype(np.float64) @ (W[e] if mode == "nn" else W[e].T) for e in range(E)]) + beta * X
+    C, a = dev(X), dev(A)
+    packed = (digits[0::2] & 15 | (digits[1::2] & 15) << 4).astype(np.uint8)
+    probs = [(a.data_ptr() + off[e] * K * 4, None, C.data_ptr() + off[e] * N * 4, e * K * N, e * K * N // group, rows[e], beta) for e in range(E)]
+    (q.gemm_nn if mode == "nn" else q.gemm_tn)(dev(packed), dev(s), group, q.problems(probs), E, K, N, pkg.ACT_F32, pkg.MATH_F32)
+    return C.cpu().numpy().astype(np.float64), want
+
+
+def f32_inputs(seed, mode, rows, K, N, group):
+    rng = np.random.default_rng(seed)
+    n = len(rows) * K * N
+    digits = rng.integers(-7, 8, n) if mode != "nt" else None
+    s = (rng.uniform(0.5, 1.5, n // group) * 0.0086).astype(f32) if mode != "nt" else None
+    return rng.standard_normal((sum(rows), K)).astype(f32), rng.standard_normal((sum(rows), N)).astype(f32), digits, s
+
+
+@pytest.mark.parametrize("mode,K,N,group,rows", [
+    ("nn", 64, 64, 64, [1, 33]), ("nn", 320, 192, 64, [31, 2, 65]), ("nn", 768, 256, 128, [4]), ("nn", 1536, 256, 256, [100]),
+    ("tn", 64, 64, 64, [1, 33]), ("tn", 320, 45, 64, [31, 0, 65]), ("tn", 1536, 72, 128, [4]), ("tn", 512, 66, 256, [100]),
+    ("nt", 1024, 1028, 0, [1]), ("nt", 1156, 1028, 0, [2, 31, 33]), ("nt", 68, 132, 0, [127, 40]), ("nt", 64, 64, 0, [128]), ("nt", 132, 260, 0, [300, 0, 97])])
+def test_f32_in_three_parts(q, mode, K, N, group, rows):
+    """The fp32 products as products of bf16 parts, at the edges of their tiles and steps. Against 64 bits: one rounding of the weight or
+    of activation times scale, and at most three (nt: six) roundings per sixteen of the contraction, each half a unit (2^-24) of a running sum
+    that is, root mean square, within the size of the result."""
+    A, X, digits, s = f32_inputs(41, mode, rows, K, N, group)
+    got, want = f32_call(q, mode, A, X, digits, s, group, rows, K, N, beta=1.0 if mode == "tn" else 0.0)
+    depth = max(rows) if mode == "nt" else K
+    assert np.linalg.norm(got - want) < 2.0 ** -24 * (1 + np.sqrt((6 if mode == "nt" else 3) * (depth / 16 + 1))) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("mode", ["nn", "tn", "nt"])
+@pytest.mark.parametrize("where,value", [("row", np.inf), ("row", np.nan), ("one", np.inf), ("one", 3.4e38), ("all", 2.0 ** 61), ("all", 2.0 ** -111),
+                                         ("all", 2.0 ** -104), ("one", 2.0 ** -140), ("scale", 2.0 ** 51), ("scale", 2.0 ** -130)])
+def test_f32_parts_leave_what_they_do_not_hold(q, mode, where, value):
+    """Infinities, values and scales at the ends of the range, and NaN: what 64 bits give, rounded to fp32, the same elements infinite or not a
+    number; finite sums to the relative error of fp32 sums."""
+    if mode == "nt" and where == "scale":
+        pytest.skip("no scales")
+    K, N, group, rows = 192, 128, 64, [40, 130]
+    A, X, digits, s = f32_inputs(42, mode, rows, K, N, group)
+    if mode == "nt" and where == "all" and value < 1:
+        X *= f32(2.0 ** 20)                              # products stay above the subnormals, whose last place is a fixed size
+    if where == "row": A[7, 3::5] = value
+    elif where == "one": A[50, 9] = value
+    elif where == "all": A *= f32(value)
+    else: s *= f32(value / 0.0086)
+    old = np.zeros_like(X)
+    got, want = f32_call(q, mode, A, X if mode == "nt" else old, digits, s, group, rows, K, N)
+    with np.errstate(all="ignore"):
+        want = want.astype(f32).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.array_equal(np.sign(got[np.isinf(got)]), np.sign(want[np.isinf(want)]))
+    scale = np.abs(want[ok]).max()
+    assert np.linalg.norm((got[ok] - want[ok]) / scale) < TOL_F32 * np.linalg.norm(want[ok] / scale)
+
+
 @pytest.mark.parametrize("mode,K,N,math,company", [("nn", 768, 2048, "f16", [600]), ("tn", 768, 2048, "mfma", [3000]), ("nn", 768, 512, "f32", [3000]),
                                                    ("nn", 768, 512, "f32", [13000]), ("tn", 768, 512, "f32", [3000])])
 @pytest.mark.parametrize("M", [3, 16])
