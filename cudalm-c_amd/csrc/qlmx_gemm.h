@@ -108,6 +108,21 @@ __device__ __forceinline__ int qx_xcd_tile_rows(int b, int g){
 }
 
 typedef float qx_f32x16 __attribute__((ext_vector_type(16)));
+typedef float qx_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 qx_bf16x2 __attribute__((ext_vector_type(2)));
+
+/* ---- fp32 values as sums of bf16 parts: hi = bf16(x), mid = bf16(x - hi), ..., every difference exact ---- */
+__device__ __forceinline__ uint32_t qx_pk_bf16(float lo, float hi){ const qx_f32x2 v = {lo, hi}; return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, qx_bf16x2)); }
+/* v_dot2_f32_bf16: x + lower half of h * lower half of m + upper * upper */
+__device__ __forceinline__ float qx_dot2(float x, uint32_t h, uint32_t m){
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(qx_bf16x2, h), __builtin_bit_cast(qx_bf16x2, m), x, false);
+}
+/* x - (the lower / upper half of h) is qx_dot2 with (-1, 0) / (0, -1): one instruction where shift and subtraction are two, exact since the
+ * difference is an fp32 value. The factors have to come from registers: as a literal the instruction takes -1 for the wrong half. */
+struct QxMinus { uint32_t lo, hi; };
+__device__ __forceinline__ QxMinus qx_minus(){ QxMinus m = {0x0000BF80u, 0xBF800000u}; asm("" : "+s"(m.lo), "+s"(m.hi)); return m; }
+/* largest magnitude so far (fmaxf would canonicalise every operand first) */
+__device__ __forceinline__ void qx_absmax(float &m, float a, float b){ asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b)); }
 /* round to nearest even, as cudalm.cu:334-338 */
 __device__ __forceinline__ unsigned short qx_f32_to_bf16(float f){
     uint32_t x = __float_as_uint(f);

@@ -26,8 +26,6 @@
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float  f32x2  __attribute__((ext_vector_type(2)));
 typedef float  f32x4  __attribute__((ext_vector_type(4)));
 /* operands named in the problem table: known to be global memory (a load from an address of unknown kind counts as an LDS access too,
  * and every wait for LDS then waits for it) */
@@ -44,31 +42,22 @@ typedef const __attribute__((address_space(1))) void glb_void;
 
 struct F3Args { const DevProb *pr; int nprob, ntiles; const signed char *d; const float *s; int group, gshift; int K, N; };
 
-__device__ __forceinline__ uint32_t f3_pk(float lo, float hi){ const f32x2 v = {lo, hi}; return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2)); }
-
-/* x - (the lower / upper half of h): v_dot2_f32_bf16 with (-1, 0) / (0, -1), one instruction where shift and subtraction are two, exact since
- * the difference is an fp32 value. The factors have to come from registers: as a literal the instruction takes -1 for the wrong half. */
-struct F3Minus { uint32_t lo, hi; };
-__device__ __forceinline__ F3Minus f3_minus(){ F3Minus m = {0x0000BF80u, 0xBF800000u}; asm("" : "+s"(m.lo), "+s"(m.hi)); return m; }
-__device__ __forceinline__ float f3_rest(float x, uint32_t h, uint32_t m){
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, h), __builtin_bit_cast(bf16x2, m), x, false);
-}
 /* the largest and the smallest non-zero of what a thread has seen, as bits less one (zero is then the largest) */
 struct F3Range { uint32_t hi, lo; };
 __device__ __forceinline__ F3Range f3_range(){ const F3Range r = {0u, 0xFFFFFFFFu}; return r; }
 __device__ __forceinline__ bool f3_odd(const F3Range &r){ return r.hi > __float_as_uint(F3_LARGE) || r.lo < __float_as_uint(F3_SMALL) - 1u; }
 __device__ __forceinline__ uint32_t f3_scale_bits(float s){ return (__float_as_uint(s) & 0x7FFFFFFFu) + (F3_SCALE << 23); }
 /* eight values into their three parts */
-__device__ __forceinline__ void f3_split(const F3Minus &k, F3Range &range, const float (&f)[8], uint4 (&p)[3]){
+__device__ __forceinline__ void f3_split(const QxMinus &k, F3Range &range, const float (&f)[8], uint4 (&p)[3]){
     uint32_t w[3][4]; float m = 0.0f;
 #pragma unroll
     for(int i = 0; i < 4; i++){
         const float a = f[2 * i], b = f[2 * i + 1];
-        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));     /* fmaxf would canonicalise every operand first */
-        w[0][i] = f3_pk(a, b);
-        const float a1 = f3_rest(a, w[0][i], k.lo), b1 = f3_rest(b, w[0][i], k.hi);
-        w[1][i] = f3_pk(a1, b1);
-        w[2][i] = f3_pk(f3_rest(a1, w[1][i], k.lo), f3_rest(b1, w[1][i], k.hi));
+        qx_absmax(m, a, b);
+        w[0][i] = qx_pk_bf16(a, b);
+        const float a1 = qx_dot2(a, w[0][i], k.lo), b1 = qx_dot2(b, w[0][i], k.hi);
+        w[1][i] = qx_pk_bf16(a1, b1);
+        w[2][i] = qx_pk_bf16(qx_dot2(a1, w[1][i], k.lo), qx_dot2(b1, w[1][i], k.hi));
     }
 #pragma unroll
     for(int q = 0; q < 3; q++) p[q] = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
@@ -134,8 +123,8 @@ template<int I, int N, class F> __device__ __forceinline__ void f3_each(const F 
 /* nt: 64 x 64 outputs per wavefront, KS of them along the contraction. Lane l loads sixteen bytes, columns 4 (l % 16) .. + 3, of rows 8 (l / 16)
  * .. + 7 of both operands: the operand of v_mfma_f32_16x16x32 for column q of each four is then in the lane that needs it, the columns of a
  * product are four apart, which only the store has to know, and a request moves four rows of 256 bytes (with four bytes per lane a step of the
- * loop waited for the issue of its requests). The loads of the next step go out as this step's values have been split. */
-template<int KS>
+ * loop waited for the issue of its requests). FEW: every problem has fewer than 32 rows. The loads of the next step go out as this step's values have been split. */
+template<int KS, bool FEW>
 __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
     constexpr int B = 64, LD = B + 4;
     extern __shared__ __attribute__((aligned(16))) unsigned char f3_lds[];
@@ -145,7 +134,7 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
     const int lt = tile - P.tile0, ti = lt / P.tiles_n, tj = lt - ti * P.tiles_n;
     const int i0 = ti * B, j0 = tj * B, M = P.M;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
-    const F3Minus minus = f3_minus();
+    const QxMinus minus = qx_minus();
     F3Range range = f3_range();
     /* the lane's byte offset in a step's rows, and with its columns alone */
     const uint32_t ca = (uint32_t)min(i0 + c * 4, a.K - 4) * 4u, cb = (uint32_t)min(j0 + c * 4, a.N - 4) * 4u;
@@ -195,7 +184,7 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
                     f32x4 small[2] = {(f32x4)(0.0f), (f32x4)(0.0f)}, large[2];
 #pragma unroll
                     for(int i = 0; i < 2; i++) large[i] = product(h + i, 0, 0, small[i]);
-                    if(M < 32)                            /* no sum for what is left out to disappear in */
+                    if(FEW)                               /* no sum for what is left out to disappear in */
 #pragma unroll
                         for(int i = 0; i < 2; i++) small[i] = product(h + i, 1, 2, product(h + i, 2, 1, small[i]));
 #pragma unroll
@@ -208,7 +197,7 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
             }
         }
     };
-    if(mine > 0){
+    if(!FEW && mine > 0){
         load(va, (gchar *)P.A, a.K, oa, 0); load(vb, (gchar *)P.B, a.N, ob, 0);
         for(int n = 0; n < mine; n++) multiply(std::true_type(), n);
     }
@@ -302,7 +291,7 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
     const int lt = tile - P.tile0, ti = lt / P.tiles_n, tj = lt - ti * P.tiles_n;
     const int i0 = ti * BM, j0 = tj * BN;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 31, hf = lane >> 5;
-    const F3Minus minus = f3_minus();
+    const QxMinus minus = qx_minus();
     F3Range range = f3_range();
     const int chunks = a.K / 64, mine = 2 * ((chunks - wave + KS - 1) / KS);        /* steps of this wavefront */
     unsigned char *base = f3_lds + wave * (ST * F3_STAGE);
@@ -442,8 +431,9 @@ int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int gr
     if(mode == GEMM_TN) return launch_tiles<GEMM_TN, 32, 64, 64 * F3_WAVES, lds, k_gemm_f32s<GEMM_TN>>(a, probs, nprob, st);
     int most = 0;
     for(int i = 0; i < nprob; i++) if(probs[i].M > most) most = probs[i].M;
-    if(f3_nt_tiles(probs, nprob, K, N) < 3LL * qlmx_cu_count() && most >= 128) return launch_tiles<GEMM_NT, 64, 64, 256, 4 * 64 * 68 * 4, k_gemm_f32s_nt<4>>(a, probs, nprob, st);
-    return launch_tiles<GEMM_NT, 64, 64, 64, 64, k_gemm_f32s_nt<1>>(a, probs, nprob, st);
+    if(f3_nt_tiles(probs, nprob, K, N) < 3LL * qlmx_cu_count() && most >= 128) return launch_tiles<GEMM_NT, 64, 64, 256, 4 * 64 * 68 * 4, k_gemm_f32s_nt<4, false>>(a, probs, nprob, st);
+    return most < 32 ? launch_tiles<GEMM_NT, 64, 64, 64, 64, k_gemm_f32s_nt<1, true>>(a, probs, nprob, st)
+                     : launch_tiles<GEMM_NT, 64, 64, 64, 64, k_gemm_f32s_nt<1, false>>(a, probs, nprob, st);
 }
 
 /* Whether these kernels take a call: 64 columns (nn) or 64 of the contraction (tn) inside one scale group, whole units of 16 bytes. Everything else
