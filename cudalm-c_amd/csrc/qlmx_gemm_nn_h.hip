@@ -13,12 +13,18 @@
  * Weights are multiplied by 2^8 before the conversion and the accumulators by 2^-8 after the last step, which
  * moves the range in which fp16 keeps all 11 bits to 2.4e-7 <= |w| <= 255.
  *
- * 256x128 output tile, 32-deep steps, four wavefronts 2x2 with 4x2 accumulators each, two LDS buffers per
- * operand. Every operand passes through registers once: a thread loads 16 bytes of four activation rows and
- * 16 weights per step two steps ahead, converts them one step ahead, and writes them into the buffer that was
- * read in the step before. Layouts in LDS as in qlmx_gemm_nn_lds.hip: activation rows of 64 bytes with the four
- * 16-byte pieces rotated by the row (conflict-free 128-bit operand reads), weight rows of 256 bytes in the
- * matrix's own order with the 16-byte units xor-swizzled, read through ds_read_b64_tr_b16.
+ * Tiles of 256 x 256 (or less, nh_tiles), steps 64 deep, eight wavefronts with 128 x 64 outputs each, two LDS buffers per operand: 128 KB, one
+ * workgroup per CU. Every operand passes through registers once: a thread loads 16 bytes of four activation rows and 32 weights per step,
+ * converts them a step later and writes them into the buffer that is not being read. What bounds it is what the wavefronts do beside
+ * the products: with the loads, conversions and LDS writes left out the gate|up launch of 3001 tokens (64 experts, top 4, 2048 x 1408) takes 137 of
+ * its 190 us, without the loads alone 165, without the conversions 159; LDS reads and barriers are in the 137 (128 without them). So the tile is
+ * as large as the registers allow -- a piece of activations or weights is prepared once for 256 columns or rows -- and the step is 64
+ * deep: activation rows are read in whole lines of 128 bytes, weights and scales with half as many loads, and there are half as many barriers.
+ * gate|up and down of those tokens, us: 228, 120 with 256 x 128 tiles on four wavefronts and steps of 32; 217, 110 with eight
+ * wavefronts and 256 x 256; 199, 100 with steps of 64; 190, 97 with the operand reads spread over the first products of a slice. Loads one
+ * step further ahead, wavefront priorities, buffer addressing or three LDS buffers change nothing.
+ * In LDS activation rows are 128 bytes with the eight 16-byte pieces xor-swizzled by the row (conflict-free 128-bit operand
+ * reads), weight rows in the matrix's own order with xor-swizzled 16-byte units, read through ds_read_b64_tr_b16.
  */
 #include "qlmx_gemm.h"
 #include <type_traits>
@@ -30,12 +36,12 @@ typedef float    f32x16 __attribute__((ext_vector_type(16)));
 typedef int      i32x2 __attribute__((ext_vector_type(2)));
 typedef int      i32x4 __attribute__((ext_vector_type(4)));
 
-#define NH_BM 256
-#define NH_BN 128
-#define NH_BK 32
-#define NH_A_BYTES (NH_BM * NH_BK * 2)          /* 16384 */
-#define NH_B_BYTES (NH_BK * NH_BN * 2)          /*  8192 */
-#define NH_B_OFF (2 * NH_A_BYTES)
+#define NH_BK 64
+#define NH_BN(WN) (64 * (WN))                    /* columns of a tile: 256 or 128, 64 for each column of wavefronts */
+#define NH_A_BYTES(ROWS) (NH_BK * (ROWS) * 2)
+#define NH_B_BYTES(WN) (NH_BK * NH_BN(WN) * 2)   /* 32768, 16384 */
+#define NH_LDS_BYTES(WN, ROWS) (2 * NH_B_BYTES(WN) + 2 * NH_A_BYTES(ROWS))
+#define NH_THREADS 512
 #define NH_WSCALE 4096.0f                       /* 16 (the digits come as digit/16) * 2^8 (range shift) */
 #define NH_UNSCALE (1.0f / 256.0f)
 
@@ -47,25 +53,25 @@ typedef int      i32x4 __attribute__((ext_vector_type(4)));
  *               points at its row indices, out[idx[r], :] = out[idx[r], :] + gate[idx[r]] * y[r, :] (gate NULL: + y[r, :]),
  *               rows with idx[r] < 0 dropped. Within one launch every output row must be named at most once. */
 enum { NH_PLAIN = 0, NH_GATHER = 1, NH_SCATTER = 2 };
-struct NhArgs { const DevProb *pr; int nprob, ntiles, nfull, tiles_n; const signed char *d; const float *s; int gshift; int K, N;
+struct NhArgs { const DevProb *pr; int nprob, ntiles, nfull, piece, rows; const signed char *d; const float *s; int gshift; int K, N;
                 const char *xsrc; float *out; const float *gate; };
 
 /* a row of zeros as long as the longest contraction a gathering launch accepts: what a dropped row reads */
 #define NH_ZERO_BYTES 32768
 static __device__ __align__(16) unsigned char nh_zero_row[NH_ZERO_BYTES];
 
-template<int OFF> __device__ __forceinline__ i32x4 nh_rd128(uint32_t addr){
+__device__ __forceinline__ i32x4 nh_rd128(uint32_t addr, int off){
     i32x4 v;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(off));
     return v;
 }
-template<int OFF> __device__ __forceinline__ i32x2 nh_tr(uint32_t addr){
+__device__ __forceinline__ i32x2 nh_tr(uint32_t addr, int off){
     i32x2 v;
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(off));
     return v;
 }
-template<int OFF> __device__ __forceinline__ void nh_wr128(uint32_t addr, i32x4 v){
-    asm volatile("ds_write_b128 %0, %1 offset:%2" :: "v"(addr), "v"(v), "n"(OFF) : "memory");
+__device__ __forceinline__ void nh_wr128(uint32_t addr, int off, i32x4 v){
+    asm volatile("ds_write_b128 %0, %1 offset:%2" :: "v"(addr), "v"(v), "i"(off) : "memory");
 }
 /* Global loads are ordinary loads here: this kernel has no load-to-LDS instruction, so the compiler's own wait
  * counts are exact (it waits, with the right count, just before the first use of a loaded value, also when that
@@ -76,11 +82,11 @@ typedef const __attribute__((address_space(1))) i32x4 g_i32x4;
 __device__ __forceinline__ int   nh_gld4(const void *p){ return *(g_i32 *)p; }
 __device__ __forceinline__ i32x2 nh_gld8(const void *p){ return *(g_i32x2 *)p; }
 __device__ __forceinline__ i32x4 nh_gld16(const void *p){ return *(g_i32x4 *)p; }
-struct NhOps { i32x4 a[4]; i32x2 b[2][2]; };
-__device__ __forceinline__ void nh_wait_lds(NhOps &o){
-    asm volatile("s_waitcnt lgkmcnt(0)"
-        : "+v"(o.a[0]), "+v"(o.a[1]), "+v"(o.a[2]), "+v"(o.a[3]),
-          "+v"(o.b[0][0]), "+v"(o.b[0][1]), "+v"(o.b[1][0]), "+v"(o.b[1][1]));
+template<int NI> struct NhOps { i32x4 a[NI]; i32x2 b[2][2]; };
+template<int NI> __device__ __forceinline__ void nh_wait_lds(NhOps<NI> &o){
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o.b[0][0]), "+v"(o.b[0][1]), "+v"(o.b[1][0]), "+v"(o.b[1][1]) :: "memory");
+#pragma unroll
+    for(int i = 0; i < NI; i++) asm volatile("" : "+v"(o.a[i]));
 }
 __device__ __forceinline__ f16x8 nh_pack(const i32x2 lo, const i32x2 hi){
     const i32x4 v = {lo[0], lo[1], hi[0], hi[1]};
@@ -96,90 +102,77 @@ __device__ __forceinline__ int nh_pk(float lo, float hi){          /* round to n
     return __builtin_bit_cast(int, __builtin_convertvector(v, f16x2));
 }
 
-struct NhW { i32x2 d; int s; };
-
-/* One output tile of NI*64 rows (NI = 4: the full 256; the last tile of a problem takes the smallest NI that
- * holds its rows). */
+/* One output tile of WM*NI*32 rows and WN*64 columns on WM x WN wavefronts; the last tile of a problem takes the smallest NI that holds its rows. */
 /* The second half of a gate|up problem (DUAL): the other weight matrix, its fp32 output, the SwiGLU output. The
- * tile's 128 LDS columns are then [gate 0-31 | up 0-31 | gate 32-63 | up 32-63] of the problem's columns
- * j0 .. j0+63: a wavefront's first accumulator column holds gate and its second up of the same 32 columns. */
+ * tile's LDS columns are then [gate 0-31 | up 0-31 | gate 32-63 | up 32-63 | ...] of the problem's columns from
+ * j0 on: a wavefront's first accumulator column holds gate and its second up of the same 32 columns. */
 struct NhDual { unsigned long long wq, wg; float *C; unsigned short *act; };
 
-template<int NI, int IO, bool DUAL = false>
+template<int NI, int WN, int IO, bool DUAL = false>
 __device__ __forceinline__ void nh_tile(const NhArgs &a, const DevProb &P, const NhDual &Q, int i0, int j0, unsigned char *lds){
-    const int rows = P.M;
+    constexpr int WM = 8 / WN, NA = NI * WM / 2, DU = WN;         /* activation pieces and weight units (8 digits) of a thread and step */
+    constexpr int BROW = NH_BN(WN) * 2, BB = NH_B_BYTES(WN), AB = NH_A_BYTES(WM * NI * 32);
+    typedef std::conditional_t<WN == 4, i32x4, i32x2> digits_t;
+    const int rows = P.M < i0 + a.rows ? P.M : i0 + a.rows;               /* a tile of 192 rows may be taken by wavefronts for 256 */
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = (wave >> 1) * (NI * 32), wj = (wave & 1) * 64;
+    const int wi = (wave / WN) * (NI * 32), wj = (wave % WN) * 64;
     const int fr = lane & 31, hf = lane >> 5;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
-    const int steps = a.K / NH_BK;
+    const int steps = a.K / NH_BK, blocks = a.K >> 5;             /* whole steps; blocks of 32 contraction indices */
+    const bool half = a.K & 32, tiny = a.K == 32;
 
-    /* ---- activations: position p = h*256 + tid of a buffer is row p/4, stored piece p%4 = ko ^ ((row >> 2) & 3) ---- */
-    const char *srcA[NI]; uint32_t posA[NI];
+    /* ---- activations: position p = h*512 + tid of a buffer is row p/8, stored piece p%8 = ko ^ (row & 7) ---- */
+    const char *srcA[NA];
 #pragma unroll
-    for(int h = 0; h < NI; h++){
-        const int p = h * 256 + tid, r = p >> 2, ko = (p & 3) ^ ((r >> 2) & 3);
+    for(int h = 0; h < NA; h++){
+        const int p = h * NH_THREADS + tid, r = p >> 3, ko = ((p & 7) ^ (r & 7)) & (tiny ? 3 : 7);
         const int rr = (i0 + r < rows) ? i0 + r : rows - 1;               /* clamp: feeds unstored rows only */
         if(IO == NH_GATHER){
             const int tok = ((const int *)P.A)[rr];
             srcA[h] = (tok >= 0 ? a.xsrc + (size_t)tok * a.K * 2 : (const char *)nh_zero_row) + ko * 16;
         } else srcA[h] = (const char *)P.A + ((size_t)rr * a.K + ko * 8) * 2;
-        posA[h] = (uint32_t)p * 16;
     }
-    /* ---- weights: thread = (contraction row kr, columns oc*16 .. +15): one 8-byte load of digits and one scale
-     * per step; its two 16-byte units are taken in opposite order by even and odd rows, so that the 16 lanes of
-     * a write phase (two rows) hit 16 different units ---- */
-    const int oc = tid & 7, kr = tid >> 3, odd = kr & 1;
-    const bool second = DUAL && ((oc >> 1) & 1);
-    const size_t e0 = (size_t)kr * a.N + j0 + (DUAL ? ((oc & 1) + ((oc >> 2) << 1)) * 16 : oc * 16);
+    /* ---- weights: thread = (contraction row kr, columns oc*8*DU .. +8*DU-1): one load of digits and one scale per
+     * step. Unit u (8 columns) of row k is stored at u ^ f(k), f(k) = (k & 3) << 2 | (k >> 2 & 3): its upper bits part the
+     * four rows of a transposing read, its lower ones the lanes of a write phase, which hold the same unit of
+     * different rows; the lanes are dealt to (kr, oc) so that 16 of them hit 16 different units. ---- */
+    const int oc = WN == 4 ? (lane & 3) | ((lane >> 2) & 4) : lane & 7;
+    const int kr = WN == 4 ? (lane & 12) | (lane >> 5) | ((wave & 1) << 1) | ((wave >> 1) << 4)
+                           : ((lane >> 1) & 4) | (lane >> 4) | (wave << 3);
+    const bool second = DUAL && (WN == 4 ? oc & 1 : (oc >> 1) & 1);
+    const int col0 = DUAL ? (WN == 4 ? (oc >> 1) * 32 : ((oc & 1) + ((oc >> 2) << 1)) * 16) : oc * (8 * DU);
+    const size_t e0 = (size_t)(tiny ? kr & 31 : kr) * a.N + j0 + col0;
     const signed char *pw = a.d + (((second ? Q.wq : P.wq) + e0) >> 1);
     const float *ps = a.s + (second ? Q.wg : P.wg) + (e0 >> a.gshift);
-    const size_t wstep = (size_t)NH_BK * a.N >> 1, sstep = (size_t)NH_BK * a.N >> a.gshift;
-    const int sw = (kr & 3) << 2;
-    const uint32_t wr0 = NH_B_OFF + (uint32_t)(kr * 256 + (((2 * oc + odd) ^ sw) << 4));         /* written first  */
-    const uint32_t wr1 = NH_B_OFF + (uint32_t)(kr * 256 + (((2 * oc + 1 - odd) ^ sw) << 4));     /* written second */
-    auto tile_of = [&](int t){ return (size_t)(t < steps ? t : steps - 1); };   /* past the end: the last one again, never used */
-    auto load_w = [&](int t) -> NhW { NhW w; w.d = nh_gld8(pw + tile_of(t) * wstep); w.s = nh_gld4(ps + tile_of(t) * sstep); return w; };
-    auto load_a = [&](int t, int h) -> i32x4 { return nh_gld16(srcA[h] + tile_of(t) * (NH_BK * 2)); };
-    auto unit_digits = [&](const NhW &w, int which) -> uint32_t { return (uint32_t)((which ^ odd) ? w.d[1] : w.d[0]); };
-    auto convert_a = [&](const i32x4 &v) -> i32x4 {
-        i32x4 r;
-#pragma unroll
-        for(int j = 0; j < 4; j++) r[j] = nh_bf16x2_to_f16x2(v[j]);
-        return r;
-    };
-    auto dequant_unit = [&](uint32_t digits, float sc) -> i32x4 {
-        const QxNibs nb = qx_nibs(digits);
-        i32x4 r;
-#pragma unroll
-        for(int j = 0; j < 4; j++) r[j] = nh_pk(sc * qx_nib16(nb, 2 * j), sc * qx_nib16(nb, 2 * j + 1));
-        return r;
-    };
+    const size_t wblock = (size_t)32 * a.N >> 1, sblock = (size_t)32 * a.N >> a.gshift;
+    /* first block of tile t: the tile behind the last whole one ends with the matrix, so that of half a tile the second half counts */
+    auto block_of = [&](int t){ const int b = 2 * t < blocks - 2 ? 2 * t : blocks - 2; return (size_t)(b < 0 ? 0 : b); };
+    digits_t wd; int wsc; i32x4 av[NA];
+    auto load_wd = [&](int t){ if constexpr(WN == 4) wd = nh_gld16(pw + block_of(t) * wblock); else wd = nh_gld8(pw + block_of(t) * wblock); };
+    auto load_ws = [&](int t){ wsc = nh_gld4(ps + block_of(t) * sblock); };
+    auto load_a = [&](int t, int h){ av[h] = nh_gld16(srcA[h] + block_of(t) * 64); };
 
     /* ---- LDS addresses. Which of an operand's two buffers a step reads or writes is known at compile time (the
-     * loop below is unrolled by two), so the buffer, the k16 slice and the second half of a transposing read all
-     * go into the instructions' immediate offsets and the loop computes no LDS address at all. ---- */
-    uint32_t ra[2][NI];                                  /* [k16 slice][row tile] activations, 128-bit reads */
+     * loop below is unrolled by two), so the buffer, the row tile, the k16 slice of the weights and the thread's piece
+     * all go into the instructions' immediate offsets and the loop computes no LDS address at all. ---- */
+    uint32_t ra[4];                                      /* [k16 slice] activations, 128-bit reads */
 #pragma unroll
-    for(int i = 0; i < NI; i++){
-        const int r = wi + i * 32 + fr, f = (r >> 2) & 3;
-#pragma unroll
-        for(int ks = 0; ks < 2; ks++) ra[ks][i] = lds_base + (uint32_t)(r * 64 + (((ks * 2 + hf) ^ f) << 4));
-    }
-    uint32_t rb[2];                                      /* [column tile] weights, transposing reads */
+    for(int ks = 0; ks < 4; ks++) ra[ks] = lds_base + 2 * BB + (uint32_t)((wi + fr) * 128 + (((ks * 2 + hf) ^ (fr & 7)) << 4));
+    uint32_t rb[2][2];                                   /* [column tile][rows 0-3, 4-7 of eight] weights, transposing reads */
     {
         const int g16 = lane >> 4, s16 = lane & 15, v = s16 >> 2, q = s16 & 3, khalf = g16 >> 1, chalf = g16 & 1;
-        const int row0 = khalf * 8 + v, swr = (row0 & 3) << 2;
 #pragma unroll
-        for(int j = 0; j < 2; j++){
-            const int col = wj + j * 32 + chalf * 16 + q * 4;
-            rb[j] = lds_base + (uint32_t)(row0 * 256 + (((col >> 3) ^ swr) << 4) + (col & 7) * 2);
-        }
+        for(int j = 0; j < 2; j++)
+#pragma unroll
+            for(int e = 0; e < 2; e++){
+                const int k = khalf * 8 + e * 4 + v, col = wj + j * 32 + chalf * 16 + q * 4, f = ((k & 3) << 2) | ((k >> 2) & 3);
+                rb[j][e] = lds_base + (uint32_t)(k * BROW + (((col >> 3) ^ f) << 4) + (col & 7) * 2);
+            }
     }
-    uint32_t wpa[NI];
+    const uint32_t wpa = lds_base + 2 * BB + (uint32_t)tid * 16;
+    uint32_t wpb[DU];
 #pragma unroll
-    for(int h = 0; h < NI; h++) wpa[h] = lds_base + posA[h];
-    const uint32_t wp0 = lds_base + wr0 - NH_B_OFF, wp1 = lds_base + wr1 - NH_B_OFF;
+    for(int u = 0; u < DU; u++) wpb[u] = lds_base + (uint32_t)(kr * BROW + (((oc * DU + u) ^ (((kr & 3) << 2) | ((kr >> 2) & 3))) << 4));
 
     f32x16 acc[NI][2];
 #pragma unroll
@@ -187,103 +180,106 @@ __device__ __forceinline__ void nh_tile(const NhArgs &a, const DevProb &P, const
 #pragma unroll
         for(int j = 0; j < 2; j++) acc[i][j] = (f32x16)(0.0f);
 
-    /* ---- prologue: tile 0 into buffer 0, tile 1 into registers; all requests go out before the first use ---- */
-    NhW wA, wB; i32x4 aA[NI], aB[NI];
-    {
-        NhW w0 = load_w(0); i32x4 a0[NI];
-#pragma unroll
-        for(int h = 0; h < NI; h++) a0[h] = load_a(0, h);
-        wB = load_w(1);
-#pragma unroll
-        for(int h = 0; h < NI; h++) aB[h] = load_a(1, h);
-#pragma unroll
-        for(int h = 0; h < NI; h++) nh_wr128<0>(wpa[h], convert_a(a0[h]));
-        const float sc = __int_as_float(w0.s) * NH_WSCALE;
-        nh_wr128<NH_B_OFF>(wp0, dequant_unit(unit_digits(w0, 0), sc));
-        nh_wr128<NH_B_OFF>(wp1, dequant_unit(unit_digits(w0, 1), sc));
-    }
-
-    /* Main loop, two steps per iteration: step `st` of parity PAR reads buffers PAR, holds tile st+1 in the
-     * register set `cur` (loaded during step st-1) and loads tile st+2 into the set `nxt`; the two sets swap
-     * roles from step to step, so no loaded value is ever copied and a tile's loads stay in flight from the first
-     * items of step st until the conversions of step st+1 need them, more than a step later (the compiler places
-     * those waits, with exact counts: this kernel has no load-to-LDS instruction to confuse it).
-     * A wavefront issues in order and an MFMA of this shape leaves room for about four vector-ALU instructions
-     * behind it, so everything else of a step is cut into small items that are dealt evenly into the gaps after
-     * the step's MFMAs (fences keep the compiler from gathering them again):
-     *   the loads of tile st+2 (weights, then the NI activation pieces),
-     *   the conversion of tile st+1's activation pieces (two words per item) and their LDS writes,
-     *   the dequantisation of tile st+1's weights (two weights per item) and their two LDS writes,
-     * the writes going to the buffers that were read in step st-1. */
-    constexpr int SLOTS = NI * 4, ITEMS = 2 + NI + 2 * NI + 8 + 2;
-    auto step = [&](auto PARC, int st, const NhW &wcur, const i32x4 (&acur)[NI], NhW &wnxt, i32x4 (&anxt)[NI]){
-        constexpr int PAR = decltype(PARC)::value;
-        constexpr int RA = PAR * NH_A_BYTES, RB = NH_B_OFF + PAR * NH_B_BYTES;                 /* read  */
-        constexpr int WA = (1 - PAR) * NH_A_BYTES, WB = NH_B_OFF + (1 - PAR) * NH_B_BYTES;     /* write */
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     /* own LDS writes of tile st are done */
-        __builtin_amdgcn_s_barrier();
-        i32x4 ah[NI], wh[2];
-        QxNibs dg[2];
-        const float sc = __int_as_float(wcur.s) * NH_WSCALE;
-        auto item = [&](int k){
-            if(k == 0)      wnxt.d = nh_gld8(pw + tile_of(st + 2) * wstep);
-            else if(k == 1) wnxt.s = nh_gld4(ps + tile_of(st + 2) * sstep);
-            else if(k < 2 + NI) anxt[k - 2] = nh_gld16(srcA[k - 2] + tile_of(st + 2) * (NH_BK * 2));
-            else if(k < 2 + 3 * NI){
-                const int q = k - 2 - NI, h = q >> 1;
-                if((q & 1) == 0){ ah[h][0] = nh_bf16x2_to_f16x2(acur[h][0]); ah[h][1] = nh_bf16x2_to_f16x2(acur[h][1]); }
-                else { ah[h][2] = nh_bf16x2_to_f16x2(acur[h][2]); ah[h][3] = nh_bf16x2_to_f16x2(acur[h][3]); nh_wr128<WA>(wpa[h], ah[h]); }
-            } else if(k < 2 + 3 * NI + 8){
-                const int q = k - 2 - 3 * NI, r = q >> 2, j = q & 3;
-                if(q == 0){ dg[0] = qx_nibs(unit_digits(wcur, 0)); dg[1] = qx_nibs(unit_digits(wcur, 1)); }
-                wh[r][j] = nh_pk(sc * qx_nib16(dg[r], 2 * j), sc * qx_nib16(dg[r], 2 * j + 1));
-            } else {
-                if(k - 2 - 3 * NI - 8 == 0) nh_wr128<WB>(wp0, wh[0]); else nh_wr128<WB>(wp1, wh[1]);
-            }
-        };
-        NhOps o0, o1;
-        if(NI < 4){                                        /* the wait names all four; the spare ones hold nothing */
-#pragma unroll
-            for(int i = NI; i < 4; i++){ o0.a[i] = (i32x4)(0); o1.a[i] = (i32x4)(0); }
-        }
-#define NH_READ(O, KS)                                                                                    \
-        _Pragma("unroll")                                                                                 \
-        for(int i = 0; i < NI; i++) O.a[i] = nh_rd128<RA>(ra[KS][i]);                                     \
-        _Pragma("unroll")                                                                                 \
-        for(int j = 0; j < 2; j++){                                                                       \
-            O.b[j][0] = nh_tr<RB + KS * 16 * 256>(rb[j]);                                                 \
-            O.b[j][1] = nh_tr<RB + KS * 16 * 256 + 4 * 256>(rb[j]);                                       \
-        }
-#define NH_MMA(O, BLOCK)                                                                                  \
-        _Pragma("unroll")                                                                                 \
-        for(int m = 0; m < NI * 2; m++){                                                                  \
-            const int i = m >> 1, j = m & 1;                                                              \
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, O.a[i]), nh_pack(O.b[j][0], O.b[j][1]), acc[i][j], 0, 0, 0); \
-            {                                                                                             \
-                const int slot = BLOCK * (SLOTS / 2) + m;                                                 \
-                __builtin_amdgcn_sched_barrier(0);                                                        \
-                _Pragma("unroll")                                                                         \
-                for(int k = slot * ITEMS / SLOTS; k < (slot + 1) * ITEMS / SLOTS; k++) item(k);           \
-                __builtin_amdgcn_sched_barrier(0);                                                        \
-            }                                                                                             \
-        }
-        NH_READ(o0, 0)
-        nh_wait_lds(o0);
-        NH_READ(o1, 1)                                     /* in flight while slice 0 multiplies */
-        NH_MMA(o0, 0)
-        nh_wait_lds(o1);
-        NH_MMA(o1, 1)
-#undef NH_READ
-#undef NH_MMA
+    /* Everything a step does beside its products, cut into small items: per activation piece two conversions (the second
+     * writes the piece) and the load of the tile after; per weight unit four pairs and the write; the weights' two loads. */
+    constexpr int ITEMS = 3 * NA + 5 * DU + 2;
+    i32x4 ah, wh; QxNibs dg; float sc = 0.0f;
+    auto item = [&](auto WPARC, int k, int t){           /* tile t goes from the registers to its buffer, tile t+1 into the registers */
+        constexpr int WA = decltype(WPARC)::value * AB, WB = decltype(WPARC)::value * BB;
+        if(k < 3 * NA){
+            const int h = k / 3, q = k % 3;
+            if(q == 0){ ah[0] = nh_bf16x2_to_f16x2(av[h][0]); ah[1] = nh_bf16x2_to_f16x2(av[h][1]); }
+            else if(q == 1){ ah[2] = nh_bf16x2_to_f16x2(av[h][2]); ah[3] = nh_bf16x2_to_f16x2(av[h][3]); nh_wr128(wpa, WA + h * (NH_THREADS * 16), ah); }
+            else load_a(t + 1, h);
+        } else if(k < 3 * NA + 5 * DU){
+            const int u = (k - 3 * NA) / 5, q = (k - 3 * NA) % 5;
+            if(k == 3 * NA) sc = __int_as_float(wsc) * NH_WSCALE;
+            if(q == 0) dg = qx_nibs((uint32_t)wd[u]);
+            if(q < 4) wh[q] = nh_pk(sc * qx_nib16(dg, 2 * q), sc * qx_nib16(dg, 2 * q + 1));
+            else nh_wr128(wpb[u], WB, wh);
+        } else if(k == 3 * NA + 5 * DU) load_wd(t + 1);
+        else load_ws(t + 1);
     };
-    {
-        int st = 0;
-        for(; st + 1 < steps; st += 2){
-            step(std::integral_constant<int, 0>(), st, wB, aB, wA, aA);
-            step(std::integral_constant<int, 1>(), st + 1, wA, aA, wB, aB);
+    typedef std::integral_constant<int, 0> P0; typedef std::integral_constant<int, 1> P1;
+
+    /* ---- prologue: tile 0 into buffer 0, tile 1 into registers ---- */
+    load_wd(0); load_ws(0);
+#pragma unroll
+    for(int h = 0; h < NA; h++) load_a(0, h);
+#pragma unroll
+    for(int k = 0; k < ITEMS; k++) item(P0(), k, 0);
+
+    /* Main loop, two steps of 64 per iteration, a step in four slices of 16: the operands of a slice are read from LDS while the slice
+     * before multiplies. Tile t+1 goes from the registers into the other buffer in the gaps between the products of tile t,
+     * and each register is loaded again (tile t+2) right after its conversion, so a load has a whole step to arrive and needs
+     * no second set of registers. One barrier per step stands in the middle of its last slice: the tile's own operands are all
+     * read by then and the next tile is complete behind it, so its first operands arrive during the slice's other half.
+     * A wavefront issues in order and an MFMA of this shape leaves room for a handful of vector-ALU instructions
+     * behind it, so the items are dealt evenly into the gaps before the barrier (fences keep the compiler from gathering them). */
+    constexpr int SLOTS = 7 * NI, PER = (4 + 3 * NI) / (2 * NI);       /* operand reads behind each of a slice's first products */
+    NhOps<NI> o0, o1;
+#define NH_READ(O, KS, RA, RB, Q)                                                                         \
+        { if((Q) < 4) O.b[((Q) >> 1) & 1][(Q) & 1] = nh_tr(rb[((Q) >> 1) & 1][(Q) & 1], (RB) + KS * 16 * BROW); \
+          else if((Q) < 4 + NI) O.a[((Q) - 4) % NI] = nh_rd128(ra[KS], (RA) + (((Q) - 4) % NI) * 4096); }
+#define NH_MFMA(O, M)                                                                                     \
+        acc[(M) >> 1][(M) & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, O.a[(M) >> 1]), nh_pack(O.b[(M) & 1][0], O.b[(M) & 1][1]), acc[(M) >> 1][(M) & 1], 0, 0, 0);
+    /* products FROM .. TO-1 of slice KS from the operands O, with N reads of slice KS2's operands behind each */
+#define NH_SLICE(KS, O, FROM, TO, N, O2, KS2, RA2, RB2)                                                   \
+        _Pragma("unroll")                                                                                 \
+        for(int m = FROM; m < TO; m++){                                                                   \
+            const int slot = KS * NI * 2 + m;                                                             \
+            NH_MFMA(O, m)                                                                                 \
+            __builtin_amdgcn_sched_barrier(0);                                                            \
+            _Pragma("unroll")                                                                             \
+            for(int q = (m - FROM) * (N); q < (m - FROM + 1) * (N); q++) NH_READ(O2, KS2, RA2, RB2, q)    \
+            if(slot < SLOTS){                                                                             \
+                _Pragma("unroll")                                                                         \
+                for(int k = slot * ITEMS / SLOTS; k < (slot + 1) * ITEMS / SLOTS; k++) item(std::integral_constant<int, 1 - PAR>(), k, t + 1); \
+            }                                                                                             \
+            __builtin_amdgcn_sched_barrier(0);                                                            \
         }
-        if(st < steps) step(std::integral_constant<int, 0>(), st, wB, aB, wA, aA);
+    auto step = [&](auto PARC, int t){
+        constexpr int PAR = decltype(PARC)::value, RA = PAR * AB, RB = PAR * BB;
+        NH_SLICE(0, o0, 0, 2 * NI, PER, o1, 1, RA, RB)
+        nh_wait_lds(o1);
+        NH_SLICE(1, o1, 0, 2 * NI, PER, o0, 2, RA, RB)
+        nh_wait_lds(o0);
+        NH_SLICE(2, o0, 0, 2 * NI, PER, o1, 3, RA, RB)
+        nh_wait_lds(o1);
+        NH_SLICE(3, o1, 0, NI, 0, o0, 0, 0, 0)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     /* this wavefront's writes */
+        __builtin_amdgcn_s_barrier();
+        NH_SLICE(3, o1, NI, 2 * NI, (4 + 2 * NI - 1) / NI, o0, 0, AB - RA, BB - RB)
+        nh_wait_lds(o0);
+    };
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for(int n = 0; n < 4 + NI; n++) NH_READ(o0, 0, 0, 0, n)
+    nh_wait_lds(o0);
+    for(int t = 0; t < steps;){
+        step(P0(), t); if(++t >= steps) break;
+        step(P1(), t); ++t;
     }
+    if(half){                                              /* the last 32: the second half of the tile that ends with the matrix */
+        const int odd = steps & 1;
+#pragma unroll
+        for(int ks = 2; ks < 4; ks++) ra[ks] += odd * AB;
+#pragma unroll
+        for(int j = 0; j < 2; j++)
+#pragma unroll
+            for(int e = 0; e < 2; e++) rb[j][e] += odd * BB;
+#pragma unroll
+        for(int n = 0; n < 4 + NI; n++){ NH_READ(o0, 2, 0, 0, n) NH_READ(o1, 3, 0, 0, n) }
+        nh_wait_lds(o0); nh_wait_lds(o1);
+#pragma unroll
+        for(int m = 0; m < 2 * NI; m++){ NH_MFMA(o0, m) }
+#pragma unroll
+        for(int m = 0; m < 2 * NI; m++){ NH_MFMA(o1, m) }
+    }
+#undef NH_READ
+#undef NH_MFMA
+#undef NH_SLICE
 
     /* ---- epilogue: undo the range shift, then the lane holds column lane%32 of each 32x32 tile, four-row band lane/32 ---- */
 #pragma unroll
@@ -298,29 +294,39 @@ __device__ __forceinline__ void nh_tile(const NhArgs &a, const DevProb &P, const
     else qx_store_tiles<NI, 2>(acc, P.C + (size_t)row * a.N + (j0 + wj + fr), row, i0 + wi, rows, (size_t)a.N, false);
 }
 
-template<int IO>
-__global__ void __launch_bounds__(256, 2) k_gemm_nn_h(NhArgs a){
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * NH_A_BYTES + 2 * NH_B_BYTES];
-    const int t = qx_lpt_tile(blockIdx.x, a.nfull, a.ntiles, a.tiles_n);
+/* the smallest NI that holds a tile's rows: 64 rows for each with four columns of wavefronts, 128 with two; a last tile
+ * of 128 columns where the launch's tiles have 256 is one of two columns */
+template<int WN, int BM, int IO, bool DUAL = false>
+__device__ __forceinline__ void nh_rows(const NhArgs &a, const DevProb &P, const NhDual &Q, int i0, int j0, int left, unsigned char *lds){
+    if(WN == 4 && j0 + NH_BN(4) / (DUAL ? 2 : 1) <= a.N){
+        if(left > 192)      nh_tile<4, 4, IO, DUAL>(a, P, Q, i0, j0, lds);
+        else if(left > 128) nh_tile<3, 4, IO, DUAL>(a, P, Q, i0, j0, lds);
+        else if(left > 64)  nh_tile<2, 4, IO, DUAL>(a, P, Q, i0, j0, lds);
+        else                nh_tile<1, 4, IO, DUAL>(a, P, Q, i0, j0, lds);
+    } else if(BM == 256 && left > 128) nh_tile<2, 2, IO, DUAL>(a, P, Q, i0, j0, lds);
+    else                               nh_tile<1, 2, IO, DUAL>(a, P, Q, i0, j0, lds);
+}
+
+template<int IO, int WN, int BM>
+__global__ void __launch_bounds__(NH_THREADS, BM == 128 ? 4 : 2) k_gemm_nn_h(NhArgs a){
+    __shared__ __attribute__((aligned(16))) unsigned char lds[NH_LDS_BYTES(WN, BM)];
+    const int t = qx_lpt_tile(blockIdx.x, a.nfull, a.ntiles, a.piece);
     if(t >= a.ntiles) return;
     const DevProb P = a.pr[qx_find_problem(a.pr, a.nprob, t)];
     const int lt = t - P.tile0;
     const int ti = lt / P.tiles_n, tj = lt - ti * P.tiles_n;
-    const int i0 = ti * NH_BM, j0 = tj * NH_BN, left = P.M - i0;
+    const int i0 = ti * a.rows, j0 = tj * NH_BN(WN), left = P.M - i0 < a.rows ? P.M - i0 : a.rows;
     const NhDual none = {0, 0, nullptr, nullptr};
-    if(left > 192)      nh_tile<4, IO>(a, P, none, i0, j0, lds);
-    else if(left > 128) nh_tile<3, IO>(a, P, none, i0, j0, lds);
-    else if(left > 64)  nh_tile<2, IO>(a, P, none, i0, j0, lds);
-    else                nh_tile<1, IO>(a, P, none, i0, j0, lds);
+    nh_rows<WN, BM, IO>(a, P, none, i0, j0, left, lds);
 }
 
-/* gate|up problems with the SwiGLU in the epilogue (mg_ab w1, mg_ab w3, e_swig; cudalm.cu:4211-4215): tiles of 256
- * rows x 64 columns of both matrices; the table entry after the problem's holds the second matrix, the up output
+/* gate|up problems with the SwiGLU in the epilogue (mg_ab w1, mg_ab w3, e_swig; cudalm.cu:4211-4215): tiles of up to 256
+ * rows x 128 columns of both matrices; the table entry after the problem's holds the second matrix, the up output
  * and the bf16 SwiGLU output. The fp32 gate / up outputs are skipped when the problem's C is NULL. */
-template<int IO>
-__global__ void __launch_bounds__(256, 2) k_gemm_nn_h_swiglu(NhArgs a){
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * NH_A_BYTES + 2 * NH_B_BYTES];
-    const int t = qx_lpt_tile(blockIdx.x, a.nfull, a.ntiles, a.tiles_n);
+template<int IO, int WN, int BM>
+__global__ void __launch_bounds__(NH_THREADS, BM == 128 ? 4 : 2) k_gemm_nn_h_swiglu(NhArgs a){
+    __shared__ __attribute__((aligned(16))) unsigned char lds[NH_LDS_BYTES(WN, BM)];
+    const int t = qx_lpt_tile(blockIdx.x, a.nfull, a.ntiles, a.piece);
     if(t >= a.ntiles) return;
     const int pi = qx_find_problem(a.pr, a.nprob, t);
     const DevProb P = a.pr[pi];
@@ -328,13 +334,73 @@ __global__ void __launch_bounds__(256, 2) k_gemm_nn_h_swiglu(NhArgs a){
     const NhDual Q = {P2.wq, P2.wg, P2.C, (unsigned short *)P2.B};
     const int lt = t - P.tile0;
     const int ti = lt / P.tiles_n, tj = lt - ti * P.tiles_n;
-    const int i0 = ti * NH_BM, j0 = tj * (NH_BN / 2), left = P.M - i0;
-    if(left > 192)      nh_tile<4, IO, true>(a, P, Q, i0, j0, lds);
-    else if(left > 128) nh_tile<3, IO, true>(a, P, Q, i0, j0, lds);
-    else if(left > 64)  nh_tile<2, IO, true>(a, P, Q, i0, j0, lds);
-    else                nh_tile<1, IO, true>(a, P, Q, i0, j0, lds);
+    const int i0 = ti * a.rows, j0 = tj * (NH_BN(WN) / 2), left = P.M - i0 < a.rows ? P.M - i0 : a.rows;
+    nh_rows<WN, BM, IO, true>(a, P, Q, i0, j0, left, lds);
 }
 
+/* The loads of the compute units of an XCD while tiles are dealt to them, longest first, each to the least loaded one: groups of
+ * units with the same load. */
+#define NH_UNITS 48
+struct NhLoads { int n; float load[NH_UNITS]; int units[NH_UNITS]; };
+static void nh_deal(NhLoads &d, long long tiles, float cost){
+    int total = 0;
+    for(int k = 0; k < d.n; k++) total += d.units[k];
+    if(tiles > 8LL * total){                               /* all but the last few rounds at once */
+        const long long r = tiles / total - 4;
+        for(int k = 0; k < d.n; k++) d.load[k] += r * cost;
+        tiles -= r * total;
+    }
+    while(tiles > 0){
+        int k = 0;
+        for(int j = 1; j < d.n; j++) if(d.load[j] < d.load[k]) k = j;
+        const int take = tiles < d.units[k] ? (int)tiles : d.units[k];
+        const float l = d.load[k] + cost;
+        tiles -= take; d.units[k] -= take;
+        if(!d.units[k]){ d.n--; d.load[k] = d.load[d.n]; d.units[k] = d.units[d.n]; }
+        int j = 0;
+        while(j < d.n && d.load[j] != l) j++;
+        if(j == d.n){ d.load[j] = l; d.units[j] = 0; d.n++; }
+        d.units[j] += take;
+    }
+}
+/* The tile of a launch: the shape whose tiles, dealt out as the launch deals them, end first. Costs in units of a whole 256 x 256 tile, by
+ * height in 64 rows, from launches of whole rounds (256 compute units, contractions of 512 to 2048: 40, 33, 28 and 20 us for 256, 192, 128 and
+ * 64 rows of 256 columns and 1024 deep, 24 and 18 for 256 and 128 rows of 128): a CU holds one such tile, or two of 128 x 128, which
+ * share it (28 us for both) and overlap one's start and end with the other's loop, of use where the contraction is short. Wide tiles do the
+ * most products per weight and activation prepared and win wherever there are rounds enough; the others where the count is unlucky. us, chosen
+ * <- 256 x 256 always: 12 experts of 530 rows, 640 x 640 gate|up 21 <- 24; 8 of 256, 768 x 2048 plain 16 <- 21 (256 x 128); 100 of
+ * 120, 512 x 768 plain 24 <- 28 (128 x 128). Over 250 calls of 1 to 200 experts the choice is within 1.2 % of the best of the five. */
+struct NhTiles { int rows, columns; };
+static NhTiles nh_tiles(const qlmx_gemm_prob *probs, int nprob, int K, int columns){
+    static const float wide[5] = {0.0f, 0.50f, 0.65f, 0.82f, 1.0f}, narrow[5] = {0.0f, 0.45f, 0.45f, 0.67f, 0.67f}, pair[3] = {0.0f, 0.36f, 0.36f}, pair_short[3] = {0.0f, 0.29f, 0.29f};
+    NhTiles best = {256, 128};
+    float least = 0.0f;
+    const int cus = qlmx_cu_count() / 8, units = cus < 1 ? 1 : cus < NH_UNITS ? cus : NH_UNITS - 1;
+    for(int rows = 256; rows >= 128; rows -= 64)
+        for(int cols = 256; cols >= 128; cols -= 128){
+            if(cols > columns || (cols == 128 && rows == 192)) continue;
+            const bool paired = rows == 128 && cols == 128;
+            const float *thin = !paired ? narrow : K > 640 ? pair : pair_short;
+            const int g_wide = cols == 256 ? columns / 256 : 0, g_thin = cols == 256 ? columns % 256 / 128 : columns / 128;
+            long long full = 0, high[5] = {0, 0, 0, 0, 0};             /* tile rows: whole ones, last ones by height */
+            for(int i = 0; i < nprob; i++){
+                const int f = probs[i].M / rows, l = (probs[i].M - f * rows + 63) / 64;
+                full += f; high[l]++;
+            }
+            NhLoads ld; ld.n = 1; ld.load[0] = paired ? 0.11f : 0.0f; ld.units[0] = units;      /* a pair's last tile runs alone */
+            nh_deal(ld, (full * g_wide + 7) / 8, wide[rows / 64]); nh_deal(ld, (full * g_thin + 7) / 8, thin[rows / 64]);
+            for(int l = rows / 64; l > 0; l--){ nh_deal(ld, (high[l] * g_wide + 7) / 8, wide[l]); nh_deal(ld, (high[l] * g_thin + 7) / 8, thin[l]); }
+            float t = 0.0f;
+            for(int k = 0; k < ld.n; k++) if(ld.load[k] > t) t = ld.load[k];
+            if(least == 0.0f || t < least){ least = t; best.rows = rows; best.columns = cols; }
+        }
+    return best;
+}
+/* How many tiles of a row of last tiles stay on one XCD: all of them (they read the same activations) where there are rows enough to go round;
+ * fewer rows than that are dealt tile by tile, or a few XCDs get two rows and the others one: 3 experts of 700 rows, 2048 x 1408 gate|up 72 -> 38 us. */
+static int nh_piece(const ProbUpload &up, int g){
+    return (up.ntiles - up.nfull) / g >= 32 ? g : 1;
+}
 /* bf16 activations only; N % 128 == 0, K % 32 == 0, group a power of two >= 32 (checked by the caller).
  * io = NH_GATHER: xsrc is the bf16 token matrix and the problems' A fields are row-index lists;
  * io = NH_SCATTER: out (and gate, may be NULL) is the destination and the problems' C fields are row-index lists. */
@@ -342,17 +408,22 @@ int qlmx_gemm_nn_h_launch(const signed char *d, const float *s, int group, const
                           int K, int N, int io, const void *xsrc, float *out, const float *gate, hipStream_t st){
     QLMX_REQUIRE(io != NH_GATHER || (size_t)K * 2 <= NH_ZERO_BYTES, "grouped gemm nn with gather: K=%d exceeds %d", K, NH_ZERO_BYTES / 2);
     if(qlmx_small_rows(probs, nprob, GEMM_NN, K, N, 1, group)) return qlmx_gemm_nn_small_launch(d, s, group, probs, nprob, K, N, io, xsrc, out, gate, st);
+    const NhTiles tl = nh_tiles(probs, nprob, K, N);
+    const int bn = tl.columns;
     ProbUpload up; int slot;
     const RowBytes rb = {io == NH_GATHER ? sizeof(int) : (size_t)K * 2, io == NH_SCATTER ? sizeof(int) : (size_t)N * 4, 0, 0, 0};
-    int rc = qlmx_upload_problems_split(probs, nullptr, nprob, GEMM_NN, K, N, NH_BM, NH_BN, &rb, st, &up, &slot); if(rc) return rc;
+    int rc = qlmx_upload_problems_split(probs, nullptr, nprob, GEMM_NN, K, N, tl.rows, bn, &rb, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
-    NhArgs a; a.pr = up.dev; a.nprob = up.nprob; a.ntiles = up.ntiles; a.nfull = up.nfull; a.tiles_n = N / NH_BN; a.d = d; a.s = s; a.K = K; a.N = N;
+    NhArgs a; a.pr = up.dev; a.nprob = up.nprob; a.ntiles = up.ntiles; a.nfull = up.nfull; a.rows = tl.rows; a.piece = nh_piece(up, (N + bn - 1) / bn); a.d = d; a.s = s; a.K = K; a.N = N;
     a.xsrc = (const char *)xsrc; a.out = out; a.gate = gate;
     a.gshift = 0; while((1 << a.gshift) < group) a.gshift++;
-    const int grid = qx_lpt_grid(up.nfull, up.ntiles, a.tiles_n);
-    if(io == NH_GATHER)       hipLaunchKernelGGL(k_gemm_nn_h<NH_GATHER>,  dim3(grid), dim3(256), 0, st, a);
-    else if(io == NH_SCATTER) hipLaunchKernelGGL(k_gemm_nn_h<NH_SCATTER>, dim3(grid), dim3(256), 0, st, a);
-    else                      hipLaunchKernelGGL(k_gemm_nn_h<NH_PLAIN>,   dim3(grid), dim3(256), 0, st, a);
+    const int grid = qx_lpt_grid(up.nfull, up.ntiles, a.piece);
+#define NH_LAUNCH(KERNEL, IO) do{ if(tl.columns == 256)            hipLaunchKernelGGL((KERNEL<IO, 4, 256>), dim3(grid), dim3(NH_THREADS), 0, st, a); \
+                                  else if(tl.rows == 128) hipLaunchKernelGGL((KERNEL<IO, 2, 128>), dim3(grid), dim3(NH_THREADS), 0, st, a); \
+                                  else                    hipLaunchKernelGGL((KERNEL<IO, 2, 256>), dim3(grid), dim3(NH_THREADS), 0, st, a); }while(0)
+    if(io == NH_GATHER)       NH_LAUNCH(k_gemm_nn_h, NH_GATHER);
+    else if(io == NH_SCATTER) NH_LAUNCH(k_gemm_nn_h, NH_SCATTER);
+    else                      NH_LAUNCH(k_gemm_nn_h, NH_PLAIN);
     QLMX_LAUNCH_CHECK("grouped gemm nn (fp16 matrix core) launch");
     return qlmx_upload_done(slot, st);
 }
@@ -364,16 +435,18 @@ int qlmx_gemm_nn_h_swiglu_launch(const signed char *d, const float *s, int group
                                  int nprob, int K, int N, const void *xsrc, hipStream_t st){
     QLMX_REQUIRE(!xsrc || (size_t)K * 2 <= NH_ZERO_BYTES, "grouped gemm nn + swiglu with gather: K=%d exceeds %d", K, NH_ZERO_BYTES / 2);
     if(N % 128 == 0 && qlmx_small_rows(gate, nprob, GEMM_NN, K, N, 1, group)) return qlmx_gemm_nn_small_swiglu_launch(d, s, group, gate, up_, nprob, K, N, xsrc, st);
+    const NhTiles tl = nh_tiles(gate, nprob, K, 2 * N);
+    const int bn = tl.columns / 2;
     ProbUpload up; int slot;
     const RowBytes rb = {xsrc ? sizeof(int) : (size_t)K * 2, (size_t)N * 4, 0, (size_t)N * 2, (size_t)N * 4};
-    int rc = qlmx_upload_problems_split(gate, up_, nprob, GEMM_NN, K, N, NH_BM, NH_BN / 2, &rb, st, &up, &slot); if(rc) return rc;
+    int rc = qlmx_upload_problems_split(gate, up_, nprob, GEMM_NN, K, N, tl.rows, bn, &rb, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
-    NhArgs a; a.pr = up.dev; a.nprob = up.nprob; a.ntiles = up.ntiles; a.nfull = up.nfull; a.tiles_n = N / (NH_BN / 2); a.d = d; a.s = s; a.K = K; a.N = N;
+    NhArgs a; a.pr = up.dev; a.nprob = up.nprob; a.ntiles = up.ntiles; a.nfull = up.nfull; a.rows = tl.rows; a.piece = nh_piece(up, (N + bn - 1) / bn); a.d = d; a.s = s; a.K = K; a.N = N;
     a.xsrc = (const char *)xsrc; a.out = nullptr; a.gate = nullptr;
     a.gshift = 0; while((1 << a.gshift) < group) a.gshift++;
-    const int grid = qx_lpt_grid(up.nfull, up.ntiles, a.tiles_n);
-    if(xsrc) hipLaunchKernelGGL(k_gemm_nn_h_swiglu<NH_GATHER>, dim3(grid), dim3(256), 0, st, a);
-    else     hipLaunchKernelGGL(k_gemm_nn_h_swiglu<NH_PLAIN>,  dim3(grid), dim3(256), 0, st, a);
+    const int grid = qx_lpt_grid(up.nfull, up.ntiles, a.piece);
+    if(xsrc) NH_LAUNCH(k_gemm_nn_h_swiglu, NH_GATHER);
+    else     NH_LAUNCH(k_gemm_nn_h_swiglu, NH_PLAIN);
     QLMX_LAUNCH_CHECK("grouped gemm nn + swiglu (fp16 matrix core) launch");
     return qlmx_upload_done(slot, st);
 }

@@ -397,6 +397,49 @@ def test_mfma_f16_forward_vs_oracle(q, orc, K, N, rows):
     assert got.size == off[-1] * N
 
 
+@pytest.mark.parametrize("E,M,K,N,group", [(16, 1000, 32, 640, 64), (12, 530, 96, 1152, 128), (16, 700, 96, 384, 64), (20, 700, 160, 384, 128),
+                                           (5, 300, 32, 384, 64), (40, 128, 224, 128, 32)])
+def test_mfma_f16_forward_tile_shapes(q, E, M, K, N, group):
+    """The five tile shapes of the fp16 forward, with and without half a step at the end and a narrow tile at a row's end, plain, behind a gather with
+    the SwiGLU and in front of a scatter. A weight is rounded once, by at most 2^-11 of it over 1 to 2, uniformly: 2^-11 / sqrt(3) of the
+    result bounds the root mean square. The fused forms see the same products: the same bits."""
+    import torch
+    rng = np.random.default_rng(77)
+    rows = [M] * (E - 3) + [M + 1, 0, M - 1]
+    off = np.concatenate([[0], np.cumsum(rows)]).astype(int)
+    R, n = int(off[-1]), E * K * N
+    digits = rng.integers(-7, 8, 2 * n).astype(np.int8)
+    s = (rng.uniform(0.5, 1.5, 2 * n // group) * 0.0086).astype(f32)
+    dd, ds = dev((digits[0::2] & 15 | (digits[1::2] & 15) << 4).astype(np.uint8)), dev(s)
+    x = dev(rng.standard_normal((R, K)).astype(f32)).bfloat16()
+    tok = torch.from_numpy(rng.permutation(R).astype(np.int32)).cuda()
+    xs = x[tok.long()].contiguous()
+    sep = [torch.full((R, N), 7.0, device="cuda") for _ in range(2)]
+    for m in range(2):
+        q.gemm_nn(dd, ds, group, q.problems([(xs.data_ptr() + off[e] * K * 2, None, sep[m].data_ptr() + off[e] * N * 4, m * n + e * K * N, (m * n + e * K * N) // group,
+                                              rows[e], 0.0) for e in range(E)]), E, K, N, pkg.ACT_BF16, pkg.MATH_MFMA_F16)
+    W = (np.repeat(s[:n // group], group).astype(np.float64) * digits[:n]).reshape(E, K, N)
+    xh = xs.float().cpu().numpy().astype(np.float64)
+    want = np.concatenate([xh[off[e]:off[e + 1]] @ W[e] for e in range(E)])
+    got = sep[0].cpu().numpy()
+    assert np.linalg.norm(got - want) < 2.0 ** -11 / np.sqrt(3) * np.linalg.norm(want)
+    if group >= 64:
+        gp, up, act = torch.full((R, N), 7.0, device="cuda"), torch.full((R, N), 7.0, device="cuda"), torch.zeros(R, N, device="cuda", dtype=torch.bfloat16)
+        q.gemm_nn_gather_swiglu(dd, ds, group, q.problems([(tok.data_ptr() + off[e] * 4, None, gp.data_ptr() + off[e] * N * 4, e * K * N, e * K * N // group, rows[e], 0.0)
+                                                           for e in range(E)]),
+                                q.problems([(0, act.data_ptr() + off[e] * N * 2, up.data_ptr() + off[e] * N * 4, n + e * K * N, (n + e * K * N) // group, rows[e], 0.0)
+                                            for e in range(E)]), E, K, N, x)
+        assert torch.equal(gp, sep[0]) and torch.equal(up, sep[1])
+        z = sep[0].double()
+        assert torch.allclose(act.double(), z * torch.sigmoid(z) * sep[1].double(), rtol=2.0 ** -8, atol=1e-6)      # one rounding to bf16
+    gate, out = dev(rng.uniform(0.1, 1.0, R).astype(f32)), dev(rng.standard_normal((R, N)).astype(f32))
+    ref = out.clone()
+    ref[tok.long()] += gate[tok.long()].unsqueeze(1) * sep[0]
+    q.gemm_nn_scatter(dd, ds, group, q.problems([(xs.data_ptr() + off[e] * K * 2, None, tok.data_ptr() + off[e] * 4, e * K * N, e * K * N // group, rows[e], 0.0)
+                                                 for e in range(E)]), E, K, N, out, gate)
+    assert torch.equal(out, ref)
+
+
 def test_mfma_f16_forward_range_edges(q, orc):
     """Where fp16 would lose bits the kernel's 2^8 range shift keeps them: weights scaled down to 1e-6 (below fp16's
     normal range unshifted) still meet the bar; activations far below fp16's normal range change nothing measurable;
