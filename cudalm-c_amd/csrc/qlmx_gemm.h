@@ -238,55 +238,80 @@ __device__ __forceinline__ void qx_swiglu_bwd1(float z, float u, float da, float
     const float sg = HW ? qx_fsig_hw(z) : qx_fsig(z), silu = z * sg, ds = sg + z * sg * (1.0f - sg);
     dg = da * u * ds; du = da * silu;
 }
-/* The SwiGLU gradient as the epilogue of the GEMM that produces its input: the NI x 2 accumulator tiles hold
- * da = d(act); gp, up (fp32) are read at the same positions and bf16(dg), bf16(du) written there, so that da
- * itself never reaches memory; the sigmoid is qx_fsig_hw. All four pointers are at the lane's first element (row `row`, its column in
- * tile (., 0)); neighbouring columns are paired into 4-byte stores as in qx_store_swiglu. */
-template<int NI>
-__device__ __forceinline__ void qx_store_swiglu_bwd(const qx_f32x16 (&acc)[NI][2], const float *gp, const float *up,
-                                                    unsigned short *dg, unsigned short *du, int row, int rows, size_t ld){
-    typedef const __attribute__((address_space(1))) float gfloat;
-    typedef __attribute__((address_space(1))) uint32_t guint;
-    const bool oddl = threadIdx.x & 1;
+/* ---- 32 x 64 strips of accumulators across the lanes ----
+ * A lane of the matrix core's result holds single elements of one column; memory wants four neighbouring columns of a row per lane. A strip
+ * goes through 8 KB of LDS that belong to the wavefront: element (r, c) at r * 64 + (c ^ 32 where bits 0 and 2 of r differ), which parts the two
+ * rows of a write and the rows of a read into different halves of the banks. */
+typedef float    qx_f4 __attribute__((ext_vector_type(4), aligned(4)));       /* memory accesses of 8 and 16 bytes, aligned to 4: what the hardware asks for */
+typedef uint32_t qx_u2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef __attribute__((address_space(1))) qx_f4 qx_gf4;
+typedef __attribute__((address_space(1))) qx_u2 qx_gu2;
+#define QX_STRIP_FLOATS (32 * 64)
+__device__ __forceinline__ void qx_strip_put(float *x, const qx_f32x16 (&acc)[2]){
+    const int lane = threadIdx.x & 63, fr = lane & 31, hf = lane >> 5;
+    float *at = x + hf * 256 + fr;
+    qx_wave_sync();
 #pragma unroll
-    for(int i = 0; i < NI; i++){
-        float z[2][16], u[2][16];
-#pragma unroll
-        for(int e = 0; e < 16; e++){
-            const int ro = i * 32 + (e >> 2) * 8 + (e & 3);
-            const bool in = row + ro < rows;
-#pragma unroll
-            for(int j = 0; j < 2; j++){
-                const size_t o = (size_t)ro * ld + j * 32;
-                z[j][e] = in ? *((gfloat *)gp + o) : 0.0f;
-                u[j][e] = in ? *((gfloat *)up + o) : 0.0f;
-            }
-        }
+    for(int e = 0; e < 16; e++)
 #pragma unroll
         for(int j = 0; j < 2; j++){
-            uint32_t a[16];                                  /* bf16(dg) | bf16(du) << 16 of the lane's 16 rows */
+            const int r = (e >> 2) * 8 + (e & 3);
+            at[r * 64 + ((j ^ (e & 1)) ? 32 - 32 * hf : 32 * hf)] = acc[j][e];
+        }
+    qx_wave_sync();
+}
+
+/* The SwiGLU gradient as the epilogue of the GEMM that produces its input: the NI x 2 accumulator tiles hold
+ * da = d(act); gp, up (fp32) are read at the same positions and bf16(dg), bf16(du) written there, so that da
+ * itself never reaches memory; the sigmoid is qx_fsig_hw. All four pointers are at the wavefront's first row and column; x is its strip.
+ * Sixteen lanes take a row of 64 columns, four each: per strip 16 loads (past the caches: gp and up are not needed again) and 16 stores of whole lines. Bound by
+ * memory: with it 32 experts of 512 rows, 768 x 2048, take 125 us, 74 without, and the difference is 270 MB. As single elements, a branch
+ * and a 64-bit address per load or store and the bf16 rounding in four integer operations, 141 us (64 of 2048, 2048 x 1408: 1186 -> 1080). */
+template<int NI, bool FULL>
+__device__ __forceinline__ void qx_swiglu_bwd_strips(const qx_f32x16 (&acc)[NI][2], float *x, const float *gp, const float *up,
+                                                     unsigned short *dg, unsigned short *du, int left, size_t ld){
+    const int lane = threadIdx.x & 63, rl = lane >> 4, c4 = (lane & 15) * 4;
+    const float *from = x + rl * 64 + (c4 ^ ((rl & 1) << 5)), *from_odd = x + rl * 64 + (c4 ^ ((rl & 1 ^ 1) << 5));
+    /* half a strip's values at a time, requested half a strip ahead */
+    qx_f4 z[2][4], u[2][4];
+    auto row_of = [&](int t) -> size_t { const int r = t * 4 + rl; return (size_t)(FULL || r < left ? r : left - 1); };
+    auto load = [&](int q){
 #pragma unroll
-            for(int e = 0; e < 16; e++){
-                float x, y;
-                qx_swiglu_bwd1<true>(z[j][e], u[j][e], acc[i][j][e], x, y);
-                a[e] = (uint32_t)qx_f32_to_bf16(x) | ((uint32_t)qx_f32_to_bf16(y) << 16);
-            }
-            /* the even lane of a pair of columns stores the first eight of its rows for both, the odd lane the rest */
+        for(int t = 0; t < 4; t++){
+            const size_t o = row_of(q * 4 + t) * ld + c4;
+            z[q & 1][t] = __builtin_nontemporal_load((const qx_gf4 *)(gp + o));
+            u[q & 1][t] = __builtin_nontemporal_load((const qx_gf4 *)(up + o));
+        }
+    };
+    load(0);
 #pragma unroll
-            for(int e = 0; e < 8; e++){
-                const uint32_t mine = oddl ? a[e + 8] : a[e];
-                const uint32_t got = (uint32_t)__shfl_xor((int)(oddl ? a[e] : a[e + 8]), 1, 64);
-                const uint32_t lo = oddl ? got : mine, hi = oddl ? mine : got;          /* even column, odd column */
-                const int e2 = oddl ? e + 8 : e;
-                const int ro = i * 32 + (e2 >> 2) * 8 + (e2 & 3);
-                if(row + ro < rows){
-                    const size_t o = (size_t)ro * ld + j * 32 - (oddl ? 1 : 0);
-                    *(guint *)(dg + o) = (lo & 0xFFFFu) | (hi << 16);
-                    *(guint *)(du + o) = (lo >> 16) | (hi & 0xFFFF0000u);
-                }
+    for(int q = 0; q < 2 * NI; q++){
+        if(!FULL && q * 16 >= left) break;
+        if(q + 1 < 2 * NI) load(q + 1);
+        if((q & 1) == 0) qx_strip_put(x, acc[q >> 1]);
+#pragma unroll
+        for(int t = 0; t < 4; t++){
+            const float4 da = *(const float4 *)((t & 1 ? from_odd : from) + ((q & 1) * 4 + t) * 256);
+            const qx_f4 zz = z[q & 1][t], uu = u[q & 1][t];
+            float g[4], v[4];
+            qx_swiglu_bwd1<true>(zz[0], uu[0], da.x, g[0], v[0]); qx_swiglu_bwd1<true>(zz[1], uu[1], da.y, g[1], v[1]);
+            qx_swiglu_bwd1<true>(zz[2], uu[2], da.z, g[2], v[2]); qx_swiglu_bwd1<true>(zz[3], uu[3], da.w, g[3], v[3]);
+            const int r = (q * 4 + t) * 4 + rl;
+            if(FULL || r < left){
+                const size_t o = (size_t)r * ld + c4;
+                const qx_u2 pg = {qx_pk_bf16(g[0], g[1]), qx_pk_bf16(g[2], g[3])}, pu = {qx_pk_bf16(v[0], v[1]), qx_pk_bf16(v[2], v[3])};
+                *(qx_gu2 *)(dg + o) = pg;
+                *(qx_gu2 *)(du + o) = pu;
             }
         }
     }
+}
+template<int NI>
+__device__ __forceinline__ void qx_store_swiglu_bwd(const qx_f32x16 (&acc)[NI][2], float *x, const float *gp, const float *up,
+                                                    unsigned short *dg, unsigned short *du, int left, size_t ld){
+    left = __builtin_amdgcn_readfirstlane(left);
+    if(left >= NI * 32)  qx_swiglu_bwd_strips<NI, true>(acc, x, gp, up, dg, du, left, ld);
+    else if(left > 0)    qx_swiglu_bwd_strips<NI, false>(acc, x, gp, up, dg, du, left, ld);
 }
 
 /* The NI x 2 accumulator tiles of one wavefront added to INDEXED output rows (the gated scatter and the
@@ -362,40 +387,42 @@ __device__ __forceinline__ void qx_chain_publish(int *flags, int flag, unsigned 
 __device__ __forceinline__ float qx_bf16_to_f32(unsigned short h){ return __uint_as_float((uint32_t)h << 16); }
 
 /* gate, up (fp32; both skipped when gp is NULL) and bf16(gate * sigmoid(gate) * up) of a gate|up tile (HW: the
- * sigmoid is qx_fsig_hw instead of the SwiGLU kernel's qx_fsig). The tile's 128 LDS columns are
- * [gate 0-31 | up 0-31 | gate 32-63 | up 32-63] of the problem's columns j0 .. j0+63, so a wavefront's first
- * accumulator column holds gate and its second holds up of the same 32 columns, element for element. */
-template<int NI, bool HW = false>
-__device__ __forceinline__ void qx_store_swiglu(const qx_f32x16 (&acc)[NI][2], float *gp, float *up, unsigned short *act,
-                                                 int row, int rows, size_t ld){
-    typedef __attribute__((address_space(1))) float gfloat;
-    typedef __attribute__((address_space(1))) uint32_t guint;
-    const bool oddl = threadIdx.x & 1;
+ * sigmoid is qx_fsig_hw instead of the SwiGLU kernel's qx_fsig). The tile's LDS columns are
+ * [gate 0-31 | up 0-31 | gate 32-63 | up 32-63 | ...] of the problem's columns from j0 on, so a wavefront's first
+ * accumulator column holds gate and its second holds up of the same 32 columns, element for element. The pointers are at the wavefront's
+ * first row and column, x is its strip; eight lanes take a row of 32 columns, four each (16384 rows, 768 x 2048, all three outputs: 175 us per
+ * launch with a branch, an address and a 4-byte store per element, 162 so). */
+template<int NI, bool HW, bool FULL>
+__device__ __forceinline__ void qx_swiglu_strips(const qx_f32x16 (&acc)[NI][2], float *x, float *gp, float *up, unsigned short *act, int left, size_t ld){
+    const int lane = threadIdx.x & 63, rl = lane >> 3, c4 = (lane & 7) * 4;
+    const float *from_g = x + rl * 64 + (c4 ^ (((rl ^ (rl >> 2)) & 1) << 5)), *from_u = x + rl * 64 + (c4 ^ (((rl ^ (rl >> 2)) & 1 ^ 1) << 5));
 #pragma unroll
     for(int i = 0; i < NI; i++){
-        uint32_t a[16];
+        if(!FULL && i * 32 >= left) break;
+        qx_strip_put(x, acc[i]);
 #pragma unroll
-        for(int e = 0; e < 16; e++){
-            const int ro = i * 32 + (e >> 2) * 8 + (e & 3);
-            const float g = acc[i][0][e], u = acc[i][1][e];
-            a[e] = qx_f32_to_bf16(g * (HW ? qx_fsig_hw(g) : qx_fsig(g)) * u);
-            if(gp && row + ro < rows){
-                const size_t o = (size_t)ro * ld;
-                __builtin_nontemporal_store(g, (gfloat *)gp + o);
-                __builtin_nontemporal_store(u, (gfloat *)up + o);
+        for(int t = 0; t < 4; t++){
+            const float4 g = *(const float4 *)(from_g + t * 512), u = *(const float4 *)(from_u + t * 512);
+            const int r = i * 32 + t * 8 + rl;
+            const size_t o = (size_t)r * ld + c4;
+            auto f = [](float a, float b) -> float { return a * (HW ? qx_fsig_hw(a) : qx_fsig(a)) * b; };
+            const qx_u2 h = {qx_pk_bf16(f(g.x, u.x), f(g.y, u.y)), qx_pk_bf16(f(g.z, u.z), f(g.w, u.w))};
+            if(FULL || r < left){
+                if(gp){
+                    const qx_f4 vg = {g.x, g.y, g.z, g.w}, vu = {u.x, u.y, u.z, u.w};
+                    __builtin_nontemporal_store(vg, (qx_gf4 *)(gp + o));
+                    __builtin_nontemporal_store(vu, (qx_gf4 *)(up + o));
+                }
+                *(qx_gu2 *)(act + o) = h;
             }
         }
-        /* two neighbouring columns per 4-byte store: the even lane of a pair writes the first eight of its
-         * rows for both, the odd lane the other eight */
-#pragma unroll
-        for(int e = 0; e < 8; e++){
-            const uint32_t got = (uint32_t)__shfl_xor((int)(oddl ? a[e] : a[e + 8]), 1, 64);
-            const int e2 = oddl ? e + 8 : e;
-            const int ro = i * 32 + (e2 >> 2) * 8 + (e2 & 3);
-            const uint32_t v = oddl ? (got | (a[e + 8] << 16)) : (a[e] | (got << 16));
-            if(row + ro < rows) *(guint *)(act + (size_t)ro * ld - (oddl ? 1 : 0)) = v;
-        }
     }
+}
+template<int NI, bool HW = false>
+__device__ __forceinline__ void qx_store_swiglu(const qx_f32x16 (&acc)[NI][2], float *x, float *gp, float *up, unsigned short *act, int left, size_t ld){
+    left = __builtin_amdgcn_readfirstlane(left);
+    if(left >= NI * 32) qx_swiglu_strips<NI, HW, true>(acc, x, gp, up, act, left, ld);
+    else if(left > 0)   qx_swiglu_strips<NI, HW, false>(acc, x, gp, up, act, left, ld);
 }
 
 

@@ -288,8 +288,9 @@ __device__ __forceinline__ void nh_tile(const NhArgs &a, const DevProb &P, const
         for(int j = 0; j < 2; j++) acc[i][j] = acc[i][j] * NH_UNSCALE;
     const int row = i0 + wi + hf * 4;
     if(DUAL){
-        const size_t o = (size_t)row * a.N + (j0 + (wj >> 1) + fr);
-        qx_store_swiglu<NI, true>(acc, P.C ? P.C + o : nullptr, Q.C + o, Q.act + o, row, rows, (size_t)a.N);
+        const size_t o = (size_t)(i0 + wi) * a.N + (j0 + (wj >> 1));
+        __syncthreads();                                   /* the buffers become the wavefronts' strips */
+        qx_store_swiglu<NI, true>(acc, (float *)lds + wave * QX_STRIP_FLOATS, P.C ? P.C + o : nullptr, Q.C + o, Q.act + o, rows - (i0 + wi), (size_t)a.N);
     } else if(IO == NH_SCATTER) qx_scatter_tiles<NI>(acc, (const int *)P.C, a.gate, a.out, row, rows, (size_t)a.N, j0 + wj + fr);
     else qx_store_tiles<NI, 2>(acc, P.C + (size_t)row * a.N + (j0 + wj + fr), row, i0 + wi, rows, (size_t)a.N, false);
 }

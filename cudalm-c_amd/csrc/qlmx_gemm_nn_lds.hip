@@ -297,8 +297,9 @@ __device__ __forceinline__ void nn3_tile(const Nn3Args &a, const DevProb &P, con
     /* ---- epilogue: the lane holds column lane%32 of each 32x32 tile, four-row band lane/32 ---- */
     const int row = i0 + wi + hf * 4;
     if(DUAL){
-        const size_t o = (size_t)row * a.N + (j0 + (wj >> 1) + fr);
-        qx_store_swiglu<NI>(acc, P.C + o, Q.C + o, Q.act + o, row, rows, (size_t)a.N);
+        const size_t o = (size_t)(i0 + wi) * a.N + (j0 + (wj >> 1));
+        __syncthreads();                                   /* the stages become the wavefronts' strips */
+        qx_store_swiglu<NI>(acc, (float *)lds + wave * QX_STRIP_FLOATS, P.C + o, Q.C + o, Q.act + o, rows - (i0 + wi), (size_t)a.N);
     } else
         qx_store_tiles<NI, 2>(acc, P.C + (size_t)row * a.N + (j0 + wj + fr), row, i0 + wi, rows, (size_t)a.N, P.beta != 0.0f);
 }

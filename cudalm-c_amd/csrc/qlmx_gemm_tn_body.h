@@ -312,8 +312,9 @@ __device__ __forceinline__ void tn3_tile(const Tn3Args &a, const DevProb &P, con
     const int row = i0 + wi + hf * 4;
     if(a.out) qx_scatter_tiles<NI>(acc, (const int *)P.C, a.gate, a.out, row, rows, (size_t)a.N, j0 + wj + fr);
     else if(a.gp){
-        const size_t o = (size_t)(P.C - a.gp) + (size_t)row * a.N + (j0 + wj + fr);
-        qx_store_swiglu_bwd<NI>(acc, a.gp + o, a.up + o, a.dg + o, a.du + o, row, rows, (size_t)a.N);
+        const size_t o = (size_t)(P.C - a.gp) + (size_t)(i0 + wi) * a.N + (j0 + wj);
+        __syncthreads();                                   /* the stages become the wavefronts' strips */
+        qx_store_swiglu_bwd<NI>(acc, (float *)lds + wave * QX_STRIP_FLOATS, a.gp + o, a.up + o, a.dg + o, a.du + o, rows - (i0 + wi), (size_t)a.N);
     } else qx_store_tiles<NI, 2>(acc, P.C + (size_t)row * a.N + (j0 + wj + fr), row, i0 + wi, rows, (size_t)a.N, P.beta != 0.0f);
 }
 

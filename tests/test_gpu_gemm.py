@@ -440,6 +440,47 @@ def test_mfma_f16_forward_tile_shapes(q, E, M, K, N, group):
     assert torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("rows", [[700, 1, 333, 257], [1024], [63, 640, 97]])
+def test_swiglu_epilogues_at_any_word(q, rows):
+    """The SwiGLU epilogues read and write four columns at a time: outputs and pre-activations that are aligned to a pair of elements only give the
+    bits of aligned ones, and nothing around them is touched."""
+    import torch
+    K, N, group, E = 128, 2048, 128, len(rows)
+    rng = np.random.default_rng(78)
+    off = np.concatenate([[0], np.cumsum(rows)]).astype(int)
+    R, n = int(off[-1]), E * K * N
+    digits = rng.integers(-7, 8, 2 * n).astype(np.int8)
+    dd = dev((digits[0::2] & 15 | (digits[1::2] & 15) << 4).astype(np.uint8))
+    ds = dev((rng.uniform(0.5, 1.5, 2 * n // group) * 0.0086).astype(f32))
+    x = dev(rng.standard_normal((R, K)).astype(f32)).bfloat16()
+    tok = torch.from_numpy(rng.permutation(R).astype(np.int32)).cuda()
+    z, u = dev(rng.standard_normal((R, N)).astype(f32)), dev(rng.standard_normal((R, N)).astype(f32))
+
+    def at(o, dtype, src=None):
+        t = torch.full((R * N + 16,), 3.0, device="cuda", dtype=dtype)
+        if src is not None:
+            t[o:o + R * N] = src.reshape(-1)
+        return t
+
+    def run(o):
+        gp, up, act = at(o, torch.float32), at(o, torch.float32), at(o, torch.bfloat16)
+        q.gemm_nn_gather_swiglu(dd, ds, group, q.problems([(tok.data_ptr() + off[e] * 4, None, gp.data_ptr() + (o + off[e] * N) * 4, e * K * N, e * K * N // group,
+                                                            rows[e], 0.0) for e in range(E)]),
+                                q.problems([(0, act.data_ptr() + (o + off[e] * N) * 2, up.data_ptr() + (o + off[e] * N) * 4, n + e * K * N, (n + e * K * N) // group,
+                                             rows[e], 0.0) for e in range(E)]), E, K, N, x)
+        zz, uu, dg, du = at(o, torch.float32, z), at(o, torch.float32, u), at(o, torch.bfloat16), at(o, torch.bfloat16)
+        cut = [t[o:] for t in (zz, uu, dg, du)]
+        q.gemm_tn_swiglu_bwd(dd, ds, group, q.problems([(x.data_ptr() + off[e] * K * 2, None, cut[0].data_ptr() + off[e] * N * 4, e * K * N, e * K * N // group, rows[e], 0.0)
+                                                        for e in range(E)]), E, K, N, *cut)
+        out = [gp, up, act, dg, du]
+        for t in out:
+            assert (t[:o] == 3.0).all() and (t[o + R * N:] == 3.0).all()
+        return [t[o:o + R * N] for t in out]
+
+    for a, b in zip(run(0), run(2)):
+        assert torch.equal(a, b)
+
+
 def test_mfma_f16_forward_range_edges(q, orc):
     """Where fp16 would lose bits the kernel's 2^8 range shift keeps them: weights scaled down to 1e-6 (below fp16's
     normal range unshifted) still meet the bar; activations far below fp16's normal range change nothing measurable;
