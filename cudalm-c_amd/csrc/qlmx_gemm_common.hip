@@ -248,6 +248,7 @@ static int unit_init(void){
     { int rc = table_alloc((void **)&g_unit_h, UNIT_SLOTS * UNIT_SLOT_BYTES, "unit ring"); if(rc) return rc; }
     QLMX_HIP(hipMalloc((void **)&g_chain_flags, CHAIN_FLAGS * sizeof(int)), "chain flags");
     QLMX_HIP(hipMemset(g_chain_flags, 0, CHAIN_FLAGS * sizeof(int)), "chain flags clear");
+    QLMX_HIP(hipStreamSynchronize(nullptr), "chain flags clear wait");     /* its first user may be a stream that does not wait for the null stream */
     QLMX_HIP(hipHostMalloc((void **)&g_chain_status, sizeof(unsigned), hipHostMallocDefault), "chain status (pinned)");
     *g_chain_status = 0;
     return QLMX_OK;

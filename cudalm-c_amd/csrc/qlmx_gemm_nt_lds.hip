@@ -138,6 +138,7 @@ int qlmx_gemm_nt_lds_launch(const qlmx_gemm_prob *probs, int nprob, int K, int N
     if(!g_nt3_zeros){
         QLMX_HIP(hipMalloc(&g_nt3_zeros, 256), "nt zero block");
         QLMX_HIP(hipMemset(g_nt3_zeros, 0, 256), "nt zero block clear");
+        QLMX_HIP(hipStreamSynchronize(nullptr), "nt zero block clear wait");     /* its first user may be a stream that does not wait for the null stream */
     }
     /* scheduled launch when the unit table holds it; the index-mapped one otherwise */
     {

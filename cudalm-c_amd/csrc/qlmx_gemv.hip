@@ -1142,6 +1142,7 @@ int qlmx_decode_setup(int device){
     dv.fixed = (unsigned char *)sym;
     QLMX_HIP(hipMalloc((void **)&dv.grown.ctl, DF_CTL_BYTES), "decode control words");
     QLMX_HIP(hipMemset(dv.grown.ctl, 0, DF_CTL_BYTES), "decode control words clear");
+    QLMX_HIP(hipStreamSynchronize(nullptr), "decode control words clear wait");     /* its first user may be a stream that does not wait for the null stream */
     dv.ready = true;
     return QLMX_OK;
 }
@@ -1159,6 +1160,7 @@ static int df_reserve(DfSpace &ws, int which, size_t words, hipStream_t st){
     ws.part[which] = nullptr; ws.words[which] = 0;
     QLMX_HIP(hipMalloc((void **)&ws.part[which], words * sizeof(u64)), "decode partial sums");
     QLMX_HIP(hipMemset(ws.part[which], 0, words * sizeof(u64)), "decode partial sums clear");
+    QLMX_HIP(hipStreamSynchronize(nullptr), "decode partial sums clear wait");     /* its first user may be a stream that does not wait for the null stream */
     ws.words[which] = words;
     return QLMX_OK;
 }
