@@ -1098,6 +1098,104 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
 }
 
 /* ------------------------------------------------------------------------------------------
+ * The decode layer of few pairs. What bounds it there is neither memory nor arithmetic but the chain inside a workgroup and, as
+ * every launch finds its instruction cache cold, the bytes of code on that chain. So no problem table (a problem is a pair), no
+ * task lists: a workgroup per task of either list and per chunk of the combine, its task read off its number by multiplications, those of list 2
+ * with their digits on the way from the start. The tasks themselves, their partial sums and the order in which these add up are
+ * k_decode_fused's, so the results are the same bits. Which calls come here: df_forward.
+ * ---------------------------------------------------------------------------------------- */
+struct DfFew { int per1, per2, n1, n2; unsigned rT, rtp1, rtp2, rS1, rS2, rNC2; };    /* tasks per XCD and in all; 2^31 / divisor, rounded up */
+__device__ __forceinline__ unsigned df_quot(unsigned a, unsigned r){ return __umulhi(2 * a, r); }      /* exact for a * divisor < 2^31 */
+__global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f){
+    __shared__ __align__(16) uint32_t xs_raw[4 * DF_NG * DF_MB * DF_XPLANE];
+    __shared__ float red[4 * DF_MB * DF_CW];
+    __shared__ int giveup;
+    const int tid = threadIdx.x;
+    const unsigned last = __hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    giveup = 0;                                            /* by every wavefront: nobody waits for another's */
+    auto tag = [&]() -> unsigned { return __builtin_amdgcn_readfirstlane(last == 0xFFFFFFFFu ? 1u : last + 1u); };
+    const unsigned xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int ng = a.group >= DF_CW ? 1 : DF_CW / a.group, cpg = a.group >= DF_CW ? a.group / DF_CW : 1;
+    const bool one = slot < (unsigned)f.per1, two = !one && slot < (unsigned)(f.per1 + f.per2);
+    if(one || two){
+        const unsigned q = one ? xcd * f.per1 + slot : xcd * f.per2 + (slot - f.per1);
+        const unsigned grp = df_quot(q, one ? f.rtp1 : f.rtp2), rest = q - grp * (one ? a.NC1 * a.S1 : a.NC2 * a.S2), ch = df_quot(rest, one ? f.rS1 : f.rS2);
+        DfT t;
+        t.list = one ? 1 : 2; t.prob = one ? grp >> 1 : grp; t.mat = one ? grp & 1 : 0; t.chunk = ch; t.sl = rest - ch * (one ? a.S1 : a.S2);
+        t.N = one ? a.F : a.D; t.k0 = t.sl * (one ? a.R1 : a.R2); t.rows = min(one ? a.R1 : a.R2, (one ? a.D : a.F) - t.k0); t.M = 1;
+        t.ngl = (ng == 2 && t.N - t.chunk * DF_CW > a.group) ? 2 : 1;
+        const bool there = q < (unsigned)(one ? f.n1 : f.n2);
+        const int ex = a.assign[there ? t.prob : 0];
+        if(there && (unsigned)ex < (unsigned)a.E){
+            const u64 DF = (u64)a.D * a.F;
+            t.wq = (one ? (t.mat ? a.w3q : a.w1q) : a.w2q) + (u64)ex * DF;
+            t.wg = (one ? (t.mat ? a.w3g : a.w1g) : a.w2g) + (u64)ex * a.dfg;
+            uint2 w0[DF_BATCH], w1[DF_BATCH];
+            float sc[DF_NG], xv = 0.0f;
+            const int r = (tid >> 6) * (t.rows >> 2) + min(tid & 63, (t.rows >> 2) - 1);        /* the row this thread stages */
+            const bool live = (tid & 63) < (t.rows >> 2);
+            const int gpr = t.N / a.group;
+            const float *sp = a.s + t.wg + (size_t)(t.k0 + r) * gpr + (a.group >= DF_CW ? t.chunk / cpg : t.chunk * (DF_CW / a.group));
+            const signed char *dp = df_digits<false>(a, t);
+#pragma unroll
+            for(int gg = 0; gg < DF_NG; gg++) sc[gg] = sp[gg < t.ngl ? gg : 0];
+            if(one) xv = a.x[(size_t)(t.prob - df_quot(t.prob, f.rT) * a.T) * a.D + t.k0 + r];
+            df_load<false>(w0, dp, (size_t)t.N >> 1, t.rows, 0, 0);
+            df_load<false>(w1, dp, (size_t)t.N >> 1, t.rows, 0, 1);
+            a.epoch = tag();
+            const size_t sstride = (size_t)DF_MB * a.F;
+            u64 *dst = one ? a.part1 + (((size_t)t.prob * 2 + t.mat) * a.S1 + t.sl) * sstride : a.part2 + ((size_t)t.prob * a.S2 + t.sl) * DF_MB * a.D;
+            auto prep = [&](float (&v)[DF_NG][DF_MB]){
+                if(two){
+                    xv = 0.0f;
+                    if(live){
+                        const u64 *p1 = a.part1 + (size_t)t.prob * 2 * a.S1 * sstride + t.k0 + r;
+                        const u64 *const src[2] = { p1, p1 + (size_t)a.S1 * sstride };
+                        float gu[2];
+                        if(a.S1 <= 3) df_sum_wait<2, 3>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                        else          df_sum_wait<2, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                        xv = (gu[0] / (1.0f + expf(-gu[0]))) * gu[1];
+                    }
+                }
+#pragma unroll
+                for(int gg = 0; gg < DF_NG; gg++){
+                    /* one scale group per chunk: in both halves (sc[1] is the first then) */
+                    const float s1 = (gg < ng ? t.chunk * DF_CW + gg * a.group < t.N : true) ? sc[gg] : 0.0f, x = xv * s1;
+                    v[gg][0] = live ? x : 0.0f; v[gg][1] = 0.0f;
+                }
+            };
+            df_task_i8(a, t, w0, w1, xs_raw + (tid >> 6) * (DF_NG * DF_MB * DF_XPLANE), red, dst, (size_t)t.N, prep, []{}, []{});
+        }
+    } else {
+        const unsigned q = (slot - f.per1 - f.per2) * 8 + xcd, n = df_quot(q, f.rNC2), col = (q - n * a.NC2) * DF_CW + tid;
+        a.epoch = tag();
+        if(n < (unsigned)a.T && col < (unsigned)a.D){
+            float o = a.out[(size_t)n * a.D + col];
+            /* two passes' sums per round trip; an invalid pair re-reads the other's words and adds nothing */
+            for(int k = 0; k < a.K; k += 2){
+                const int j0 = k * a.T + n, j1 = min(k + 1, a.K - 1) * a.T + n;
+                const bool v0 = (unsigned)a.assign[j0] < (unsigned)a.E, v1 = k + 1 < a.K && (unsigned)a.assign[j1] < (unsigned)a.E;
+                if(!v0 && !v1) continue;
+                const size_t pair = (size_t)a.S2 * DF_MB * a.D;
+                const u64 *const src[2] = { a.part2 + (v0 ? j0 : j1) * pair + col, a.part2 + (v1 ? j1 : j0) * pair + col };
+                float y[2];
+                df_sum_wait<2, 4>(src, (size_t)DF_MB * a.D, a.S2, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, y);
+                if(v0) o = o + a.gate[j0] * y[0];
+                if(v1) o = o + a.gate[j1] * y[1];
+            }
+            a.out[(size_t)n * a.D + col] = o;
+        }
+    }
+    if(tid == 0){
+        const unsigned done = __hip_atomic_fetch_add(a.ctl + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if(done == gridDim.x - 1){
+            __hip_atomic_store(a.ctl + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.ctl, tag(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
+/* ------------------------------------------------------------------------------------------
  * Host side. Per device: the launch shape, a status word in pinned host memory, a grow-only
  * workspace for qlmx_moe_decode_forward, and the address of the fixed device array that
  * qlmx_moe_decode_forward_noalloc uses instead. All of it is set up by qlmx_init (nothing is
@@ -1237,8 +1335,18 @@ static int df_forward(bool fixed, const char *who, const float *x, const int *as
     a.T = T; a.K = K; a.E = E; a.D = D; a.F = F;
     a.NC1 = (F + DF_CW - 1) / DF_CW; a.NC2 = (D + DF_CW - 1) / DF_CW;
     const double hits = E * (1.0 - pow(1.0 - 1.0 / E, (double)npair));
-    a.R1 = df_rows(D, 2.0 * hits * a.NC1, dv.grid); a.S1 = (D + a.R1 - 1) / a.R1;
     a.R2 = df_rows_down(F, hits * a.NC2, dv.grid);   a.S2 = (F + a.R2 - 1) / a.R2;
+    a.R1 = DF_RMAX; a.S1 = (D + a.R1 - 1) / a.R1;
+    /* k_decode_few takes a workgroup per task, all resident at once, with 256 rows to a task of list 1 whatever their number. Up to 5/8 of the
+     * workgroups that fit it is the faster one, by a microsecond to seven, beyond it the same or slower (a pair is a problem there: experts that
+     * several tokens hit are read once for each). us per layer, recorded in a graph, k_decode_fused and this: 32 experts top-2,
+     * 768 x 2048: one token 13.7, 9.8; two 13.0, 11.7; four (588 workgroups) 14.8, 14.6; five (735) 15.8, 16.2; six 17.5, 18.2. 8 experts top-2,
+     * 512 x 896, ten tokens 15.8, 12.6; 8 experts top-4, 256 x 512, sixteen tokens 20.4, 13.4; 64 experts top-4, 2048 x 1408, one token
+     * 17.4, 17.1. With 128 rows to a task the first of these is 10.6. */
+    const long long n1 = 2LL * npair * a.NC1 * a.S1, n2 = (long long)npair * a.NC2 * a.S2, n3 = (long long)T * a.NC2;
+    const long long few_grid = 8 * ((n1 + 7) / 8 + (n2 + 7) / 8 + (n3 + 7) / 8);
+    const bool few = !df_math_fp16() && few_grid <= dv.grid * 5 / 8;
+    if(!few){ a.R1 = df_rows(D, 2.0 * hits * a.NC1, dv.grid); a.S1 = (D + a.R1 - 1) / a.R1; }
     const size_t words1 = (size_t)npair * 2 * a.S1 * DF_MB * F, words2 = (size_t)npair * a.S2 * DF_MB * D;
     if(fixed){
         if((words1 + words2) * sizeof(u64) > (size_t)QLMX_DECODE_SCRATCH_BYTES){
@@ -1253,6 +1361,17 @@ static int df_forward(bool fixed, const char *who, const float *x, const int *as
         rc = df_reserve(dv.grown, 1, words2, st); if(rc) return rc;
         a.ctl = dv.grown.ctl; a.part1 = dv.grown.part[0]; a.part2 = dv.grown.part[1];
     }
+    a.status = dv.status; a.epoch = 0;
+    a.wait_xor = 0; a.spin_limit = DF_SPIN_LIMIT;
+    if(qlmx_test_take_forced_timeout(1)){ a.wait_xor = 0x40000000u; a.spin_limit = 0; }
+    if(few){
+        DfFew f; f.n1 = (int)n1; f.n2 = (int)n2; f.per1 = (int)((n1 + 7) / 8); f.per2 = (int)((n2 + 7) / 8);
+        auto rec = [](int d){ return (unsigned)(((1ULL << 31) + d - 1) / d); };
+        f.rT = rec(T); f.rtp1 = rec(a.NC1 * a.S1); f.rtp2 = rec(a.NC2 * a.S2); f.rS1 = rec(a.S1); f.rS2 = rec(a.S2); f.rNC2 = rec(a.NC2);
+        hipLaunchKernelGGL(k_decode_few, dim3((unsigned)few_grid), dim3(DF_THREADS), 0, st, a, f);
+        QLMX_LAUNCH_CHECK("decode launch");
+        return QLMX_OK;
+    }
     /* n groups left over after the last full round of 8: the number of pieces (a divisor of the chunk count) that
      * leaves the fullest XCD with the fewest chunks, the smallest such number */
     a.parts1 = 0; a.parts2 = 0;
@@ -1264,9 +1383,6 @@ static int df_forward(bool fixed, const char *who, const float *x, const int *as
         a.parts1 |= (u64)pieces(a.NC1) << (8 * n); a.parts2 |= (u64)pieces(a.NC2) << (8 * n);
     }
     a.full_at = dv.grid / 16;
-    a.status = dv.status; a.epoch = 0;
-    a.wait_xor = 0; a.spin_limit = DF_SPIN_LIMIT;
-    if(qlmx_test_take_forced_timeout(1)){ a.wait_xor = 0x40000000u; a.spin_limit = 0; }
     const long long most = (long long)2 * npair * a.NC1 * a.S1;
     const int grid = (int)std::min<long long>(dv.grid, (most + 7) & ~7LL);
     {   /* a workgroup lists its tasks once, one candidate per thread: bound them for the worst case (every pair its own expert) */

@@ -140,6 +140,31 @@ def test_decode_token_counts_cover_leftover_groups(q, orc, tol, T):
     assert orc.relerr(out.cpu().numpy(), want) < tol
 
 
+@pytest.mark.parametrize("T,E,D,F,K", [(1, 8, 128, 128, 8), (64, 5, 128, 384, 1), (8, 16, 384, 640, 8), (1, 4, 1152, 2816, 2)]
+                         + [(T, 16, 512, 2048, 2) for T in (7, 8, 9, 10, 11, 12, 13, 14, 15, 16)])
+def test_decode_few_pairs_and_many(q, orc, tol, T, E, D, F, K):
+    """Both sides of the line between the kernel of few pairs and the one with a problem table -- the smallest shapes, chunks that end in the
+    middle, the most pairs, an expert that is none, every remainder of problems modulo 8 -- by either entry point, to the same bits."""
+    import torch
+    d, s, P, n = encode_layer(orc, 90 + T, E, D, F)
+    x = orc.normal(T * D, 90 + T, 2)
+    rt = orc.normal(T * E, 90 + T, 3)
+    pr = np.zeros(T * E, f32); asn = np.zeros(K * T, np.int32); gate = np.zeros(K * T, f32)
+    orc.router_topk(rt, pr, asn, gate, T, E, K)
+    ref_gate = gate.copy(); ref_gate[K * T - 1] = 0.0
+    want = np.zeros(T * D, f32)
+    rc, ws = orc.moe_forward(x, P[:n], P[n:2 * n], P[2 * n:], asn, ref_gate, want, T, D, F, E, K)
+    orc.moe_ws_free(ws)
+    assert rc == 0
+    bad = asn.copy(); bad[K * T - 1] = E
+    outs = [torch.zeros(T * D, device="cuda") for _ in range(3)]
+    for o, f in zip(outs, (q.decode_forward, q.decode_forward, q.decode_forward_noalloc)):
+        f(dev(x), dev(bad), dev(gate), o, dev(d), dev(s), 128, 0, n, 2 * n, T, K, E, D, F)
+    torch.cuda.synchronize()
+    assert orc.relerr(outs[0].cpu().numpy(), want) < tol
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 def test_decode_all_tokens_one_expert(q, orc, tol):
     """Collision case: 16 tokens on the same two experts -> problems are cut into row pairs."""
     import torch
