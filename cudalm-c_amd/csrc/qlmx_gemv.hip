@@ -1026,6 +1026,14 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                     float gu[2 * DF_MB];
                     if(a.S1 <= 3) df_sum_wait<2 * DF_MB, 3>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
                     else if(a.S1 == 5 || a.S1 == 6) df_sum_wait<2 * DF_MB, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                    else if(a.S1 > 6 && M == 1){
+                        /* one input row: eight slices in one trip (64 experts top-4, 2048 x 1408, eleven tokens: 54.6 -> 53.6 us per layer
+                         * against two trips of four slices of the row twice) */
+                        const u64 *const row[2] = { src[0], src[1] };
+                        float y[2];
+                        df_sum_wait<2, 8>(row, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, y);
+                        gu[0] = y[0]; gu[1] = y[1];
+                    }
                     else          df_sum_wait<2 * DF_MB, 4>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
 #pragma unroll
                     for(int m = 0; m < DF_MB; m++)
@@ -1153,7 +1161,8 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f)
                         const u64 *const src[2] = { p1, p1 + (size_t)a.S1 * sstride };
                         float gu[2];
                         if(a.S1 <= 3) df_sum_wait<2, 3>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
-                        else          df_sum_wait<2, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                        else if(a.S1 <= 6) df_sum_wait<2, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                        else df_sum_wait<2, 8>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
                         xv = (gu[0] / (1.0f + expf(-gu[0]))) * gu[1];
                     }
                 }
