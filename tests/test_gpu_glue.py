@@ -206,6 +206,25 @@ def test_row_moves_larger_than_the_last_level_cache(q, bf16):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("N,D", [(1, 4), (33, 1028), (70, 768)])
+def test_combine_any_number_of_passes(q, K, N, D):
+    """The passes in their order whatever number of them is requested at a time, dropped ones and rows that are not a multiple of the workgroup's included."""
+    import torch
+    g = torch.Generator(device="cuda"); g.manual_seed(9)
+    y = torch.randn(N * K, D, device="cuda", generator=g); gate = torch.rand(N * K, device="cuda", generator=g)
+    inv = torch.randperm(N * K, device="cuda", generator=g).to(torch.int32)
+    inv[torch.rand(N * K, device="cuda", generator=g) < 0.3] = -1
+    for w in (gate, None):
+        out = torch.randn(N, D, device="cuda", generator=g); want = out.clone()
+        q.moe_combine(y, inv, w, out, N, K, D)
+        for k in range(K):
+            p = inv[k * N:(k + 1) * N].long()
+            b = y[p.clamp(min=0)]
+            want = torch.where((p >= 0)[:, None], want + (b if w is None else gate[k * N:(k + 1) * N, None] * b), want)
+        assert torch.equal(out, want)
+
+
 def test_perm_reports_bad_expert_of_any_chunk(q):
     asn = np.zeros(9000, np.int32); asn[8999] = 77
     with pytest.raises(pkg.QlmxError, match="index 77 out of range"):
