@@ -18,13 +18,22 @@
  * gradient multiplies exact digits and applies the scale to the fp32 sums of each group of k.
  *
  * Which calls come here (qlmx_small_rows): all whose problems have at most 32 rows, and those that would leave the tiled
- * kernels with few workgroups, each walking the whole contraction at 0.3 (64 rows) to 0.7 us (256) per 32 of it. Counted in
- * tiles of 64 rows: forward, 128 columns, up to 256 tiles where the contraction is not shorter than the width and up to 512
- * where it is twice as long (a wide gate | up has tiles enough for the tiled kernel), and any number where one row tile
- * holds every problem and the contraction is long (64 experts of 40 rows, 2048 x 1408: 102 -> 82 us and 48 -> 41); input
- * gradient, 64 columns, up to 512, 1024 where the contraction is twice the width. Around these lines both take about the
- * same time. The forward's rule looks at what the forms of a call that are documented to agree bit for bit have in common
- * -- with and without gather, SwiGLU, scatter -- so that they run the same arithmetic in the same order.
+ * kernels with few workgroups, each walking the whole contraction. The forward's rule looks at what the forms of a call that
+ * are documented to agree bit for bit have in common -- with and without gather, SwiGLU, scatter -- so that they run the same
+ * arithmetic in the same order. Counted in strips of 64 rows x 128 columns (a SwiGLU call has twice as many); us for the plain
+ * and the SwiGLU call, these : tiled --
+ *   up to 128, always: one round of workgroups here. 1024 x 4096, 8 experts of 40 rows 13:16 and 16:16; 1408 x 2048, 512 rows
+ *     of one expert 16:18 and 18:19; 768 x 2048, 8 of 64 11:12 and 14:15.
+ *   up to 256, where the contraction is not shorter than the width, or over 1024 with no problem of more than 64 rows: the plain
+ *     call gains what the SwiGLU call (two rounds) loses. 1536 x 512, 64 of 40 18:22 and 29:28; 1408 x 2048, 16 of 40 17:20 and 32:28.
+ *   up to 512, where the contraction is four times the width: the down projection of a wide layer, whose SwiGLU call has other
+ *     sizes. 2304 x 512, 64 of 77 39:43 (a SwiGLU call 79:59, as at twice the width: 2048 x 768, 32 of 100 30:26 and 56:38).
+ *   beyond, contractions over 1024 with few rows to a problem on average, which the tiled kernel pads to 128 each:
+ *     contraction not shorter than the width: 48, or 32 where the largest is over 64 (the others have fewer still). 2048 x 768,
+ *     64 of 40 31:33 and 57:68; 2048 x 1408, 128 of 24 (largest 144) 70:93 and 207:202, of 12 61:86 and 194:201; on the other side
+ *     128 of 36 (largest 172) 84:96 and 230:208, 64 of 64 56:63 and 121:103; 4096 x 1024, 32 of 36 (largest 170) 54:65 and 112:83.
+ *     shorter: 24, none over 64. 1408 x 2048, 64 of 18 (largest 55) 44:46 and 98:101; on the other side 32 of 36 26:24 and 63:53.
+ * Input gradient, 64 columns: up to 512, 1024 where the contraction is twice the width.
  * us per call, tiled kernels -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16
  * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
@@ -60,15 +69,18 @@ static __device__ __align__(16) unsigned char sm_zero_row[32768];       /* what 
 /* see the head of this file */
 bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, int N, int nseg, int group){
     if(group < 64) return false;
-    long long tiles = 0; int most = 0;
+    long long tiles = 0, rows = 0; int most = 0, busy = 0;
     for(int i = 0; i < nprob; i++){
         if(probs[i].M > most) most = probs[i].M;
+        rows += probs[i].M; busy += probs[i].M > 0;
         tiles += (probs[i].M + 63) / 64;
     }
     if(most <= 32) return true;
     if(mode == GEMM_NN){
         tiles *= N / SM_COLS;
-        return (most <= 64 && K > 1024) || (tiles <= 256 && K >= N) || (tiles <= 512 && K >= 2 * N);
+        if(tiles <= 256) return tiles <= 128 || K >= N || (most <= 64 && K > 1024);
+        if(tiles <= 512 && K >= 4 * N) return true;
+        return K > 1024 && rows <= busy * (K >= N ? most <= 64 ? 48LL : 32 : most <= 64 ? 24 : 0);
     }
     tiles *= N / SM_TCOLS;
     return tiles <= 512 || (tiles <= 1024 && (long long)K * nseg >= 2 * N);

@@ -368,6 +368,19 @@ def test_mfma_few_tiles(q, orc, K, N, group, rows):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("K,N,rows", [(128, 512, [256, 1792]), (128, 512, [257, 1792]),                       # 128 strips of 64 x 128, and over
+                                      (1152, 1152, [33] + [20] * 40), (1152, 1152, [65] + [40] * 40),        # 41 of 9: few rows to a problem, and more
+                                      (1152, 1280, [50] + [23] * 40), (1152, 1280, [65] + [23] * 40),
+                                      (1024, 256, [1000] * 11), (1024, 256, [1000] * 17)])                   # four times the width, up to 512 strips
+def test_f16_forward_on_both_sides_of_the_lines(q, orc, K, N, rows):
+    """The sizes of a call choose between the kernels for few rows and the tiled ones; on either side of each line the SwiGLU call
+    gives the bits of the separate ones, and both the oracle's values."""
+    (f, sep), want = _swiglu_case(q, orc, rows, K, N, pkg.ACT_BF16, pkg.MATH_MFMA_F16, seed=26)
+    assert orc.relerr(f[0], want) < 4e-4            # one rounding of the weights to 11 bits
+    for a, b in zip(f[:2], sep[:2]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 @pytest.mark.parametrize("mode,K,N", [("nn", 768, 2048), ("nn", 2048, 768), ("tn", 768, 2048), ("tn", 2048, 768),
                                       ("nt", 768, 2048), ("nt", 2048, 768)])
 def test_mfma_layer_shapes(q, orc, mode, K, N):
