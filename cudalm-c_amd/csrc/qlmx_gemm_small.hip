@@ -22,8 +22,8 @@
  * are documented to agree bit for bit have in common -- with and without gather, SwiGLU, scatter -- so that they run the same
  * arithmetic in the same order. Counted in strips of 64 rows x 128 columns (a SwiGLU call has twice as many); us for the plain
  * and the SwiGLU call, these : tiled --
- *   up to 128, always: one round of workgroups here. 1024 x 4096, 8 experts of 40 rows 13:16 and 16:16; 1408 x 2048, 512 rows
- *     of one expert 16:18 and 18:19; 768 x 2048, 8 of 64 11:12 and 14:15.
+ *   up to 128, contractions over 512: one round of workgroups here. 1024 x 4096, 8 experts of 40 rows 13:16 and 16:16; 1408 x
+ *     2048, 512 rows of one expert 16:18 and 18:19; 768 x 2048, 8 of 64 11:12 and 14:15; but 512 x 1536, 512 of one 9:9 and 10:9.
  *   up to 256, where the contraction is not shorter than the width, or over 1024 with no problem of more than 64 rows: the plain
  *     call gains what the SwiGLU call (two rounds) loses. 1536 x 512, 64 of 40 18:22 and 29:28; 1408 x 2048, 16 of 40 17:20 and 32:28.
  *   up to 512, where the contraction is four times the width: the down projection of a wide layer, whose SwiGLU call has other
@@ -78,7 +78,7 @@ bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, in
     if(most <= 32) return true;
     if(mode == GEMM_NN){
         tiles *= N / SM_COLS;
-        if(tiles <= 256) return tiles <= 128 || K >= N || (most <= 64 && K > 1024);
+        if(tiles <= 256) return (tiles <= 128 && K > 512) || K >= N || (most <= 64 && K > 1024);
         if(tiles <= 512 && K >= 4 * N) return true;
         return K > 1024 && rows <= busy * (K >= N ? most <= 64 ? 48LL : 32 : most <= 64 ? 24 : 0);
     }

@@ -368,7 +368,7 @@ def test_mfma_few_tiles(q, orc, K, N, group, rows):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-@pytest.mark.parametrize("K,N,rows", [(128, 512, [256, 1792]), (128, 512, [257, 1792]),                       # 128 strips of 64 x 128, and over
+@pytest.mark.parametrize("K,N,rows", [(576, 1024, [100, 896]), (576, 1024, [129, 896]), (512, 1024, [100, 896]),     # 128 strips of 64 x 128, and over
                                       (1152, 1152, [33] + [20] * 40), (1152, 1152, [65] + [40] * 40),        # 41 of 9: few rows to a problem, and more
                                       (1152, 1280, [50] + [23] * 40), (1152, 1280, [65] + [23] * 40),
                                       (1024, 256, [1000] * 11), (1024, 256, [1000] * 17)])                   # four times the width, up to 512 strips
