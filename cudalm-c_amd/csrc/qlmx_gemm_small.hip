@@ -2,7 +2,7 @@
  * experts with few rows: a short prompt, a small training batch.
  *
  * The tiled kernels (qlmx_gemm_nn_h.hip, qlmx_gemm_tn_body.h) give a workgroup a column strip of an expert and the
- * whole contraction, one LDS tile and one barrier per 32 of it. With a dozen rows a step is some 1000 cycles of
+ * whole contraction, one LDS tile and one barrier per 32 or 64 of it. With a dozen rows a step is some 1000 cycles of
  * LDS, barrier and issue latency around four matrix products, and a call has too few strips to hide it: 36 us for the
  * down projection of 32 experts (2048 x 768, 12 rows each), whose 25 MB of weights take 5. Here nothing meets
  * a barrier on the way in, four wavefronts split the contraction and add up at the end:
@@ -31,10 +31,10 @@
  *   beyond, contractions over 1024 with few rows to a problem on average, which the tiled kernel pads to 128 each:
  *     contraction not shorter than the width: 48, or 32 where the largest is over 64 (the others have fewer still). 2048 x 768,
  *     64 of 40 31:33 and 57:68; 2048 x 1408, 128 of 24 (largest 144) 70:93 and 207:202, of 12 61:86 and 194:201; on the other side
- *     128 of 36 (largest 172) 84:96 and 230:208, 64 of 64 56:63 and 121:103; 4096 x 1024, 32 of 36 (largest 170) 54:65 and 112:83.
+ *     128 of 36 (largest 172) 84:96 and 230:208, 64 of 64 56:63 and 121:103.
  *     shorter: 24, none over 64. 1408 x 2048, 64 of 18 (largest 55) 44:46 and 98:101; on the other side 32 of 36 26:24 and 63:53.
  * Input gradient, 64 columns: up to 512, 1024 where the contraction is twice the width.
- * us per call, tiled kernels -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
+ * us per call, tiled kernels of 256 x 128 (128 x 128) as these were written -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16
  * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
  * What bounds them now: a wavefront's chain -- the round trip in front of its loop, the steps one behind the other, the sum over

@@ -1110,7 +1110,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
  * every launch finds its instruction cache cold, the bytes of code on that chain. So no problem table (a problem is a pair), no
  * task lists: a workgroup per task of either list and per chunk of the combine, its task read off its number by multiplications, those of list 2
  * with their digits on the way from the start. The tasks themselves, their partial sums and the order in which these add up are
- * k_decode_fused's, so the results are the same bits. Which calls come here: df_forward.
+ * k_decode_fused's: the same bits where both cut a problem into the same slices. Which calls come here: df_forward.
  * ---------------------------------------------------------------------------------------- */
 struct DfFew { int per1, per2, n1, n2; unsigned rT, rtp1, rtp2, rS1, rS2, rNC2; };    /* tasks per XCD and in all; 2^31 / divisor, rounded up */
 __device__ __forceinline__ unsigned df_quot(unsigned a, unsigned r){ return __umulhi(2 * a, r); }      /* exact for a * divisor < 2^31 */
