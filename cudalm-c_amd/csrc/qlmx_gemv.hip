@@ -793,6 +793,16 @@ __device__ __forceinline__ void df_task_h(const DfArgs &a, const DfT &t, uint2 (
     DF_STAMP(14);
 }
 
+/* The call's tag from the last one's. Every wavefront loads the word for itself, and the last workgroup to finish moves it on; thread 0
+ * counts its workgroup as finished. So a wavefront has the word in a register in front of a barrier of the workgroup: a barrier
+ * alone waits for no load, which would be waited for where the value is used. (Barriers at the kernels' ends instead: one token
+ * 98.7 -> 100 us for eight layers, sixteen 231.9 -> 232.7.) */
+__device__ __forceinline__ unsigned df_tag(unsigned last){
+    const unsigned t = __builtin_amdgcn_readfirstlane(last == 0xFFFFFFFFu ? 1u : last + 1u);
+    asm volatile("" :: "s"(t) : "memory");
+    return t;
+}
+
 template<bool H>
 __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
     __shared__ DfMeta mt;
@@ -920,11 +930,10 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
         }
         if(tid == 0){ mt.ntasks = min(DF_MAXTASKS, n); mt.full = lim1 > a.full_at; }
     }
+    /* the tag's load (past the caches) has had the table and the task list to come back */
+    a.epoch = df_tag(last);
     __syncthreads();
     DF_STAMP(2);
-    /* the tag is first needed when a partial sum is stored: its load (past the caches) has had the table and the
-     * task list to come back */
-    a.epoch = __builtin_amdgcn_readfirstlane(last == 0xFFFFFFFFu ? 1u : last + 1u);
     const int ntasks = mt.ntasks;
     int ti = 0;
     auto fetch = [&]() -> DfT {
@@ -1121,7 +1130,6 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f)
     const int tid = threadIdx.x;
     const unsigned last = __hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     giveup = 0;                                            /* by every wavefront: nobody waits for another's */
-    auto tag = [&]() -> unsigned { return __builtin_amdgcn_readfirstlane(last == 0xFFFFFFFFu ? 1u : last + 1u); };
     const unsigned xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int ng = a.group >= DF_CW ? 1 : DF_CW / a.group, cpg = a.group >= DF_CW ? a.group / DF_CW : 1;
     const bool one = slot < (unsigned)f.per1, two = !one && slot < (unsigned)(f.per1 + f.per2);
@@ -1150,7 +1158,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f)
             if(one) xv = a.x[(size_t)(t.prob - df_quot(t.prob, f.rT) * a.T) * a.D + t.k0 + r];
             df_load<false>(w0, dp, (size_t)t.N >> 1, t.rows, 0, 0);
             df_load<false>(w1, dp, (size_t)t.N >> 1, t.rows, 0, 1);
-            a.epoch = tag();
+            a.epoch = df_tag(last);                       /* the barrier behind it is df_task_i8's */
             const size_t sstride = (size_t)DF_MB * a.F;
             u64 *dst = one ? a.part1 + (((size_t)t.prob * 2 + t.mat) * a.S1 + t.sl) * sstride : a.part2 + ((size_t)t.prob * a.S2 + t.sl) * DF_MB * a.D;
             auto prep = [&](float (&v)[DF_NG][DF_MB]){
@@ -1177,7 +1185,8 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f)
         }
     } else {
         const unsigned q = (slot - f.per1 - f.per2) * 8 + xcd, n = df_quot(q, f.rNC2), col = (q - n * a.NC2) * DF_CW + tid;
-        a.epoch = tag();
+        a.epoch = df_tag(last);
+        __syncthreads();
         if(n < (unsigned)a.T && col < (unsigned)a.D){
             float o = a.out[(size_t)n * a.D + col];
             /* two passes' sums per round trip; an invalid pair re-reads the other's words and adds nothing */
@@ -1199,7 +1208,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f)
         const unsigned done = __hip_atomic_fetch_add(a.ctl + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if(done == gridDim.x - 1){
             __hip_atomic_store(a.ctl + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(a.ctl, tag(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.ctl, df_tag(last), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }

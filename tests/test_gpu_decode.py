@@ -281,6 +281,54 @@ def test_decode_wait_timeout_is_reported_once(q, orc, tol):
     assert orc.relerr(out.cpu().numpy(), want) < tol
 
 
+def test_decode_on_two_streams_in_turn(q, orc):
+    """Calls of both kernels that follow each other on two streams, one event apart, over the one workspace: every call finds the tag
+    of the call before it, whichever stream that was on. Behind a workspace that has just grown, too: its new memory is
+    cleared before a stream that does not wait for the null stream uses it."""
+    import torch
+    q.call("qlmx_decode_math", 0)
+    calls = []
+    for seed, (T, E, D, F, K) in enumerate([(1, 4, 256, 512, 2), (16, 8, 768, 1024, 2), (2, 4, 512, 256, 3), (12, 8, 768, 1024, 2)]):
+        d, s, P, n = encode_layer(orc, 60 + seed, E, D, F)
+        x = orc.normal(T * D, 60 + seed, 2); rt = orc.normal(T * E, 60 + seed, 3)
+        pr = np.zeros(T * E, f32); asn = np.zeros(K * T, np.int32); gate = np.zeros(K * T, f32)
+        orc.router_topk(rt, pr, asn, gate, T, E, K)
+        want = np.zeros(T * D, f32)
+        rc, ws = orc.moe_forward(x, P[:n], P[n:2 * n], P[2 * n:], asn, gate, want, T, D, F, E, K)
+        orc.moe_ws_free(ws)
+        assert rc == 0
+        calls.append((dev(x), dev(asn), dev(gate), dev(d), dev(s), n, (T, K, E, D, F), want))
+    # 64 pairs of a wide layer: more partial sums than any other call of these tests
+    T, E, D, F, K = 64, 1, 1024, 8192, 1
+    g = torch.Generator(device="cuda").manual_seed(1)
+    big = (torch.randn(T * D, generator=g, device="cuda"), torch.zeros(T, dtype=torch.int32, device="cuda"), torch.ones(T, device="cuda"),
+           torch.randint(0, 256, (3 * D * F // 2,), generator=g, dtype=torch.uint8, device="cuda"), torch.full((3 * D * F // 128,), 0.01, device="cuda"))
+    grown = [torch.zeros(T * D, device="cuda") for _ in range(2)]
+    outs = [[torch.zeros(c[6][0] * c[6][3], device="cuda") for c in calls] for _ in range(20)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    turn = 0
+
+    def run(x, asn, gate, out, d, s, n, shape):
+        nonlocal turn
+        here, other = streams[turn & 1], streams[1 - (turn & 1)]
+        here.wait_stream(other)
+        q.decode_forward(x, asn, gate, out, d, s, 128, 0, n, 2 * n, *shape, stream=here.cuda_stream)
+        turn += 1
+
+    run(*big[:3], grown[0], *big[3:], D * F, (T, K, E, D, F))
+    for row in outs:
+        for out, (x, asn, gate, d, s, n, shape, _) in zip(row, calls):
+            run(x, asn, gate, out, d, s, n, shape)
+    run(*big[:3], grown[1], *big[3:], D * F, (T, K, E, D, F))
+    torch.cuda.synchronize()
+    q.call("qlmx_decode_status")
+    assert torch.isfinite(grown[0]).all() and torch.equal(*grown)
+    for row in outs:
+        for out, first, c in zip(row, outs[0], calls):
+            assert torch.equal(out, first) and orc.relerr(out.cpu().numpy(), c[7]) < 2e-5
+
+
 def test_decode_limits(q):
     import torch
     z = torch.zeros(65536, device="cuda")
