@@ -1126,10 +1126,10 @@ __device__ __forceinline__ unsigned df_quot(unsigned a, unsigned r){ return __um
 __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f){
     __shared__ __align__(16) uint32_t xs_raw[4 * DF_NG * DF_MB * DF_XPLANE];
     __shared__ float red[4 * DF_MB * DF_CW];
-    __shared__ int giveup;
+    __shared__ int giveup[4];
     const int tid = threadIdx.x;
     const unsigned last = __hip_atomic_load(a.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    giveup = 0;                                            /* by every wavefront: nobody waits for another's */
+    giveup[tid >> 6] = 0;                                  /* a wavefront's own: nothing orders it between wavefronts here */
     const unsigned xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int ng = a.group >= DF_CW ? 1 : DF_CW / a.group, cpg = a.group >= DF_CW ? a.group / DF_CW : 1;
     const bool one = slot < (unsigned)f.per1, two = !one && slot < (unsigned)(f.per1 + f.per2);
@@ -1168,9 +1168,9 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f)
                         const u64 *p1 = a.part1 + (size_t)t.prob * 2 * a.S1 * sstride + t.k0 + r;
                         const u64 *const src[2] = { p1, p1 + (size_t)a.S1 * sstride };
                         float gu[2];
-                        if(a.S1 <= 3) df_sum_wait<2, 3>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
-                        else if(a.S1 <= 6) df_sum_wait<2, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
-                        else df_sum_wait<2, 8>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
+                        if(a.S1 <= 3) df_sum_wait<2, 3>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup[tid >> 6], a.status, gu);
+                        else if(a.S1 <= 6) df_sum_wait<2, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup[tid >> 6], a.status, gu);
+                        else df_sum_wait<2, 8>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup[tid >> 6], a.status, gu);
                         xv = (gu[0] / (1.0f + expf(-gu[0]))) * gu[1];
                     }
                 }
@@ -1197,7 +1197,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_few(DfArgs a, DfFew f)
                 const size_t pair = (size_t)a.S2 * DF_MB * a.D;
                 const u64 *const src[2] = { a.part2 + (v0 ? j0 : j1) * pair + col, a.part2 + (v1 ? j1 : j0) * pair + col };
                 float y[2];
-                df_sum_wait<2, 4>(src, (size_t)DF_MB * a.D, a.S2, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, y);
+                df_sum_wait<2, 4>(src, (size_t)DF_MB * a.D, a.S2, a.epoch ^ a.wait_xor, a.spin_limit, &giveup[tid >> 6], a.status, y);
                 if(v0) o = o + a.gate[j0] * y[0];
                 if(v1) o = o + a.gate[j1] * y[1];
             }

@@ -48,3 +48,10 @@ def test_every_wavefront_has_the_tag_in_front_of_a_barrier(name):
     for at, end in zip(taken, taken[1:] + [close]):
         assert body[at:].startswith("df_tag(last);"), name
         assert re.match(r"df_tag\(last\);\s*__syncthreads\(\);", body[at:]) or "df_task_i8(" in body[at:end], name
+
+
+def test_nobody_clears_the_give_up_word_of_another_wavefront():
+    """k_decode_few has no barrier between the clearing and the first wait, so a wavefront's word is its own."""
+    body = closing_kernels()["k_decode_few"]
+    assert "__shared__ int giveup[4];" in body and "giveup[tid >> 6] = 0;" in body
+    assert body.count("&giveup") == body.count("&giveup[tid >> 6]") > 0
