@@ -121,8 +121,6 @@ __device__ __forceinline__ float qx_dot2(float x, uint32_t h, uint32_t m){
  * difference is an fp32 value. The factors have to come from registers: as a literal the instruction takes -1 for the wrong half. */
 struct QxMinus { uint32_t lo, hi; };
 __device__ __forceinline__ QxMinus qx_minus(){ QxMinus m = {0x0000BF80u, 0xBF800000u}; asm("" : "+s"(m.lo), "+s"(m.hi)); return m; }
-/* largest magnitude so far (fmaxf would canonicalise every operand first) */
-__device__ __forceinline__ void qx_absmax(float &m, float a, float b){ asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b)); }
 /* round to nearest even, as cudalm.cu:334-338 */
 __device__ __forceinline__ unsigned short qx_f32_to_bf16(float f){
     uint32_t x = __float_as_uint(f);

@@ -17,10 +17,13 @@
  * pace: splitting (4 instructions a value), converting digits (1.6), addresses. 1024 rows, 512 x 1536: 10-12 us a forward or input gradient, 16-18
  * a weight gradient (22-29 all six before), of which about 4 are the launch and the ends of a workgroup.
  *
- * What the parts do not hold: infinities, values near the ends of the exponent range. Whoever splits eight values looks at the
- * largest: 0 < largest < 2^-110 (lo may underflow), or beyond 2^60 (a sum of products could overflow that fp32 holds); scales
- * beyond 2^50 alike. A workgroup that has met one drops its sums and runs the plain fp32 matrix core loop (f3_plain). NaN goes
- * through the parts as it is.
+ * Small values: the last bit of lo is the value's own, 23 places below its first, and bf16 ends where fp32 ends, at 2^-133. So what is
+ * split has been multiplied by a power of two, F3_UP, that makes the parts of every fp32 value normal numbers; the sums are divided by it at the
+ * end. In nn that rides in the scale, in tn and nt it is an instruction per value.
+ * Large ones: infinities have no parts, and what has been multiplied can overflow where fp32 sums do not. Either leaves sums that are not
+ * finite: a workgroup that has one, or a NaN, drops its sums and runs the plain fp32 matrix core loop (f3_plain). Looking at the sums
+ * and not for the largest of what is split pays for most of the multiplication: six launches of 1024 rows, 512 x 1536 and back, 83.5 us
+ * when small values beside large ones kept as little as eight bits, 85 so, 88.5 with both.
  */
 #include "qlmx_gemm.h"
 #include <type_traits>
@@ -36,24 +39,19 @@ typedef const __attribute__((address_space(1))) char gchar;
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void glb_void;
 
-#define F3_LARGE 0x1p60f
-#define F3_SMALL 0x1p-110f
-#define F3_SCALE 10          /* a scale may be so many binades below F3_LARGE */
+/* Powers of two on what is split and back: the smallest fp32 value, 2^-149, has its parts at 2^-121 (2^-125 in nt, where both operands are
+ * multiplied), and a sixteenth of that (digits come as digit / 16) is still a normal number. */
+#define F3_UP(MODE)   ((MODE) == GEMM_NT ? 0x1p24f : 0x1p28f)
+#define F3_DOWN(MODE) ((MODE) == GEMM_NT ? 0x1p-48f : (MODE) == GEMM_NN ? 0x1p-24f : 0x1p-28f)     /* nn: with digit / 16 */
 
 struct F3Args { const DevProb *pr; int nprob, ntiles; const signed char *d; const float *s; int group, gshift; int K, N; };
 
-/* the largest and the smallest non-zero of what a thread has seen, as bits less one (zero is then the largest) */
-struct F3Range { uint32_t hi, lo; };
-__device__ __forceinline__ F3Range f3_range(){ const F3Range r = {0u, 0xFFFFFFFFu}; return r; }
-__device__ __forceinline__ bool f3_odd(const F3Range &r){ return r.hi > __float_as_uint(F3_LARGE) || r.lo < __float_as_uint(F3_SMALL) - 1u; }
-__device__ __forceinline__ uint32_t f3_scale_bits(float s){ return (__float_as_uint(s) & 0x7FFFFFFFu) + (F3_SCALE << 23); }
 /* eight values into their three parts */
-__device__ __forceinline__ void f3_split(const QxMinus &k, F3Range &range, const float (&f)[8], uint4 (&p)[3]){
-    uint32_t w[3][4]; float m = 0.0f;
+__device__ __forceinline__ void f3_split(const QxMinus &k, const float (&f)[8], uint4 (&p)[3]){
+    uint32_t w[3][4];
 #pragma unroll
     for(int i = 0; i < 4; i++){
         const float a = f[2 * i], b = f[2 * i + 1];
-        qx_absmax(m, a, b);
         w[0][i] = qx_pk_bf16(a, b);
         const float a1 = qx_dot2(a, w[0][i], k.lo), b1 = qx_dot2(b, w[0][i], k.hi);
         w[1][i] = qx_pk_bf16(a1, b1);
@@ -61,8 +59,6 @@ __device__ __forceinline__ void f3_split(const QxMinus &k, F3Range &range, const
     }
 #pragma unroll
     for(int q = 0; q < 3; q++) p[q] = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
-    range.hi = max(range.hi, __float_as_uint(m));
-    range.lo = min(range.lo, __float_as_uint(m) - 1u);
 }
 /* eight digits as bf16(digit / 16) */
 __device__ __forceinline__ uint4 f3_digits(uint32_t w){
@@ -103,17 +99,17 @@ __device__ __forceinline__ void f3_plain(const F3Args &a, const DevProb &P, int 
     }
 }
 
-/* whether a thread of the workgroup's NWAVE wavefronts has met an odd value; the LDS at hand may be used again afterwards */
-template<int NWAVE> __device__ __forceinline__ bool f3_any(bool odd, unsigned char *lds){
-    int *flag = (int *)lds;
-    __syncthreads();
-    const bool mine = __ballot(odd) != 0;
+/* zero if the four sums are finite, else NaN */
+__device__ __forceinline__ float f3_odd(f32x4 v){ return fmaf(v[0], 0.0f, v[1] * 0.0f) + fmaf(v[2], 0.0f, v[3] * 0.0f); }
+/* whether a thread of the workgroup's NWAVE wavefronts has an odd sum; `flag`: LDS words that nothing else is in */
+template<int NWAVE> __device__ __forceinline__ bool f3_any(float odd, int *flag){
+    const bool mine = __ballot(odd != 0.0f) != 0;         /* NaN is not equal to zero */
+    if(NWAVE == 1) return mine;
     if((threadIdx.x & 63) == 0) flag[threadIdx.x >> 6] = mine;
     __syncthreads();
     int any = 0;
 #pragma unroll
     for(int w = 0; w < NWAVE; w++) any |= flag[w];
-    __syncthreads();
     return any != 0;
 }
 
@@ -127,6 +123,7 @@ template<int I, int N, class F> __device__ __forceinline__ void f3_each(const F 
 template<int KS, bool FEW>
 __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
     constexpr int B = 64, LD = B + 4;
+    constexpr float up = F3_UP(GEMM_NT), down = F3_DOWN(GEMM_NT);
     extern __shared__ __attribute__((aligned(16))) unsigned char f3_lds[];
     const int tile = qx_xcd_tile(blockIdx.x, gridDim.x);
     if(tile >= a.ntiles) return;
@@ -135,7 +132,6 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
     const int i0 = ti * B, j0 = tj * B, M = P.M;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
     const QxMinus minus = qx_minus();
-    F3Range range = f3_range();
     /* the lane's byte offset in a step's rows, and with its columns alone */
     const uint32_t ca = (uint32_t)min(i0 + c * 4, a.K - 4) * 4u, cb = (uint32_t)min(j0 + c * 4, a.N - 4) * 4u;
     const uint32_t oa = (uint32_t)(g * 8 * a.K) * 4u + ca, ob = (uint32_t)(g * 8 * a.N) * 4u + cb;
@@ -157,15 +153,15 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
         uint4 x[4][3];
 #pragma unroll
         for(int i = 0; i < 4; i++){
-            const float f[8] = {va[0][i], va[1][i], va[2][i], va[3][i], va[4][i], va[5][i], va[6][i], va[7][i]};
-            f3_split(minus, range, f, x[i]);
+            const float f[8] = {up * va[0][i], up * va[1][i], up * va[2][i], up * va[3][i], up * va[4][i], up * va[5][i], up * va[6][i], up * va[7][i]};
+            f3_split(minus, f, x[i]);
         }
         if(next) load(va, (gchar *)P.A, a.K, oa, n + 1);
 #pragma unroll
         for(int j = 0; j < 4; j++){
-            const float f[8] = {vb[0][j], vb[1][j], vb[2][j], vb[3][j], vb[4][j], vb[5][j], vb[6][j], vb[7][j]};
+            const float f[8] = {up * vb[0][j], up * vb[1][j], up * vb[2][j], up * vb[3][j], up * vb[4][j], up * vb[5][j], up * vb[6][j], up * vb[7][j]};
             uint4 y[3];
-            f3_split(minus, range, f, y);
+            f3_split(minus, f, y);
             if(next && j == 3) load(vb, (gchar *)P.B, a.N, ob, n + 1);
             auto product = [&](int i, int p, int q, f32x4 v){
                 return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[i][p]), __builtin_bit_cast(bf16x8, y[q]), v, 0, 0, 0);
@@ -211,20 +207,27 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
         }
         multiply(std::false_type(), 0);
     }
-    if(f3_any<KS>(f3_odd(range), f3_lds)){ f3_plain<GEMM_NT, B, B, KS>(a, P, i0, j0); return; }
     /* element e of acc[i][j]: row 4 (4 g + e) + i, column 4 c + j; four columns at a time */
     auto out = [&](int r, int col, f32x4 v){
         if(i0 + r >= a.K || j0 + col >= a.N) return;
-        qx_gfloat *o = (qx_gfloat *)P.C + (size_t)(i0 + r) * a.N + j0 + col;
-#pragma unroll
-        for(int q = 0; q < 4; q++) o[q] = P.beta != 0.0f ? o[q] + v[q] : v[q];
+        v *= down;
+        qx_gf4 *o = (qx_gf4 *)((qx_gfloat *)P.C + (size_t)(i0 + r) * a.N + j0 + col);      /* at any float */
+        if(P.beta != 0.0f){ const qx_f4 old = *o; v += (f32x4){old[0], old[1], old[2], old[3]}; }
+        *o = (qx_f4){v[0], v[1], v[2], v[3]};
     };
+    float odd = 0.0f;
     if constexpr(KS == 1){
+#pragma unroll
+        for(int i = 0; i < 4; i++)
+#pragma unroll
+            for(int j = 0; j < 4; j++) odd += f3_odd(acc[i][j]);
+        if(f3_any<KS>(odd, nullptr)){ f3_plain<GEMM_NT, B, B, KS>(a, P, i0, j0); return; }
 #pragma unroll
         for(int i = 0; i < 4; i++)
 #pragma unroll
             for(int e = 0; e < 4; e++) out((g * 4 + e) * 4 + i, c * 4, (f32x4){acc[i][0][e], acc[i][1][e], acc[i][2][e], acc[i][3][e]});
     } else {
+        constexpr int U = B * B / 4 / (64 * KS);
         float *red = (float *)f3_lds;
 #pragma unroll
         for(int i = 0; i < 4; i++)
@@ -232,13 +235,20 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
             for(int e = 0; e < 4; e++)
                 *(f32x4 *)(red + (wave * B + (g * 4 + e) * 4 + i) * LD + c * 4) = (f32x4){acc[i][0][e], acc[i][1][e], acc[i][2][e], acc[i][3][e]};
         __syncthreads();
+        f32x4 v[U];
 #pragma unroll
-        for(int u = 0; u < B * B / 4 / (64 * KS); u++){
+        for(int u = 0; u < U; u++){
             const int x = u * 64 * KS + threadIdx.x, r = x / (B / 4), col = x % (B / 4) * 4;
-            f32x4 v = *(const f32x4 *)(red + r * LD + col);
+            v[u] = *(const f32x4 *)(red + r * LD + col);
 #pragma unroll
-            for(int q = 1; q < KS; q++) v += *(const f32x4 *)(red + (q * B + r) * LD + col);
-            out(r, col, v);
+            for(int q = 1; q < KS; q++) v[u] += *(const f32x4 *)(red + (q * B + r) * LD + col);
+            odd += f3_odd(v[u]);
+        }
+        if(f3_any<KS>(odd, (int *)(red + KS * B * LD))){ f3_plain<GEMM_NT, B, B, KS>(a, P, i0, j0); return; }
+#pragma unroll
+        for(int u = 0; u < U; u++){
+            const int x = u * 64 * KS + threadIdx.x;
+            out(x / (B / 4), x % (B / 4) * 4, v[u]);
         }
     }
 }
@@ -284,6 +294,7 @@ template<int I> __device__ __forceinline__ float f3_bcast(float v){
 template<int MODE>
 __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
     constexpr int BM = 32, BN = 64, LD = BM + 4, KS = F3_WAVES, ST = F3_ST, AB = F3_A_BYTES;
+    constexpr float up = F3_UP(MODE), down = F3_DOWN(MODE);
     extern __shared__ __attribute__((aligned(16))) unsigned char f3_lds[];
     const int tile = qx_xcd_tile(blockIdx.x, gridDim.x);
     if(tile >= a.ntiles) return;
@@ -292,7 +303,6 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
     const int i0 = ti * BM, j0 = tj * BN;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 31, hf = lane >> 5;
     const QxMinus minus = qx_minus();
-    F3Range range = f3_range();
     const int chunks = a.K / 64, mine = 2 * ((chunks - wave + KS - 1) / KS);        /* steps of this wavefront */
     unsigned char *base = f3_lds + wave * (ST * F3_STAGE);
     uint32_t ra[4];
@@ -337,9 +347,8 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
         /* everything is in registers before the stage is loaded again */
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(w[0]), "+v"(w[1]), "+v"(sv[0]), "+v"(sv[1]) :: "memory");
         if(n + ST < mine) load(stage, n + ST);
-        range.hi = max(range.hi, f3_scale_bits(sv[0]));
-        if(MODE == GEMM_TN) range.hi = max(range.hi, f3_scale_bits(sv[1]));
-        sv[0] *= 16.0f; sv[1] *= 16.0f;                   /* digits come as digit / 16 */
+        if(MODE == GEMM_NN) sv[0] *= up;
+        else { sv[0] *= 16.0f; sv[1] *= 16.0f; }          /* digits come as digit / 16 */
         constexpr bool first = decltype(HALF)::value == 0;
         if(MODE == GEMM_TN && first) part[0] = part[1] = (qx_f32x16)(0.0f);
         qx_f32x16 (&sum)[2] = MODE == GEMM_TN ? part : acc;
@@ -350,9 +359,9 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
             for(int j = 0; j < 2; j++) y[j] = f3_digits((uint32_t)w[j][u]);
             float f[8];
 #pragma unroll
-            for(int q = 0; q < 8; q++) f[q] = x[u * 2 + (q >> 2)][q & 3];
+            for(int q = 0; q < 8; q++) f[q] = MODE == GEMM_TN ? up * x[u * 2 + (q >> 2)][q & 3] : x[u * 2 + (q >> 2)][q & 3];
             if constexpr(MODE == GEMM_NN) f3_each<0, 8>([&](auto QC){ constexpr int q = decltype(QC)::value; f[q] *= f3_bcast<u * 8 + q>(sv[0]); });
-            f3_split(minus, range, f, xp);
+            f3_split(minus, f, xp);
 #pragma unroll
             for(int q = 2; q >= 0; q--)
 #pragma unroll
@@ -372,29 +381,39 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
         step(std::integral_constant<int, 1>(), 1, n + 1);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);                   /* vmcnt(0): no load may land in a stage any more */
-    if(f3_any<KS>(f3_odd(range), f3_lds)){ f3_plain<MODE, BM, BN, KS>(a, P, i0, j0); return; }
-    /* Sums of a wavefront as columns of 32 rows (a lane holds four consecutive rows of a column), columns 36 words apart: the 16-byte
-     * writes and reads of eight lanes hit all banks once. */
+    /* Sums of a wavefront, in its own stages, as columns of 32 rows (a lane holds four consecutive rows of a column), columns 36 words
+     * apart: the 16-byte writes and reads of eight lanes hit all banks once. */
+    constexpr int U = BM * BN / 4 / (64 * KS), STRIDE = ST * F3_STAGE / 4;
+    static_assert(BN * LD + KS <= STRIDE, "a wavefront's sums and a flag fit its stages");
     float *red = (float *)f3_lds;
 #pragma unroll
     for(int j = 0; j < 2; j++)
 #pragma unroll
         for(int q = 0; q < 4; q++)
-            *(f32x4 *)(red + (wave * BN + j * 32 + c) * LD + q * 8 + hf * 4) = (f32x4){acc[j][q * 4], acc[j][q * 4 + 1], acc[j][q * 4 + 2], acc[j][q * 4 + 3]};
+            *(f32x4 *)(red + wave * STRIDE + (j * 32 + c) * LD + q * 8 + hf * 4) = (f32x4){acc[j][q * 4], acc[j][q * 4 + 1], acc[j][q * 4 + 2], acc[j][q * 4 + 3]};
     __syncthreads();
+    f32x4 v[U];
+    float odd = 0.0f;
 #pragma unroll
-    for(int u = 0; u < BM * BN / 4 / (64 * KS); u++){
+    for(int u = 0; u < U; u++){
+        const int x = u * 64 * KS + threadIdx.x, col = x % BN, row = x / BN * 4;
+        v[u] = *(const f32x4 *)(red + col * LD + row);
+#pragma unroll
+        for(int q = 1; q < KS; q++) v[u] += *(const f32x4 *)(red + q * STRIDE + col * LD + row);
+        odd += f3_odd(v[u]);
+    }
+    if(f3_any<KS>(odd, (int *)(red + (KS - 1) * STRIDE + BN * LD))){ f3_plain<MODE, BM, BN, KS>(a, P, i0, j0); return; }
+#pragma unroll
+    for(int u = 0; u < U; u++){
         const int x = u * 64 * KS + threadIdx.x, col = x % BN, row = x / BN * 4, left = P.M - (i0 + row);
-        f32x4 v = *(const f32x4 *)(red + col * LD + row);
-#pragma unroll
-        for(int q = 1; q < KS; q++) v += *(const f32x4 *)(red + (q * BN + col) * LD + row);
         if(j0 + col >= a.N) continue;
+        v[u] *= down;
         qx_gfloat *o = (qx_gfloat *)P.C + (size_t)(i0 + row) * a.N + j0 + col;
         if(P.beta != 0.0f)
 #pragma unroll
-            for(int e = 0; e < 4; e++) if(e < left) v[e] += o[(size_t)e * a.N];
+            for(int e = 0; e < 4; e++) if(e < left) v[u][e] += o[(size_t)e * a.N];
 #pragma unroll
-        for(int e = 0; e < 4; e++) if(e < left) o[(size_t)e * a.N] = v[e];
+        for(int e = 0; e < 4; e++) if(e < left) o[(size_t)e * a.N] = v[u][e];
     }
 }
 
@@ -426,12 +445,12 @@ static long long f3_nt_tiles(const qlmx_gemm_prob *probs, int nprob, int K, int 
 int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N, hipStream_t st){
     F3Args a; a.pr = nullptr; a.nprob = a.ntiles = 0; a.d = d; a.s = s; a.gshift = 0; a.K = K; a.N = N;
     while(mode != GEMM_NT && (1 << a.gshift) < group) a.gshift++;
-    constexpr int stages = F3_WAVES * F3_ST * F3_STAGE, red = F3_WAVES * 64 * 36 * 4, lds = stages > red ? stages : red;
+    constexpr int lds = F3_WAVES * F3_ST * F3_STAGE;
     if(mode == GEMM_NN) return launch_tiles<GEMM_NN, 32, 64, 64 * F3_WAVES, lds, k_gemm_f32s<GEMM_NN>>(a, probs, nprob, st);
     if(mode == GEMM_TN) return launch_tiles<GEMM_TN, 32, 64, 64 * F3_WAVES, lds, k_gemm_f32s<GEMM_TN>>(a, probs, nprob, st);
     int most = 0;
     for(int i = 0; i < nprob; i++) if(probs[i].M > most) most = probs[i].M;
-    if(f3_nt_tiles(probs, nprob, K, N) < 3LL * qlmx_cu_count() && most >= 128) return launch_tiles<GEMM_NT, 64, 64, 256, 4 * 64 * 68 * 4, k_gemm_f32s_nt<4, false>>(a, probs, nprob, st);
+    if(f3_nt_tiles(probs, nprob, K, N) < 3LL * qlmx_cu_count() && most >= 128) return launch_tiles<GEMM_NT, 64, 64, 256, (4 * 64 * 68 + 4) * 4, k_gemm_f32s_nt<4, false>>(a, probs, nprob, st);
     return most < 32 ? launch_tiles<GEMM_NT, 64, 64, 64, 64, k_gemm_f32s_nt<1, true>>(a, probs, nprob, st)
                      : launch_tiles<GEMM_NT, 64, 64, 64, 64, k_gemm_f32s_nt<1, false>>(a, probs, nprob, st);
 }

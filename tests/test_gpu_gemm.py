@@ -288,6 +288,39 @@ def test_f32_parts_leave_what_they_do_not_hold(q, mode, where, value):
     assert np.linalg.norm((got[ok] - want[ok]) / scale) < TOL_F32 * np.linalg.norm(want[ok] / scale)
 
 
+@pytest.mark.parametrize("mode", ["nn", "tn", "nt"])
+@pytest.mark.parametrize("rows", [[40], [130]])
+@pytest.mark.parametrize("n,big", [(104, 0), (109, 0), (112, 0), (118, 0), (121, 0), (125, 0), (130, 0), (138, 0), (145, 0), (121, 60), (130, 110)])
+def test_f32_small_values_beside_large_ones(q, mode, n, big, rows):
+    """Values of some 2^-n beside others, of some 2^big, whose products vanish -- the digit is 0, the gradient is 0 -- so that the small values are the
+    result, column by column: the sums of K products to the roundings of up to K/16 + 24 additions (2^-24 of the terms' magnitudes each) and,
+    where the numbers end, half the last place (2^-150) per product and addition."""
+    K, N, group = 256, 128, 64
+    rng = np.random.default_rng(43)
+    A, X, digits, s = f32_inputs(43, mode, rows, K, N, group)
+    small = f32(2.0) ** f32(-n)
+    if mode == "nt":                                     # a token every eight is ordinary in A and 0 in X
+        lift = f32(2.0 ** 40)
+        keep = np.arange(rows[0]) % 8 == 0
+        A[~keep] *= small; A[keep] *= f32(2.0 ** big); X[keep] = 0.0; X *= lift
+        terms = np.abs(A.astype(np.float64)).T @ np.abs(X.astype(np.float64))
+        grid, depth = 0.0, rows[0]
+    else:                                                # one of the contraction every eight is ordinary in A and has digits 0
+        keep = np.arange(K) % 8 == 0
+        A[:, ~keep] *= small; A[:, keep] *= f32(2.0 ** big)
+        W = digits.reshape((K, N) if mode == "nn" else (N, K))
+        if mode == "nn": W[keep] = 0
+        else: W[:, keep] = 0
+        digits = np.ascontiguousarray(W).reshape(-1)
+        s[:] = rng.uniform(0.5, 1.5, s.shape).astype(f32)
+        w = np.repeat(s, group).astype(np.float64) * np.abs(digits)
+        terms = np.abs(A.astype(np.float64)) @ (w.reshape(K, N) if mode == "nn" else w.reshape(N, K).T)
+        grid, depth = 1.0, K
+    got, want = f32_call(q, mode, A, X if mode == "nt" else np.zeros_like(X), digits, s, group, rows, K, N)
+    bound = (depth / 16 + 24) * 2.0 ** -24 * terms.reshape(want.shape) + 8 * (1 + depth * grid) * 2.0 ** -150
+    assert (np.abs(got - want) <= bound).all(), (np.abs(got - want) / bound).max()
+
+
 @pytest.mark.parametrize("mode,K,N,math,company", [("nn", 768, 2048, "f16", [600]), ("tn", 768, 2048, "mfma", [3000]), ("nn", 768, 512, "f32", [3000]),
                                                    ("nn", 768, 512, "f32", [13000]), ("tn", 768, 512, "f32", [3000])])
 @pytest.mark.parametrize("M", [3, 16])
