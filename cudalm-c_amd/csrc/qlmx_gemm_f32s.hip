@@ -7,15 +7,21 @@
  *   nn: out[m,n] = sum_k fl(A[m,k] * s[k, group of n]) * digit[k,n]: a tile's columns lie in one scale group, so the scale is
  *       a factor of the activation; one rounding of the product as in fl(s * digit) before, then three exact products.
  *   tn: out[m,n] = sum over groups of s[n, group] * sum_{k in group} A[m,k] * digit[n,k]: three exact products.
- *   nt: out[k,n] (+)= sum_m A[m,k] * B[m,n]: six of the nine products of the parts; mid*lo, lo*mid and lo*lo are left out,
- *       together below 2^-24 of a product (2^-26.8 root mean square, against 2^-24.8 for the rounding of one addition).
+ *   nt: out[k,n] (+)= sum_m A[m,k] * B[m,n]: of the nine products of the parts six; mid*lo, lo*mid and lo*lo, together below
+ *       2^-24 of a product (2^-27.5 root mean square), are left out of sums of 32 rows, where 1 % of the error comes from that.
+ *       In the last rows of a problem, which may be one or two and all it has, only lo*lo is, below 2^-32.
  *
- * Products are added smallest parts first, so that small sums take one rounding at full size. A matrix product adds sixteen
- * terms per accumulation where the fp32 core adds two.
+ * Every matrix product rounds what it adds to, so the parts of a step (64 of the contraction, 32 rows in nt) are added up by themselves, smallest
+ * first, and the total takes one rounding a step. With the total in the matrix core it took six per 32 rows (nt) or three per 16 (nn), and long
+ * sums of few outputs, which the fp32 core spreads over sixteen wavefronts, came out further off than there. Error against 64 bits, so / with
+ * the total in the matrix core / fp32 core: nt 32 rows 3.8e-8 / 3.9e-8 / 7.9e-8, 1024 rows 512 x 512 8.6e-8 / 2.3e-7 / 2.9e-7, 4096 rows 256 x 512 1.4e-7 /
+ * 4.9e-7 / 3.0e-7, 16384 rows 256 x 256 2.6e-7 / 1.1e-6 / 5.8e-7; nn one row, 8192 x 512, 1.6e-7 / 4.4e-7 / 3.4e-7; 1024 x 1024 1.0e-7 /
+ * 1.6e-7 / 1.7e-7; tn, which always did, 1.4e-7 / 4.0e-7 (core) and 9.6e-8 / 1.8e-7.
  *
  * What bounds it: with three (six) bf16 products for an fp32 one the matrix core needs a fifth (two fifths) of the time, and vector issue sets the
- * pace: splitting (4 instructions a value), converting digits (1.6), addresses. 1024 rows, 512 x 1536: 10-12 us a forward or input gradient, 16-18
- * a weight gradient (22-29 all six before), of which about 4 are the launch and the ends of a workgroup.
+ * pace: splitting (4 instructions a value, 5 in tn and nt), converting digits (1.6), addresses; a wavefront's splitting and products hardly overlap.
+ * 1024 rows, 512 x 1536: 10-12 us a forward or input gradient, 17-20 a weight gradient (22-29 all six before; 16-18 with the total in the
+ * matrix core and no factor), of which about 4 are the launch and the ends of a workgroup.
  *
  * Small values: the last bit of lo is the value's own, 23 places below its first, and bf16 ends where fp32 ends, at 2^-133. So what is
  * split has been multiplied by a power of two, F3_UP, that makes the parts of every fp32 value normal numbers; the sums are divided by it at the
@@ -23,7 +29,7 @@
  * Large ones: infinities have no parts, and what has been multiplied can overflow where fp32 sums do not. Either leaves sums that are not
  * finite: a workgroup that has one, or a NaN, drops its sums and runs the plain fp32 matrix core loop (f3_plain). Looking at the sums
  * and not for the largest of what is split pays for most of the multiplication: six launches of 1024 rows, 512 x 1536 and back, 83.5 us
- * when small values beside large ones kept as little as eight bits, 85 so, 88.5 with both.
+ * when small values beside large ones kept as little as eight bits, 85 so, 88.5 with both (all three with the total in the matrix core).
  */
 #include "qlmx_gemm.h"
 #include <type_traits>
@@ -166,25 +172,25 @@ __global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
             auto product = [&](int i, int p, int q, f32x4 v){
                 return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[i][p]), __builtin_bit_cast(bf16x8, y[q]), v, 0, 0, 0);
             };
-            constexpr int order[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
-            if constexpr(KS > 1){
+            constexpr int order[8][2] = {{2, 1}, {1, 2}, {2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+            if constexpr(next){                           /* a whole step: one rounding of the total */
+                f32x4 t[4] = {(f32x4)(0.0f), (f32x4)(0.0f), (f32x4)(0.0f), (f32x4)(0.0f)};
 #pragma unroll
-                for(int o = 0; o < 6; o++)
+                for(int o = 2; o < 8; o++)
 #pragma unroll
-                    for(int i = 0; i < 4; i++) acc[i][j] = product(i, order[o][0], order[o][1], acc[i][j]);
+                    for(int i = 0; i < 4; i++) t[i] = product(i, order[o][0], order[o][1], t[i]);
+#pragma unroll
+                for(int i = 0; i < 4; i++) acc[i][j] += t[i];
             } else {
-                /* one wavefront has all rows, perhaps one or two: the large products and the small ones of a step apart, added to the total by
-                 * rounded additions, which keeps the error below that of fp32 products at every number of rows */
+                /* The last rows, perhaps one or two and no others: eight of the products, the large ones and the small ones apart, added to
+                 * the total by rounded additions, which is what a single product needs to be as close as fp32's. */
 #pragma unroll
                 for(int h = 0; h < 4; h += 2){
                     f32x4 small[2] = {(f32x4)(0.0f), (f32x4)(0.0f)}, large[2];
 #pragma unroll
                     for(int i = 0; i < 2; i++) large[i] = product(h + i, 0, 0, small[i]);
-                    if(FEW)                               /* no sum for what is left out to disappear in */
 #pragma unroll
-                        for(int i = 0; i < 2; i++) small[i] = product(h + i, 1, 2, product(h + i, 2, 1, small[i]));
-#pragma unroll
-                    for(int o = 0; o < 5; o++)
+                    for(int o = 0; o < 7; o++)
 #pragma unroll
                         for(int i = 0; i < 2; i++) small[i] = product(h + i, order[o][0], order[o][1], small[i]);
 #pragma unroll
@@ -350,8 +356,7 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
         if(MODE == GEMM_NN) sv[0] *= up;
         else { sv[0] *= 16.0f; sv[1] *= 16.0f; }          /* digits come as digit / 16 */
         constexpr bool first = decltype(HALF)::value == 0;
-        if(MODE == GEMM_TN && first) part[0] = part[1] = (qx_f32x16)(0.0f);
-        qx_f32x16 (&sum)[2] = MODE == GEMM_TN ? part : acc;
+        if(first) part[0] = part[1] = (qx_f32x16)(0.0f);
         f3_each<0, 2>([&](auto UC){
             constexpr int u = decltype(UC)::value;
             uint4 y[2], xp[3];
@@ -366,13 +371,13 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 2) k_gemm_f32s(F3Args a){
             for(int q = 2; q >= 0; q--)
 #pragma unroll
                 for(int j = 0; j < 2; j++)
-                    sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xp[q]), __builtin_bit_cast(bf16x8, y[j]), sum[j], 0, 0, 0);
+                    part[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xp[q]), __builtin_bit_cast(bf16x8, y[j]), part[j], 0, 0, 0);
         });
-        if(MODE == GEMM_TN && !first)
+        if(!first)
 #pragma unroll
             for(int j = 0; j < 2; j++)
 #pragma unroll
-                for(int e = 0; e < 16; e++) acc[j][e] = fmaf(sv[j], part[j][e], acc[j][e]);
+                for(int e = 0; e < 16; e++) acc[j][e] = MODE == GEMM_TN ? fmaf(sv[j], part[j][e], acc[j][e]) : acc[j][e] + part[j][e];
     };
 #pragma unroll
     for(int n = 0; n < ST; n++) if(n < mine) load(n, n);
@@ -440,8 +445,8 @@ static long long f3_nt_tiles(const qlmx_gemm_prob *probs, int nprob, int K, int 
     return n;
 }
 /* Weight gradients: four wavefronts along the rows where there are too few tiles to fill the device with one each and rows enough for all four
- * (us, one / four: 1024 rows, 1536 x 512, 192 tiles: 41 / 16; 4096, 1024 x 2048, 512: 166 / 110; 4 x 75, 640 x 1408, 880: 11 / 14; 4 x 1024,
- * 2048 x 1024, 2048: 100 / 111; eight never gained), else one, without LDS. */
+ * (us, one / four: 1024 rows, 1536 x 512, 192 tiles: 41 / 17; 4096, 1024 x 2048, 512: 166 / 106; 4 x 75, 640 x 1408, 880: 11 / 14; 4 x 1024,
+ * 2048 x 1024, 2048: 99 / 111; eight never gained), else one, without LDS. */
 int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N, hipStream_t st){
     F3Args a; a.pr = nullptr; a.nprob = a.ntiles = 0; a.d = d; a.s = s; a.gshift = 0; a.K = K; a.N = N;
     while(mode != GEMM_NT && (1 << a.gshift) < group) a.gshift++;
@@ -459,8 +464,8 @@ int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int gr
  * goes to qlmx_gemm_f32.hip, as do weight gradients of few rows and few tiles, whose rows it spreads over more wavefronts (2 to 16 rows of 256 x
  * 512: 4.5 us against 5.0). Elsewhere these are the faster ones, few-row forwards included (us, before / here: two rows of eight experts, 512 x
  * 1024, 24.8 / 5.4 with the GEMV; 1024 rows, 512 x 1536, and back, forward 28.2, 27.6 / 11.6, 10.3, input gradient 28.7, 25.3 / 11.2, 10.5,
- * weight gradient 23.7, 22.4 / 17.3, 15.7; 4096 rows, 1024 x 2048: 175, 168, 197 / 80, 74, 103). Relative error against 64 bits, before / here:
- * 3.4e-7 / 1.9e-7 (nn, K 1536), 3.4e-7 / 1.0e-7 (tn), 2.9e-7 / 2.3e-7 (nt, 1024 rows), and no larger at any size tried. */
+ * weight gradient 23.7, 22.4 / 19.8, 17.3; 4096 rows, 1024 x 2048: 175, 168, 197 / 77, 69, 106). The error against 64 bits is no larger at any size
+ * tried, one to 32768 rows and contractions of up to 16384 (head of the file). */
 bool qlmx_gemm_f32s_takes(int mode, const signed char *d, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N){
     if(mode == GEMM_NT){
         int most = 0;

@@ -321,6 +321,37 @@ def test_f32_small_values_beside_large_ones(q, mode, n, big, rows):
     assert (np.abs(got - want) <= bound).all(), (np.abs(got - want) / bound).max()
 
 
+@pytest.mark.parametrize("mode,M,K,N", [("nt", 1, 512, 256), ("nt", 2, 512, 256), ("nt", 31, 512, 256), ("nt", 32, 512, 256), ("nt", 64, 512, 260),
+                                        ("nt", 1024, 64, 128), ("nt", 1024, 512, 512), ("nt", 4096, 256, 512), ("nt", 16384, 64, 64),
+                                        ("nn", 1, 8192, 512), ("nn", 40, 8192, 128), ("nn", 64, 16384, 128), ("nn", 300, 512, 512),
+                                        ("tn", 1, 8192, 512), ("tn", 40, 8192, 64), ("tn", 64, 16384, 128)])
+def test_f32_parts_are_no_further_off_than_the_fp32_core(q, mode, M, K, N):
+    """Relative error against 64 bits of a call whose operands lie on 16 bytes (bf16 parts) and of the same call on operands a float further (fp32
+    matrix core), many additions of few outputs among them. Nothing is added to the core's error but 2 % for chance in the last bits."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rnd = lambda n: torch.randn(n + 4, generator=g, device="cuda")
+    err = []
+    a, b, group = rnd(M * K), rnd(M * N), 64
+    digits = torch.randint(-7, 8, (K * N,), generator=g, device="cuda")
+    packed = ((digits[0::2] & 15) | (digits[1::2] & 15) << 4).to(torch.uint8)
+    s = torch.rand(K * N // group, generator=g, device="cuda") * 0.0086 + 0.001
+    if mode != "nt":
+        W = (s.double().repeat_interleave(group) * digits.double()).view((K, N) if mode == "nn" else (N, K))
+    for off in (0, 1):
+        A, B = a[off:off + M * K], b[off:off + M * N]
+        C = torch.zeros(K * N if mode == "nt" else M * N, device="cuda")
+        if mode == "nt":
+            q.gemm_nt(q.problems([(A.data_ptr(), B.data_ptr(), C.data_ptr(), 0, 0, M, 0.0)]), 1, K, N, pkg.ACT_F32, pkg.MATH_F32)
+            want = A.view(M, K).double().t() @ B.view(M, N).double()
+        else:
+            (q.gemm_nn if mode == "nn" else q.gemm_tn)(packed, s, group, q.problems([(A.data_ptr(), None, C.data_ptr(), 0, 0, M, 0.0)]), 1, K, N,
+                                                       pkg.ACT_F32, pkg.MATH_F32)
+            want = A.view(M, K).double() @ (W if mode == "nn" else W.t())
+        err.append(float((C.view(want.shape).double() - want).norm() / want.norm()))
+    assert err[0] <= 1.02 * err[1], err
+
+
 @pytest.mark.parametrize("mode,K,N,math,company", [("nn", 768, 2048, "f16", [600]), ("tn", 768, 2048, "mfma", [3000]), ("nn", 768, 512, "f32", [3000]),
                                                    ("nn", 768, 512, "f32", [13000]), ("tn", 768, 512, "f32", [3000])])
 @pytest.mark.parametrize("M", [3, 16])
