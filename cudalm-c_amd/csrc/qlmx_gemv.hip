@@ -51,15 +51,17 @@ struct GvArgs {
 __device__ __forceinline__ float ub(uint32_t w, int k){ return (float)((w >> (8 * k)) & 0xFFu); }
 
 #define GV_MAXSPLIT 16
-/* sum of S <= GV_MAXSPLIT partial sums `stride` apart, added in slice order; all loads are issued
- * before the first add so the chain costs one memory latency, not S of them */
+/* sum of S partial sums `stride` apart, added in slice order; the loads of GV_MAXSPLIT of them are issued before the first add, so
+ * the chain costs one memory latency per GV_MAXSPLIT slices (more than those only where K is over GV_MAXSPLIT * GV_MAXSLICE) */
 __device__ __forceinline__ float sum_slices(const float *src, size_t stride, int S){
-    float t[GV_MAXSPLIT];
-#pragma unroll
-    for(int u = 0; u < GV_MAXSPLIT; u++) t[u] = u < S ? src[(size_t)u * stride] : 0.0f;
     float v = 0.0f;
+    for(int b = 0; b < S; b += GV_MAXSPLIT){
+        float t[GV_MAXSPLIT];
 #pragma unroll
-    for(int u = 0; u < GV_MAXSPLIT; u++) v += t[u];
+        for(int u = 0; u < GV_MAXSPLIT; u++) t[u] = b + u < S ? src[(size_t)(b + u) * stride] : 0.0f;
+#pragma unroll
+        for(int u = 0; u < GV_MAXSPLIT; u++) v += t[u];
+    }
     return v;
 }
 
@@ -208,7 +210,7 @@ static int ws_reserve(int which, size_t floats, hipStream_t st){
 }
 
 /* number of K slices: about four workgroups per CU over the expected tasks, at least two row
- * sweeps per slice, at most GV_MAXSLICE rows per slice, at most 16 slices (partial-sum traffic) */
+ * sweeps per slice, at most 16 slices (partial-sum traffic), but at most GV_MAXSLICE rows per slice, whatever their number */
 static void choose_split(int K, int N, int ntask, int *S, int *rps){
     const int ncc = N / 32, nph = GV_THREADS / ncc > 0 ? GV_THREADS / ncc : 1;
     int want = (1024 + ntask - 1) / (ntask > 0 ? ntask : 1);

@@ -91,6 +91,34 @@ def test_gemv_small_rows_vs_oracle(q, orc, K, N):
         assert orc.relerr(o.cpu().numpy(), want) < 1e-5
 
 
+def run_few_rows(q, K, N, rows, floats_off):
+    """qlmx_moe_gemm_nn in fp32 on rows that start so many floats behind 16 bytes, against 64 bits"""
+    import torch
+    E, group, rng = len(rows), 64, np.random.default_rng(K + N)
+    digits = rng.integers(-7, 8, (E, K, N))
+    s = (0.0086 * rng.uniform(0.5, 1.5, (E, K, N // group))).astype(f32)
+    A = rng.standard_normal((sum(rows), K), dtype=f32)
+    off = np.concatenate([[0], np.cumsum(rows)])
+    flat = digits.reshape(-1) & 15
+    dA, dC = dev(np.concatenate([np.zeros(floats_off, f32), A.reshape(-1)])), torch.full((sum(rows), N), 7.0, device="cuda")
+    dd, ds = dev((flat[0::2] | flat[1::2] << 4).astype(np.uint8)), dev(s)
+    items = [(dA.data_ptr() + (floats_off + int(off[e]) * K) * 4, None, dC.data_ptr() + int(off[e]) * N * 4, e * K * N, e * K * N // group, rows[e], 0.0)
+             for e in range(E)]
+    q.gemm_nn(dd, ds, group, q.problems(items), E, K, N, pkg.ACT_F32, pkg.MATH_F32)
+    got = dC.cpu().numpy()
+    for e in range(E):
+        if rows[e]:
+            want = A[off[e]:off[e + 1]].astype(np.float64) @ (digits[e] * np.repeat(s[e].astype(np.float64), group, axis=1))
+            assert np.linalg.norm(got[off[e]:off[e + 1]] - want) < np.sqrt(K / 4) * 2.0 ** -24 * np.linalg.norm(want), e
+
+
+@pytest.mark.parametrize("K,N,rows", [(768, 2048, [1, 4]), (8000, 320, [2]), (8192, 320, [3, 4]), (8192, 128, [1, 0, 2]), (8224, 64, [4]), (16384, 64, [1] * 8), (20000, 512, [1, 4])])
+def test_gemv_of_long_contractions(q, K, N, rows):
+    """The streaming path (which rows a float off 16 bytes take) at contractions of more slices than are added up in one go, against 64 bits: K
+    additions spread over at least four partial sums, each a random walk of at most sqrt(K / 4) roundings of 2^-24."""
+    run_few_rows(q, K, N, rows, 1)
+
+
 @pytest.mark.parametrize("T,E,D,F,K", [(1, 32, 768, 2048, 2), (4, 32, 768, 2048, 2), (16, 32, 768, 2048, 2), (4, 8, 768, 2048, 2), (16, 8, 768, 2048, 2),
                                        (16, 4, 256, 384, 4), (5, 3, 128, 256, 1), (7, 6, 1024, 640, 3), (3, 4, 2048, 256, 2)])
 def test_decode_forward_vs_oracle_layer(q, orc, tol, T, E, D, F, K):
