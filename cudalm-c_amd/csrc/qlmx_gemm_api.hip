@@ -6,6 +6,7 @@
 int qlmx_gemm_f32_dispatch(int mode, const signed char *d, const float *s, int group,
                            const qlmx_gemm_prob *probs, int nprob, int K, int N, int act_dtype, hipStream_t st);
 bool qlmx_gemm_f32s_takes(int mode, const signed char *d, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N);
+bool qlmx_gemv_nn_gains(const qlmx_gemm_prob *probs, int nprob, int K, int N);
 int qlmx_gemv_nn_dispatch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob,
                           int K, int N, hipStream_t st);
 int qlmx_gemm_mfma_dispatch(int mode, const signed char *d, const float *s, int group,
@@ -34,9 +35,10 @@ static int gemm_entry(const char *who, int mode, const signed char *d, const flo
         return qlmx_gemm_mfma_dispatch(mode, d, s, group, probs, second, nprob, K, N, act_dtype, (hipStream_t)stream, math == QLMX_MATH_MFMA_F16);
     QLMX_REQUIRE(!second, "%s: continued contractions need the MFMA path", who);
     if(mode == GEMM_NN && act_dtype == QLMX_ACT_F32 && N % 32 == 0 && group % 32 == 0 && ((uintptr_t)d & 15) == 0){
-        /* every problem has a few rows only: stream the weights once */
-        bool small = nprob > 0 && !qlmx_gemm_f32s_takes(mode, d, group, probs, nprob, K, N);
+        /* every problem has a few rows only: spread the contraction over workgroups, unless the kernels in parts are faster */
+        bool small = nprob > 0;
         for(int i = 0; i < nprob && small; i++) small = probs[i].M <= 4 && probs[i].wq % 32 == 0;
+        if(small) small = qlmx_gemv_nn_gains(probs, nprob, K, N) || !qlmx_gemm_f32s_takes(mode, d, group, probs, nprob, K, N);
         if(small) return qlmx_gemv_nn_dispatch(d, s, group, probs, nprob, K, N, (hipStream_t)stream);
     }
     return qlmx_gemm_f32_dispatch(mode, d, s, group, probs, nprob, K, N, act_dtype, (hipStream_t)stream);

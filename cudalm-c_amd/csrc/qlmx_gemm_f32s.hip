@@ -462,7 +462,7 @@ int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int gr
 
 /* Whether these kernels take a call: 64 columns (nn) or 64 of the contraction (tn) inside one scale group, whole units of 16 bytes. Everything else
  * goes to qlmx_gemm_f32.hip, as do weight gradients of few rows and few tiles, whose rows it spreads over more wavefronts (2 to 16 rows of 256 x
- * 512: 4.5 us against 5.0). Elsewhere these are the faster ones, few-row forwards included (us, before / here: two rows of eight experts, 512 x
+ * 512: 4.5 us against 5.0). Elsewhere these are the faster ones, few-row forwards but those of qlmx_gemv_nn_gains included (us, before / here: two rows of eight experts, 512 x
  * 1024, 24.8 / 5.4 with the GEMV; 1024 rows, 512 x 1536, and back, forward 28.2, 27.6 / 11.6, 10.3, input gradient 28.7, 25.3 / 11.2, 10.5,
  * weight gradient 23.7, 22.4 / 19.8, 17.3; 4096 rows, 1024 x 2048: 175, 168, 197 / 77, 69, 106). The error against 64 bits is no larger at any size
  * tried, one to 32768 rows and contractions of up to 16384 (head of the file). */

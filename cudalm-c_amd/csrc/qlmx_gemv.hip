@@ -223,6 +223,18 @@ static void choose_split(int K, int N, int ntask, int *S, int *rps){
     *S = s; *rps = r;
 }
 
+/* Whether this path gains over k_gemm_f32s, which has a workgroup per 64 columns and problem, each walking the whole contraction: that
+ * takes some 3 + K / 244 us, this path 14 + N / 20 and 5 for every row behind the first, as long as its workgroups, busy * S, all run at once (one
+ * to a CU; then in turns: 32 experts of 8192 x 128 37, 46, 56, 65 us for one to four rows, k_gemm_f32s 37). us, k_gemm_f32s / this path with one, two, four rows:
+ * 4096 x 128 20 / 17, 22, 32; 5504 x 128 26 / 19, 24, 34; 7168 x 256 32 / 23, 26, 33; 8192 x 128 36 / 20, 25, 35, x 320 36 / 26, 31, 40; 12288 x 512
+ * 52 / 35, 39, 47; 16384 x 640 69 / 43, 47, 57; 32768 x 1024 135 / 65, 71, 82. */
+bool qlmx_gemv_nn_gains(const qlmx_gemm_prob *probs, int nprob, int K, int N){
+    int most = 0, busy = 0, S, rps;
+    for(int i = 0; i < nprob; i++){ if(probs[i].M > most) most = probs[i].M; busy += probs[i].M > 0; }
+    choose_split(K, N, busy, &S, &rps);
+    return K >= 1500LL + 12LL * N + 1200LL * most && (long long)busy * S <= qlmx_cu_count();
+}
+
 template<int MR>
 static int launch_gemv(GvArgs &a, int ntask_max, hipStream_t st){
     hipLaunchKernelGGL((k_qlmx_gemv<MR>), dim3(a.S, ntask_max), dim3(GV_THREADS), 0, st, a);

@@ -119,6 +119,13 @@ def test_gemv_of_long_contractions(q, K, N, rows):
     run_few_rows(q, K, N, rows, 1)
 
 
+@pytest.mark.parametrize("K,N,rows", [(4224, 128, [1]), (4288, 128, [1, 0, 1]), (4288, 192, [1]), (6656, 64, [1, 3]), (5888, 64, [2, 2]), (7040, 64, [4]), (7104, 64, [4]),
+                                      (10112, 320, [3, 4]), (10176, 320, [3, 4]), (16384, 64, [1] * 8), (16384, 64, [1] * 9), (16384, 640, [1])])
+def test_few_rows_of_long_and_narrow_matrices(q, K, N, rows):
+    """Both sides of the lines between the streaming path and the kernels in parts for few rows and a long contraction; bound as above."""
+    run_few_rows(q, K, N, rows, 0)
+
+
 @pytest.mark.parametrize("T,E,D,F,K", [(1, 32, 768, 2048, 2), (4, 32, 768, 2048, 2), (16, 32, 768, 2048, 2), (4, 8, 768, 2048, 2), (16, 8, 768, 2048, 2),
                                        (16, 4, 256, 384, 4), (5, 3, 128, 256, 1), (7, 6, 1024, 640, 3), (3, 4, 2048, 256, 2)])
 def test_decode_forward_vs_oracle_layer(q, orc, tol, T, E, D, F, K):
