@@ -23,6 +23,10 @@
  * gate|up and down of those tokens, us: 228, 120 with 256 x 128 tiles on four wavefronts and steps of 32; 217, 110 with eight
  * wavefronts and 256 x 256; 199, 100 with steps of 64; 190, 97 with the operand reads spread over the first products of a slice. Loads one
  * step further ahead, wavefront priorities, buffer addressing or three LDS buffers change nothing.
+ * What the larger tile costs: with a short contraction a tile is mostly its ends, which nothing covers with one workgroup per CU, where two of 192 x 128
+ * on four wavefronts covered each other's. Against those over 2081 calls (sizes as at nh_tiles) these take 0.865 of the time in the mean, but more
+ * than a twentieth longer in 81 of the 648 plain calls no deeper than 256 (2 of 645 with SwiGLU), at worst some 130 rows to an expert: 64 experts of
+ * 130, 64 x 1408, 13.6 -> 16.6 us, 256 x 1408 20.0 -> 23.3; 128 of 130, 128 x 2048 36.2 -> 40.2; 64 of 190, 256 x 1408 22.8 -> 25.1.
  * In LDS activation rows are 128 bytes with the eight 16-byte pieces xor-swizzled by the row (conflict-free 128-bit operand
  * reads), weight rows in the matrix's own order with xor-swizzled 16-byte units, read through ds_read_b64_tr_b16.
  */
@@ -367,30 +371,34 @@ static void nh_deal(NhLoads &d, long long tiles, float cost){
 /* The tile of a launch: the shape whose tiles, dealt out as the launch deals them, end first. Costs in units of a whole 256 x 256 tile, by
  * height in 64 rows, from launches of whole rounds (256 compute units, contractions of 512 to 2048: 40, 33, 28 and 20 us for 256, 192, 128 and
  * 64 rows of 256 columns and 1024 deep, 24 and 18 for 256 and 128 rows of 128): a CU holds one such tile, or two of 128 x 128, which
- * share it (28 us for both) and overlap one's start and end with the other's loop, of use where the contraction is short. Wide tiles do the
+ * share it (28 us for both) and overlap one's start and end with the other's loop, of use where the contraction is short: up to 384 such a tile
+ * counts 0.29 instead of 0.36 (slower than the best of the five shapes by, in the mean over 3727 calls, with 0.29 / with 0.36: contractions of 256
+ * 1.0 / 1.3 %, 384 0.9 / 1.0, 512 1.0 / 0.8, 640 1.2 / 0.8, 1024 1.2 / 0.6). Wide tiles do the
  * most products per weight and activation prepared and win wherever there are rounds enough; the others where the count is unlucky. us, chosen
  * <- 256 x 256 always: 12 experts of 530 rows, 640 x 640 gate|up 21 <- 24; 8 of 256, 768 x 2048 plain 16 <- 21 (256 x 128); 100 of
- * 120, 512 x 768 plain 24 <- 28 (128 x 128). Over 250 calls of 1 to 200 experts the choice is within 1.2 % of the best of the five. */
+ * 120, 512 x 768 plain 24 <- 28 (128 x 128). Over those 3727 calls (4 to 128 experts of 70 to 400 rows, 64 to 1024 deep, 256 to 2048 wide, plain and
+ * SwiGLU) the choice is within 0.9 % of the best of the five in the mean and more than 5 % behind it in 166. */
 struct NhTiles { int rows, columns; };
 static NhTiles nh_tiles(const qlmx_gemm_prob *probs, int nprob, int K, int columns){
     static const float wide[5] = {0.0f, 0.50f, 0.65f, 0.82f, 1.0f}, narrow[5] = {0.0f, 0.45f, 0.45f, 0.67f, 0.67f}, pair[3] = {0.0f, 0.36f, 0.36f}, pair_short[3] = {0.0f, 0.29f, 0.29f};
     NhTiles best = {256, 128};
     float least = 0.0f;
+    long long full[3] = {0, 0, 0}, high[3][5] = {};                    /* tile rows, for tiles of 256, 192 and 128: whole ones, last ones by height */
+    for(int i = 0; i < nprob; i++){
+        const int m = probs[i].M, f[3] = {m / 256, m / 192, m / 128};
+        for(int r = 0; r < 3; r++){ full[r] += f[r]; high[r][(m - f[r] * (256 - 64 * r) + 63) / 64]++; }
+    }
     const int cus = qlmx_cu_count() / 8, units = cus < 1 ? 1 : cus < NH_UNITS ? cus : NH_UNITS - 1;
     for(int rows = 256; rows >= 128; rows -= 64)
         for(int cols = 256; cols >= 128; cols -= 128){
             if(cols > columns || (cols == 128 && rows == 192)) continue;
             const bool paired = rows == 128 && cols == 128;
-            const float *thin = !paired ? narrow : K > 640 ? pair : pair_short;
+            const float *thin = !paired ? narrow : K > 384 ? pair : pair_short;
             const int g_wide = cols == 256 ? columns / 256 : 0, g_thin = cols == 256 ? columns % 256 / 128 : columns / 128;
-            long long full = 0, high[5] = {0, 0, 0, 0, 0};             /* tile rows: whole ones, last ones by height */
-            for(int i = 0; i < nprob; i++){
-                const int f = probs[i].M / rows, l = (probs[i].M - f * rows + 63) / 64;
-                full += f; high[l]++;
-            }
+            const int r = (256 - rows) / 64;
             NhLoads ld; ld.n = 1; ld.load[0] = paired ? 0.11f : 0.0f; ld.units[0] = units;      /* a pair's last tile runs alone */
-            nh_deal(ld, (full * g_wide + 7) / 8, wide[rows / 64]); nh_deal(ld, (full * g_thin + 7) / 8, thin[rows / 64]);
-            for(int l = rows / 64; l > 0; l--){ nh_deal(ld, (high[l] * g_wide + 7) / 8, wide[l]); nh_deal(ld, (high[l] * g_thin + 7) / 8, thin[l]); }
+            nh_deal(ld, (full[r] * g_wide + 7) / 8, wide[rows / 64]); nh_deal(ld, (full[r] * g_thin + 7) / 8, thin[rows / 64]);
+            for(int l = rows / 64; l > 0; l--){ nh_deal(ld, (high[r][l] * g_wide + 7) / 8, wide[l]); nh_deal(ld, (high[r][l] * g_thin + 7) / 8, thin[l]); }
             float t = 0.0f;
             for(int k = 0; k < ld.n; k++) if(ld.load[k] > t) t = ld.load[k];
             if(least == 0.0f || t < least){ least = t; best.rows = rows; best.columns = cols; }
