@@ -33,6 +33,8 @@
  *     64 of 40 31:33 and 57:68; 2048 x 1408, 128 of 24 (largest 144) 70:93 and 207:202, of 12 61:86 and 194:201; on the other side
  *     128 of 36 (largest 172) 84:96 and 230:208, 64 of 64 56:63 and 121:103.
  *     shorter: 24, none over 64. 1408 x 2048, 64 of 18 (largest 55) 44:46 and 98:101; on the other side 32 of 36 26:24 and 63:53.
+ * The lines look at a call's own sizes, so a layer whose passes run one by one may take the one path and its merged list the other: bits that
+ * agree between the two are not promised and not looked for here.
  * Input gradient, 64 columns: up to 512, 1024 where the contraction is twice the width.
  * us per call, tiled kernels of 256 x 128 (128 x 128) as these were written -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16

@@ -517,6 +517,44 @@ def test_mfma_f16_forward_tile_shapes(q, E, M, K, N, group):
     assert torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("rows,K,N", [([700] * 14 + [701, 699, 0], 96, 192), ([300, 65, 129, 193, 255], 160, 320), ([130] * 40, 64, 704), ([1000, 1, 257], 96, 64),
+                                      ([530] * 12, 608, 448), ([190] * 64, 224, 192)])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_swiglu_forward_of_odd_halves(q, rows, K, N, gathered):
+    """gate | up with SwiGLU where the columns are an odd multiple of 64, so that a launch of wide tiles ends in narrow ones: pre-activations against 64
+    bits (bound as above), the activation from them, and nothing behind the last row."""
+    import torch
+    group, E, rng = 64, len(rows), np.random.default_rng(79)
+    off = np.concatenate([[0], np.cumsum(rows)]).astype(int)
+    R, n = int(off[-1]), E * K * N
+    digits = rng.integers(-7, 8, 2 * n).astype(np.int8)
+    s = (rng.uniform(0.5, 1.5, 2 * n // group) * 0.0086).astype(f32)
+    dd, ds = dev((digits[0::2] & 15 | (digits[1::2] & 15) << 4).astype(np.uint8)), dev(s)
+    x = dev(rng.standard_normal((R, K)).astype(f32)).bfloat16()
+    tok = torch.from_numpy((rng.permutation(R) if gathered else np.arange(R)).astype(np.int32)).cuda()
+    xs = x[tok.long()]
+    pre, act = [torch.full((R + 1, N), 7.0, device="cuda") for _ in range(2)], torch.full((R + 1, N), 7.0, device="cuda", dtype=torch.bfloat16)
+    rows_of = (lambda e: tok.data_ptr() + off[e] * 4) if gathered else (lambda e: x.data_ptr() + off[e] * K * 2)
+    gate = q.problems([(rows_of(e), None, pre[0].data_ptr() + off[e] * N * 4, e * K * N, e * K * N // group, rows[e], 0.0) for e in range(E)])
+    up = q.problems([(0, act.data_ptr() + off[e] * N * 2, pre[1].data_ptr() + off[e] * N * 4, n + e * K * N, (n + e * K * N) // group, rows[e], 0.0) for e in range(E)])
+    if gathered:
+        q.gemm_nn_gather_swiglu(dd, ds, group, gate, up, E, K, N, x)
+    else:
+        q.gemm_nn_swiglu(dd, ds, group, gate, up, E, K, N, pkg.ACT_BF16, pkg.MATH_MFMA_F16)
+    for m in range(2):
+        W = (np.repeat(s[m * n // group:(m + 1) * n // group], group).astype(np.float64) * digits[m * n:(m + 1) * n]).reshape(E, K, N)
+        xh = xs.float().cpu().numpy().astype(np.float64)
+        got = pre[m][:R].cpu().numpy()
+        for e in range(E):
+            want = xh[off[e]:off[e + 1]] @ W[e]
+            for c in range(0, N, 64):
+                d = np.linalg.norm(got[off[e]:off[e + 1], c:c + 64] - want[:, c:c + 64])
+                assert d <= 2.0 ** -11 / np.sqrt(3) * np.linalg.norm(want[:, c:c + 64]), (m, e, c)
+    z = pre[0][:R].double()
+    assert torch.allclose(act[:R].double(), z * torch.sigmoid(z) * pre[1][:R].double(), rtol=2.0 ** -8, atol=1e-6)
+    assert (pre[0][R] == 7.0).all() and (pre[1][R] == 7.0).all() and (act[R] == 7.0).all()
+
+
 @pytest.mark.parametrize("rows", [[700, 1, 333, 257], [1024], [63, 640, 97]])
 def test_swiglu_epilogues_at_any_word(q, rows):
     """The SwiGLU epilogues read and write four columns at a time: outputs and pre-activations that are aligned to a pair of elements only give the
