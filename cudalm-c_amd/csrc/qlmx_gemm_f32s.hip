@@ -14,14 +14,14 @@
  * Every matrix product rounds what it adds to, so the parts of a step (64 of the contraction, 32 rows in nt) are added up by themselves, smallest
  * first, and the total takes one rounding a step. With the total in the matrix core it took six per 32 rows (nt) or three per 16 (nn), and long
  * sums of few outputs, which the fp32 core spreads over sixteen wavefronts, came out further off than there. Error against 64 bits, so / with
- * the total in the matrix core / fp32 core: nt 32 rows 3.8e-8 / 3.9e-8 / 7.9e-8, 1024 rows 512 x 512 8.6e-8 / 2.3e-7 / 2.9e-7, 4096 rows 256 x 512 1.4e-7 /
- * 4.9e-7 / 3.0e-7, 16384 rows 256 x 256 2.6e-7 / 1.1e-6 / 5.8e-7; nn one row, 8192 x 512, 1.6e-7 / 4.4e-7 / 3.4e-7; 1024 x 1024 1.0e-7 /
+ * the total in the matrix core / fp32 core: nt 32 rows 3.8e-8 / 3.9e-8 / 7.9e-8, 1024 rows 512 x 512 8.6e-8 / 2.3e-7 / 2.9e-7, 4096 rows 256 x 512 1.2e-7 /
+ * 4.9e-7 / 3.0e-7, 16384 rows 256 x 256 2.2e-7 / 1.1e-6 / 5.8e-7; nn one row, 8192 x 512, 1.6e-7 / 4.4e-7 / 3.4e-7; 1024 x 1024 1.0e-7 /
  * 1.6e-7 / 1.7e-7; tn, which always did, 1.4e-7 / 4.0e-7 (core) and 9.6e-8 / 1.8e-7.
  *
  * What bounds it: with three (six) bf16 products for an fp32 one the matrix core needs a fifth (two fifths) of the time, and vector issue sets the
- * pace: splitting (4 instructions a value, 5 in tn and nt), converting digits (1.6), addresses; a wavefront's splitting and products hardly overlap.
- * 1024 rows, 512 x 1536: 10-12 us a forward or input gradient, 17-20 a weight gradient (22-29 all six before; 16-18 with the total in the
- * matrix core and no factor), of which about 4 are the launch and the ends of a workgroup.
+ * pace: splitting (4 instructions a value, 5 in tn and nt), converting digits (1.6), addresses; one wavefront's splitting and products hardly overlap.
+ * 1024 rows, 512 x 1536: 10-12 us a forward or input gradient, 16-17 a weight gradient (22-29 all six before; 20 with four wavefronts to a
+ * tile), of which about 4 are the launch and the ends of a workgroup.
  *
  * Small values: the last bit of lo is the value's own, 23 places below its first, and bf16 ends where fp32 ends, at 2^-133. So what is
  * split has been multiplied by a power of two, F3_UP, that makes the parts of every fp32 value normal numbers; the sums are divided by it at the
@@ -127,7 +127,7 @@ template<int I, int N, class F> __device__ __forceinline__ void f3_each(const F 
  * product are four apart, which only the store has to know, and a request moves four rows of 256 bytes (with four bytes per lane a step of the
  * loop waited for the issue of its requests). FEW: every problem has fewer than 32 rows. The loads of the next step go out as this step's values have been split. */
 template<int KS, bool FEW>
-__global__ void __launch_bounds__(64 * KS, 2) k_gemm_f32s_nt(F3Args a){
+__global__ void __launch_bounds__(64 * KS, KS == 8 ? 1 : 2) k_gemm_f32s_nt(F3Args a){
     constexpr int B = 64, LD = B + 4;
     constexpr float up = F3_UP(GEMM_NT), down = F3_DOWN(GEMM_NT);
     extern __shared__ __attribute__((aligned(16))) unsigned char f3_lds[];
@@ -444,9 +444,10 @@ static long long f3_nt_tiles(const qlmx_gemm_prob *probs, int nprob, int K, int 
     for(int i = 0; i < nprob; i++) if(probs[i].M > 0) n += (long long)((K + 63) / 64) * ((N + 63) / 64);
     return n;
 }
-/* Weight gradients: four wavefronts along the rows where there are too few tiles to fill the device with one each and rows enough for all four
- * (us, one / four: 1024 rows, 1536 x 512, 192 tiles: 41 / 17; 4096, 1024 x 2048, 512: 166 / 106; 4 x 75, 640 x 1408, 880: 11 / 14; 4 x 1024,
- * 2048 x 1024, 2048: 99 / 111; eight never gained), else one, without LDS. */
+/* Weight gradients: eight wavefronts along the rows where every compute unit has at most one tile, two wavefronts to a matrix core, one splitting
+ * while the other multiplies; four up to three tiles per unit; each where there are rows enough for all of them; else one, without LDS. us with one /
+ * four / eight: 192 tiles of 512 x 1536, 128 rows 9 / 6.0 / 6.1, 192 rows 12 / 7.5 / 7.2, 1024 rows 55 / 20 / 17; 256 tiles, 1024 rows 55 / 20 / 18; 320 tiles
+ * 55 / 28 / 29; 512 tiles, 4096 rows 213 / 111 / 111; 4 x 75 rows, 640 x 1408, 880 tiles 11 / 14; 4 x 1024, 2048 x 1024, 2048 tiles 99 / 111. */
 int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N, hipStream_t st){
     F3Args a; a.pr = nullptr; a.nprob = a.ntiles = 0; a.d = d; a.s = s; a.gshift = 0; a.K = K; a.N = N;
     while(mode != GEMM_NT && (1 << a.gshift) < group) a.gshift++;
@@ -455,7 +456,9 @@ int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int gr
     if(mode == GEMM_TN) return launch_tiles<GEMM_TN, 32, 64, 64 * F3_WAVES, lds, k_gemm_f32s<GEMM_TN>>(a, probs, nprob, st);
     int most = 0;
     for(int i = 0; i < nprob; i++) if(probs[i].M > most) most = probs[i].M;
-    if(f3_nt_tiles(probs, nprob, K, N) < 3LL * qlmx_cu_count() && most >= 128) return launch_tiles<GEMM_NT, 64, 64, 256, (4 * 64 * 68 + 4) * 4, k_gemm_f32s_nt<4, false>>(a, probs, nprob, st);
+    const long long tiles = f3_nt_tiles(probs, nprob, K, N);
+    if(tiles <= qlmx_cu_count() && most >= 192) return launch_tiles<GEMM_NT, 64, 64, 512, (8 * 64 * 68 + 8) * 4, k_gemm_f32s_nt<8, false>>(a, probs, nprob, st);
+    if(tiles < 3LL * qlmx_cu_count() && most >= 128) return launch_tiles<GEMM_NT, 64, 64, 256, (4 * 64 * 68 + 4) * 4, k_gemm_f32s_nt<4, false>>(a, probs, nprob, st);
     return most < 32 ? launch_tiles<GEMM_NT, 64, 64, 64, 64, k_gemm_f32s_nt<1, true>>(a, probs, nprob, st)
                      : launch_tiles<GEMM_NT, 64, 64, 64, 64, k_gemm_f32s_nt<1, false>>(a, probs, nprob, st);
 }
@@ -464,7 +467,7 @@ int qlmx_gemm_f32s_launch(int mode, const signed char *d, const float *s, int gr
  * goes to qlmx_gemm_f32.hip, as do weight gradients of few rows and few tiles, whose rows it spreads over more wavefronts (2 to 16 rows of 256 x
  * 512: 4.5 us against 5.0). Elsewhere these are the faster ones, few-row forwards but those of qlmx_gemv_nn_gains included (us, before / here: two rows of eight experts, 512 x
  * 1024, 24.8 / 5.4 with the GEMV; 1024 rows, 512 x 1536, and back, forward 28.2, 27.6 / 11.6, 10.3, input gradient 28.7, 25.3 / 11.2, 10.5,
- * weight gradient 23.7, 22.4 / 19.8, 17.3; 4096 rows, 1024 x 2048: 175, 168, 197 / 77, 69, 106). The error against 64 bits is no larger at any size
+ * weight gradient 23.7, 22.4 / 17.0, 15.8; 4096 rows, 1024 x 2048: 175, 168, 197 / 77, 69, 106). The error against 64 bits is no larger at any size
  * tried, one to 32768 rows and contractions of up to 16384 (head of the file). */
 bool qlmx_gemm_f32s_takes(int mode, const signed char *d, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N){
     if(mode == GEMM_NT){

@@ -250,7 +250,8 @@ def f32_inputs(seed, mode, rows, K, N, group):
 @pytest.mark.parametrize("mode,K,N,group,rows", [
     ("nn", 64, 64, 64, [1, 33]), ("nn", 320, 192, 64, [31, 2, 65]), ("nn", 768, 256, 128, [4]), ("nn", 1536, 256, 256, [100]),
     ("tn", 64, 64, 64, [1, 33]), ("tn", 320, 45, 64, [31, 0, 65]), ("tn", 1536, 72, 128, [4]), ("tn", 512, 66, 256, [100]),
-    ("nt", 1024, 1028, 0, [1]), ("nt", 1156, 1028, 0, [2, 31, 33]), ("nt", 68, 132, 0, [127, 40]), ("nt", 64, 64, 0, [128]), ("nt", 132, 260, 0, [300, 0, 97])])
+    ("nt", 1024, 1028, 0, [1]), ("nt", 1156, 1028, 0, [2, 31, 33]), ("nt", 68, 132, 0, [127, 40]), ("nt", 64, 64, 0, [128]), ("nt", 132, 260, 0, [300, 0, 97]),
+    ("nt", 1028, 964, 0, [192, 1]), ("nt", 64, 132, 0, [191, 63]), ("nt", 68, 64, 0, [193, 224, 256, 289]), ("nt", 4, 4, 0, [1000])])
 def test_f32_in_three_parts(q, mode, K, N, group, rows):
     """The fp32 products as products of bf16 parts, at the edges of their tiles and steps. Against 64 bits: one rounding of the weight or
     of activation times scale, and at most three (nt: six) roundings per sixteen of the contraction, each half a unit (2^-24) of a running sum
