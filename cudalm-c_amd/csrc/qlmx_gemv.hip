@@ -1050,7 +1050,7 @@ __global__ void __launch_bounds__(DF_THREADS, 4) k_decode_fused(DfArgs a){
                     if(a.S1 <= 3) df_sum_wait<2 * DF_MB, 3>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
                     else if(a.S1 == 5 || a.S1 == 6) df_sum_wait<2 * DF_MB, 6>(src, sstride, a.S1, a.epoch ^ a.wait_xor, a.spin_limit, &giveup, a.status, gu);
                     else if(a.S1 > 6 && M == 1){
-                        /* one input row: eight slices in one trip (64 experts top-4, 2048 x 1408, eleven tokens: 54.6 -> 53.6 us per layer
+                        /* one input row: eight slices in one trip (64 experts top-4, 2048 x 1408, eleven tokens: 52.7 -> 51.1 us per layer
                          * against two trips of four slices of the row twice) */
                         const u64 *const row[2] = { src[0], src[1] };
                         float y[2];
@@ -1295,11 +1295,12 @@ static int df_reserve(DfSpace &ws, int which, size_t words, hipStream_t st){
     return QLMX_OK;
 }
 
-/* Rows per task of list 1: 256 keeps the per-task fixed cost (staging, reduction, hand-over) small against
- * the streaming part; the slices are halved only while they leave fewer than 0.15 x the grid with a gate|up task
- * (a single token: 128 rows, 192 tasks). More, shorter slices cost the down tasks a second round trip for their
- * sums: measured at E=32 D=768 F=2048 top-2, rows 256 / 128 / 64 give 16.3 / 15.6 / 18.2 us per layer for one
- * token, 18.8 / 21.4 / 26.4 for four, 29.7 / 32.7 / 42.0 for sixteen. The number of problems is only known on the
+/* Rows per task of list 1 in k_decode_fused: 256 keeps the per-task fixed cost (staging, reduction, hand-over) small
+ * against the streaming part; the slices are halved only while they leave fewer than 0.15 x the grid with a gate|up
+ * task. With the default loop such calls are k_decode_few's, which keeps 256; here come those of the fp16 loop (a single token:
+ * 128 rows, 192 tasks) and many tokens on few experts. More, shorter slices cost the down tasks a second round trip for
+ * their sums: measured at E=32 D=768 F=2048 top-2, when one token took this kernel, rows 256 / 128 / 64 gave 16.3 / 15.6 / 18.2 us per layer for
+ * it, 18.8 / 21.4 / 26.4 for four, 29.7 / 32.7 / 42.0 for sixteen. The number of problems is only known on the
  * device; the host uses the expected number of distinct experts hit by `npair` uniform picks out of E. */
 static int df_rows(int Kdim, double tasks_per_slice, int grid){
     int R = DF_RMAX;

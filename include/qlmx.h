@@ -177,12 +177,19 @@ int qlmx_servo(signed char *d, signed char *r, float *s,
  * Which kernel a call runs -- tiles of 256 rows or of 64 and fewer, the contraction in one piece or shared by several
  * wavefronts or workgroups and added up -- depends on the row counts of all its problems, on K, N and the group. Calls of the
  * same sizes give the same bits, and so do the forms below that are said to. A problem's rows beside other problems than
- * before (a sequence served in another batch) may differ in the last bits: by the order of K fp32 additions, about 1e-6 of
- * the result and never by the precision of a product. A caller that needs bits that do not depend on the batch keeps the sizes.
+ * before (a sequence served in another batch) may differ in the last bits: by the order of K fp32 additions and by roundings of
+ * their size, about 1e-6 of the result, never by operands or weights of fewer bits. A caller that needs bits that do not depend on
+ * the batch keeps the sizes.
  * ===================================================================================== */
 #define QLMX_ACT_F32   0     /* activation operands are fp32                         */
 #define QLMX_ACT_BF16  1     /* activation operands are bf16 (high half of an fp32)  */
-#define QLMX_MATH_F32  0     /* fp32 products and sums (fp32 matrix core)            */
+#define QLMX_MATH_F32  0     /* fp32 operands, products and sums. fp32 activations in the aligned sizes of everyday use run on the bf16
+                              * matrix core as exact sums of three bf16 parts each, the rest on the fp32 matrix core or, with a few
+                              * rows, a streaming path. Operands keep all their bits over fp32's whole range, infinities and NaN
+                              * included. nn and tn multiply exactly, up to one rounding of a factor by its scale; nt (the weight
+                              * gradient) drops what is below 2^-24 of a product, in the last rows of a problem below 2^-32.
+                              * Relative L2 error against 64 bits: 1e-7 to 2e-7 (nn, tn, up to 16384 of the contraction), 3e-8 to
+                              * 3e-7 (nt, one to 32768 rows), no larger than fp32 multiply-adds' */
 #define QLMX_MATH_MFMA 1     /* bf16 MFMA, fp32 accumulate                           */
 #define QLMX_MATH_MFMA_F16 2 /* as QLMX_MATH_MFMA, except that qlmx_moe_gemm_nn on bf16 activations runs on the fp16
                               * matrix core: the activations are converted exactly (|x| in [2^-14, 65504]; smaller ones
@@ -285,8 +292,9 @@ int qlmx_moe_gemm_nt(const qlmx_gemm_prob *probs_host, int nprob, int K, int N,
  *
  * The reference's decoder runs the training forward on N = batch rows (dec_step, cudalm.cu:7163-7204
  * -> moe_forward 7193), so each expert GEMM has 0..few rows and the work is reading the experts'
- * packed weights once. qlmx_moe_gemm_nn with QLMX_MATH_F32 already takes a streaming GEMV path when
- * every problem has at most 4 rows (the counterpart of the reference's R<=4 path, cpu_rt.h:233-258).
+ * packed weights once. qlmx_moe_gemm_nn with QLMX_MATH_F32 has a streaming GEMV path for calls whose problems
+ * all have at most 4 rows (the counterpart of the reference's R<=4 path, cpu_rt.h:233-258); it takes those that
+ * the matrix-core kernels do not, or are slower at: long and narrow matrices.
  * qlmx_moe_decode_forward fuses the whole expert part of moe_forward for such batches: it groups
  * the (pass, token) pairs by expert on the device (no host round trip, unlike cudalm.cu:3576-3602),
  * streams w1|w3 with the SwiGLU applied on the fly, streams w2, and adds gate*y into `out` in pass
