@@ -112,9 +112,10 @@ def run_few_rows(q, K, N, rows, floats_off):
             assert np.linalg.norm(got[off[e]:off[e + 1]] - want) < np.sqrt(K / 4) * 2.0 ** -24 * np.linalg.norm(want), e
 
 
-@pytest.mark.parametrize("K,N,rows", [(768, 2048, [1, 4]), (8000, 320, [2]), (8192, 320, [3, 4]), (8192, 128, [1, 0, 2]), (8224, 64, [4]), (16384, 64, [1] * 8), (20000, 512, [1, 4])])
+@pytest.mark.parametrize("K,N,rows", [(768, 2048, [1, 4]), (8000, 320, [2]), (8192, 320, [3, 4]), (8192, 128, [1, 0, 2]), (8224, 64, [4]), (16384, 64, [1] * 8), (20000, 512, [1, 4]),
+                                      (96, 8256, [2]), (130, 16384, [4, 1]), (8704, 8256, [1])])
 def test_gemv_of_long_contractions(q, K, N, rows):
-    """The streaming path (which rows a float off 16 bytes take) at contractions of more slices than are added up in one go, against 64 bits: K
+    """The streaming path (which rows a float off 16 bytes take) at contractions of more slices than are added up in one go, and rows wider than a workgroup, against 64 bits: K
     additions spread over at least four partial sums, each a random walk of at most sqrt(K / 4) roundings of 2^-24."""
     run_few_rows(q, K, N, rows, 1)
 
