@@ -39,9 +39,21 @@
  * us per call, tiled kernels of 256 x 128 (128 x 128) as these were written -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16
  * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
+ * Shapes of the forward of at most 32 rows per problem, groups of 128 or 256 (sm_few_shape). What takes the time there is the CU's address unit
+ * as much as vector issue: an instruction that loads a word per lane from four rows of weights takes it as long as one that loads two.
+ *   wide: 256 columns to a strip, a lane's words of a row of weights in one load (RT * 64 registers of sums). Four wavefronts to a workgroup, two workgroups to a CU, from 176
+ *     strips on (wide : narrow, us, 8 / 20 rows, 1408 x N: 64 experts of 512 14.9:11.3 / 17.9:13.4, of 768 14.6:16.7 / 18.1:18.3, 40 of 1408 15.2:17.4 / 18.6:19.4,
+ *     28 of 2048 15.3:20.5 / 18.7:22.8, 64 of 2816 34.9:45.7 / 42.3:52.2). Gate|up is eight wavefronts and one workgroup to a CU, so that its strips come in rounds of 256:
+ *     up to 16 rows from 176 strips on, but not between 257 and 351 (768 x N: 64 of 512 17:13.1, 64 of 768 16.6:20.4, 40 of 1408 17.4:20.9, 28 of 2048 17.4:24.6, 40 of 2048 31.4:30.4, 48 of
+ *     2048 32.4:35.7, 64 of 2816 48:59.6); above 16 rows only for one round with rows of weights a multiple of 1 KB apart, where narrow strips meet in the same memory
+ *     channels (28 of 2048 23.4:24.6, a mixture around twelve rows 22.4:26.9; but 40 of 1408 23.7:21.9, 64 of 2048 45.5:44.6).
+ *   eight wavefronts along the contraction, where few strips walk a long one: K from 2048, up to 224 strips of 128, above 16 rows K from 2 N (8 : 4 wavefronts, 2048 x 768, 8 rows of 16 experts
+ *     11.6:13.3, of 32 11.7:13.9, 20 rows of 32 14.6:16.7; gate|up the same with up to 16 rows, 20 rows of 8, 2048 x 1408, 25.5:22.6). One step of a wavefront
+ *     is on its way in both: two are slower (18.3 -> 19.6 for gate|up of 32, 768 x 2048).
  * What bounds them now: a wavefront's chain -- the round trip in front of its loop, the steps one behind the other, the sum over
- * the wavefronts behind it. Vector issue is at 36-38 % in the forward (231 to 261 vector instructions for 32 x 128 weights,
- * everything included) and 15-29 % in the input gradient, the address units at 24-51 %, the matrix cores at 4-14 %.
+ * the wavefronts behind it: 7 us of a gate|up call of 18, whose 50 MB stream at 4 TB/s beside it. Without the conversions it took 10. Other ways to them: scales on the
+ * activations, as two bf16 parts, and digits as denormal bf16 took half the vector instructions and no less time, the address unit being as busy; and they round otherwise than
+ * the tiled kernel. Vector issue is at 15-29 % in the input gradient, the address units at 24-51 %, the matrix cores at 4-14 %.
  */
 #include "qlmx_gemm.h"
 #include <type_traits>
@@ -57,7 +69,7 @@ typedef int    i32x4 __attribute__((ext_vector_type(4)));
 
 #define SM_COLS 128                             /* of a forward strip */
 #define SM_TCOLS 64                             /* of an input-gradient strip */
-#define SM_WAVES 4                              /* along the contraction (eight: the same for 2048, 20 % slower for 768) */
+#define SM_WAVES 4                              /* along the contraction (the forward of few rows: eight where sm_few_shape says so) */
 #define SM_WSCALE 4096.0f                       /* 16 (digits come as digit/16) * 2^8, as NH_WSCALE */
 #define SM_UNSCALE (1.0f / 256.0f)
 
@@ -103,26 +115,40 @@ template<int I> __device__ __forceinline__ float sm_bcast_hi(float low, float v)
 }
 template<int I, int N, class F> __device__ __forceinline__ void sm_each(const F &f){ if constexpr(I < N){ f(std::integral_constant<int, I>()); sm_each<I + 1, N>(f); } }
 
-/* The sums of the four wavefronts from `first` on, of one 16-row tile, through LDS: acc holds a lane's sums of rows
- * (lane/16)*4 + e, columns (lane%16)*8 + j. */
-__device__ __forceinline__ void sm_put(float *red, int first, const f32x4 (&acc)[8]){
+/* The sums of four wavefronts from `first` on, of one 16-row tile, through LDS: acc holds a lane's sums of rows
+ * (lane/16)*4 + e, columns (lane%16)*CL + j. */
+template<int CL> __device__ __forceinline__ void sm_put(float *red, int first, const f32x4 (&acc)[CL]){
     const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) - first, c = lane & 15, g = lane >> 4;
     __syncthreads();                                      /* the tile before has been read */
-    if(wave >= 0 && wave < SM_WAVES){
-        float *w = red + wave * (16 * SM_COLS);
+    if(wave >= 0 && wave < 4){
+        float *w = red + wave * (16 * 16 * CL);
 #pragma unroll
-        for(int e = 0; e < 4; e++){
-            *(f32x4 *)&w[(g * 4 + e) * SM_COLS + c * 8]     = (f32x4){acc[0][e], acc[1][e], acc[2][e], acc[3][e]};
-            *(f32x4 *)&w[(g * 4 + e) * SM_COLS + c * 8 + 4] = (f32x4){acc[4][e], acc[5][e], acc[6][e], acc[7][e]};
-        }
+        for(int e = 0; e < 4; e++)
+#pragma unroll
+            for(int j = 0; j < CL; j += 4)
+                *(f32x4 *)&w[(g * 4 + e) * (16 * CL) + c * CL + j] = (f32x4){acc[j][e], acc[j + 1][e], acc[j + 2][e], acc[j + 3][e]};
     }
     __syncthreads();
 }
-/* four columns of a row */
-__device__ __forceinline__ f32x4 sm_get(const float *red, int row, int col){
-    f32x4 v = *(const f32x4 *)&red[row * SM_COLS + col];
+/* what wavefront w + 4 has put, added to wavefront w's own, w from `first` on */
+template<int CL> __device__ __forceinline__ void sm_add(const float *red, int first, f32x4 (&acc)[CL]){
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) - first, c = lane & 15, g = lane >> 4;
+    if(wave < 0 || wave >= 4) return;
+    const float *w = red + wave * (16 * 16 * CL);
 #pragma unroll
-    for(int k = 1; k < SM_WAVES; k++) v += *(const f32x4 *)&red[k * (16 * SM_COLS) + row * SM_COLS + col];
+    for(int e = 0; e < 4; e++)
+#pragma unroll
+        for(int j = 0; j < CL; j += 4){
+            const f32x4 v = *(const f32x4 *)&w[(g * 4 + e) * (16 * CL) + c * CL + j];
+#pragma unroll
+            for(int q = 0; q < 4; q++) acc[j + q][e] += v[q];
+        }
+}
+/* four columns of a row */
+template<int CL> __device__ __forceinline__ f32x4 sm_get(const float *red, int row, int col){
+    f32x4 v = *(const f32x4 *)&red[row * (16 * CL) + col];
+#pragma unroll
+    for(int k = 1; k < 4; k++) v += *(const f32x4 *)&red[k * (16 * 16 * CL) + row * (16 * CL) + col];
     return v * SM_UNSCALE;
 }
 
@@ -132,39 +158,45 @@ __device__ __forceinline__ f32x4 sm_get(const float *red, int row, int col){
  * 20.6 against 26.3 us); by lane a workgroup is half as large and twice as many fit where 64 rows need 216 registers (8
  * experts of 250 rows, 512 x 1536: 24.5 against 30.2). TWO: the halves of the strip have scales of their own. ---- */
 enum { SM_ONE = 0, SM_BY_WAVE = 1, SM_BY_LANE = 2 };
-template<int RT, int IO, int DUAL, bool TWO>
+template<int RT, int IO, int DUAL, bool TWO, int CL, int KW>
 __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, const DevProb &Q, int i0, int j0, float *red){
-    constexpr int PF = RT == 1 ? (DUAL == SM_BY_WAVE ? 3 : 4) : RT == 2 ? (DUAL == SM_BY_WAVE ? 1 : 2) : 1;        /* steps on their way */
+    constexpr int COLS = 16 * CL, PF = CL == 16 || KW == 8 ? 1 : RT == 1 ? (DUAL == SM_BY_WAVE ? 3 : 4) : RT == 2 ? (DUAL == SM_BY_WAVE ? 1 : 2) : 1;        /* steps on their way */
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
-    const int steps = a.K / 32, ks = wave & (SM_WAVES - 1), st0 = steps * ks / SM_WAVES, st1 = steps * (ks + 1) / SM_WAVES;
-    const char *pa[RT];
-#pragma unroll
-    for(int r = 0; r < RT; r++){
-        const int row = min(i0 + r * 16 + c, P.M - 1);
-        if(IO == SM_GATHER){
-            const int tok = ((const int *)P.A)[row];
-            pa[r] = tok >= 0 ? a.xsrc + (size_t)tok * a.K * 2 : (const char *)sm_zero_row;
-        } else pa[r] = (const char *)P.A + (size_t)row * a.K * 2;
-        pa[r] += g * 16;
-    }
+    const int steps = a.K / 32, ks = wave & (KW - 1), st0 = steps * ks / KW, st1 = steps * (ks + 1) / KW;
     const size_t gpr = (size_t)a.N >> a.gshift, rowb = (size_t)a.N >> 1;       /* scale groups and bytes per row of weights */
-    const bool second = DUAL == SM_BY_WAVE ? wave >= SM_WAVES : DUAL == SM_BY_LANE && c >= 8;
-    const signed char *pw = a.d + (((second ? Q.wq : P.wq) + (size_t)(g * 8) * a.N + j0 + (DUAL == SM_BY_LANE ? c & 7 : c) * 8) >> 1);
-    const float *ps = a.s + (second ? Q.wg : P.wg) + (size_t)(g * 8 + (c & 7)) * gpr + (j0 >> a.gshift) + (TWO && DUAL != SM_BY_LANE ? c >> 3 : 0);
-    f32x4 acc[RT][8];
+    const bool second = DUAL == SM_BY_WAVE ? wave >= KW : DUAL == SM_BY_LANE && c >= 8;
+    /* where the strip's weights and scales start, the same in all lanes (by lane: in those of a half), and the lane's way from there */
+    const signed char *pw = a.d + (((second ? Q.wq : P.wq) + j0) >> 1);
+    const float *ps = a.s + (second ? Q.wg : P.wg) + (j0 >> a.gshift);
+    const int cw = DUAL == SM_BY_LANE || (CL == 16 && j0 + 128 >= a.N) ? c & 7 : c;      /* past the last column: the strip's first half once more, not stored */
+    const uint32_t vw = (uint32_t)((g * 8) * rowb) + cw * (CL / 2);
+    const uint32_t vs = (uint32_t)((g * 8 + (c & 7)) * gpr) + (CL == 16 ? ((j0 + (cw & 8) * 16) >> a.gshift) - (j0 >> a.gshift) : TWO && DUAL != SM_BY_LANE ? c >> 3 : 0);
+    const char *pa[RT];
+    f32x4 acc[RT][CL];
 #pragma unroll
     for(int r = 0; r < RT; r++)
 #pragma unroll
-        for(int j = 0; j < 8; j++) acc[r][j] = (f32x4)(0.0f);
-    uint32_t w[PF][8]; float s[PF]; i32x4 x[PF][RT];
-    auto load = [&](int set, int st){
+        for(int j = 0; j < CL; j++) acc[r][j] = (f32x4)(0.0f);
+    typedef uint32_t Word __attribute__((ext_vector_type(CL / 8)));
+    Word w[PF][8]; float s[PF]; i32x4 x[PF][RT];
+    auto load_w = [&](int set, int st){
         const int t = min(st, st1 - 1);                   /* past the end: the last step again, never used */
-        s[set] = ps[(size_t)t * 32 * gpr];
+        const float *sc = ps + (size_t)t * 32 * gpr;
+        const signed char *row = pw + (size_t)t * 32 * rowb;
+        s[set] = sc[vs];
 #pragma unroll
-        for(int i = 0; i < 8; i++) w[set][i] = *(const uint32_t *)(pw + ((size_t)t * 32 + i) * rowb);
+        for(int i = 0; i < 8; i++){
+            if(DUAL != SM_BY_LANE) asm("" : "+s"(row));   /* stays in scalar registers: seen through, every load adds 64 bits per lane */
+            w[set][i] = *(const Word *)(row + vw);
+            row += rowb;
+        }
+    };
+    auto load_x = [&](int set, int st){
+        const int t = min(st, st1 - 1);
 #pragma unroll
         for(int r = 0; r < RT; r++) x[set][r] = *(const i32x4 *)(pa[r] + (size_t)t * 64);
     };
+    auto load = [&](int set, int st){ load_w(set, st); load_x(set, st); };
     auto step = [&](auto IC, int st){
         constexpr int I = decltype(IC)::value;
         f16x8 xa[RT];
@@ -176,20 +208,21 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
             xa[r] = __builtin_bit_cast(f16x8, v);
         }
         const float sv = s[I] * SM_WSCALE;
-        float sk[8]; QxNibs nb[8];
+        float sk[8]; QxNibs nb[8][CL / 8];
         sm_each<0, 8>([&](auto KC){
             constexpr int k = decltype(KC)::value;
             sk[k] = sm_bcast<k>(sv);
             if(TWO) sk[k] = sm_bcast_hi<k>(sk[k], sv);
-            nb[k] = qx_nibs(w[I][k]);
+#pragma unroll
+            for(int h = 0; h < CL / 8; h++) nb[k][h] = qx_nibs(w[I][k][h]);
         });
         load(I, st + PF);
         /* two operands at a time: left alone, the compiler builds all eight first and runs out of registers */
 #pragma unroll
-        for(int j = 0; j < 8; j++){
+        for(int j = 0; j < CL; j++){
             i32x4 b;
 #pragma unroll
-            for(int q = 0; q < 4; q++) b[q] = sm_pk_f16(sk[2 * q] * qx_nib16(nb[2 * q], j), sk[2 * q + 1] * qx_nib16(nb[2 * q + 1], j));
+            for(int q = 0; q < 4; q++) b[q] = sm_pk_f16(sk[2 * q] * qx_nib16(nb[2 * q][j / 8], j & 7), sk[2 * q + 1] * qx_nib16(nb[2 * q + 1][j / 8], j & 7));
 #pragma unroll
             for(int r = 0; r < RT; r++)
                 acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[r], __builtin_bit_cast(f16x8, b), acc[r][j], 0, 0, 0);
@@ -197,14 +230,25 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
         }
     };
     if(st0 < st1){
-        sm_each<0, PF>([&](auto IC){ load(decltype(IC)::value, st0 + decltype(IC)::value); });
+        sm_each<0, PF>([&](auto IC){ load_w(decltype(IC)::value, st0 + decltype(IC)::value); });
+        /* a gather's row indices are a round trip of their own: behind the first weights */
+#pragma unroll
+        for(int r = 0; r < RT; r++){
+            const int row = min(i0 + r * 16 + c, P.M - 1);
+            if(IO == SM_GATHER){
+                const int tok = ((const int *)P.A)[row];
+                pa[r] = tok >= 0 ? a.xsrc + (size_t)tok * a.K * 2 : (const char *)sm_zero_row;
+            } else pa[r] = (const char *)P.A + (size_t)row * a.K * 2;
+            pa[r] += g * 16;
+        }
+        sm_each<0, PF>([&](auto IC){ load_x(decltype(IC)::value, st0 + decltype(IC)::value); });
         int st = st0;
         for(; st + PF <= st1; st += PF) sm_each<0, PF>([&](auto IC){ step(IC, st + decltype(IC)::value); });
         sm_each<0, PF - 1>([&](auto IC){ if(st + decltype(IC)::value < st1) step(IC, st + decltype(IC)::value); });
     }
     /* ---- totals ---- */
     auto swiglu = [&](int lr, int col, const f32x4 &y, const f32x4 &u){
-        if(lr >= P.M) return;
+        if(lr >= P.M || (CL == 16 && j0 + col >= a.N)) return;
         const size_t o = (size_t)lr * a.N + j0 + col;
         if(P.C){ *(f32x4 *)(P.C + o) = y; *(f32x4 *)(Q.C + o) = u; }
         ushort4 h;
@@ -212,24 +256,34 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
         h.z = qx_f32_to_bf16(y[2] * qx_fsig_hw(y[2]) * u[2]); h.w = qx_f32_to_bf16(y[3] * qx_fsig_hw(y[3]) * u[3]);
         *(ushort4 *)((unsigned short *)Q.B + o) = h;
     };
+    constexpr int THREADS = 64 * KW * (DUAL == SM_BY_WAVE ? 2 : 1), PER_ROW = COLS / 4, V = (16 * PER_ROW + THREADS - 1) / THREADS;
+    auto together = [&](int first, f32x4 (&v)[CL]){       /* the sums of the wavefronts from `first` on, for sm_get */
+        if(KW == 8){ sm_put<CL>(red, first + 4, v); sm_add<CL>(red, first, v); }
+        sm_put<CL>(red, first, v);
+    };
 #pragma unroll
     for(int r = 0; r < RT; r++){
         const int i = i0 + r * 16;
-        sm_put(red, 0, acc[r]);
+        together(0, acc[r]);
         if constexpr(DUAL == SM_BY_LANE){
             const int row = tid >> 4, col = (tid & 15) * 4;
-            swiglu(i + row, col, sm_get(red, row, col), sm_get(red, row, 64 + col));
+            swiglu(i + row, col, sm_get<CL>(red, row, col), sm_get<CL>(red, row, 64 + col));
         } else if constexpr(DUAL == SM_BY_WAVE){
-            const int row = tid >> 5, col = (tid & 31) * 4;
-            const f32x4 y = sm_get(red, row, col);
-            sm_put(red, SM_WAVES, acc[r]);
-            swiglu(i + row, col, y, sm_get(red, row, col));
+            f32x4 y[V];
+#pragma unroll
+            for(int v = 0; v < V; v++){ const int at = (v * THREADS + tid) % (16 * PER_ROW); y[v] = sm_get<CL>(red, at / PER_ROW, at % PER_ROW * 4); }
+            together(KW, acc[r]);
+#pragma unroll
+            for(int v = 0; v < V; v++){
+                const int at = v * THREADS + tid, row = at / PER_ROW, col = at % PER_ROW * 4;
+                if(at < 16 * PER_ROW) swiglu(i + row, col, y[v], sm_get<CL>(red, row, col));
+            }
         } else {
 #pragma unroll
-            for(int v = 0; v < 2; v++){
-                const int row = v * 8 + (tid >> 5), col = (tid & 31) * 4, lr = i + row;
-                const f32x4 y = sm_get(red, row, col);
-                if(lr >= P.M) continue;
+            for(int v = 0; v < V; v++){
+                const int at = v * THREADS + tid, row = at / PER_ROW, col = at % PER_ROW * 4, lr = i + row;
+                const f32x4 y = sm_get<CL>(red, row, col);
+                if(lr >= P.M || (CL == 16 && j0 + col >= a.N)) continue;
                 if constexpr(IO == SM_SCATTER){
                     const int tok = ((const int *)P.C)[lr];
                     if(tok >= 0){
@@ -244,24 +298,24 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
     }
 }
 
-template<int RT, int IO, int DUAL>
-__global__ void __launch_bounds__(64 * SM_WAVES * (DUAL == SM_BY_WAVE ? 2 : 1), RT == 1 || DUAL == SM_BY_WAVE ? 4 : 2) k_gemm_nn_small(SmArgs a){
-    __shared__ __attribute__((aligned(16))) float red[SM_WAVES * 16 * SM_COLS];
+template<int RT, int IO, int DUAL, int CL, int KW>
+__global__ void __launch_bounds__(64 * KW * (DUAL == SM_BY_WAVE ? 2 : 1), CL == 16 ? 2 : RT == 1 || DUAL == SM_BY_WAVE ? 4 : 2) k_gemm_nn_small(SmArgs a){
+    __shared__ __attribute__((aligned(16))) float red[4 * 16 * 16 * CL];
     const int t = qx_xcd_tile(blockIdx.x, gridDim.x);
     if(t >= a.ntiles) return;
     const int pi = qx_find_problem(a.pr, a.nprob, t);
     const DevProb P = a.pr[pi], Q = a.pr[DUAL ? pi + 1 : pi];
     const int lt = t - P.tile0, ti = lt / P.tiles_n, tj = lt - ti * P.tiles_n;
-    const int i0 = ti * (RT * 16), j0 = tj * (DUAL == SM_BY_LANE ? SM_COLS / 2 : SM_COLS), left = P.M - i0;
-    if(DUAL == SM_BY_LANE || a.gshift == 6){
-        if(RT == 4 && left > 32)      sm_nn_tile<RT, IO, DUAL, true>(a, P, Q, i0, j0, red);
-        else if(RT >= 2 && left > 16) sm_nn_tile<RT >= 2 ? 2 : 1, IO, DUAL, true>(a, P, Q, i0, j0, red);
-        else                          sm_nn_tile<1, IO, DUAL, true>(a, P, Q, i0, j0, red);
-    } else {
-        if(RT == 4 && left > 32)      sm_nn_tile<RT, IO, DUAL, DUAL == SM_BY_LANE>(a, P, Q, i0, j0, red);
-        else if(RT >= 2 && left > 16) sm_nn_tile<RT >= 2 ? 2 : 1, IO, DUAL, DUAL == SM_BY_LANE>(a, P, Q, i0, j0, red);
-        else                          sm_nn_tile<1, IO, DUAL, DUAL == SM_BY_LANE>(a, P, Q, i0, j0, red);
-    }
+    const int i0 = ti * (RT * 16), j0 = tj * (DUAL == SM_BY_LANE ? 8 * CL : 16 * CL), left = P.M - i0;
+    auto tile = [&](auto TW){
+        constexpr bool TWO = decltype(TW)::value;
+        if(RT == 4 && left > 32)      sm_nn_tile<RT, IO, DUAL, TWO, CL, KW>(a, P, Q, i0, j0, red);
+        else if(RT >= 2 && left > 16) sm_nn_tile<RT >= 2 ? 2 : 1, IO, DUAL, TWO, CL, KW>(a, P, Q, i0, j0, red);
+        else                          sm_nn_tile<1, IO, DUAL, TWO, CL, KW>(a, P, Q, i0, j0, red);
+    };
+    if constexpr(DUAL == SM_BY_LANE || CL == 16) tile(std::true_type());
+    else if(a.gshift == 6) tile(std::true_type());
+    else tile(std::false_type());
 }
 
 /* ---- input gradient: 64 columns per workgroup; nseg operand pairs (a continued problem's second pair comes from the
@@ -441,6 +495,18 @@ static int sm_row_tiles(const qlmx_gemm_prob *probs, int nprob){
     for(int i = 0; i < nprob; i++) if(probs[i].M > most) most = probs[i].M;
     return most > 32 ? 4 : most > 16 ? 2 : 1;
 }
+/* Shape of the forward of at most 32 rows per problem. Eight wavefronts along the contraction change the order of the sums, so that line looks at what the
+ * forms of a call have in common; the width of a strip does not, and looks at the form too. See the head of this file. */
+enum { SM_NARROW = 0, SM_WIDE = 1, SM_EIGHT = 2 };
+static int sm_few_shape(const qlmx_gemm_prob *probs, int nprob, int K, int N, int group, bool dual, int rt){
+    if(group < 128) return SM_NARROW;                     /* a wide strip has room for two scales in a row of weights */
+    long long narrow = 0, wide = 0;
+    for(int i = 0; i < nprob; i++) if(probs[i].M > 0){ narrow += N / SM_COLS; wide += (N + 2 * SM_COLS - 1) / (2 * SM_COLS); }
+    if(narrow <= 224 && K >= 2048 && (rt == 1 || K >= 2 * N)) return SM_EIGHT;
+    if(!dual) return wide >= 176 ? SM_WIDE : SM_NARROW;
+    if(rt == 2) return wide >= 160 && wide <= 256 && N % 2048 == 0 ? SM_WIDE : SM_NARROW;
+    return wide >= 176 && (wide <= 256 || wide >= 352) ? SM_WIDE : SM_NARROW;
+}
 static SmArgs sm_args(const signed char *d, const float *s, int group, int K, int N, const ProbUpload &up){
     SmArgs a = {};
     a.pr = up.dev; a.nprob = up.nprob; a.ntiles = up.ntiles; a.d = d; a.s = s; a.K = K; a.N = N;
@@ -454,14 +520,17 @@ int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, c
                               int io, const void *xsrc, float *out, const float *gate, hipStream_t st){
     const int rt = sm_row_tiles(probs, nprob);
     ProbUpload up; int slot;
-    int rc = qlmx_upload_problems(probs, nprob, GEMM_NN, K, N, rt * 16, SM_COLS, st, &up, &slot); if(rc) return rc;
+    const int shape = rt <= 2 ? sm_few_shape(probs, nprob, K, N, group, false, rt) : SM_NARROW;
+    int rc = qlmx_upload_problems(probs, nprob, GEMM_NN, K, N, rt * 16, shape == SM_WIDE ? 2 * SM_COLS : SM_COLS, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
     a.xsrc = (const char *)xsrc; a.out = out; a.gate = gate;
-#define SM_NN(IO) do{ if(rt == 1) SM_LAUNCH((k_gemm_nn_small<1, IO, SM_ONE>), SM_WAVES, 0); else if(rt == 2) SM_LAUNCH((k_gemm_nn_small<2, IO, SM_ONE>), SM_WAVES, 0); \
-                      else SM_LAUNCH((k_gemm_nn_small<4, IO, SM_ONE>), SM_WAVES, 0); }while(0)
+#define SM_FEW(RT, IO) do{ if(shape == SM_WIDE) SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_ONE, 16, 4>), 4, 0); \
+                           else if(shape == SM_EIGHT) SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_ONE, 8, 8>), 8, 0); else SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_ONE, 8, 4>), 4, 0); }while(0)
+#define SM_NN(IO) do{ if(rt == 1) SM_FEW(1, IO); else if(rt == 2) SM_FEW(2, IO); else SM_LAUNCH((k_gemm_nn_small<4, IO, SM_ONE, 8, 4>), 4, 0); }while(0)
     if(io == SM_GATHER) SM_NN(SM_GATHER); else if(io == SM_SCATTER) SM_NN(SM_SCATTER); else SM_NN(SM_PLAIN);
 #undef SM_NN
+#undef SM_FEW
     QLMX_LAUNCH_CHECK("grouped gemm nn (few rows) launch");
     return qlmx_upload_done(slot, st);
 }
@@ -470,14 +539,17 @@ int qlmx_gemm_nn_small_swiglu_launch(const signed char *d, const float *s, int g
                                      int K, int N, const void *xsrc, hipStream_t st){
     const int rt = sm_row_tiles(gate, nprob);
     ProbUpload up; int slot;
-    int rc = qlmx_upload_problem_pairs(gate, up_, nprob, GEMM_NN, K, N, rt * 16, rt == 4 ? SM_COLS / 2 : SM_COLS, st, &up, &slot); if(rc) return rc;
+    const int shape = rt <= 2 ? sm_few_shape(gate, nprob, K, N, group, true, rt) : SM_NARROW;
+    int rc = qlmx_upload_problem_pairs(gate, up_, nprob, GEMM_NN, K, N, rt * 16, rt == 4 ? SM_COLS / 2 : shape == SM_WIDE ? 2 * SM_COLS : SM_COLS, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
     a.xsrc = (const char *)xsrc;
-#define SM_DUAL(IO) do{ if(rt == 1) SM_LAUNCH((k_gemm_nn_small<1, IO, SM_BY_WAVE>), 2 * SM_WAVES, 0); else if(rt == 2) SM_LAUNCH((k_gemm_nn_small<2, IO, SM_BY_WAVE>), 2 * SM_WAVES, 0); \
-                        else SM_LAUNCH((k_gemm_nn_small<4, IO, SM_BY_LANE>), SM_WAVES, 0); }while(0)
+#define SM_FEW(RT, IO) do{ if(shape == SM_WIDE) SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_BY_WAVE, 16, 4>), 8, 0); \
+                           else if(shape == SM_EIGHT) SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_BY_WAVE, 8, 8>), 16, 0); else SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_BY_WAVE, 8, 4>), 8, 0); }while(0)
+#define SM_DUAL(IO) do{ if(rt == 1) SM_FEW(1, IO); else if(rt == 2) SM_FEW(2, IO); else SM_LAUNCH((k_gemm_nn_small<4, IO, SM_BY_LANE, 8, 4>), 4, 0); }while(0)
     if(xsrc) SM_DUAL(SM_GATHER); else SM_DUAL(SM_PLAIN);
 #undef SM_DUAL
+#undef SM_FEW
     QLMX_LAUNCH_CHECK("grouped gemm nn + swiglu (few rows) launch");
     return qlmx_upload_done(slot, st);
 }

@@ -394,6 +394,57 @@ def test_mfma_few_rows(q, orc, mode, K, N, group, rows):
         assert orc.relerr(got, want) < (4e-4 if mode == "nn" else 3e-6)
 
 
+@pytest.mark.parametrize("K,N,rows,group", [(32, 2048, [1, 16, 0, 9] * 7, 128),              # strips of 256 columns, gate|up too; fewer steps than wavefronts
+                                            (160, 1408, [16, 3] * 16, 128),                   # half a strip at the end
+                                            (96, 2048, [17, 32, 1, 16] * 6, 256),             # one scale for both halves, more than 16 rows
+                                            (64, 1408, [31, 5, 16, 17] * 9, 128),             # wide, gate|up on strips of 128
+                                            (64, 1152, [20, 0] * 35, 128), (64, 1152, [7] * 36, 128), (64, 1152, [7] * 35, 128),     # either side of the line for wide strips
+                                            (2048, 384, [16, 1, 0, 7], 128), (2048, 512, [32, 17, 9], 256), (2080, 128, [5], 128),     # eight wavefronts along the contraction
+                                            (2048, 1152, [32, 17, 9], 128)])
+def test_f16_forward_of_few_rows_in_every_form(q, K, N, rows, group):
+    """The shapes of the forward of at most 32 rows per problem: products with the weights rounded once to fp16, within what K fp32 additions
+    in some order differ from 64 bits by (sqrt(K) * 2^-24 relative to the sums, four times that for their cancelling), and the same bits with the row moves and the SwiGLU
+    folded in."""
+    import torch
+    E, R = len(rows), sum(rows)
+    g = torch.Generator(device="cuda"); g.manual_seed(K + N + E)
+    digit = torch.randint(-8, 8, (2, E, K, N), generator=g, device="cuda", dtype=torch.int8)
+    scale = (torch.rand(2, E, K, N // group, generator=g, device="cuda") + 0.5) * 0.01
+    nib = digit.reshape(-1).to(torch.uint8) & 15
+    d, s = (nib[0::2] | nib[1::2] << 4).view(torch.int8), scale.reshape(-1)
+    w = (scale.repeat_interleave(group, 3) * digit * 256).half().double() / 256
+    x = torch.randn(R + 5, K, generator=g, device="cuda").bfloat16()
+    idx = torch.randperm(R + 5, generator=g, device="cuda")[:R].int()
+    A = x[idx.long()].contiguous()
+    at = np.concatenate([[0], np.cumsum(rows)]).astype(int)
+    n = E * K * N
+    out = {k: torch.full((R, N), 3.0, device="cuda") for k in ("g", "u", "gg", "gp", "up")}
+    act = torch.zeros(R, N, device="cuda", dtype=torch.bfloat16)
+    spread = torch.zeros(R + 5, N, device="cuda")
+
+    def lists(C, first, src=None, B=None):
+        return q.problems([((src.data_ptr() + int(at[e]) * 4) if src is not None else A.data_ptr() + int(at[e]) * K * 2, None if B is None else B.data_ptr() + int(at[e]) * N * 2,
+                            C.data_ptr() + int(at[e]) * (4 if C is idx else N * 4), first * n + e * K * N, (first * n + e * K * N) // group, rows[e], 0.0) for e in range(E)])
+    bf = pkg.ACT_BF16, pkg.MATH_MFMA_F16
+    q.gemm_nn(d, s, group, lists(out["g"], 0), E, K, N, *bf)
+    q.gemm_nn(d, s, group, lists(out["u"], 1), E, K, N, *bf)
+    q.gemm_nn_gather(d, s, group, lists(out["gg"], 0, idx), E, K, N, x)
+    q.gemm_nn_scatter(d, s, group, lists(idx, 0), E, K, N, spread, None)
+    q.gemm_nn_gather_swiglu(d, s, group, lists(out["gp"], 0, idx), lists(out["up"], 1, None, act), E, K, N, x)
+    torch.cuda.synchronize()
+    tol = 4 * K ** 0.5 * 2.0 ** -24
+    for m, k in enumerate("gu"):
+        for e in range(E):
+            if rows[e]:
+                want = A[at[e]:at[e + 1]].double().cpu() @ w[m, e].cpu()
+                got = out[k][at[e]:at[e + 1]].double().cpu()
+                assert float((got - want).norm() / want.norm()) < tol, (k, e)
+    assert torch.equal(out["gg"], out["g"]) and torch.equal(out["gp"], out["g"]) and torch.equal(out["up"], out["u"])
+    assert torch.equal(spread[idx.long()], out["g"])
+    fused = (out["g"] * torch.sigmoid(out["g"]) * out["u"]).bfloat16().float()
+    assert float((act.float() - fused).abs().max()) <= float(fused.abs().max()) * 2.0 ** -7
+
+
 @pytest.mark.parametrize("mode,math", [("nn", "f16"), ("tn", "mfma"), ("nn", "f32"), ("tn", "f32")])
 @pytest.mark.parametrize("M", [5, 40, 100])
 def test_few_rows_outputs_at_any_float(q, orc, mode, math, M):
