@@ -118,7 +118,8 @@ def build_all(jobs=8):
             _drain(procs)
     _drain(procs)
     check_device_asm(objdir)
-    _run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC"] + objs + ["-o", LIB])
+    # nodelete: threads of the library may be asleep in it when a program closes it
+    _run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-Wl,-z,nodelete"] + objs + ["-o", LIB])
     host_src = os.path.join(HERE, "host", "qlm_host.cpp")
     if os.path.exists(host_src):
         _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-I", os.path.join(HERE, "..", "include"),

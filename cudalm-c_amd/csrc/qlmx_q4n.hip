@@ -15,46 +15,117 @@
 #include <immintrin.h>
 #include <math.h>
 #include <string.h>
+#include <signal.h>
+#include <unistd.h>
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <functional>
+#include <mutex>
 #include <new>
 #include <stdexcept>
 #include <thread>
 #include <vector>
 
-/* What bounds it: one division per value when a group is tried against a scale, then the copy of the bytes. Eight
- * values at a time where the CPU has AVX2 (division, rounding and product are the IEEE ones of the scalar form, so the
- * bytes are the same), and by several threads where each has a share worth the 10 us or so that it takes to start: 128 K
- * values when writing, 256 K when reading, eight threads at most (sixteen were slower). The writer finds the groups'
- * scales first, which says where each part's bytes start, and the digits again behind that; the reader walks the group
- * headers first. 4 M values, a tenth of the groups raw, on the 16 CPUs of a GPU's share: write 7.9 ms -> 0.65,
- * read 0.99 -> 0.22. */
-#define Q4N_WRITE_SHARE (128 * 1024)
-#define Q4N_READ_SHARE (256 * 1024)
+/* What bounds it: reading the values, twice when writing -- the writer finds the groups' scales first, which says where each part's bytes
+ * start, and the digits again behind that -- the first touch of the output's pages, and the reader's walk over the group headers. Whether a group fits a scale is
+ * tried eight values at a time where the CPU has AVX2, with one reciprocal for the group instead of a division per value (fits_avx2), and all of it in parts by up
+ * to eight threads (sixteen were slower). Seven threads take 80 us to start and 15 to wake, so they are kept (Q4nCrew below).
+ * 4 M values, a tenth of the groups raw, on the 16 CPUs of a GPU's share, us: write and read by one thread with scalar arithmetic 7900 + 990, divisions and threads started in
+ * each call 330-500 + 180, as here 160-200 + 95-125; half the groups raw, groups of 64: 560 + 420 -> 290 + 340. */
+#define Q4N_WRITE_PART (48 * 1024)              /* values to a part: several parts a thread, since threads wake one after the other */
+#define Q4N_READ_PART (128 * 1024)
 #define Q4N_MAX_THREADS 8
-static int q4n_parts(size_t n, size_t ngroups, size_t share){
-    const unsigned hw = std::thread::hardware_concurrency();
-    return (int)std::max<size_t>(1, std::min({n / share, ngroups, (size_t)std::min<unsigned>(Q4N_MAX_THREADS, hw)}));
-}
 static size_t q4n_groups(size_t n, int group){ return n / (size_t)group + (n % (size_t)group != 0); }
-/* first(part) for every part, and once all are done, second(part) */
-template<class F, class S> static void q4n_run(int parts, const F &first, const S &second){
-    std::atomic<int> done(0);
-    auto finish = [&](int p0, int p1){
-        done.fetch_add(p1 - p0, std::memory_order_acq_rel);
-        while(done.load(std::memory_order_acquire) < parts) std::this_thread::yield();
-        for(int p = p0; p < p1; p++) second(p);
-    };
-    std::thread th[Q4N_MAX_THREADS];
-    int own = 0;                                           /* parts from here on are this thread's */
-    for(; own + 1 < parts; own++){
-        const int p = own;
-        try { th[p] = std::thread([&, p]{ first(p); finish(p, p + 1); }); }
-        catch(const std::exception &){ break; }            /* no more threads, or no memory for one, to be had */
+/* groups longer than 4096: no more parts than threads, as each part has scratch for the digits of a group */
+static int q4n_parts(size_t n, size_t ngroups, int group, size_t part){ return (int)std::max<size_t>(1, std::min<size_t>({n / part, ngroups, (size_t)(group > 4096 ? Q4N_MAX_THREADS : 4096)})); }
+
+/* Threads for the calls' parts: started as calls ask for them, at most seven whatever the number of callers, and gone after a second without work. A call
+ * takes part in its own job and needs none of them; several calls at once share them. A job is on its caller's stack: the caller leaves when its
+ * parts are done and no thread has hold of it any more. The crew itself is never destroyed, so threads asleep at exit touch nothing that is; a
+ * child of fork() has none of the threads and starts with a crew of its own. */
+struct Q4nJob {
+    const std::function<void(int)> *phase[2]; int parts;
+    std::atomic<int> next[2], done[2];
+    int holders; Q4nJob *link;                             /* both under the crew's lock */
+    Q4nJob() : parts(0), holders(0), link(nullptr) { for(int i = 0; i < 2; i++){ phase[i] = nullptr; next[i] = 0; done[i] = 0; } }
+    bool open() const { return next[0].load(std::memory_order_relaxed) < parts || (phase[1] && next[1].load(std::memory_order_relaxed) < parts); }
+    /* parts that nobody has begun; the second phase only when all of the first are done */
+    void work(){
+        for(int ph = 0; ph < 2 && phase[ph]; ph++){
+            for(int p; (p = next[ph].fetch_add(1, std::memory_order_relaxed)) < parts; ){
+                (*phase[ph])(p);
+                done[ph].fetch_add(1, std::memory_order_acq_rel);
+            }
+            while(done[ph].load(std::memory_order_acquire) < parts) std::this_thread::yield();
+        }
     }
-    for(int p = own; p < parts; p++) first(p);
-    finish(own, parts);
-    for(int p = 0; p < own; p++) th[p].join();
+};
+struct Q4nCrew {
+    std::mutex lock; std::condition_variable wake, left;
+    Q4nJob *jobs = nullptr; int threads = 0, idle = 0;
+    const pid_t owner = getpid();
+
+    void member(){
+        sigset_t all;                                      /* signals are for the program's own threads */
+        sigfillset(&all); pthread_sigmask(SIG_BLOCK, &all, nullptr);
+        std::unique_lock<std::mutex> l(lock);
+        for(;;){
+            Q4nJob *j = jobs;
+            while(j && !j->open()) j = j->link;
+            if(!j){
+                idle++;
+                const bool late = wake.wait_for(l, std::chrono::seconds(1)) == std::cv_status::timeout;
+                idle--;
+                if(late){
+                    for(j = jobs; j && !j->open(); j = j->link) ;
+                    if(!j) break;
+                }
+                continue;
+            }
+            j->holders++;
+            l.unlock();
+            j->work();
+            l.lock();
+            if(--j->holders == 0) left.notify_all();
+        }
+        threads--;
+    }
+    void run(Q4nJob &j, int wanted){
+        {
+            std::lock_guard<std::mutex> l(lock);
+            j.link = jobs; jobs = &j;
+            for(int more = wanted - idle; more > 0 && threads < Q4N_MAX_THREADS - 1; more--){
+                try { std::thread([this]{ member(); }).detach(); threads++; }
+                catch(const std::exception &){ break; }    /* no more threads, or no memory for one, to be had */
+            }
+        }
+        wake.notify_all();
+        j.work();
+        std::unique_lock<std::mutex> l(lock);
+        Q4nJob **at = &jobs;
+        while(*at != &j) at = &(*at)->link;
+        *at = j.link;
+        while(j.holders) left.wait(l);
+    }
+};
+static Q4nCrew *q4n_crew(){
+    static std::atomic<Q4nCrew *> crew(nullptr);
+    Q4nCrew *c = crew.load(std::memory_order_acquire);
+    while(!c || c->owner != getpid()){
+        Q4nCrew *n = new Q4nCrew;
+        if(crew.compare_exchange_strong(c, n, std::memory_order_acq_rel)) return n;
+        delete n;
+    }
+    return c;
+}
+/* first(part) for every part, and once all are done, second(part) for every part */
+static void q4n_run(int parts, const std::function<void(int)> &first, const std::function<void(int)> *second){
+    Q4nJob j;
+    j.parts = parts; j.phase[0] = &first; j.phase[1] = second;
+    const int wanted = std::min({parts, Q4N_MAX_THREADS, (int)std::thread::hardware_concurrency()}) - 1;
+    if(wanted > 0) q4n_crew()->run(j, wanted); else j.work();
 }
 static bool q4n_avx2(){ static const bool yes = __builtin_cpu_supports("avx2"); return yes; }
 
@@ -84,13 +155,60 @@ static void unpack_from(const unsigned char *b, int j0, int g, float scale, floa
 }
 __attribute__((target("avx2"))) static float amax_avx2(const float *v, int g){
     const __m256 mag = _mm256_castsi256_ps(_mm256_set1_epi32(0x7FFFFFFF));
-    __m256 m = _mm256_setzero_ps();
+    __m256 m = _mm256_setzero_ps(), m1 = m, m2 = m, m3 = m;       /* four chains: a maximum takes four cycles */
     int j = 0;
-    for(; j + 8 <= g; j += 8) m = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j), mag), m);     /* a NaN leaves m, as fmaxf does */
-    float e[8]; _mm256_storeu_ps(e, m);
-    float amax = 0.0f;
-    for(int k = 0; k < 8; k++) amax = fmaxf(amax, e[k]);
+    for(; j + 32 <= g; j += 32){
+        m  = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j), mag), m);                             /* a NaN leaves m, as fmaxf does */
+        m1 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j + 8), mag), m1);
+        m2 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j + 16), mag), m2);
+        m3 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j + 24), mag), m3);
+    }
+    m = _mm256_max_ps(_mm256_max_ps(m, m1), _mm256_max_ps(m2, m3));
+    __m128 t = _mm_max_ps(_mm256_castps256_ps128(m), _mm256_extractf128_ps(m, 1));
+    t = _mm_max_ps(t, _mm_movehl_ps(t, t));
+    const float amax = _mm_cvtss_f32(_mm_max_ss(t, _mm_shuffle_ps(t, t, 1)));
     return amax_from(v, j, g, amax);
+}
+/* A group against one of its candidates amax / k, in the range that q4n_mid names: whether every value is a digit times the scale, with a reciprocal for the division. The
+ * answer is that of try_from. A digit d passes there when |d| <= 7 and the rounded product d * scale is v. Then v is d * scale within 2^-24 of itself, and v * (1/scale), two
+ * roundings further, d within 2^-22 of itself: it rounds to the same d. The other way round, a digit that passes here has v = rounded d * scale, so that
+ * v / scale rounds to it too; and it is at most 7, as no value is more than amax and no candidate less than amax / 7 by more than two units in its last place. */
+__attribute__((target("avx2"))) static bool fits_avx2(const float *v, int g, float scale){
+    const __m256 s = _mm256_set1_ps(scale), inv = _mm256_set1_ps(1.0f / scale);
+    int j = 0;
+    for(; j + 32 <= g; j += 32){
+        __m256 off = _mm256_setzero_ps();
+        for(int i = 0; i < 32; i += 8){
+            const __m256 x = _mm256_loadu_ps(v + j + i), d = _mm256_round_ps(_mm256_mul_ps(x, inv), _MM_FROUND_CUR_DIRECTION);
+            off = _mm256_or_ps(off, _mm256_cmp_ps(_mm256_mul_ps(d, s), x, _CMP_NEQ_UQ));
+        }
+        if(_mm256_movemask_ps(off)) return false;
+    }
+    for(; j < g; j++){
+        const float d = rintf(v[j] / scale);
+        if(fabsf(d) > 7.0f || d * scale != v[j]) return false;
+    }
+    return true;
+}
+/* the nibbles of a group that fits, one of the range */
+__attribute__((target("avx2"))) static void put_avx2(const float *v, int g, float scale, unsigned char *b){
+    const __m256 inv = _mm256_set1_ps(1.0f / scale);
+    const __m256i low = _mm256_set1_epi32(0x000F000F), byte = _mm256_set1_epi32(0xFF);
+    int j = 0;
+    for(; j + 32 <= g; j += 32){
+        __m256i h[2];
+        for(int i = 0; i < 2; i++){
+            const __m256i u = _mm256_cvtps_epi32(_mm256_mul_ps(_mm256_loadu_ps(v + j + 16 * i), inv)), w = _mm256_cvtps_epi32(_mm256_mul_ps(_mm256_loadu_ps(v + j + 16 * i + 8), inv));
+            const __m256i x = _mm256_and_si256(_mm256_permute4x64_epi64(_mm256_packs_epi32(u, w), 0xD8), low);      /* 16 digits in order, a 16-bit word each */
+            h[i] = _mm256_and_si256(_mm256_or_si256(x, _mm256_srli_epi32(x, 12)), byte);
+        }
+        const __m256i t = _mm256_permute4x64_epi64(_mm256_packus_epi32(h[0], h[1]), 0xD8);
+        _mm_storeu_si128((__m128i *)(b + (j >> 1)), _mm_packus_epi16(_mm256_castsi256_si128(t), _mm256_extracti128_si256(t, 1)));
+    }
+    for(; j < g; j += 2){
+        const int d0 = (int)rintf(v[j] / scale), d1 = j + 1 < g ? (int)rintf(v[j + 1] / scale) : 0;
+        b[j >> 1] = (unsigned char)((d0 & 15) | ((d1 & 15) << 4));
+    }
 }
 __attribute__((target("avx2"))) static bool try_avx2(const float *v, int g, float scale, signed char *digit){
     const __m256 s = _mm256_set1_ps(scale), seven = _mm256_set1_ps(7.0f), mag = _mm256_castsi256_ps(_mm256_set1_epi32(0x7FFFFFFF));
@@ -127,6 +245,23 @@ __attribute__((target("avx2"))) static void unpack_avx2(const unsigned char *b, 
     }
     unpack_from(b, j, g, scale, P);
 }
+/* Whether the first eight values may be amax / k times whole numbers, for the candidates of this k: a value that is a digit times one of them, rounded, is
+ * amax / k times that digit within 2^-21 of itself, so that v * (1 / amax) * k is within 2^-17 of a whole number. What fails here fails with all five; a raw group, which has no
+ * scale, is seen off with 7 of these instead of 35 tries (4 M values, half the groups raw: 580 -> 376 us). */
+__attribute__((target("avx2"))) static bool maybe_avx2(__m256 share, int k){
+    const __m256 t = _mm256_mul_ps(share, _mm256_set1_ps((float)k)), off = _mm256_sub_ps(t, _mm256_round_ps(t, _MM_FROUND_CUR_DIRECTION));
+    const __m256 mag = _mm256_castsi256_ps(_mm256_set1_epi32(0x7FFFFFFF));
+    return _mm256_movemask_ps(_mm256_cmp_ps(_mm256_and_ps(off, mag), _mm256_set1_ps(0x1p-17f), _CMP_NLE_UQ)) == 0;
+}
+__attribute__((target("avx2"))) static unsigned maybe_scales(const float *v, int g, float amax){       /* bit k: amax / k has to be tried */
+    if(g < 8) return 0xFEu;
+    const __m256 share = _mm256_mul_ps(_mm256_loadu_ps(v), _mm256_set1_ps(1.0f / amax));
+    unsigned m = 0;
+    for(int k = 7; k >= 1; k--) m |= (unsigned)maybe_avx2(share, k) << k;
+    return m;
+}
+/* largest magnitudes, and scales, whose quotients and products neither overflow nor lose bits */
+static bool q4n_mid(float x){ return q4n_avx2() && x >= 0x1p-90f && x <= 0x1p90f; }
 static float group_amax(const float *v, int g){ return q4n_avx2() ? amax_avx2(v, g) : amax_from(v, 0, g, 0.0f); }
 static bool group_try(const float *v, int g, float scale, signed char *digit){ return q4n_avx2() ? try_avx2(v, g, scale, digit) : try_from(v, 0, g, scale, digit); }
 static void group_pack(const signed char *digit, int g, unsigned char *b){ if(q4n_avx2()) pack_avx2(digit, g, b); else pack_from(digit, 0, g, b); }
@@ -139,11 +274,14 @@ static inline float toward_inf(float x){ unsigned u; memcpy(&u, &x, 4); if(u != 
 static float group_scale(const float *v, int g, signed char *digit){
     const float amax = group_amax(v, g);
     if(amax == 0.0f) return 0.0f;
+    const bool mid = q4n_mid(amax);
+    const unsigned worth = mid ? maybe_scales(v, g, amax) : 0xFEu;
     for(int k = 7; k >= 1; k--){
+        if(!(worth >> k & 1)) continue;
         const float s0 = amax / (float)k;
         const float below = toward_zero(s0), above = toward_inf(s0);
         const float cand[5] = {s0, below, above, toward_zero(below), toward_inf(above)};
-        for(int t = 0; t < 5; t++) if(group_try(v, g, cand[t], digit)) return cand[t];
+        for(int t = 0; t < 5; t++) if(mid ? fits_avx2(v, g, cand[t]) : group_try(v, g, cand[t], digit)) return cand[t];
     }
     return NAN;
 }
@@ -155,14 +293,14 @@ extern "C" size_t qlmx_q4n_bound(size_t n, int group){
 
 static int q4n_write(const float *P, size_t n, int group, unsigned char *out, size_t *out_len, size_t *nraw){
     const size_t ngroups = q4n_groups(n, group);
-    const int parts = q4n_parts(n, ngroups, Q4N_WRITE_SHARE);
+    const int parts = q4n_parts(n, ngroups, group, Q4N_WRITE_PART);
     std::vector<float> scales(ngroups);
     const size_t stride = std::min((size_t)group, n) + 256;     /* a part's digits share no cache line with another's */
     std::vector<signed char> digits((size_t)parts * stride);
-    size_t len[Q4N_MAX_THREADS] = {}, raw[Q4N_MAX_THREADS] = {};
+    std::vector<size_t> len(parts), raw(parts);
     auto begin = [&](int p){ return ngroups * (size_t)p / (size_t)parts; };
     auto size_of = [&](size_t q){ return (int)std::min((size_t)group, n - q * (size_t)group); };
-    q4n_run(parts, [&](int p){
+    const std::function<void(int)> find = [&](int p){
         signed char *digit = digits.data() + (size_t)p * stride;
         size_t l = 0, r = 0;
         for(size_t q = begin(p); q < begin(p + 1); q++){
@@ -172,7 +310,7 @@ static int q4n_write(const float *P, size_t n, int group, unsigned char *out, si
             if(s != s){ l += 4 + 4 * (size_t)g; r++; } else l += 4 + (size_t)(g + 1) / 2;
         }
         len[p] = l; raw[p] = r;
-    }, [&](int p){
+    }, put = [&](int p){
         signed char *digit = digits.data() + (size_t)p * stride;
         unsigned char *o = out;
         for(int i = 0; i < p; i++) o += len[i];
@@ -182,11 +320,16 @@ static int q4n_write(const float *P, size_t n, int group, unsigned char *out, si
             const float s = scales[q];
             memcpy(o, &s, 4); o += 4;
             if(s != s){ memcpy(o, v, 4 * (size_t)g); o += 4 * (size_t)g; continue; }
-            if(s == 0.0f) memset(digit, 0, (size_t)g); else group_try(v, g, s, digit);
-            digit[g] = 0;                                  /* the partner of an odd group's last digit */
-            group_pack(digit, g, o); o += (g + 1) / 2;
+            if(q4n_mid(s)) put_avx2(v, g, s, o);
+            else {
+                if(s == 0.0f) memset(digit, 0, (size_t)g); else group_try(v, g, s, digit);
+                digit[g] = 0;                              /* the partner of an odd group's last digit */
+                group_pack(digit, g, o);
+            }
+            o += (g + 1) / 2;
         }
-    });
+    };
+    q4n_run(parts, find, &put);
     size_t o = 0, nr = 0;
     for(int p = 0; p < parts; p++){ o += len[p]; nr += raw[p]; }
     *out_len = o;
@@ -213,7 +356,7 @@ static int q4n_read(const unsigned char *buf, size_t len, float *P, size_t n, in
             o += (g + 1) / 2;
         }
     }
-    const int parts = q4n_parts(n, ngroups, Q4N_READ_SHARE);
+    const int parts = q4n_parts(n, ngroups, group, Q4N_READ_PART);
     q4n_run(parts, [&](int p){
         for(size_t q = ngroups * (size_t)p / (size_t)parts; q < ngroups * (size_t)(p + 1) / (size_t)parts; q++){
             const size_t i = q * (size_t)group;
@@ -223,7 +366,7 @@ static int q4n_read(const unsigned char *buf, size_t len, float *P, size_t n, in
             if(scale != scale) memcpy(P + i, b + 4, 4 * (size_t)g);
             else group_unpack(b + 4, g, scale, P + i);
         }
-    }, [](int){});
+    }, nullptr);
     if(used) *used = o;
     return QLMX_OK;
 }

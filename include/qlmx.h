@@ -444,7 +444,8 @@ int qlmx_test_step_wide(int on);
  * qlmx_q4n_bound: bytes that always suffice for n values. quantize: *out_len bytes written, *nraw
  * (may be NULL) = groups stored raw. dequantize: *used (may be NULL) = bytes consumed.
  * Scratch is a few bytes per group of the values (writer) or per group that len bytes can hold (reader), and one group's digits
- * for each of at most eight threads; QLMX_E_LIMIT if it cannot be had.
+ * for each 48 K values (groups longer than 4096: eight times); QLMX_E_LIMIT if it cannot be had.
+ * Large calls share up to seven threads of the library with all callers; the threads end after a second without work.
  * ===================================================================================== */
 size_t qlmx_q4n_bound(size_t n, int group);
 int qlmx_q4n_quantize(const float *P, size_t n, int group, unsigned char *out, size_t cap, size_t *out_len, size_t *nraw);

@@ -96,6 +96,61 @@ def test_sizes_around_the_vector_and_thread_shares(lib, orc, n, group):
     assert ok == 1 and used == want.size and np.array_equal(back.view(np.uint32), wback.view(np.uint32))
 
 
+@pytest.mark.parametrize("exponent", [-126, -100, -93, -91, -90, -89, 0, 86, 87, 88, 89, 90, 91, 120])
+@pytest.mark.parametrize("group", [128, 64, 34])
+def test_groups_that_fit_and_groups_that_nearly_do(lib, orc, exponent, group):
+    """Scales of any mantissa at both ends of the range in which a reciprocal stands for the division: digits up to 7 down to 1, values one unit in the last
+    place off at the front and at the back, negative zeros, one value between the digits."""
+    rng = np.random.default_rng((exponent + 200) * 1000 + group)
+    groups = []
+    for i in range(420):
+        most = 7 - i % 7
+        d = rng.integers(-most, most + 1, group).astype(f32)
+        d[rng.integers(group)] = most if i % 2 else -most
+        scale = np.ldexp(f32(1 + rng.random()), exponent).astype(f32)
+        v = (d * scale).astype(f32)
+        at = (0, group - 1, int(rng.integers(group)))[i % 3]
+        if i % 5 == 1: v[at] = np.nextafter(v[at], f32(np.inf))
+        elif i % 5 == 2: v[v == 0] = f32(-0.0)
+        elif i % 5 == 3: v[at] = f32(0.5) * scale
+        groups.append(v)
+    P = np.concatenate(groups)
+    want, wraw = orc.q4n_quantize(P, group)
+    got, raw = lib.q4n_quantize(P, group)
+    assert raw == wraw and np.array_equal(got, want)
+    back, used = lib.q4n_dequantize(got, P.size, group)
+    assert used == got.size and np.array_equal(back + f32(0), P + f32(0))       # a zero comes back positive
+
+
+def test_callers_share_the_threads_and_a_child_has_its_own(lib):
+    """Calls from several threads at once, calls after the threads have gone for want of work, and calls in a child process."""
+    import threading
+    import time
+    rng = np.random.default_rng(9)
+    data = [(rng.integers(-7, 8, n) * f32(0.031)).astype(f32) for n in (900001, 60000, 400000, 1300000)]
+    alone = [lib.q4n_quantize(P, 128)[0] for P in data]
+    ok = [0] * len(data)
+
+    def caller(i):
+        for _ in range(20):
+            buf, raw = lib.q4n_quantize(data[i], 128)
+            back, _ = lib.q4n_dequantize(buf, data[i].size, 128)
+            ok[i] += raw == 0 and np.array_equal(buf, alone[i]) and np.array_equal(back, data[i])
+    for pause in (0.0, 1.3):
+        time.sleep(pause)
+        ts = [threading.Thread(target=caller, args=(i,)) for i in range(len(data))]
+        [t.start() for t in ts]
+        [t.join() for t in ts]
+    assert ok == [40] * len(data)
+    child = os.fork()
+    if child == 0:
+        try:
+            os._exit(0 if np.array_equal(lib.q4n_quantize(data[0], 128)[0], alone[0]) else 1)
+        finally:
+            os._exit(2)
+    assert os.waitstatus_to_exitcode(os.waitpid(child, 0)[1]) == 0
+
+
 def test_truncated_buffer_is_refused(lib, orc, golden):
     g = golden("q4n")
     n, group = (int(v) for v in g["dims"])
