@@ -509,6 +509,17 @@ static int sm_few_shape(const qlmx_gemm_prob *probs, int nprob, int K, int N, in
     if(rt == 2) return wide >= 160 && wide <= 256 && N % 2048 == 0 ? SM_WIDE : SM_NARROW;
     return wide >= 176 && (wide <= 256 || wide >= 352) ? SM_WIDE : SM_NARROW;
 }
+/* Height of the row tiles of a call with more than 32 rows to a problem: 64, which share the weights' conversion or loads; 32 where these are at most one to a CU
+ * and the contraction is long enough for a workgroup's loop to be what takes the time. The order of a sum is the same in both. us, 32 : 64 rows: forward, 8 experts of 125, 1536 x 512,
+ * 11.9:15.1, of 100, 1408 x 1024, 11.6:15.2, 16 of 64, 2048 x 768 16.5:20.8, one of 500 14.5:18.1; more than one to a CU, 8 of 250, 1536 x 512, 18.0:15.9; gate|up the
+ * same within 4 % (not taken). Paired input gradient 8 of 125, 1536 x 512, 11.6:14.5, of 64, 2048 x 768 14:18.1; more than one to a CU 16 of 64, 1536 x 768 19.5:16.2, 32
+ * of 64, 2048 x 1024 47:40; short, 8 of 64, 512 x 512, 7.5:6.5. */
+static int sm_tile_rows(const qlmx_gemm_prob *probs, int nprob, int contraction, int strips){
+    const int rt = sm_row_tiles(probs, nprob);
+    long long tiles = 0;
+    for(int i = 0; i < nprob; i++) tiles += (probs[i].M + 31) / 32 * strips;
+    return rt == 4 && tiles <= qlmx_cu_count() && contraction >= 1024 ? 2 : rt;
+}
 static SmArgs sm_args(const signed char *d, const float *s, int group, int K, int N, const ProbUpload &up){
     SmArgs a = {};
     a.pr = up.dev; a.nprob = up.nprob; a.ntiles = up.ntiles; a.d = d; a.s = s; a.K = K; a.N = N;
@@ -520,9 +531,9 @@ static SmArgs sm_args(const signed char *d, const float *s, int group, int K, in
 /* N % 128 == 0, K % 32 == 0, group a power of two >= 64; io, xsrc, out, gate as in qlmx_gemm_nn_h_launch */
 int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N,
                               int io, const void *xsrc, float *out, const float *gate, hipStream_t st){
-    const int rt = sm_row_tiles(probs, nprob);
+    const int high = sm_row_tiles(probs, nprob), rt = sm_tile_rows(probs, nprob, K, N / SM_COLS);
     ProbUpload up; int slot;
-    const int shape = rt <= 2 ? sm_few_shape(probs, nprob, K, N, group, false, rt) : SM_NARROW;
+    const int shape = high <= 2 ? sm_few_shape(probs, nprob, K, N, group, false, rt) : SM_NARROW;
     int rc = qlmx_upload_problems(probs, nprob, GEMM_NN, K, N, rt * 16, shape == SM_WIDE ? 2 * SM_COLS : SM_COLS, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
@@ -558,7 +569,7 @@ int qlmx_gemm_nn_small_swiglu_launch(const signed char *d, const float *s, int g
 /* N % 128 == 0, K % 64 == 0, group a power of two >= 64; the rest as in qlmx_gemm_tn_lds_launch */
 int qlmx_gemm_tn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, const qlmx_gemm_prob *second, int nprob,
                               int K, int N, float *out, const float *gp, const float *up_, void *dg, void *du, hipStream_t st){
-    const int rt = sm_row_tiles(probs, nprob);
+    const int rt = sm_tile_rows(probs, nprob, K * (second ? 2 : 1), N / SM_TCOLS);
     ProbUpload up; int slot;
     int rc = second ? qlmx_upload_problem_pairs(probs, second, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot)
                     : qlmx_upload_problems(probs, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot);
