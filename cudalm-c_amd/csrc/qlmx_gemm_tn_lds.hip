@@ -25,10 +25,8 @@ int qlmx_gemm_tn_lds_issue(const Tn3Args &a, int grid, int slot, hipStream_t st)
 int qlmx_gemm_tn_lds_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs,
                             const qlmx_gemm_prob *second, int nprob, int K, int N, float *out, const float *gate,
                             const float *gp, const float *up_, void *dg, void *du, hipStream_t st){
-    if(qlmx_small_rows(probs, nprob, GEMM_TN, K, N, second ? 2 : 1, group)){
-        int rc = qlmx_pair_flush(); if(rc) return rc;          /* not a kernel that is held for a pair: what is held goes first */
+    if(qlmx_small_rows(probs, nprob, GEMM_TN, K, N, second ? 2 : 1, group))
         return qlmx_gemm_tn_small_launch(d, s, group, probs, second, nprob, K, N, out, gp, up_, dg, du, st);
-    }
     ProbUpload up; int slot;
     /* a problem's C field is its output rows, its rows of gp (SwiGLU gradient behind), or a list of row indices */
     const RowBytes rb = {(size_t)K * 2, out ? sizeof(int) : (size_t)N * 4, (size_t)K * 2, 0, 0};

@@ -76,7 +76,7 @@ int         qlmx_side_join(void *stream);
  * kind's tiles take the compute units as the first kind's last round leaves them -- without the wait between
  * hardware queues that the side stream costs at its fork and join. The caller promises what it promises for the
  * side stream: neither of the two reads what the other writes. Everything else keeps its order on the stream:
- * a second launch of a kind already held, a launch of a shape the two direct-to-LDS kernels do not take, and any
+ * a second launch of a kind already held, a launch of a shape that none of these kernels takes, and any
  * other library call that queues work first issue what is held. One pair at a time; not for use across host
  * synchronisation (nothing held runs before qlmx_pair_end or one of the calls just named). */
 int         qlmx_pair_begin(void *stream);

@@ -1014,6 +1014,61 @@ def test_side_stream_fork_join(q, orc):
     assert float(outs[0][1].abs().max()) > 0.0
 
 
+@pytest.mark.parametrize("form", ["plain", "added", "continued", "swiglu", "scatter"])
+@pytest.mark.parametrize("rows,K,N", [([9, 16, 0, 1], 256, 512), ([40, 33, 64, 17, 1], 128, 1024), ([125, 131, 97], 512, 384), ([1200, 3], 256, 256)])
+def test_backward_pair_of_few_rows(q, form, rows, K, N):
+    """The kernels for few rows in one grid with the weight gradient: the bits of the two launches, for every form of the input gradient, row tiles of
+    one and two sixteens, a sliced weight gradient behind it, no weight gradient at all, and a second one of each kind."""
+    import torch
+    cur = torch.cuda.current_stream().cuda_stream
+    E, R, bf = len(rows), sum(rows), (pkg.ACT_BF16, pkg.MATH_MFMA)
+    at = np.concatenate([[0], np.cumsum(rows)]).astype(int)
+    g = torch.Generator(device="cuda"); g.manual_seed(R + K)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    digit = torch.randint(-7, 8, (2 * E * K * N // 2, 2), generator=g, device="cuda")
+    d = ((digit[:, 0] & 15) | (digit[:, 1] & 15) << 4).to(torch.uint8).view(torch.int8)
+    s = torch.rand(2 * E * K * N // 128, generator=g, device="cuda") * 0.01 + 0.005
+    dY, dY2, X = rnd(R, N).bfloat16(), rnd(R, N).bfloat16(), rnd(R, K).bfloat16()
+    gp, up = rnd(R, K), rnd(R, K)
+    idx = torch.randperm(R + 3, generator=g, device="cuda")[:R].int()
+    wgrad = lambda G, src, beta: q.problems([(X.data_ptr() + int(at[e]) * K * 2, src.data_ptr() + int(at[e]) * N * 2, G.data_ptr() + e * K * N * 4, 0, 0, rows[e], beta) for e in range(E)])
+
+    def igrad(C, src, first, beta=0.0, size=4):
+        width = 1 if C is idx else K
+        return q.problems([(src.data_ptr() + int(at[e]) * N * 2, None, C.data_ptr() + int(at[e]) * width * 4, (first + e) * N * K, (first + e) * N * K // 128, rows[e], beta) for e in range(E)])
+    outs = []
+    for pair in (False, True):
+        for partner in ("after", "before", "none", "twice"):
+            G, dX, spread = torch.ones(E * K * N, device="cuda"), torch.ones(R, K, device="cuda"), torch.ones(R + 3, K, device="cuda")
+            dg, du = torch.zeros(R, K, device="cuda", dtype=torch.bfloat16), torch.zeros(R, K, device="cuda", dtype=torch.bfloat16)
+
+            def weights(beta=0.0, src=dY): q.gemm_nt(wgrad(G, src, beta), E, K, N, *bf, cur)
+
+            def inputs():
+                if form == "plain": q.gemm_tn(d, s, 128, igrad(dX, dY, 0), E, N, K, *bf, cur)
+                elif form == "added": q.gemm_tn(d, s, 128, igrad(dX, dY, 0, 1.0), E, N, K, *bf, cur)
+                elif form == "continued": q.gemm_tn_pair(d, s, 128, igrad(dX, dY, 0), igrad(dX, dY2, E, 1.0), E, N, K, *bf, cur)
+                elif form == "swiglu": q.gemm_tn_swiglu_bwd(d, s, 128, igrad(gp, dY, 0), E, N, K, gp, up, dg, du, cur)
+                else: q.gemm_tn_pair_scatter(d, s, 128, igrad(idx, dY, 0), igrad(idx, dY2, E), E, N, K, spread, cur)
+            if pair:
+                q.pair_begin(cur)
+            if partner in ("before", "twice"): weights()
+            inputs()
+            if partner == "twice":
+                weights(1.0, dY2)
+                inputs()
+            if partner == "after": weights()
+            if pair:
+                q.pair_end(cur)
+            torch.cuda.synchronize()
+            outs.append((G, dX, spread, dg, du))
+    for a, b in zip(outs[:4], outs[4:]):
+        for x, y in zip(a, b):
+            assert torch.equal(x, y)
+    changed = {"plain": 1, "added": 1, "continued": 1, "swiglu": 3, "scatter": 2}[form]
+    assert float((outs[4][changed].float() - 1).abs().max()) > 0.0 and float((outs[4][0] - 1).abs().max()) > 0.0
+
+
 def test_backward_pair_is_one_launch_with_the_same_bits(q, orc):
     """qlmx_pair_begin / qlmx_pair_end: the input gradient and the weight gradient of a flush held back and issued as
     one grid give the bits of the two launches one after the other -- plain, with a sliced weight-gradient contraction
