@@ -18,24 +18,26 @@
  * gradient multiplies exact digits and applies the scale to the fp32 sums of each group of k.
  *
  * Which calls come here (qlmx_small_rows): all whose problems have at most 32 rows, and those that would leave the tiled
- * kernels with few workgroups, each walking the whole contraction. The forward's rule looks at what the forms of a call that
- * are documented to agree bit for bit have in common -- with and without gather, SwiGLU, scatter -- so that they run the same
- * arithmetic in the same order. Counted in strips of 64 rows x 128 columns (a SwiGLU call has twice as many); us for the plain
- * and the SwiGLU call, these : tiled --
- *   up to 128, contractions over 512: one round of workgroups here. 1024 x 4096, 8 experts of 40 rows 13:16 and 16:16; 1408 x
- *     2048, 512 rows of one expert 16:18 and 18:19; 768 x 2048, 8 of 64 11:12 and 14:15; but 512 x 1536, 512 of one 9:9 and 10:9.
- *   up to 256, where the contraction is not shorter than the width, or over 1024 with no problem of more than 64 rows: the plain
+ * kernels with few workgroups, each walking the whole contraction, or with tiles that are mostly padding: a prompt or a small batch whose router prefers
+ * some experts has a few problems of a hundred rows beside many of five, each a tile of 128 there and of 32 here. The forward's rule looks at what the
+ * forms of a call that are documented to agree bit for bit have in common -- with and without gather, SwiGLU, scatter -- so that they run the same
+ * arithmetic in the same order. us for the plain and the SwiGLU call, these : tiled --
+ *   tiles of 32 rows x 128 columns up to 256, one to a CU. 16 problems, largest 43 rows, 896 x 1152 8.3:13.6, 1152 x 896 14.6:19.0; 8, largest 69,
+ *     384 x 1152 6.0:8.3 and 8.6:9.0; one of 292, 1024 x 1920 9.8:11.9 and 13.5:13.1;
+ *   beyond, tiles of 32 rows at most 1.5 times the 128-row tiles; up to 352 of them 1.125 times (a second round that is nearly empty). Zipf shares: 1096 rows of 64, 896 x 512
+ *     12.5:18.0, 512 x 896 22:24; 617 of 64, 1664 x 1920 41:60, 1920 x 1664 62:109; 362 of 32, 2304 x 896 18:31, 896 x 2304 32:50. On the other side 4832 of 64,
+ *     1536 x 768 41:33, 768 x 1536 77:70; and with 330 tiles, 16 of 31 rows, 1024 x 1920 14:16 and 26:20;
+ *   strips of 64 x 128 up to 256, where the contraction is not shorter than the width, or over 1024 with no problem of more than 64 rows: the plain
  *     call gains what the SwiGLU call (two rounds) loses. 1536 x 512, 64 of 40 18:22 and 29:28; 1408 x 2048, 16 of 40 17:20 and 32:28.
  *   up to 512, where the contraction is four times the width: the down projection of a wide layer, whose SwiGLU call has other
  *     sizes. 2304 x 512, 64 of 77 39:43 (a SwiGLU call 79:59, as at twice the width: 2048 x 768, 32 of 100 30:26 and 56:38).
- *   beyond, contractions over 1024 with few rows to a problem on average, which the tiled kernel pads to 128 each:
- *     contraction not shorter than the width: 48, or 32 where the largest is over 64 (the others have fewer still). 2048 x 768,
- *     64 of 40 31:33 and 57:68; 2048 x 1408, 128 of 24 (largest 144) 70:93 and 207:202, of 12 61:86 and 194:201; on the other side
- *     128 of 36 (largest 172) 84:96 and 230:208, 64 of 64 56:63 and 121:103.
- *     shorter: 24, none over 64. 1408 x 2048, 64 of 18 (largest 55) 44:46 and 98:101; on the other side 32 of 36 26:24 and 63:53.
+ *   beyond, contractions over 1024 and not shorter than the width, of at most 64 rows to a problem and 48 on average, which the tiled kernel pads to 128: 2048 x 1664,
+ *     64 of 41 59:63 and 102:116, 2048 x 768, 64 of 40 31:33 and 57:68; on the other side 64 of 64 56:63 and 121:103.
+ * Over 160 calls of 1 to 64 problems of 5 to 400 rows on average, in even and in Zipf shares, 256 to 2048 in and out, a plain call takes 0.86 and a SwiGLU call 0.96 of what they took
+ * when the rule counted strips of 64 rows only and problems of over 32 rows had tiles of 64 (mean of the ratios; over half of the calls are as they were).
  * The lines look at a call's own sizes, so a layer whose passes run one by one may take the one path and its merged list the other: bits that
  * agree between the two are not promised and not looked for here.
- * Input gradient, 64 columns: up to 512, 1024 where the contraction is twice the width.
+ * Input gradient, strips of 64 x 64: up to 512, 1024 where the contraction is twice the width.
  * us per call, tiled kernels of 256 x 128 (128 x 128) as these were written -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16
  * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
@@ -67,23 +69,36 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 static __device__ __align__(16) unsigned char sm_zero_row[32768];       /* what a dropped row of a gather reads */
 
+/* a call's row tiles of 32, 64 and 128 */
+struct SmRows { long long t32, t64, t128, rows, busy; int most; };
+static SmRows sm_rows(const qlmx_gemm_prob *probs, int nprob){
+    SmRows r = {0, 0, 0, 0, 0, 0};
+    for(int i = 0; i < nprob; i++){
+        const int m = probs[i].M;
+        r.t32 += (m + 31) / 32; r.t64 += (m + 63) / 64; r.t128 += (m + 127) / 128;
+        r.rows += m; r.busy += m > 0;
+        if(m > r.most) r.most = m;
+    }
+    return r;
+}
+/* tiles of 32 rows against `high` taller ones, on so many strips: at most one to a CU, or not many more of them; see the head of this file */
+static bool sm_low(long long t32, long long high, int strips){
+    const long long tiles = t32 * strips;
+    return tiles <= 256 || (tiles <= 352 ? 8 * t32 <= 9 * high : 2 * t32 <= 3 * high);
+}
 /* see the head of this file */
 bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, int N, int nseg, int group){
     if(group < 64) return false;
-    long long tiles = 0, rows = 0; int most = 0, busy = 0;
-    for(int i = 0; i < nprob; i++){
-        if(probs[i].M > most) most = probs[i].M;
-        rows += probs[i].M; busy += probs[i].M > 0;
-        tiles += (probs[i].M + 63) / 64;
-    }
-    if(most <= 32) return true;
+    const SmRows r = sm_rows(probs, nprob);
+    if(r.most <= 32) return true;
     if(mode == GEMM_NN){
-        tiles *= N / SM_COLS;
-        if(tiles <= 256) return (tiles <= 128 && K > 512) || K >= N || (most <= 64 && K > 1024);
+        const long long tiles = r.t64 * (N / SM_COLS);
+        if(sm_low(r.t32, r.t128, N / SM_COLS)) return true;
+        if(tiles <= 256) return K >= N || (r.most <= 64 && K > 1024);
         if(tiles <= 512 && K >= 4 * N) return true;
-        return K > 1024 && rows <= busy * (K >= N ? most <= 64 ? 48LL : 32 : most <= 64 ? 24 : 0);
+        return K > 1024 && K >= N && r.most <= 64 && r.rows <= 48 * r.busy;
     }
-    tiles *= N / SM_TCOLS;
+    const long long tiles = r.t64 * (N / SM_TCOLS);
     return tiles <= 512 || (tiles <= 1024 && (long long)K * nseg >= 2 * N);
 }
 
@@ -312,11 +327,6 @@ __global__ void __launch_bounds__(64 * SM_WAVES, 2) k_gemm_tn_small(SmArgs a){
 }
 
 /* ---- launches ---- */
-static int sm_row_tiles(const qlmx_gemm_prob *probs, int nprob){
-    int most = 0;
-    for(int i = 0; i < nprob; i++) if(probs[i].M > most) most = probs[i].M;
-    return most > 32 ? 4 : most > 16 ? 2 : 1;
-}
 /* Shape of the forward of at most 32 rows per problem. Eight wavefronts along the contraction change the order of the sums, so that line looks at what the
  * forms of a call have in common; the width of a strip does not, and looks at the form too. See the head of this file. */
 enum { SM_NARROW = 0, SM_WIDE = 1, SM_EIGHT = 2 };
@@ -329,16 +339,22 @@ static int sm_few_shape(const qlmx_gemm_prob *probs, int nprob, int K, int N, in
     if(rt == 2) return wide >= 160 && wide <= 256 && N % 2048 == 0 ? SM_WIDE : SM_NARROW;
     return wide >= 176 && (wide <= 256 || wide >= 352) ? SM_WIDE : SM_NARROW;
 }
-/* Height of the row tiles of a call with more than 32 rows to a problem: 64, which share the weights' conversion or loads; 32 where these are at most one to a CU
- * and the contraction is long enough for a workgroup's loop to be what takes the time. The order of a sum is the same in both. us, 32 : 64 rows: forward, 8 experts of 125, 1536 x 512,
- * 11.9:15.1, of 100, 1408 x 1024, 11.6:15.2, 16 of 64, 2048 x 768 16.5:20.8, one of 500 14.5:18.1; more than one to a CU, 8 of 250, 1536 x 512, 18.0:15.9; gate|up the
- * same within 4 % (not taken). Paired input gradient 8 of 125, 1536 x 512, 11.6:14.5, of 64, 2048 x 768 14:18.1; more than one to a CU 16 of 64, 1536 x 768 19.5:16.2, 32
- * of 64, 2048 x 1024 47:40; short, 8 of 64, 512 x 512, 7.5:6.5. */
-static int sm_tile_rows(const qlmx_gemm_prob *probs, int nprob, int contraction, int strips){
-    const int rt = sm_row_tiles(probs, nprob);
-    long long tiles = 0;
-    for(int i = 0; i < nprob; i++) tiles += (probs[i].M + 31) / 32 * strips;
-    return rt == 4 && tiles <= qlmx_cu_count() && contraction >= 1024 ? 2 : rt;
+/* Height, in sixteens, of the row tiles of a call with more than 32 rows to a problem: 64 rows share the weights' conversion or loads, 32 are less padding and more
+ * workgroups. The order of a sum is the same in both, so the forms of a call need not agree on it. us, 32 : 64 rows:
+ *   forward: 32 where these are at most one to a CU, or beyond that not many more than the tiles of 64 (sm_low): 8 problems of 125, 1536 x 512, 11.9:15.1, 16 of 64, 2048 x 768
+ *     16.5:20.8, 107 rows of 16, largest 41, 896 x 1920 8.4:10.9, 1040 of 64, largest 245, 1920 x 1152 33.5:46.3; on the other side 16, largest 555, 1920 x 896, 20.5:18.4, 64 of 31, 1024 x 384, 13.0:11.6;
+ *   gate|up: also 64 where there are at most 128 of 32, whose strips would leave half the CUs idle (those of 64 rows are half as wide): 8 of 11, 896 x 256, 11.8:10.7, 32 of 9,
+ *     1152 x 384, 13.8:12.8; but 16 of 23, 1792 x 1024, 22.7:28.9, and 1040 of 64, 1920 x 1152, 56:78;
+ *   input gradient: 32 where at most one to a CU and the contraction is long enough for a workgroup's loop to be what takes the time: paired, 8 of 125, 1536 x 512, 11.6:14.5, of 64, 2048 x 768
+ *     14:18.1; more than one to a CU 16 of 64, 1536 x 768 19.5:16.2, 32 of 64, 2048 x 1024 47:40; short, 8 of 64, 512 x 512, 7.5:6.5. */
+static int sm_few_height(const SmRows &r){ return r.most > 16 ? 2 : 1; }
+static int sm_nn_height(const SmRows &r, int strips, bool dual){
+    if(r.most <= 32) return sm_few_height(r);
+    return sm_low(r.t32, r.t64, strips) && !(dual && r.t32 * strips <= 128) ? 2 : 4;
+}
+static int sm_tn_height(const SmRows &r, long long contraction, int strips){
+    if(r.most <= 32) return sm_few_height(r);
+    return r.t32 * strips <= qlmx_cu_count() && contraction >= 1024 ? 2 : 4;
 }
 bool qlmx_pair_open(hipStream_t st);
 int qlmx_pair_hold_tn_few(const SmArgs &a, int io, int slot, hipStream_t st, bool *held);
@@ -353,9 +369,10 @@ static SmArgs sm_args(const signed char *d, const float *s, int group, int K, in
 /* N % 128 == 0, K % 32 == 0, group a power of two >= 64; io, xsrc, out, gate as in qlmx_gemm_nn_h_launch */
 int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, int nprob, int K, int N,
                               int io, const void *xsrc, float *out, const float *gate, hipStream_t st){
-    const int high = sm_row_tiles(probs, nprob), rt = sm_tile_rows(probs, nprob, K, N / SM_COLS);
+    const SmRows rows = sm_rows(probs, nprob);
+    const int rt = sm_nn_height(rows, N / SM_COLS, false);
     ProbUpload up; int slot;
-    const int shape = high <= 2 ? sm_few_shape(probs, nprob, K, N, group, false, rt) : SM_NARROW;
+    const int shape = rows.most <= 32 ? sm_few_shape(probs, nprob, K, N, group, false, rt) : SM_NARROW;
     int rc = qlmx_upload_problems(probs, nprob, GEMM_NN, K, N, rt * 16, shape == SM_WIDE ? 2 * SM_COLS : SM_COLS, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
@@ -372,9 +389,10 @@ int qlmx_gemm_nn_small_launch(const signed char *d, const float *s, int group, c
 /* gate|up with the SwiGLU behind; N % 128 == 0 */
 int qlmx_gemm_nn_small_swiglu_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *gate, const qlmx_gemm_prob *up_, int nprob,
                                      int K, int N, const void *xsrc, hipStream_t st){
-    const int rt = sm_row_tiles(gate, nprob);
+    const SmRows rows = sm_rows(gate, nprob);
+    const int rt = sm_nn_height(rows, N / SM_COLS, true);
     ProbUpload up; int slot;
-    const int shape = rt <= 2 ? sm_few_shape(gate, nprob, K, N, group, true, rt) : SM_NARROW;
+    const int shape = rows.most <= 32 ? sm_few_shape(gate, nprob, K, N, group, true, rt) : SM_NARROW;
     int rc = qlmx_upload_problem_pairs(gate, up_, nprob, GEMM_NN, K, N, rt * 16, rt == 4 ? SM_COLS / 2 : shape == SM_WIDE ? 2 * SM_COLS : SM_COLS, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
@@ -407,7 +425,7 @@ int qlmx_gemm_tn_small_launch(const signed char *d, const float *s, int group, c
     /* one grid with a weight gradient: tiles of 32 rows, two workgroups to a CU, as that kernel's */
     const bool pair = qlmx_pair_open(st);
     if(!pair){ const int rc = qlmx_pair_flush(); if(rc) return rc; }
-    const int rt = pair ? 2 : sm_tile_rows(probs, nprob, K * (second ? 2 : 1), N / SM_TCOLS);
+    const int rt = pair ? 2 : sm_tn_height(sm_rows(probs, nprob), (long long)K * (second ? 2 : 1), N / SM_TCOLS);
     ProbUpload up; int slot;
     int rc = second ? qlmx_upload_problem_pairs(probs, second, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot)
                     : qlmx_upload_problems(probs, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot);

@@ -487,7 +487,11 @@ def test_mfma_few_tiles(q, orc, K, N, group, rows):
 @pytest.mark.parametrize("K,N,rows", [(576, 1024, [100, 896]), (576, 1024, [129, 896]), (512, 1024, [100, 896]),     # 128 strips of 64 x 128, and over
                                       (1152, 1152, [33] + [20] * 40), (1152, 1152, [65] + [40] * 40),        # 41 of 9: few rows to a problem, and more
                                       (1152, 1280, [50] + [23] * 40), (1152, 1280, [65] + [23] * 40),
-                                      (1024, 256, [1000] * 11), (1024, 256, [1000] * 17)])                   # four times the width, up to 512 strips
+                                      (1024, 256, [1000] * 11), (1024, 256, [1000] * 17),                    # four times the width, up to 512 strips
+                                      (64, 1024, [33] * 16), (64, 1024, [33] * 17), (64, 2048, [40] + [9] * 14), (64, 2048, [40] + [9] * 15),     # 32 rows x 128: 256, and over
+                                      (96, 1408, [97] + [7] * 27), (96, 1408, [97] + [7] * 28), (64, 2816, [65, 33] + [32] * 13),     # to 352 and over, more or less of them than taller ones
+                                      (64, 1408, [300, 0, 64] + [1, 31, 33] * 11), (64, 1408, [33] * 64),
+                                      (96, 128, [33] + [5] * 40), (96, 256, [70] + [5] * 61), (96, 256, [70] + [5] * 62)])     # gate|up on 64 rows, up to 128 of 32; on 32
 def test_f16_forward_on_both_sides_of_the_lines(q, orc, K, N, rows):
     """The sizes of a call choose between the kernels for few rows and the tiled ones; on either side of each line the SwiGLU call
     gives the bits of the separate ones, and both the oracle's values."""
