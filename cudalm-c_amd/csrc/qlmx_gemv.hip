@@ -1301,7 +1301,9 @@ static int df_reserve(DfSpace &ws, int which, size_t words, hipStream_t st){
  * 128 rows, 192 tasks) and many tokens on few experts. More, shorter slices cost the down tasks a second round trip for
  * their sums: measured at E=32 D=768 F=2048 top-2, when one token took this kernel, rows 256 / 128 / 64 gave 16.3 / 15.6 / 18.2 us per layer for
  * it, 18.8 / 21.4 / 26.4 for four, 29.7 / 32.7 / 42.0 for sixteen. The number of problems is only known on the
- * device; the host uses the expected number of distinct experts hit by `npair` uniform picks out of E. */
+ * device; the host uses what `npair` uniform picks out of E make on average: of an expert's x pairs (x + 1) / 2 problems, rounded down. (Counted as
+ * one problem to an expert that is hit, many tokens on few experts had slices a half or a quarter as long: 8 experts top-2, 16 tokens, 512 x 640
+ * 19.4 -> 16.4 us per layer, 12 tokens, 640 x 768 19.1 -> 16.5, 31 tokens, 640 x 512 22.6 -> 20.6.) */
 static int df_rows(int Kdim, double tasks_per_slice, int grid){
     int R = DF_RMAX;
     while(R > 64 && tasks_per_slice * ((Kdim + R - 1) / R) < 0.15 * grid) R >>= 1;
@@ -1367,8 +1369,8 @@ static int df_forward(bool fixed, const char *who, const float *x, const int *as
     a.w1g = w1q / group; a.w3g = w3q / group; a.w2g = w2q / group; a.dfg = (u64)D * F / group;
     a.T = T; a.K = K; a.E = E; a.D = D; a.F = F;
     a.NC1 = (F + DF_CW - 1) / DF_CW; a.NC2 = (D + DF_CW - 1) / DF_CW;
-    const double hits = E * (1.0 - pow(1.0 - 1.0 / E, (double)npair));
-    a.R2 = df_rows_down(F, hits * a.NC2, dv.grid);   a.S2 = (F + a.R2 - 1) / a.R2;
+    const double problems = 0.5 * npair + 0.25 * E * (1.0 - pow(1.0 - 2.0 / E, (double)npair));
+    a.R2 = df_rows_down(F, problems * a.NC2, dv.grid);   a.S2 = (F + a.R2 - 1) / a.R2;
     a.R1 = DF_RMAX; a.S1 = (D + a.R1 - 1) / a.R1;
     /* k_decode_few takes a workgroup per task, all resident at once, with 256 rows to a task of list 1 whatever their number. Up to 5/8 of the
      * workgroups that fit it is the faster one, by a microsecond to seven, beyond it the same or slower (a pair is a problem there: experts that
@@ -1379,7 +1381,7 @@ static int df_forward(bool fixed, const char *who, const float *x, const int *as
     const long long n1 = 2LL * npair * a.NC1 * a.S1, n2 = (long long)npair * a.NC2 * a.S2, n3 = (long long)T * a.NC2;
     const long long few_grid = 8 * ((n1 + 7) / 8 + (n2 + 7) / 8 + (n3 + 7) / 8);
     const bool few = !df_math_fp16() && few_grid <= dv.grid * 5 / 8;
-    if(!few){ a.R1 = df_rows(D, 2.0 * hits * a.NC1, dv.grid); a.S1 = (D + a.R1 - 1) / a.R1; }
+    if(!few){ a.R1 = df_rows(D, 2.0 * problems * a.NC1, dv.grid); a.S1 = (D + a.R1 - 1) / a.R1; }
     const size_t words1 = (size_t)npair * 2 * a.S1 * DF_MB * F, words2 = (size_t)npair * a.S2 * DF_MB * D;
     if(fixed){
         if((words1 + words2) * sizeof(u64) > (size_t)QLMX_DECODE_SCRATCH_BYTES){
