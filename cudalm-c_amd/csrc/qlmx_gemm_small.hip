@@ -22,9 +22,10 @@
  * some experts has a few problems of a hundred rows beside many of five, each a tile of 128 there and of 32 here. The forward's rule looks at what the
  * forms of a call that are documented to agree bit for bit have in common -- with and without gather, SwiGLU, scatter -- so that they run the same
  * arithmetic in the same order. us for the plain and the SwiGLU call, these : tiled --
- *   tiles of 32 rows x 128 columns up to 256, one to a CU. 16 problems, largest 43 rows, 896 x 1152 8.3:13.6, 1152 x 896 14.6:19.0; 8, largest 69,
- *     384 x 1152 6.0:8.3 and 8.6:9.0; one of 292, 1024 x 1920 9.8:11.9 and 13.5:13.1;
- *   beyond, tiles of 32 rows at most 1.5 times the 128-row tiles; up to 352 of them 1.125 times (a second round that is nearly empty). Zipf shares: 1096 rows of 64, 896 x 512
+ *   contractions over 512, tiles of 32 rows x 128 columns up to 256, one to a CU. 16 problems, largest 43 rows, 896 x 1152 8.3:13.6, 1152 x 896 14.6:19.0; 8 of 49,
+ *     768 x 896 8.3:11.9, 896 x 768 12.2:13.8. Shorter ones, whose SwiGLU call gains little (8 of 104, 384 x 384 6.0:7.7 and 8.3:8.6; 8 of 21, 384 x 1152 6.0:8.3 and 8.6:9.0), stay
+ *     with the tiled kernel, which also takes a small layer's passes merged into one list: the same bits either way;
+ *   tiles of 32 rows at most 1.5 times the 128-row tiles; from 257 to 352 of them 1.125 times (a second round that is nearly empty). Zipf shares: 1096 rows of 64, 896 x 512
  *     12.5:18.0, 512 x 896 22:24; 617 of 64, 1664 x 1920 41:60, 1920 x 1664 62:109; 362 of 32, 2304 x 896 18:31, 896 x 2304 32:50. On the other side 4832 of 64,
  *     1536 x 768 41:33, 768 x 1536 77:70; and with 330 tiles, 16 of 31 rows, 1024 x 1920 14:16 and 26:20;
  *   strips of 64 x 128 up to 256, where the contraction is not shorter than the width, or over 1024 with no problem of more than 64 rows: the plain
@@ -33,8 +34,8 @@
  *     sizes. 2304 x 512, 64 of 77 39:43 (a SwiGLU call 79:59, as at twice the width: 2048 x 768, 32 of 100 30:26 and 56:38).
  *   beyond, contractions over 1024 and not shorter than the width, of at most 64 rows to a problem and 48 on average, which the tiled kernel pads to 128: 2048 x 1664,
  *     64 of 41 59:63 and 102:116, 2048 x 768, 64 of 40 31:33 and 57:68; on the other side 64 of 64 56:63 and 121:103.
- * Over 160 calls of 1 to 64 problems of 5 to 400 rows on average, in even and in Zipf shares, 256 to 2048 in and out, a plain call takes 0.86 and a SwiGLU call 0.96 of what they took
- * when the rule counted strips of 64 rows only and problems of over 32 rows had tiles of 64 (mean of the ratios; over half of the calls are as they were).
+ * Over 160 calls of 1 to 64 problems of 5 to 400 rows on average, in even and in Zipf shares, 256 to 2048 in and out, a plain call takes 0.88 and a SwiGLU call 0.96 of what they took
+ * when the rule counted strips of 64 rows only and problems of over 32 rows had tiles of 64 (mean of the ratios; 68 of the calls are as they were).
  * The lines look at a call's own sizes, so a layer whose passes run one by one may take the one path and its merged list the other: bits that
  * agree between the two are not promised and not looked for here.
  * Input gradient, strips of 64 x 64: up to 512, 1024 where the contraction is twice the width.
@@ -81,10 +82,10 @@ static SmRows sm_rows(const qlmx_gemm_prob *probs, int nprob){
     }
     return r;
 }
-/* tiles of 32 rows against `high` taller ones, on so many strips: at most one to a CU, or not many more of them; see the head of this file */
+/* tiles of 32 rows on so many strips, against `high` taller ones: not many more of them, by a line that depends on whether they come in two rounds; see the head of this file */
 static bool sm_low(long long t32, long long high, int strips){
     const long long tiles = t32 * strips;
-    return tiles <= 256 || (tiles <= 352 ? 8 * t32 <= 9 * high : 2 * t32 <= 3 * high);
+    return tiles > 256 && tiles <= 352 ? 8 * t32 <= 9 * high : 2 * t32 <= 3 * high;
 }
 /* see the head of this file */
 bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, int N, int nseg, int group){
@@ -93,7 +94,7 @@ bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, in
     if(r.most <= 32) return true;
     if(mode == GEMM_NN){
         const long long tiles = r.t64 * (N / SM_COLS);
-        if(sm_low(r.t32, r.t128, N / SM_COLS)) return true;
+        if((K > 512 && r.t32 * (N / SM_COLS) <= 256) || sm_low(r.t32, r.t128, N / SM_COLS)) return true;
         if(tiles <= 256) return K >= N || (r.most <= 64 && K > 1024);
         if(tiles <= 512 && K >= 4 * N) return true;
         return K > 1024 && K >= N && r.most <= 64 && r.rows <= 48 * r.busy;
@@ -350,7 +351,8 @@ static int sm_few_shape(const qlmx_gemm_prob *probs, int nprob, int K, int N, in
 static int sm_few_height(const SmRows &r){ return r.most > 16 ? 2 : 1; }
 static int sm_nn_height(const SmRows &r, int strips, bool dual){
     if(r.most <= 32) return sm_few_height(r);
-    return sm_low(r.t32, r.t64, strips) && !(dual && r.t32 * strips <= 128) ? 2 : 4;
+    const long long tiles = r.t32 * strips;
+    return tiles <= 256 ? (dual && tiles <= 128 ? 4 : 2) : sm_low(r.t32, r.t64, strips) ? 2 : 4;
 }
 static int sm_tn_height(const SmRows &r, long long contraction, int strips){
     if(r.most <= 32) return sm_few_height(r);

@@ -488,7 +488,7 @@ def test_mfma_few_tiles(q, orc, K, N, group, rows):
                                       (1152, 1152, [33] + [20] * 40), (1152, 1152, [65] + [40] * 40),        # 41 of 9: few rows to a problem, and more
                                       (1152, 1280, [50] + [23] * 40), (1152, 1280, [65] + [23] * 40),
                                       (1024, 256, [1000] * 11), (1024, 256, [1000] * 17),                    # four times the width, up to 512 strips
-                                      (64, 1024, [33] * 16), (64, 1024, [33] * 17), (64, 2048, [40] + [9] * 14), (64, 2048, [40] + [9] * 15),     # 32 rows x 128: 256, and over
+                                      (544, 1024, [33] * 16), (544, 1024, [33] * 17), (512, 1024, [33] * 16),                 # 32 rows x 128: 256 of them, and over
                                       (96, 1408, [97] + [7] * 27), (96, 1408, [97] + [7] * 28), (64, 2816, [65, 33] + [32] * 13),     # to 352 and over, more or less of them than taller ones
                                       (64, 1408, [300, 0, 64] + [1, 31, 33] * 11), (64, 1408, [33] * 64),
                                       (96, 128, [33] + [5] * 40), (96, 256, [70] + [5] * 61), (96, 256, [70] + [5] * 62)])     # gate|up on 64 rows, up to 128 of 32; on 32
