@@ -400,9 +400,12 @@ def test_mfma_few_rows(q, orc, mode, K, N, group, rows):
                                             (64, 1408, [31, 5, 16, 17] * 9, 128),             # wide, gate|up on strips of 128
                                             (64, 1152, [20, 0] * 35, 128), (64, 1152, [7] * 36, 128), (64, 1152, [7] * 35, 128),     # either side of the line for wide strips
                                             (2048, 384, [16, 1, 0, 7], 128), (2048, 512, [32, 17, 9], 256), (2080, 128, [5], 128),     # eight wavefronts along the contraction
-                                            (2048, 1152, [32, 17, 9], 128)])
+                                            (2048, 1152, [32, 17, 9], 128),
+                                            (160, 384, [70, 5, 0, 33, 9, 9, 2], 128), (576, 384, [129, 64, 1], 64),               # larger problems on 32 rows, gate|up on 64
+                                            (96, 256, [70, 3] + [5] * 70, 128), (544, 1152, [97, 34, 0, 31] * 4, 64),    # both on 32
+                                            (1056, 896, [64, 40, 34] * 16, 128)])                                        # both on 64
 def test_f16_forward_of_few_rows_in_every_form(q, K, N, rows, group):
-    """The shapes of the forward of at most 32 rows per problem: products with the weights rounded once to fp16, within what K fp32 additions
+    """The shapes of the forward of few rows, at most 32 per problem and more: products with the weights rounded once to fp16, within what K fp32 additions
     in some order differ from 64 bits by (sqrt(K) * 2^-24 relative to the sums, four times that for their cancelling), and the same bits with the row moves and the SwiGLU
     folded in."""
     import torch
