@@ -43,10 +43,12 @@ static int q4n_parts(size_t n, size_t ngroups, int group, size_t part){ return (
 
 /* Threads for the calls' parts: started as calls ask for them, at most seven whatever the number of callers, and gone after a second without work. A call
  * takes part in its own job and needs none of them; several calls at once share them. A job is on its caller's stack: the caller leaves when its
- * parts are done and no thread has hold of it any more. The crew itself is never destroyed, so threads asleep at exit touch nothing that is; a
+ * parts are done and no thread has hold of it any more. A thread works on a job in its caller's floating-point mode (rounding, small values flushed to
+ * zero or not): a new thread has that of whoever started it, which here is some earlier caller. The crew itself is never destroyed, so threads asleep at exit touch nothing that is; a
  * child of fork() has none of the threads and starts with a crew of its own. */
 struct Q4nJob {
     const std::function<void(int)> *phase[2]; int parts;
+    const unsigned mode = _mm_getcsr() & ~(unsigned)_MM_EXCEPT_MASK;
     std::atomic<int> next[2], done[2];
     int holders; Q4nJob *link;                             /* both under the crew's lock */
     Q4nJob() : parts(0), holders(0), link(nullptr) { for(int i = 0; i < 2; i++){ phase[i] = nullptr; next[i] = 0; done[i] = 0; } }
@@ -86,7 +88,10 @@ struct Q4nCrew {
             }
             j->holders++;
             l.unlock();
+            const unsigned own = _mm_getcsr();
+            _mm_setcsr(j->mode);
             j->work();
+            _mm_setcsr(own);
             l.lock();
             if(--j->holders == 0) left.notify_all();
         }
@@ -169,7 +174,7 @@ __attribute__((target("avx2"))) static float amax_avx2(const float *v, int g){
     const float amax = _mm_cvtss_f32(_mm_max_ss(t, _mm_shuffle_ps(t, t, 1)));
     return amax_from(v, j, g, amax);
 }
-/* A group against one of its candidates amax / k, in the range that q4n_mid names: whether every value is a digit times the scale, with a reciprocal for the division. The
+/* A group against one of its candidates amax / k, in the range and the direction of rounding that q4n_mid names: whether every value is a digit times the scale, with a reciprocal for the division. The
  * answer is that of try_from. A digit d passes there when |d| <= 7 and the rounded product d * scale is v. Then v is d * scale within 2^-24 of itself, and v * (1/scale), two
  * roundings further, d within 2^-22 of itself: it rounds to the same d. The other way round, a digit that passes here has v = rounded d * scale, so that
  * v / scale rounds to it too; and it is at most 7, as no value is more than amax and no candidate less than amax / 7 by more than two units in its last place. */
@@ -260,8 +265,10 @@ __attribute__((target("avx2"))) static unsigned maybe_scales(const float *v, int
     for(int k = 7; k >= 1; k--) m |= (unsigned)maybe_avx2(share, k) << k;
     return m;
 }
-/* largest magnitudes, and scales, whose quotients and products neither overflow nor lose bits */
-static bool q4n_mid(float x){ return q4n_avx2() && x >= 0x1p-90f && x <= 0x1p90f; }
+/* the callers that round to nearest, as the bounds of fits_avx2 and maybe_scales have it; asked once per part */
+static bool q4n_nearest(){ return q4n_avx2() && _MM_GET_ROUNDING_MODE() == _MM_ROUND_NEAREST; }
+/* and largest magnitudes, and scales, whose quotients and products neither overflow nor lose bits */
+static bool q4n_mid(float x, bool nearest){ return nearest && x >= 0x1p-90f && x <= 0x1p90f; }
 static float group_amax(const float *v, int g){ return q4n_avx2() ? amax_avx2(v, g) : amax_from(v, 0, g, 0.0f); }
 static bool group_try(const float *v, int g, float scale, signed char *digit){ return q4n_avx2() ? try_avx2(v, g, scale, digit) : try_from(v, 0, g, scale, digit); }
 static void group_pack(const signed char *digit, int g, unsigned char *b){ if(q4n_avx2()) pack_avx2(digit, g, b); else pack_from(digit, 0, g, b); }
@@ -271,10 +278,10 @@ static void group_unpack(const unsigned char *b, int g, float scale, float *P){ 
 static inline float toward_zero(float x){ unsigned u; memcpy(&u, &x, 4); if(u) u--; memcpy(&x, &u, 4); return x; }
 static inline float toward_inf(float x){ unsigned u; memcpy(&u, &x, 4); if(u != 0x7F800000u) u++; memcpy(&x, &u, 4); return x; }
 /* the group's scale, the first candidate that fits (0 for a group of zeros), or NaN for a group that is kept raw */
-static float group_scale(const float *v, int g, signed char *digit){
+static float group_scale(const float *v, int g, bool nearest, signed char *digit){
     const float amax = group_amax(v, g);
     if(amax == 0.0f) return 0.0f;
-    const bool mid = q4n_mid(amax);
+    const bool mid = q4n_mid(amax, nearest);
     const unsigned worth = mid ? maybe_scales(v, g, amax) : 0xFEu;
     for(int k = 7; k >= 1; k--){
         if(!(worth >> k & 1)) continue;
@@ -302,16 +309,18 @@ static int q4n_write(const float *P, size_t n, int group, unsigned char *out, si
     auto size_of = [&](size_t q){ return (int)std::min((size_t)group, n - q * (size_t)group); };
     const std::function<void(int)> find = [&](int p){
         signed char *digit = digits.data() + (size_t)p * stride;
+        const bool nearest = q4n_nearest();
         size_t l = 0, r = 0;
         for(size_t q = begin(p); q < begin(p + 1); q++){
             const int g = size_of(q);
-            const float s = group_scale(P + q * (size_t)group, g, digit);
+            const float s = group_scale(P + q * (size_t)group, g, nearest, digit);
             scales[q] = s;
             if(s != s){ l += 4 + 4 * (size_t)g; r++; } else l += 4 + (size_t)(g + 1) / 2;
         }
         len[p] = l; raw[p] = r;
     }, put = [&](int p){
         signed char *digit = digits.data() + (size_t)p * stride;
+        const bool nearest = q4n_nearest();
         unsigned char *o = out;
         for(int i = 0; i < p; i++) o += len[i];
         for(size_t q = begin(p); q < begin(p + 1); q++){
@@ -320,7 +329,7 @@ static int q4n_write(const float *P, size_t n, int group, unsigned char *out, si
             const float s = scales[q];
             memcpy(o, &s, 4); o += 4;
             if(s != s){ memcpy(o, v, 4 * (size_t)g); o += 4 * (size_t)g; continue; }
-            if(q4n_mid(s)) put_avx2(v, g, s, o);
+            if(q4n_mid(s, nearest)) put_avx2(v, g, s, o);
             else {
                 if(s == 0.0f) memset(digit, 0, (size_t)g); else group_try(v, g, s, digit);
                 digit[g] = 0;                              /* the partner of an odd group's last digit */

@@ -151,6 +151,59 @@ def test_callers_share_the_threads_and_a_child_has_its_own(lib):
     assert os.waitstatus_to_exitcode(os.waitpid(child, 0)[1]) == 0
 
 
+MODES = ("default", "flush", "up", "down", "zero")
+MODE_CODE = """
+import ctypes, threading
+libm = ctypes.CDLL("libm.so.6")
+def mode(name):            # of the calling thread: flush-to-zero with denormals-are-zero, or a direction of rounding
+    env = (ctypes.c_uint32 * 8)()
+    libm.fegetenv(env)
+    env[7] = env[7] & ~0xE040 | {"default": 0, "flush": 0x8040, "up": 0x4000, "down": 0x2000, "zero": 0x6000}[name]
+    libm.fesetenv(env)
+def threaded(f, *args):
+    t = threading.Thread(target=f, args=args); t.start(); t.join()
+"""
+
+
+@pytest.mark.parametrize("first", MODES)
+def test_a_caller_has_its_own_floating_point_mode_and_no_other(first):
+    """A caller that rounds otherwise or flushes small values to zero, and right behind it callers in every mode: each gets what one thread in its mode gives, on the
+    threads that the first has left too. In the default mode that is every value, bit for bit, subnormal ones among them."""
+    code = MODE_CODE + """
+import numpy as np
+from __graft_entry__ import load_package
+from oracle.binding import Oracle
+lib, orc, f32 = load_package().Qlmx(init=False), Oracle(), np.float32
+rng = np.random.default_rng(3)
+P = rng.integers(-7, 8, 1200000).astype(f32).reshape(-1, 100)
+P[:, 0] = 7
+P *= (0.01 + 0.01 * rng.random((len(P), 1))).astype(f32)
+P[1::5] = rng.integers(-7, 8, P[1::5].shape) * f32(2.0 ** -140)
+P[2::5] = rng.normal(size=P[2::5].shape)
+P[3::5] *= f32(2.0 ** -100)
+P[4::5, ::9] = f32(2.0 ** -145)          # beside values that are not small
+P = np.ascontiguousarray(P.reshape(-1))
+def check(name):
+    mode(name)
+    got, raw = lib.q4n_quantize(P, 100)
+    want, wraw = orc.q4n_quantize(P, 100)
+    back, used = lib.q4n_dequantize(want, P.size, 100)
+    ok, wback = orc.q4n_dequantize(want, P.size, 100)
+    mode("default")
+    assert ok == 1 and used == want.size and raw == wraw and np.array_equal(got, want), name
+    assert np.array_equal(back.view(np.uint32), wback.view(np.uint32)), name
+    if name == "default":
+        assert np.array_equal(back + f32(0), P + f32(0))
+    done.append(name)
+done = []
+for name in (%r,) + %r:
+    threaded(check, name)
+assert len(done) == 6, done
+""" % (first, MODES)
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_truncated_buffer_is_refused(lib, orc, golden):
     g = golden("q4n")
     n, group = (int(v) for v in g["dims"])
