@@ -15,6 +15,7 @@
 #include <immintrin.h>
 #include <math.h>
 #include <string.h>
+#include <sched.h>
 #include <signal.h>
 #include <unistd.h>
 #include <algorithm>
@@ -44,11 +45,13 @@ static int q4n_parts(size_t n, size_t ngroups, int group, size_t part){ return (
 /* Threads for the calls' parts: started as calls ask for them, at most seven whatever the number of callers, and gone after a second without work. A call
  * takes part in its own job and needs none of them; several calls at once share them. A job is on its caller's stack: the caller leaves when its
  * parts are done and no thread has hold of it any more. A thread works on a job in its caller's floating-point mode (rounding, small values flushed to
- * zero or not): a new thread has that of whoever started it, which here is some earlier caller. The crew itself is never destroyed, so threads asleep at exit touch nothing that is; a
+ * zero or not) and on the CPUs that the caller may run on: a new thread has those of whoever started it, which here is some earlier caller (4 M values written behind a
+ * call bound to one CPU, 8 CPUs, us: on the CPU of that call 1600-2000, with this 580-630, as behind any other). The crew itself is never destroyed, so threads asleep at exit touch nothing that is; a
  * child of fork() has none of the threads and starts with a crew of its own. */
 struct Q4nJob {
     const std::function<void(int)> *phase[2]; int parts;
     const unsigned mode = _mm_getcsr() & ~(unsigned)_MM_EXCEPT_MASK;
+    cpu_set_t cpus; const bool placed = sched_getaffinity(0, sizeof cpus, &cpus) == 0;      /* false: more CPUs than the set has room for */
     std::atomic<int> next[2], done[2];
     int holders; Q4nJob *link;                             /* both under the crew's lock */
     Q4nJob() : parts(0), holders(0), link(nullptr) { for(int i = 0; i < 2; i++){ phase[i] = nullptr; next[i] = 0; done[i] = 0; } }
@@ -72,6 +75,7 @@ struct Q4nCrew {
     void member(){
         sigset_t all;                                      /* signals are for the program's own threads */
         sigfillset(&all); pthread_sigmask(SIG_BLOCK, &all, nullptr);
+        cpu_set_t cpus; CPU_ZERO(&cpus);
         std::unique_lock<std::mutex> l(lock);
         for(;;){
             Q4nJob *j = jobs;
@@ -88,6 +92,7 @@ struct Q4nCrew {
             }
             j->holders++;
             l.unlock();
+            if(j->placed && !CPU_EQUAL(&cpus, &j->cpus) && sched_setaffinity(0, sizeof cpus, &j->cpus) == 0) cpus = j->cpus;
             const unsigned own = _mm_getcsr();
             _mm_setcsr(j->mode);
             j->work();

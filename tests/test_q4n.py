@@ -204,6 +204,46 @@ assert len(done) == 6, done
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+CREW_CODE = MODE_CODE + """
+import numpy as np, os, time
+from __graft_entry__ import load_package
+lib, f32 = load_package().Qlmx(init=False), np.float32
+P = (np.arange(1200000) % 15 - 7).astype(f32) * f32(0.25)
+wire = lib.q4n_quantize(P[:1280], 128)[0]
+own = set(os.listdir("/proc/self/task"))        # before any thread of the library
+def call(): assert lib.q4n_quantize(P, 128)[1] == 0
+def crew(): return sorted(int(t) for t in set(os.listdir("/proc/self/task")) - own)
+def ran(t): return int(open("/proc/self/task/%d/schedstat" % t).read().split()[0])
+"""
+
+
+@pytest.mark.skipif(len(os.sched_getaffinity(0)) < 4, reason="needs four CPUs")
+def test_kept_threads_run_where_their_caller_may():
+    """A caller bound to two CPUs starts the threads; those that work for the next caller, which is not bound, are not bound either, and the bound caller's are again."""
+    code = CREW_CODE + """
+everywhere = os.sched_getaffinity(0)
+two = set(sorted(everywhere)[:2])
+def bound():
+    os.sched_setaffinity(0, two)
+    for i in range(5): call()
+    own.discard(str(threading.get_native_id()))
+threaded(bound)
+for want, many in ((everywhere, 20), (two, 20)):
+    os.sched_setaffinity(0, want)
+    worked, wrong = set(), set()
+    for i in range(many):
+        before = {t: ran(t) for t in crew()}
+        call()
+        for t in crew():
+            if ran(t) - before.get(t, 0) > 100000:          # more than to wake and find nothing left
+                worked.add(t)
+                if os.sched_getaffinity(t) != want: wrong.add(t)
+    assert worked and not wrong, (want, worked, wrong)
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_truncated_buffer_is_refused(lib, orc, golden):
     g = golden("q4n")
     n, group = (int(v) for v in g["dims"])
