@@ -17,6 +17,7 @@
 #include <string.h>
 #include <sched.h>
 #include <signal.h>
+#include <sys/resource.h>
 #include <unistd.h>
 #include <algorithm>
 #include <atomic>
@@ -46,7 +47,8 @@ static int q4n_parts(size_t n, size_t ngroups, int group, size_t part){ return (
  * takes part in its own job and needs none of them; several calls at once share them. A job is on its caller's stack: the caller leaves when its
  * parts are done and no thread has hold of it any more. A thread works on a job in its caller's floating-point mode (rounding, small values flushed to
  * zero or not) and on the CPUs that the caller may run on: a new thread has those of whoever started it, which here is some earlier caller (4 M values written behind a
- * call bound to one CPU, 8 CPUs, us: on the CPU of that call 1600-2000, with this 580-630, as behind any other). The crew itself is never destroyed, so threads asleep at exit touch nothing that is; a
+ * call bound to one CPU, 8 CPUs, us: on the CPU of that call 1600-2000, with this 580-630, as behind any other). A priority cannot be
+ * given back once lowered, so the threads serve callers of the one that they were started with; a caller of another starts its own for the call. The crew itself is never destroyed, so threads asleep at exit touch nothing that is; a
  * child of fork() has none of the threads and starts with a crew of its own. */
 struct Q4nJob {
     const std::function<void(int)> *phase[2]; int parts;
@@ -67,9 +69,15 @@ struct Q4nJob {
         }
     }
 };
+struct Q4nPriority {                                      /* of the calling thread */
+    int policy = sched_getscheduler(0), level = 0, nice = getpriority(PRIO_PROCESS, 0);
+    Q4nPriority(){ sched_param p; if(sched_getparam(0, &p) == 0) level = p.sched_priority; }
+    bool operator==(const Q4nPriority &o) const { return policy == o.policy && level == o.level && nice == o.nice; }
+};
 struct Q4nCrew {
     std::mutex lock; std::condition_variable wake, left;
     Q4nJob *jobs = nullptr; int threads = 0, idle = 0;
+    Q4nPriority theirs;                                    /* while there are threads */
     const pid_t owner = getpid();
 
     void member(){
@@ -102,9 +110,12 @@ struct Q4nCrew {
         }
         threads--;
     }
-    void run(Q4nJob &j, int wanted){
+    bool run(Q4nJob &j, int wanted){                       /* false: not for this caller */
+        const Q4nPriority mine;
         {
             std::lock_guard<std::mutex> l(lock);
+            if(threads == 0) theirs = mine;
+            else if(!(theirs == mine)) return false;
             j.link = jobs; jobs = &j;
             for(int more = wanted - idle; more > 0 && threads < Q4N_MAX_THREADS - 1; more--){
                 try { std::thread([this]{ member(); }).detach(); threads++; }
@@ -118,6 +129,7 @@ struct Q4nCrew {
         while(*at != &j) at = &(*at)->link;
         *at = j.link;
         while(j.holders) left.wait(l);
+        return true;
     }
 };
 static Q4nCrew *q4n_crew(){
@@ -135,7 +147,14 @@ static void q4n_run(int parts, const std::function<void(int)> &first, const std:
     Q4nJob j;
     j.parts = parts; j.phase[0] = &first; j.phase[1] = second;
     const int wanted = std::min({parts, Q4N_MAX_THREADS, (int)std::thread::hardware_concurrency()}) - 1;
-    if(wanted > 0) q4n_crew()->run(j, wanted); else j.work();
+    if(wanted > 0 && q4n_crew()->run(j, wanted)) return;
+    std::thread own[Q4N_MAX_THREADS];
+    for(int i = 0; i < wanted; i++){
+        try { own[i] = std::thread([&j]{ j.work(); }); }
+        catch(const std::exception &){ break; }
+    }
+    j.work();
+    for(std::thread &t : own) if(t.joinable()) t.join();
 }
 static bool q4n_avx2(){ static const bool yes = __builtin_cpu_supports("avx2"); return yes; }
 

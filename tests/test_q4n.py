@@ -226,7 +226,7 @@ two = set(sorted(everywhere)[:2])
 def bound():
     os.sched_setaffinity(0, two)
     for i in range(5): call()
-    own.discard(str(threading.get_native_id()))
+    own.add(str(threading.get_native_id()))
 threaded(bound)
 for want, many in ((everywhere, 20), (two, 20)):
     os.sched_setaffinity(0, want)
@@ -239,6 +239,35 @@ for want, many in ((everywhere, 20), (two, 20)):
                 worked.add(t)
                 if os.sched_getaffinity(t) != want: wrong.add(t)
     assert worked and not wrong, (want, worked, wrong)
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
+def test_kept_threads_serve_callers_of_their_own_priority():
+    """Threads started by a caller of low priority do nothing for one of ordinary priority, which has threads of its own as long as they are there, and the other
+    way round; once they have gone the next caller's are kept."""
+    code = CREW_CODE + """
+def low():
+    os.setpriority(os.PRIO_PROCESS, 0, 19)
+    for i in range(5): call()
+    own.add(str(threading.get_native_id()))
+def worked(): return [t for t in kept if ran(t) - before[t] > 100000]
+threaded(low)
+kept = crew()
+assert kept and all(os.getpriority(os.PRIO_PROCESS, t) == 19 for t in kept)
+for i in range(10):
+    before = {t: ran(t) for t in kept}
+    call()
+    assert not worked()
+time.sleep(2.5)
+assert not crew()
+call()
+kept = crew()
+assert kept and all(os.getpriority(os.PRIO_PROCESS, t) == 0 for t in kept)
+before = {t: ran(t) for t in kept}
+threaded(low)
+assert not worked()
 """
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr[-2000:]
