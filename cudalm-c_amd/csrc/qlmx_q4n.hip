@@ -81,8 +81,10 @@ struct Q4nCrew {
     const pid_t owner = getpid();
 
     void member(){
-        sigset_t all;                                      /* signals are for the program's own threads */
-        sigfillset(&all); pthread_sigmask(SIG_BLOCK, &all, nullptr);
+        sigset_t sent;                                     /* signals are for the program's own threads, but a fault is the faulting thread's: blocked, it ends the process past any handler */
+        sigfillset(&sent);
+        for(int fault : {SIGSEGV, SIGBUS, SIGFPE, SIGILL, SIGTRAP, SIGSYS}) sigdelset(&sent, fault);
+        pthread_sigmask(SIG_BLOCK, &sent, nullptr);
         cpu_set_t cpus; CPU_ZERO(&cpus);
         std::unique_lock<std::mutex> l(lock);
         for(;;){

@@ -273,6 +273,26 @@ assert not worked()
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+def test_kept_threads_leave_faults_to_the_programs_handlers():
+    """A program may answer a fault on its buffers in a handler (pages mapped or unprotected on first use), and has to be asked on the library's threads as on its own;
+    signals sent to the process are for the program's threads."""
+    code = CREW_CODE + """
+import signal
+call()
+time.sleep(0.2)          # a thread starts with all signals blocked
+assert crew()
+for t in crew():
+    status = dict(line.split(":", 1) for line in open("/proc/self/task/%d/status" % t))
+    blocked = int(status["SigBlk"], 16)
+    for name in ("SIGSEGV", "SIGBUS", "SIGFPE", "SIGILL", "SIGTRAP", "SIGSYS"):
+        assert not blocked >> (getattr(signal, name) - 1) & 1, name
+    for name in ("SIGINT", "SIGTERM", "SIGALRM", "SIGUSR1"):
+        assert blocked >> (getattr(signal, name) - 1) & 1, name
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_truncated_buffer_is_refused(lib, orc, golden):
     g = golden("q4n")
     n, group = (int(v) for v in g["dims"])
