@@ -32,8 +32,9 @@
 
 /* What bounds it: reading the values, twice when writing -- the writer finds the groups' scales first, which says where each part's bytes
  * start, and the digits again behind that -- the first touch of the output's pages, and the reader's walk over the group headers. Whether a group fits a scale is
- * tried eight values at a time where the CPU has AVX2, with one reciprocal for the group instead of a division per value (fits_avx2), and all of it in parts by up
- * to eight threads (sixteen were slower). Seven threads take 80 us to start and 15 to wake, so they are kept (Q4nCrew below).
+ * tried eight values at a time where the CPU has AVX2, with one reciprocal for the group instead of a division per value (fits_avx2), also behind the last whole 32 of a
+ * group: with scalar divisions there, as the remainders of 32 had, 40 K values in groups of 24 took 350 us to write, of 16 384, of 56 175; now 66, 91, 42 (with divisions eight at a time
+ * 87, 116, 67). All of it in parts by up to eight threads (sixteen were slower). Seven threads take 80 us to start and 15 to wake, so they are kept (Q4nCrew below).
  * 4 M values, a tenth of the groups raw, on the 16 CPUs of a GPU's share, us: write and read by one thread with scalar arithmetic 7900 + 990, divisions and threads started in
  * each call 330-500 + 180, as here 160-200 + 95-125; half the groups raw, groups of 64: 560 + 420 -> 290 + 340. */
 #define Q4N_WRITE_PART (48 * 1024)              /* values to a part: several parts a thread, since threads wake one after the other */
@@ -194,6 +195,7 @@ __attribute__((target("avx2"))) static float amax_avx2(const float *v, int g){
         m2 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j + 16), mag), m2);
         m3 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j + 24), mag), m3);
     }
+    for(; j + 8 <= g; j += 8) m1 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(v + j), mag), m1);
     m = _mm256_max_ps(_mm256_max_ps(m, m1), _mm256_max_ps(m2, m3));
     __m128 t = _mm_max_ps(_mm256_castps256_ps128(m), _mm256_extractf128_ps(m, 1));
     t = _mm_max_ps(t, _mm_movehl_ps(t, t));
@@ -207,14 +209,14 @@ __attribute__((target("avx2"))) static float amax_avx2(const float *v, int g){
 __attribute__((target("avx2"))) static bool fits_avx2(const float *v, int g, float scale){
     const __m256 s = _mm256_set1_ps(scale), inv = _mm256_set1_ps(1.0f / scale);
     int j = 0;
-    for(; j + 32 <= g; j += 32){
-        __m256 off = _mm256_setzero_ps();
-        for(int i = 0; i < 32; i += 8){
-            const __m256 x = _mm256_loadu_ps(v + j + i), d = _mm256_round_ps(_mm256_mul_ps(x, inv), _MM_FROUND_CUR_DIRECTION);
-            off = _mm256_or_ps(off, _mm256_cmp_ps(_mm256_mul_ps(d, s), x, _CMP_NEQ_UQ));
-        }
-        if(_mm256_movemask_ps(off)) return false;
-    }
+    auto off8 = [&](int at) __attribute__((target("avx2"))) {
+        const __m256 x = _mm256_loadu_ps(v + at), d = _mm256_round_ps(_mm256_mul_ps(x, inv), _MM_FROUND_CUR_DIRECTION);
+        return _mm256_cmp_ps(_mm256_mul_ps(d, s), x, _CMP_NEQ_UQ);
+    };
+    for(; j + 32 <= g; j += 32)
+        if(_mm256_movemask_ps(_mm256_or_ps(_mm256_or_ps(off8(j), off8(j + 8)), _mm256_or_ps(off8(j + 16), off8(j + 24))))) return false;
+    for(; j + 8 <= g; j += 8) if(_mm256_movemask_ps(off8(j))) return false;
+    if(j < g && g >= 8) return !_mm256_movemask_ps(off8(g - 8));          /* the last eight, some of them once more */
     for(; j < g; j++){
         const float d = rintf(v[j] / scale);
         if(fabsf(d) > 7.0f || d * scale != v[j]) return false;
@@ -236,6 +238,15 @@ __attribute__((target("avx2"))) static void put_avx2(const float *v, int g, floa
         const __m256i t = _mm256_permute4x64_epi64(_mm256_packus_epi32(h[0], h[1]), 0xD8);
         _mm_storeu_si128((__m128i *)(b + (j >> 1)), _mm_packus_epi16(_mm256_castsi256_si128(t), _mm256_extracti128_si256(t, 1)));
     }
+    auto put8 = [&](int at) __attribute__((target("avx2"))) {
+        const __m256i u = _mm256_cvtps_epi32(_mm256_mul_ps(_mm256_loadu_ps(v + at), inv));
+        const __m128i x = _mm_and_si128(_mm_packs_epi32(_mm256_castsi256_si128(u), _mm256_extracti128_si256(u, 1)), _mm256_castsi256_si128(low));
+        const __m128i h = _mm_and_si128(_mm_or_si128(x, _mm_srli_epi32(x, 12)), _mm256_castsi256_si128(byte)), t = _mm_packus_epi32(h, h);
+        const int four = _mm_cvtsi128_si32(_mm_packus_epi16(t, t));
+        memcpy(b + (at >> 1), &four, 4);
+    };
+    for(; j + 8 <= g; j += 8) put8(j);
+    if(j < g && g >= 8 && !(g & 1)){ put8(g - 8); return; }                /* the last eight, some of them once more */
     for(; j < g; j += 2){
         const int d0 = (int)rintf(v[j] / scale), d1 = j + 1 < g ? (int)rintf(v[j + 1] / scale) : 0;
         b[j >> 1] = (unsigned char)((d0 & 15) | ((d1 & 15) << 4));
@@ -279,19 +290,12 @@ __attribute__((target("avx2"))) static void unpack_avx2(const unsigned char *b, 
 /* Whether the first eight values may be amax / k times whole numbers, for the candidates of this k: a value that is a digit times one of them, rounded, is
  * amax / k times that digit within 2^-21 of itself, so that v * (1 / amax) * k is within 2^-17 of a whole number. What fails here fails with all five; a raw group, which has no
  * scale, is seen off with 7 of these instead of 35 tries (4 M values, half the groups raw: 580 -> 376 us). */
-__attribute__((target("avx2"))) static bool maybe_avx2(__m256 share, int k){
-    const __m256 t = _mm256_mul_ps(share, _mm256_set1_ps((float)k)), off = _mm256_sub_ps(t, _mm256_round_ps(t, _MM_FROUND_CUR_DIRECTION));
+__attribute__((target("avx2"))) static bool maybe_avx2(const float *v, float inv, int k){       /* inv = 1 / amax */
+    const __m256 t = _mm256_mul_ps(_mm256_mul_ps(_mm256_loadu_ps(v), _mm256_set1_ps(inv)), _mm256_set1_ps((float)k)), off = _mm256_sub_ps(t, _mm256_round_ps(t, _MM_FROUND_CUR_DIRECTION));
     const __m256 mag = _mm256_castsi256_ps(_mm256_set1_epi32(0x7FFFFFFF));
     return _mm256_movemask_ps(_mm256_cmp_ps(_mm256_and_ps(off, mag), _mm256_set1_ps(0x1p-17f), _CMP_NLE_UQ)) == 0;
 }
-__attribute__((target("avx2"))) static unsigned maybe_scales(const float *v, int g, float amax){       /* bit k: amax / k has to be tried */
-    if(g < 8) return 0xFEu;
-    const __m256 share = _mm256_mul_ps(_mm256_loadu_ps(v), _mm256_set1_ps(1.0f / amax));
-    unsigned m = 0;
-    for(int k = 7; k >= 1; k--) m |= (unsigned)maybe_avx2(share, k) << k;
-    return m;
-}
-/* the callers that round to nearest, as the bounds of fits_avx2 and maybe_scales have it; asked once per part */
+/* the callers that round to nearest, as the bounds of fits_avx2 and maybe_avx2 have it; asked once per part */
 static bool q4n_nearest(){ return q4n_avx2() && _MM_GET_ROUNDING_MODE() == _MM_ROUND_NEAREST; }
 /* and largest magnitudes, and scales, whose quotients and products neither overflow nor lose bits */
 static bool q4n_mid(float x, bool nearest){ return nearest && x >= 0x1p-90f && x <= 0x1p90f; }
@@ -303,20 +307,26 @@ static void group_unpack(const unsigned char *b, int g, float scale, float *P){ 
 /* the neighbours of a value >= 0: nextafterf towards 0 and towards infinity, without the calls (35 candidates in a raw group) */
 static inline float toward_zero(float x){ unsigned u; memcpy(&u, &x, 4); if(u) u--; memcpy(&x, &u, 4); return x; }
 static inline float toward_inf(float x){ unsigned u; memcpy(&u, &x, 4); if(u != 0x7F800000u) u++; memcpy(&x, &u, 4); return x; }
-/* the group's scale, the first candidate that fits (0 for a group of zeros), or NaN for a group that is kept raw */
-static float group_scale(const float *v, int g, bool nearest, signed char *digit){
-    const float amax = group_amax(v, g);
-    if(amax == 0.0f) return 0.0f;
-    const bool mid = q4n_mid(amax, nearest);
-    const unsigned worth = mid ? maybe_scales(v, g, amax) : 0xFEu;
+/* the first candidate that fits, or NaN for a group that is kept raw */
+template<class Worth, class Fits> static inline float first_scale(float amax, const Worth &worth, const Fits &fits){
     for(int k = 7; k >= 1; k--){
-        if(!(worth >> k & 1)) continue;
+        if(!worth(k)) continue;
         const float s0 = amax / (float)k;
         const float below = toward_zero(s0), above = toward_inf(s0);
         const float cand[5] = {s0, below, above, toward_zero(below), toward_inf(above)};
-        for(int t = 0; t < 5; t++) if(mid ? fits_avx2(v, g, cand[t]) : group_try(v, g, cand[t], digit)) return cand[t];
+        for(int t = 0; t < 5; t++) if(fits(cand[t])) return cand[t];
     }
     return NAN;
+}
+/* the group's scale: 0 for a group of zeros, NaN for one that is kept raw */
+static float group_scale(const float *v, int g, bool nearest, signed char *digit){
+    const float amax = group_amax(v, g);
+    if(amax == 0.0f) return 0.0f;
+    if(q4n_mid(amax, nearest)){
+        const float inv = 1.0f / amax;
+        return first_scale(amax, [&](int k){ return g < 8 || maybe_avx2(v, inv, k); }, [&](float s){ return fits_avx2(v, g, s); });
+    }
+    return first_scale(amax, [](int){ return true; }, [&](float s){ return group_try(v, g, s, digit); });
 }
 
 extern "C" size_t qlmx_q4n_bound(size_t n, int group){

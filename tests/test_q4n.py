@@ -122,6 +122,25 @@ def test_groups_that_fit_and_groups_that_nearly_do(lib, orc, exponent, group):
     assert used == got.size and np.array_equal(back + f32(0), P + f32(0))       # a zero comes back positive
 
 
+@pytest.mark.parametrize("tail", [0, 1, 6, 7, 8, 9, 15, 31, 33, 39])
+def test_every_even_group_up_to_eighty(lib, orc, tail):
+    """Groups and last groups of every remainder of 8 and of 32: ones that fit, with the digits of the last eight looked at twice, and ones that a value at
+    the back keeps raw."""
+    rng = np.random.default_rng(tail)
+    for group in range(2, 82, 2):
+        n = 36 * group + min(tail, group - 1)
+        P = rng.integers(-7, 8, n).astype(f32) * f32(0.0173)
+        P[group * np.arange(36)] = f32(7) * f32(0.0173)
+        for q in range(0, 37, 3):
+            v = P[q * group:(q + 1) * group]
+            if v.size: v[-1 - q % min(9, v.size)] += f32(0.003)
+        want, wraw = orc.q4n_quantize(P, group)
+        got, raw = lib.q4n_quantize(P, group)
+        assert raw == wraw and np.array_equal(got, want), group
+        back, used = lib.q4n_dequantize(got, n, group)
+        assert used == got.size and np.array_equal(back + f32(0), P + f32(0)), group
+
+
 def test_callers_share_the_threads_and_a_child_has_its_own(lib):
     """Calls from several threads at once, calls after the threads have gone for want of work, and calls in a child process."""
     import threading
