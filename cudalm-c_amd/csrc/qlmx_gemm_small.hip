@@ -44,12 +44,17 @@
  * (35 -> 17), its input gradient 18 -> 13 (28 -> 22), paired input gradient 50 -> 14 (72 -> 16).
  * Shapes of the forward of at most 32 rows per problem, groups of 128 or 256 (sm_few_shape). What takes the time there is the CU's address unit
  * as much as vector issue: an instruction that loads a word per lane from four rows of weights takes it as long as one that loads two.
- *   wide: 256 columns to a strip, a lane's words of a row of weights in one load (RT * 64 registers of sums). Four wavefronts to a workgroup, two workgroups to a CU, from 176
- *     strips on (wide : narrow, us, 8 / 20 rows, 1408 x N: 64 experts of 512 14.9:11.3 / 17.9:13.4, of 768 14.6:16.7 / 18.1:18.3, 40 of 1408 15.2:17.4 / 18.6:19.4,
- *     28 of 2048 15.3:20.5 / 18.7:22.8, 64 of 2816 34.9:45.7 / 42.3:52.2). Gate|up is eight wavefronts and one workgroup to a CU, so that its strips come in rounds of 256:
- *     up to 16 rows from 176 strips on, but not between 257 and 351 (768 x N: 64 of 512 17:13.1, 64 of 768 16.6:20.4, 40 of 1408 17.4:20.9, 28 of 2048 17.4:24.6, 40 of 2048 31.4:30.4, 48 of
- *     2048 32.4:35.7, 64 of 2816 48:59.6); above 16 rows only for one round with rows of weights a multiple of 1 KB apart, where narrow strips meet in the same memory
- *     channels (28 of 2048 23.4:24.6, a mixture around twelve rows 22.4:26.9; but 40 of 1408 23.7:21.9, 64 of 2048 45.5:44.6).
+ *   wide: 256 columns to a strip, a lane's words of a row of weights in one load (RT * 64 registers of sums), two workgroups of four wavefronts to a CU; gate|up is eight wavefronts and one
+ *     workgroup to a CU. Lines (sm_wide) from 2700 pairs of calls, K 256-2048, N 512-4096, 136-512 strips, and 3000 drawn ones; time of wide over narrow, with rows, K x N:
+ *     one round of CUs, from 11/16 of it on (gate|up 10/16; with half of the CUs 1.3-1.7). Up to 16 rows K from 512: 0.66-0.97, at 384 and 256 0.97-1.13; gate|up from 384: 0.67-0.94, at 256 1.02-1.16.
+ *       More rows, plain: K from 768 0.72-1.04, at 512 1.0-1.1 and at 256 1.07-1.18. More rows, gate|up: twice the registers against half the loads, and it takes a large matrix: from
+ *       3 M weights 0.78-1.02 (20 rows, 1408 x 2304 0.98, 2048 x 1536 0.96, 1280 x 2560 0.94; below it 768 x 1536 1.08, 1408 x 768 1.04, 2048 x 768 1.02). Rows of weights a
+ *       multiple of 1 KB apart, where narrow strips meet in the same memory channels, gain earlier: 768 x 2048 0.93-0.99, 896 x 4096 0.90, beside 768 x 2304 1.08, 768 x 2816 1.06, 896 x 3072
+ *       0.99; 512 x 2048 1.05. They take the plain call from K = 512: 0.93, others 1.0-1.05. More rows and two strips for three narrow ones (N = 384): 1.07;
+ *     beyond: plain, not where narrow strips, 2 to a CU, still come in one round (43 of 1408 1.40-1.44), K from 512: up to 16 rows 0.60-1.03, more rows from three narrow strips to a CU 0.64-0.97, with
+ *       fewer a large matrix or rows 1 KB apart 0.85-1.04, others, and half strips, up to 1.14. Shorter ones with six rounds and more 0.85-0.98, fewer 0.9-1.3. Gate|up of up to 16 rows, K from 768,
+ *       where the rounds are 25/32 full (a large matrix 22/32 or 23/32): 0.70-1.09; K from 384 two that are 27/32 full, or five: 0.84-1.0; others up to 1.25, at 256 1.1-1.5. Gate|up of more rows in
+ *       one round only (1.0-1.5, with a round and a half and more 0.8-1.2).
  *   eight wavefronts along the contraction, where few strips walk a long one: K from 2048, up to 224 strips of 128, above 16 rows K from 2 N (8 : 4 wavefronts, 2048 x 768, 8 rows of 16 experts
  *     11.6:13.3, of 32 11.7:13.9, 20 rows of 32 14.6:16.7; gate|up the same with up to 16 rows, 20 rows of 8, 2048 x 1408, 25.5:22.6). One step of a wavefront
  *     is on its way in both: two are slower (18.3 -> 19.6 for gate|up of 32, 768 x 2048).
@@ -331,14 +336,27 @@ __global__ void __launch_bounds__(64 * SM_WAVES, 2) k_gemm_tn_small(SmArgs a){
 /* Shape of the forward of at most 32 rows per problem. Eight wavefronts along the contraction change the order of the sums, so that line looks at what the
  * forms of a call have in common; the width of a strip does not, and looks at the form too. See the head of this file. */
 enum { SM_NARROW = 0, SM_WIDE = 1, SM_EIGHT = 2 };
+static bool sm_wide(long long narrow, long long wide, int K, int N, bool dual, int rt){
+    const int cu = qlmx_cu_count();
+    const bool apart = N % 2048 == 0, large = (long long)K * N >= 3000000;
+    if(16 * wide < (dual ? 10 : 11) * cu || (rt == 2 && 8 * wide > 5 * narrow)) return false;
+    if(wide <= cu) return rt == 1 ? K >= (dual ? 384 : 512) : dual ? K >= 768 && (apart || large) : K >= (apart ? 512 : 768);
+    if(dual){
+        const long long rounds = (wide + cu - 1) / cu, full = 32 * wide / (rounds * cu);          /* in 32nds */
+        if(rt == 2) return false;
+        if(K < 768) return K >= 384 && (rounds == 2 ? full >= 27 : rounds >= 5);
+        return full >= (!large ? 25 : rounds == 2 ? 22 : 23);
+    }
+    if(narrow <= 2 * cu) return false;
+    if(rt == 2 && narrow < 3 * cu && (N % 256 != 0 || !(large || apart))) return false;
+    return K >= 512 || wide >= 6 * cu;
+}
 static int sm_few_shape(const qlmx_gemm_prob *probs, int nprob, int K, int N, int group, bool dual, int rt){
     if(group < 128) return SM_NARROW;                     /* a wide strip has room for two scales in a row of weights */
     long long narrow = 0, wide = 0;
     for(int i = 0; i < nprob; i++) if(probs[i].M > 0){ narrow += N / SM_COLS; wide += (N + 2 * SM_COLS - 1) / (2 * SM_COLS); }
     if(narrow <= 224 && K >= 2048 && (rt == 1 || K >= 2 * N)) return SM_EIGHT;
-    if(!dual) return wide >= 176 ? SM_WIDE : SM_NARROW;
-    if(rt == 2) return wide >= 160 && wide <= 256 && N % 2048 == 0 ? SM_WIDE : SM_NARROW;
-    return wide >= 176 && (wide <= 256 || wide >= 352) ? SM_WIDE : SM_NARROW;
+    return sm_wide(narrow, wide, K, N, dual, rt) ? SM_WIDE : SM_NARROW;
 }
 /* Height, in sixteens, of the row tiles of a call with more than 32 rows to a problem: 64 rows share the weights' conversion or loads, 32 are less padding and more
  * workgroups. The order of a sum is the same in both, so the forms of a call need not agree on it. us, 32 : 64 rows:

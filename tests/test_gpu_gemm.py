@@ -394,13 +394,17 @@ def test_mfma_few_rows(q, orc, mode, K, N, group, rows):
         assert orc.relerr(got, want) < (4e-4 if mode == "nn" else 3e-6)
 
 
-@pytest.mark.parametrize("K,N,rows,group", [(32, 2048, [1, 16, 0, 9] * 7, 128),              # strips of 256 columns, gate|up too; fewer steps than wavefronts
-                                            (160, 1408, [16, 3] * 16, 128),                   # half a strip at the end
-                                            (96, 2048, [17, 32, 1, 16] * 6, 256),             # one scale for both halves, more than 16 rows
-                                            (64, 1408, [31, 5, 16, 17] * 9, 128),             # wide, gate|up on strips of 128
-                                            (64, 1152, [20, 0] * 35, 128), (64, 1152, [7] * 36, 128), (64, 1152, [7] * 35, 128),     # either side of the line for wide strips
+@pytest.mark.parametrize("K,N,rows,group", [(32, 2048, [1, 16, 0, 9] * 7, 128), (64, 1152, [20, 0] * 35, 128),          # strips of 128 columns; fewer steps than wavefronts
+                                            (32, 2048, [1, 16, 0, 9] * 17, 128),                                          # the plain call on strips of 256: 408 of them, from three of 128 to a CU
+                                            (512, 2048, [1, 16, 0, 9] * 8, 128), (512, 2048, [1, 16, 0, 9] * 8, 256),     # 192 of 256, gate|up too
+                                            (384, 2048, [7] * 20, 128), (384, 2048, [7] * 19, 128),                       # 160, gate|up only, and fewer
+                                            (512, 1408, [16, 3] * 16, 128), (512, 1408, [7] * 43, 128),                   # half a strip at the end; 258 of 256 and 473 of 128
+                                            (512, 2048, [7] * 32, 128), (512, 2048, [7] * 33, 256),                       # a full round, and 264: the plain call
+                                            (512, 2048, [5] * 48, 128), (768, 4096, [7] * 22, 128),                       # beyond: three of 128 to a CU; 352, a large matrix
+                                            (768, 2048, [17, 32, 1, 16] * 6, 256), (640, 2048, [17, 32, 1, 16] * 6, 128),      # more than 16 rows, one scale for both halves; gate|up on 128
+                                            (768, 3968, [31, 5, 16, 17, 2] * 2 + [3], 128), (768, 3840, [31, 5, 16] * 4, 128),      # either side of 3 M weights; half a strip at the end
                                             (2048, 384, [16, 1, 0, 7], 128), (2048, 512, [32, 17, 9], 256), (2080, 128, [5], 128),     # eight wavefronts along the contraction
-                                            (2048, 1152, [32, 17, 9], 128),
+                                            (2048, 256, [3, 17] * 33, 128), (2048, 1152, [32, 17, 9], 128),                    # 132 strips; eight no more
                                             (160, 384, [70, 5, 0, 33, 9, 9, 2], 128), (576, 384, [129, 64, 1], 64),               # larger problems on 32 rows, gate|up on 64
                                             (96, 256, [70, 3] + [5] * 70, 128), (544, 1152, [97, 34, 0, 31] * 4, 64),    # both on 32
                                             (1056, 896, [64, 40, 34] * 16, 128)])                                        # both on 64
