@@ -55,9 +55,11 @@
  *       fewer a large matrix or rows 1 KB apart 0.85-1.04, others, and half strips, up to 1.14. Shorter ones with six rounds and more 0.85-0.98, fewer 0.9-1.3. Gate|up of up to 16 rows, K from 768,
  *       where the rounds are 25/32 full (a large matrix 22/32 or 23/32): 0.70-1.09; K from 384 two that are 27/32 full, or five: 0.84-1.0; others up to 1.25, at 256 1.1-1.5. Gate|up of more rows in
  *       one round only (1.0-1.5, with a round and a half and more 0.8-1.2).
- *   eight wavefronts along the contraction, where few strips walk a long one: K from 2048, up to 224 strips of 128, above 16 rows K from 2 N (8 : 4 wavefronts, 2048 x 768, 8 rows of 16 experts
- *     11.6:13.3, of 32 11.7:13.9, 20 rows of 32 14.6:16.7; gate|up the same with up to 16 rows, 20 rows of 8, 2048 x 1408, 25.5:22.6). One step of a wavefront
- *     is on its way in both: two are slower (18.3 -> 19.6 for gate|up of 32, 768 x 2048).
+ *   eight wavefronts along the contraction, where few strips walk a long one: K from 2048, up to 7/8 of a strip of 128 to a CU, above 16 rows K from 2 N. All forms of a call split alike. Eight over four,
+ *     K 1024-4096, N 128-3840: plain 0.81-0.95. Gate|up, up to half a strip to a CU, on strips of 64 columns of each matrix, one to a CU: 0.59-0.88; on strips of 128, as with more of them, 0.97-1.03
+ *     up to 16 rows and 1.04-1.10 above, where the rule takes that for the plain call's 0.75-0.90 (2048 x 768, 20 rows of 32: 14.3:16.7). Shorter contractions: plain 0.86-0.95 and 0.90-0.99 from K = 1024 on,
+ *     gate|up on strips of 128 0.96-1.07 and 1.05-1.2. All eight put their sums into LDS at once; four after four took gate|up 2-4 % longer. One step of a wavefront is on its way in both: two are slower (18.3 -> 19.6
+ *     for gate|up of 32, 768 x 2048).
  * What bounds them now: a wavefront's chain -- the round trip in front of its loop, the steps one behind the other, the sum over
  * the wavefronts behind it: 7 us of a gate|up call of 18, whose 50 MB stream at 4 TB/s beside it. Without the conversions it took 10. Other ways to them: scales on the
  * activations, as two bf16 parts, and digits as denormal bf16 took half the vector instructions and no less time, the address unit being as busy; and they round otherwise than
@@ -121,12 +123,12 @@ template<int I> __device__ __forceinline__ float sm_bcast_hi(float low, float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(low), __float_as_int(v), 0x158 + I, 0xF, 0xC, false));
 }
 
-/* The sums of four wavefronts from `first` on, of one 16-row tile, through LDS: acc holds a lane's sums of rows
+/* The sums of KW wavefronts from `first` on, of one 16-row tile, through LDS: acc holds a lane's sums of rows
  * (lane/16)*4 + e, columns (lane%16)*CL + j. */
-template<int CL> __device__ __forceinline__ void sm_put(float *red, int first, const f32x4 (&acc)[CL]){
+template<int CL, int KW> __device__ __forceinline__ void sm_put(float *red, int first, const f32x4 (&acc)[CL]){
     const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) - first, c = lane & 15, g = lane >> 4;
     __syncthreads();                                      /* the tile before has been read */
-    if(wave >= 0 && wave < 4){
+    if(wave >= 0 && wave < KW){
         float *w = red + wave * (16 * 16 * CL);
 #pragma unroll
         for(int e = 0; e < 4; e++)
@@ -136,26 +138,16 @@ template<int CL> __device__ __forceinline__ void sm_put(float *red, int first, c
     }
     __syncthreads();
 }
-/* what wavefront w + 4 has put, added to wavefront w's own, w from `first` on */
-template<int CL> __device__ __forceinline__ void sm_add(const float *red, int first, f32x4 (&acc)[CL]){
-    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) - first, c = lane & 15, g = lane >> 4;
-    if(wave < 0 || wave >= 4) return;
-    const float *w = red + wave * (16 * 16 * CL);
+/* four columns of a row; of eight wavefronts, first k and k + 4 */
+template<int CL, int KW> __device__ __forceinline__ f32x4 sm_get(const float *red, int row, int col){
+    f32x4 sum;
 #pragma unroll
-    for(int e = 0; e < 4; e++)
-#pragma unroll
-        for(int j = 0; j < CL; j += 4){
-            const f32x4 v = *(const f32x4 *)&w[(g * 4 + e) * (16 * CL) + c * CL + j];
-#pragma unroll
-            for(int q = 0; q < 4; q++) acc[j + q][e] += v[q];
-        }
-}
-/* four columns of a row */
-template<int CL> __device__ __forceinline__ f32x4 sm_get(const float *red, int row, int col){
-    f32x4 v = *(const f32x4 *)&red[row * (16 * CL) + col];
-#pragma unroll
-    for(int k = 1; k < 4; k++) v += *(const f32x4 *)&red[k * (16 * 16 * CL) + row * (16 * CL) + col];
-    return v * SM_UNSCALE;
+    for(int k = 0; k < 4; k++){
+        f32x4 v = *(const f32x4 *)&red[k * (16 * 16 * CL) + row * (16 * CL) + col];
+        if(KW == 8) v += *(const f32x4 *)&red[(k + 4) * (16 * 16 * CL) + row * (16 * CL) + col];
+        sum = k ? sum + v : v;
+    }
+    return sum * SM_UNSCALE;
 }
 
 /* ---- forward, and gate | up in one (the second matrix at wq, wg of Q): SM_BY_WAVE, four more wavefronts work on 128 columns
@@ -265,32 +257,28 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
         *(ushort4 *)((unsigned short *)Q.B + o) = h;
     };
     constexpr int THREADS = 64 * KW * (DUAL == SM_BY_WAVE ? 2 : 1), PER_ROW = COLS / 4, V = (16 * PER_ROW + THREADS - 1) / THREADS;
-    auto together = [&](int first, f32x4 (&v)[CL]){       /* the sums of the wavefronts from `first` on, for sm_get */
-        if(KW == 8){ sm_put<CL>(red, first + 4, v); sm_add<CL>(red, first, v); }
-        sm_put<CL>(red, first, v);
-    };
 #pragma unroll
     for(int r = 0; r < RT; r++){
         const int i = i0 + r * 16;
-        together(0, acc[r]);
+        sm_put<CL, KW>(red, 0, acc[r]);
         if constexpr(DUAL == SM_BY_LANE){
             const int row = tid >> 4, col = (tid & 15) * 4;
-            swiglu(i + row, col, sm_get<CL>(red, row, col), sm_get<CL>(red, row, 64 + col));
+            if(THREADS <= 256 || row < 16) swiglu(i + row, col, sm_get<CL, KW>(red, row, col), sm_get<CL, KW>(red, row, 64 + col));
         } else if constexpr(DUAL == SM_BY_WAVE){
             f32x4 y[V];
 #pragma unroll
-            for(int v = 0; v < V; v++){ const int at = (v * THREADS + tid) % (16 * PER_ROW); y[v] = sm_get<CL>(red, at / PER_ROW, at % PER_ROW * 4); }
-            together(KW, acc[r]);
+            for(int v = 0; v < V; v++){ const int at = (v * THREADS + tid) % (16 * PER_ROW); y[v] = sm_get<CL, KW>(red, at / PER_ROW, at % PER_ROW * 4); }
+            sm_put<CL, KW>(red, KW, acc[r]);
 #pragma unroll
             for(int v = 0; v < V; v++){
                 const int at = v * THREADS + tid, row = at / PER_ROW, col = at % PER_ROW * 4;
-                if(at < 16 * PER_ROW) swiglu(i + row, col, y[v], sm_get<CL>(red, row, col));
+                if(at < 16 * PER_ROW) swiglu(i + row, col, y[v], sm_get<CL, KW>(red, row, col));
             }
         } else {
 #pragma unroll
             for(int v = 0; v < V; v++){
                 const int at = v * THREADS + tid, row = at / PER_ROW, col = at % PER_ROW * 4, lr = i + row;
-                const f32x4 y = sm_get<CL>(red, row, col);
+                const f32x4 y = sm_get<CL, KW>(red, row, col);
                 if(lr >= P.M || (CL == 16 && j0 + col >= a.N)) continue;
                 if constexpr(IO == SM_SCATTER){
                     const int tok = ((const int *)P.C)[lr];
@@ -308,7 +296,7 @@ __device__ __forceinline__ void sm_nn_tile(const SmArgs &a, const DevProb &P, co
 
 template<int RT, int IO, int DUAL, int CL, int KW>
 __global__ void __launch_bounds__(64 * KW * (DUAL == SM_BY_WAVE ? 2 : 1), CL == 16 ? 2 : RT == 1 || DUAL == SM_BY_WAVE ? 4 : 2) k_gemm_nn_small(SmArgs a){
-    __shared__ __attribute__((aligned(16))) float red[4 * 16 * 16 * CL];
+    __shared__ __attribute__((aligned(16))) float red[KW * 16 * 16 * CL];
     const int t = qx_xcd_tile(blockIdx.x, gridDim.x);
     if(t >= a.ntiles) return;
     const int pi = qx_find_problem(a.pr, a.nprob, t);
@@ -335,7 +323,7 @@ __global__ void __launch_bounds__(64 * SM_WAVES, 2) k_gemm_tn_small(SmArgs a){
 /* ---- launches ---- */
 /* Shape of the forward of at most 32 rows per problem. Eight wavefronts along the contraction change the order of the sums, so that line looks at what the
  * forms of a call have in common; the width of a strip does not, and looks at the form too. See the head of this file. */
-enum { SM_NARROW = 0, SM_WIDE = 1, SM_EIGHT = 2 };
+enum { SM_NARROW = 0, SM_WIDE = 1, SM_EIGHT = 2, SM_EIGHT_HALF = 3 };
 static bool sm_wide(long long narrow, long long wide, int K, int N, bool dual, int rt){
     const int cu = qlmx_cu_count();
     const bool apart = N % 2048 == 0, large = (long long)K * N >= 3000000;
@@ -355,7 +343,7 @@ static int sm_few_shape(const qlmx_gemm_prob *probs, int nprob, int K, int N, in
     if(group < 128) return SM_NARROW;                     /* a wide strip has room for two scales in a row of weights */
     long long narrow = 0, wide = 0;
     for(int i = 0; i < nprob; i++) if(probs[i].M > 0){ narrow += N / SM_COLS; wide += (N + 2 * SM_COLS - 1) / (2 * SM_COLS); }
-    if(narrow <= 224 && K >= 2048 && (rt == 1 || K >= 2 * N)) return SM_EIGHT;
+    if(8 * narrow <= 7 * qlmx_cu_count() && K >= 2048 && (rt == 1 || K >= 2 * N)) return dual && 2 * narrow <= qlmx_cu_count() ? SM_EIGHT_HALF : SM_EIGHT;
     return sm_wide(narrow, wide, K, N, dual, rt) ? SM_WIDE : SM_NARROW;
 }
 /* Height, in sixteens, of the row tiles of a call with more than 32 rows to a problem: 64 rows share the weights' conversion or loads, 32 are less padding and more
@@ -413,11 +401,12 @@ int qlmx_gemm_nn_small_swiglu_launch(const signed char *d, const float *s, int g
     const int rt = sm_nn_height(rows, N / SM_COLS, true);
     ProbUpload up; int slot;
     const int shape = rows.most <= 32 ? sm_few_shape(gate, nprob, K, N, group, true, rt) : SM_NARROW;
-    int rc = qlmx_upload_problem_pairs(gate, up_, nprob, GEMM_NN, K, N, rt * 16, rt == 4 ? SM_COLS / 2 : shape == SM_WIDE ? 2 * SM_COLS : SM_COLS, st, &up, &slot); if(rc) return rc;
+    int rc = qlmx_upload_problem_pairs(gate, up_, nprob, GEMM_NN, K, N, rt * 16, rt == 4 || shape == SM_EIGHT_HALF ? SM_COLS / 2 : shape == SM_WIDE ? 2 * SM_COLS : SM_COLS, st, &up, &slot); if(rc) return rc;
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
     a.xsrc = (const char *)xsrc;
 #define SM_FEW(RT, IO) do{ if(shape == SM_WIDE) SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_BY_WAVE, 16, 4>), 8, 0); \
+                           else if(shape == SM_EIGHT_HALF) SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_BY_LANE, 8, 8>), 8, 0); \
                            else if(shape == SM_EIGHT) SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_BY_WAVE, 8, 8>), 16, 0); else SM_LAUNCH((k_gemm_nn_small<RT, IO, SM_BY_WAVE, 8, 4>), 8, 0); }while(0)
 #define SM_DUAL(IO) do{ if(rt == 1) SM_FEW(1, IO); else if(rt == 2) SM_FEW(2, IO); else SM_LAUNCH((k_gemm_nn_small<4, IO, SM_BY_LANE, 8, 4>), 4, 0); }while(0)
     if(xsrc) SM_DUAL(SM_GATHER); else SM_DUAL(SM_PLAIN);

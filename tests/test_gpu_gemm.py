@@ -404,7 +404,8 @@ def test_mfma_few_rows(q, orc, mode, K, N, group, rows):
                                             (768, 2048, [17, 32, 1, 16] * 6, 256), (640, 2048, [17, 32, 1, 16] * 6, 128),      # more than 16 rows, one scale for both halves; gate|up on 128
                                             (768, 3968, [31, 5, 16, 17, 2] * 2 + [3], 128), (768, 3840, [31, 5, 16] * 4, 128),      # either side of 3 M weights; half a strip at the end
                                             (2048, 384, [16, 1, 0, 7], 128), (2048, 512, [32, 17, 9], 256), (2080, 128, [5], 128),     # eight wavefronts along the contraction
-                                            (2048, 256, [3, 17] * 33, 128), (2048, 1152, [32, 17, 9], 128),                    # 132 strips; eight no more
+                                            (2048, 256, [3, 17] * 33, 128), (2048, 256, [16, 3] * 33, 256),                    # 132 strips: gate|up on 128 columns, up to there on 64
+                                            (2048, 1152, [32, 17, 9], 128),                                               # four
                                             (160, 384, [70, 5, 0, 33, 9, 9, 2], 128), (576, 384, [129, 64, 1], 64),               # larger problems on 32 rows, gate|up on 64
                                             (96, 256, [70, 3] + [5] * 70, 128), (544, 1152, [97, 34, 0, 31] * 4, 64),    # both on 32
                                             (1056, 896, [64, 40, 34] * 16, 128)])                                        # both on 64
