@@ -21,7 +21,7 @@
  * kernels with few workgroups, each walking the whole contraction, or with tiles that are mostly padding: a prompt or a small batch whose router prefers
  * some experts has a few problems of a hundred rows beside many of five, each a tile of 128 there and of 32 here. The forward's rule looks at what the
  * forms of a call that are documented to agree bit for bit have in common -- with and without gather, SwiGLU, scatter -- so that they run the same
- * arithmetic in the same order. us for the plain and the SwiGLU call, these : tiled --
+ * arithmetic in the same order. The lines count in CUs of the device; the numbers here are a device's with 256. us for the plain and the SwiGLU call, these : tiled --
  *   contractions over 512, tiles of 32 rows x 128 columns up to 256, one to a CU. 16 problems, largest 43 rows, 896 x 1152 8.3:13.6, 1152 x 896 14.6:19.0; 8 of 49,
  *     768 x 896 8.3:11.9, 896 x 768 12.2:13.8. Shorter ones, whose SwiGLU call gains little (8 of 104, 384 x 384 6.0:7.7 and 8.3:8.6; 8 of 21, 384 x 1152 6.0:8.3 and 8.6:9.0), stay
  *     with the tiled kernel, which also takes a small layer's passes merged into one list: the same bits either way;
@@ -91,23 +91,24 @@ static SmRows sm_rows(const qlmx_gemm_prob *probs, int nprob){
 }
 /* tiles of 32 rows on so many strips, against `high` taller ones: not many more of them, by a line that depends on whether they come in two rounds; see the head of this file */
 static bool sm_low(long long t32, long long high, int strips){
-    const long long tiles = t32 * strips;
-    return tiles > 256 && tiles <= 352 ? 8 * t32 <= 9 * high : 2 * t32 <= 3 * high;
+    const long long tiles = t32 * strips, cu = qlmx_cu_count();
+    return tiles > cu && 8 * tiles <= 11 * cu ? 8 * t32 <= 9 * high : 2 * t32 <= 3 * high;
 }
 /* see the head of this file */
 bool qlmx_small_rows(const qlmx_gemm_prob *probs, int nprob, int mode, int K, int N, int nseg, int group){
     if(group < 64) return false;
     const SmRows r = sm_rows(probs, nprob);
+    const int cu = qlmx_cu_count();
     if(r.most <= 32) return true;
     if(mode == GEMM_NN){
         const long long tiles = r.t64 * (N / SM_COLS);
-        if((K > 512 && r.t32 * (N / SM_COLS) <= 256) || sm_low(r.t32, r.t128, N / SM_COLS)) return true;
-        if(tiles <= 256) return K >= N || (r.most <= 64 && K > 1024);
-        if(tiles <= 512 && K >= 4 * N) return true;
+        if((K > 512 && r.t32 * (N / SM_COLS) <= cu) || sm_low(r.t32, r.t128, N / SM_COLS)) return true;
+        if(tiles <= cu) return K >= N || (r.most <= 64 && K > 1024);
+        if(tiles <= 2 * cu && K >= 4 * N) return true;
         return K > 1024 && K >= N && r.most <= 64 && r.rows <= 48 * r.busy;
     }
     const long long tiles = r.t64 * (N / SM_TCOLS);
-    return tiles <= 512 || (tiles <= 1024 && (long long)K * nseg >= 2 * N);
+    return tiles <= 2 * cu || (tiles <= 4 * cu && (long long)K * nseg >= 2 * N);
 }
 
 __device__ __forceinline__ int sm_pk_f16(float lo, float hi){ f32x2 v = {lo, hi}; return __builtin_bit_cast(int, __builtin_convertvector(v, f16x2)); }
@@ -357,8 +358,8 @@ static int sm_few_shape(const qlmx_gemm_prob *probs, int nprob, int K, int N, in
 static int sm_few_height(const SmRows &r){ return r.most > 16 ? 2 : 1; }
 static int sm_nn_height(const SmRows &r, int strips, bool dual){
     if(r.most <= 32) return sm_few_height(r);
-    const long long tiles = r.t32 * strips;
-    return tiles <= 256 ? (dual && tiles <= 128 ? 4 : 2) : sm_low(r.t32, r.t64, strips) ? 2 : 4;
+    const long long tiles = r.t32 * strips, cu = qlmx_cu_count();
+    return tiles <= cu ? (dual && 2 * tiles <= cu ? 4 : 2) : sm_low(r.t32, r.t64, strips) ? 2 : 4;
 }
 static int sm_tn_height(const SmRows &r, long long contraction, int strips){
     if(r.most <= 32) return sm_few_height(r);
