@@ -23,8 +23,9 @@
  * forms of a call that are documented to agree bit for bit have in common -- with and without gather, SwiGLU, scatter -- so that they run the same
  * arithmetic in the same order. The lines count in CUs of the device; the numbers here are a device's with 256. us for the plain and the SwiGLU call, these : tiled --
  *   contractions over 512, tiles of 32 rows x 128 columns up to 256, one to a CU. 16 problems, largest 43 rows, 896 x 1152 8.3:13.6, 1152 x 896 14.6:19.0; 8 of 49,
- *     768 x 896 8.3:11.9, 896 x 768 12.2:13.8. Shorter ones, whose SwiGLU call gains little (8 of 104, 384 x 384 6.0:7.7 and 8.3:8.6; 8 of 21, 384 x 1152 6.0:8.3 and 8.6:9.0), stay
- *     with the tiled kernel, which also takes a small layer's passes merged into one list: the same bits either way;
+ *     768 x 896 8.3:11.9, 896 x 768 12.2:13.8. Shorter ones stay with the tiled kernel (plain and SwiGLU call, 8 of 104,
+ *     384 x 384 6.0:7.7 and 8.3:8.6; 8 of 21, 384 x 1152 6.0:8.3 and 8.6:9.0): the SwiGLU call gains little, and the plain call's gain is given up for layers of such widths, whose passes one by one
+ *     and merged into one list then run the same kernel in more cases;
  *   tiles of 32 rows at most 1.5 times the 128-row tiles; from 257 to 352 of them 1.125 times (a second round that is nearly empty). Zipf shares: 1096 rows of 64, 896 x 512
  *     12.5:18.0, 512 x 896 22:24; 617 of 64, 1664 x 1920 41:60, 1920 x 1664 62:109; 362 of 32, 2304 x 896 18:31, 896 x 2304 32:50. On the other side 4832 of 64,
  *     1536 x 768 41:33, 768 x 1536 77:70; and with 330 tiles, 16 of 31 rows, 1024 x 1920 14:16 and 26:20;
@@ -36,8 +37,8 @@
  *     64 of 41 59:63 and 102:116, 2048 x 768, 64 of 40 31:33 and 57:68; on the other side 64 of 64 56:63 and 121:103.
  * Over 160 calls of 1 to 64 problems of 5 to 400 rows on average, in even and in Zipf shares, 256 to 2048 in and out, a plain call takes 0.88 and a SwiGLU call 0.96 of what they took
  * when the rule counted strips of 64 rows only and problems of over 32 rows had tiles of 64 (mean of the ratios; 68 of the calls are as they were).
- * The lines look at a call's own sizes, so a layer whose passes run one by one may take the one path and its merged list the other: bits that
- * agree between the two are not promised and not looked for here.
+ * The lines look at a call's own sizes, so a layer whose passes run one by one may take the one path and its merged list the other: where both take the same, bits agree, and that is
+ * promised for no size.
  * Input gradient, strips of 64 x 64: up to 512, 1024 where the contraction is twice the width.
  * us per call, tiled kernels of 256 x 128 (128 x 128) as these were written -> these: 32 experts, 768 x 2048, 12 rows each: gate|up + SwiGLU 34 -> 21, down 26 -> 12, its
  * input gradient + SwiGLU 21 -> 13, paired input gradient 56 -> 19; 8 experts of 125 (250) rows, 512 x 1536: down 24 -> 16

@@ -379,7 +379,8 @@ int qlmx_moe_dgate(const float *dout, const float *yp, const int *perm, const fl
                    float *d_gate, void *dyp, int N, int D, int out_dtype, void *stream);
 /* All K passes of a layer as ONE expert-grouped list of K*N rows (the reference's merged top-K: moe_gperm with
  * mrg, k_gather_bfm, k_combine_bf, k_moe_dgate_bfm; cudalm.cu:3532-3561, 4022-4047), so that every grouped GEMM
- * runs once per layer on K times the rows instead of once per pass. The grouping itself is qlmx_moe_perm over the
+ * runs once per layer on K times the rows instead of once per pass (calls of other sizes than the passes': a row's products
+ * agree with the passes' to the order of their additions, bit for bit only where both run the same kernel). The grouping itself is qlmx_moe_perm over the
  * K*N assignments as a single pass (N' = K*N, K' = 1): its perm names entries m = pass * N + token.
  *   qlmx_moe_merge_rows: tok[p] = perm[p] % N (the token row p holds; what a gather or a gathering GEMM takes as
  *     its index list) and inv[m] = the row that holds entry m (-1 if none), both int32 [K*N]; tok may be perm.
