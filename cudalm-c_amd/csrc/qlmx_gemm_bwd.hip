@@ -46,7 +46,7 @@ struct PairState {
     bool open; hipStream_t st;
     bool has_tn, has_nt, few;                              /* few: the input gradient held is `small` */
     Tn3Args tn; int tn_grid, tn_slot;
-    SmArgs small; int io;
+    SmArgs small; int rt, io;                              /* rt: its height on its own, 16 or 32 rows */
     Nt3Args nt; int nt_grid, nt_slot; bool nt_units;
 };
 static PairState g_pair = {};
@@ -74,7 +74,7 @@ int qlmx_pair_flush(void){
     if(!p.has_tn && !p.has_nt) return QLMX_OK;
     const bool tn = p.has_tn, nt = p.has_nt;
     p.has_tn = p.has_nt = false;
-    if(tn && !nt) return p.few ? qlmx_gemm_tn_small_issue(p.small, 2, p.io, p.tn_slot, p.st) : qlmx_gemm_tn_lds_issue(p.tn, p.tn_grid, p.tn_slot, p.st);
+    if(tn && !nt) return p.few ? qlmx_gemm_tn_small_issue(p.small, p.rt, p.io, p.tn_slot, p.st) : qlmx_gemm_tn_lds_issue(p.tn, p.tn_grid, p.tn_slot, p.st);
     if(nt && !tn) return qlmx_gemm_nt_lds_issue(p.nt, p.nt_grid, p.nt_slot, p.nt_units, p.st);
     if(p.few){
         const int rc = p.io == SM_SCATTER ? launch_few<SM_SCATTER>(p) : p.io == SM_SWIGLU_BWD ? launch_few<SM_SWIGLU_BWD>(p) : launch_few<SM_PLAIN>(p);
@@ -113,15 +113,18 @@ int qlmx_pair_hold_tn(const Tn3Args &a, int grid, int slot, hipStream_t st, bool
     p.tn = a; p.tn_grid = grid; p.tn_slot = slot; p.has_tn = true; p.few = false; *held = true;
     return QLMX_OK;
 }
-int qlmx_pair_hold_tn_few(const SmArgs &a, int io, int slot, hipStream_t st, bool *held){
+/* a table of tiles of 16 rows (rt 1) is one of 32 too: no problem has more than 16 */
+int qlmx_pair_hold_tn_few(const SmArgs &a, int rt, int io, int slot, hipStream_t st, bool *held){
     PairState &p = g_pair;
     *held = false;
     if(!p.open || st != p.st) return QLMX_OK;
     if(p.has_tn){ const int rc = qlmx_pair_flush(); if(rc) return rc; }
-    p.small = a; p.io = io; p.tn_slot = slot; p.has_tn = true; p.few = true; *held = true;
+    p.small = a; p.rt = rt; p.io = io; p.tn_slot = slot; p.has_tn = true; p.few = true; *held = true;
     return QLMX_OK;
 }
 bool qlmx_pair_open(hipStream_t st){ return g_pair.open && g_pair.st == st; }
+/* a weight gradient is held that has no input gradient yet */
+bool qlmx_pair_waits(hipStream_t st){ return qlmx_pair_open(st) && g_pair.has_nt && !g_pair.has_tn; }
 int qlmx_pair_hold_nt(const Nt3Args &a, int grid, int slot, bool units, hipStream_t st, bool *held){
     PairState &p = g_pair;
     *held = false;

@@ -67,6 +67,7 @@
  * the tiled kernel. Vector issue is at 15-29 % in the input gradient, the address units at 24-51 %, the matrix cores at 4-14 %.
  */
 #include "qlmx_gemm_tn_small_body.h"
+#include <algorithm>
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -367,7 +368,8 @@ static int sm_tn_height(const SmRows &r, long long contraction, int strips){
     return r.t32 * strips <= qlmx_cu_count() && contraction >= 1024 ? 2 : 4;
 }
 bool qlmx_pair_open(hipStream_t st);
-int qlmx_pair_hold_tn_few(const SmArgs &a, int io, int slot, hipStream_t st, bool *held);
+bool qlmx_pair_waits(hipStream_t st);
+int qlmx_pair_hold_tn_few(const SmArgs &a, int rt, int io, int slot, hipStream_t st, bool *held);
 static SmArgs sm_args(const signed char *d, const float *s, int group, int K, int N, const ProbUpload &up){
     SmArgs a = {};
     a.pr = up.dev; a.nprob = up.nprob; a.ntiles = up.ntiles; a.d = d; a.s = s; a.K = K; a.N = N;
@@ -433,21 +435,29 @@ int qlmx_gemm_tn_small_issue(const SmArgs &a, int rt, int io, int slot, hipStrea
 /* N % 128 == 0, K % 64 == 0, group a power of two >= 64; the rest as in qlmx_gemm_tn_lds_launch */
 int qlmx_gemm_tn_small_launch(const signed char *d, const float *s, int group, const qlmx_gemm_prob *probs, const qlmx_gemm_prob *second, int nprob,
                               int K, int N, float *out, const float *gp, const float *up_, void *dg, void *du, hipStream_t st){
-    /* one grid with a weight gradient: tiles of 32 rows, two workgroups to a CU, as that kernel's */
-    const bool pair = qlmx_pair_open(st);
+    /* In one grid with a weight gradient the tiles are of 32 rows, two workgroups to a CU as that kernel's: 0.58-0.99 of the two launches, this one on its own height (60 drawn pairs).
+     * On its own where it would be 64 rows, that takes 0.63-1.25, so it is held only for a weight gradient that is there already: one that comes later finds it launched. */
+    const int alone = sm_tn_height(sm_rows(probs, nprob), (long long)K * (second ? 2 : 1), N / SM_TCOLS);
+    bool pair = alone <= 2 ? qlmx_pair_open(st) : qlmx_pair_waits(st);
     if(!pair){ const int rc = qlmx_pair_flush(); if(rc) return rc; }
-    const int rt = pair ? 2 : sm_tn_height(sm_rows(probs, nprob), (long long)K * (second ? 2 : 1), N / SM_TCOLS);
+    int rt = pair ? std::min(alone, 2) : alone;
     ProbUpload up; int slot;
-    int rc = second ? qlmx_upload_problem_pairs(probs, second, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot)
-                    : qlmx_upload_problems(probs, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot);
-    if(rc) return rc;
+    auto upload = [&]{
+        return second ? qlmx_upload_problem_pairs(probs, second, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot)
+                      : qlmx_upload_problems(probs, nprob, GEMM_TN, K, N, rt * 16, SM_TCOLS, st, &up, &slot);
+    };
+    int rc = upload(); if(rc) return rc;
+    if(rt != alone && !qlmx_pair_waits(st)){               /* the slot opened a segment of the ring, which issues what is held */
+        pair = false; rt = alone;
+        rc = upload(); if(rc) return rc;
+    }
     if(up.ntiles == 0) return QLMX_OK;
     SmArgs a = sm_args(d, s, group, K, N, up);
     a.out = out; a.gp = gp; a.up = up_; a.dg = (unsigned short *)dg; a.du = (unsigned short *)du;
     const int io = out ? SM_SCATTER : gp ? SM_SWIGLU_BWD : SM_PLAIN;
     if(pair){
         bool held;
-        rc = qlmx_pair_hold_tn_few(a, io, slot, st, &held); if(rc) return rc;
+        rc = qlmx_pair_hold_tn_few(a, rt, io, slot, st, &held); if(rc) return rc;
         if(held) return QLMX_OK;
     }
     return qlmx_gemm_tn_small_issue(a, rt, io, slot, st);

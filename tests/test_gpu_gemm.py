@@ -1027,10 +1027,11 @@ def test_side_stream_fork_join(q, orc):
 
 
 @pytest.mark.parametrize("form", ["plain", "added", "continued", "swiglu", "scatter"])
-@pytest.mark.parametrize("rows,K,N", [([9, 16, 0, 1], 256, 512), ([40, 33, 64, 17, 1], 128, 1024), ([125, 131, 97], 512, 384), ([1200, 3], 256, 256)])
-def test_backward_pair_of_few_rows(q, form, rows, K, N):
+@pytest.mark.parametrize("rows,K,N,tall", [([9, 16, 0, 1], 256, 512, False), ([40, 33, 64, 17, 1], 128, 1024, False), ([125, 131, 97], 512, 384, True), ([1200, 3], 256, 256, True)])
+def test_backward_pair_of_few_rows(q, form, rows, K, N, tall):
     """The kernels for few rows in one grid with the weight gradient: the bits of the two launches, for every form of the input gradient, row tiles of
-    one and two sixteens, a sliced weight gradient behind it, no weight gradient at all, and a second one of each kind."""
+    one and two sixteens, a sliced weight gradient behind it, no weight gradient at all, and a second one of each kind. Before the end nothing of a pair has run; an
+    input gradient whose tiles are of 64 rows on its own has, where no weight gradient was there before it."""
     import torch
     cur = torch.cuda.current_stream().cuda_stream
     E, R, bf = len(rows), sum(rows), (pkg.ACT_BF16, pkg.MATH_MFMA)
@@ -1070,6 +1071,10 @@ def test_backward_pair_of_few_rows(q, form, rows, K, N):
                 weights(1.0, dY2)
                 inputs()
             if partner == "after": weights()
+            if pair and partner != "twice":
+                torch.cuda.synchronize()
+                ran = [bool((t != fresh).any()) for t, fresh in ((G, 1), (dX, 1), (spread, 1), (dg, 0), (du, 0))]
+                assert not ran[0] and any(ran[1:]) == (tall and partner != "before"), (partner, ran)
             if pair:
                 q.pair_end(cur)
             torch.cuda.synchronize()
