@@ -1049,36 +1049,45 @@ def test_backward_pair_of_few_rows(q, form, rows, K, N, tall):
     def igrad(C, src, first, beta=0.0, size=4):
         width = 1 if C is idx else K
         return q.problems([(src.data_ptr() + int(at[e]) * N * 2, None, C.data_ptr() + int(at[e]) * width * 4, (first + e) * N * K, (first + e) * N * K // 128, rows[e], beta) for e in range(E)])
+
+    def one(pair, partner):
+        """The outputs, and what has run before the pair's end (a launch that opens a segment of the table ring issues what is held, once in several launches)."""
+        G, dX, spread = torch.ones(E * K * N, device="cuda"), torch.ones(R, K, device="cuda"), torch.ones(R + 3, K, device="cuda")
+        dg, du = torch.zeros(R, K, device="cuda", dtype=torch.bfloat16), torch.zeros(R, K, device="cuda", dtype=torch.bfloat16)
+
+        def weights(beta=0.0, src=dY): q.gemm_nt(wgrad(G, src, beta), E, K, N, *bf, cur)
+
+        def inputs():
+            if form == "plain": q.gemm_tn(d, s, 128, igrad(dX, dY, 0), E, N, K, *bf, cur)
+            elif form == "added": q.gemm_tn(d, s, 128, igrad(dX, dY, 0, 1.0), E, N, K, *bf, cur)
+            elif form == "continued": q.gemm_tn_pair(d, s, 128, igrad(dX, dY, 0), igrad(dX, dY2, E, 1.0), E, N, K, *bf, cur)
+            elif form == "swiglu": q.gemm_tn_swiglu_bwd(d, s, 128, igrad(gp, dY, 0), E, N, K, gp, up, dg, du, cur)
+            else: q.gemm_tn_pair_scatter(d, s, 128, igrad(idx, dY, 0), igrad(idx, dY2, E), E, N, K, spread, cur)
+        if pair:
+            q.pair_begin(cur)
+        if partner in ("before", "twice"): weights()
+        inputs()
+        if partner == "twice":
+            weights(1.0, dY2)
+            inputs()
+        if partner == "after": weights()
+        ran = None
+        if pair:
+            torch.cuda.synchronize()
+            ran = [bool((G != 1).any()), bool((dX != 1).any() or (spread != 1).any() or dg.any() or du.any())]
+            q.pair_end(cur)
+        torch.cuda.synchronize()
+        return (G, dX, spread, dg, du), ran
     outs = []
     for pair in (False, True):
         for partner in ("after", "before", "none", "twice"):
-            G, dX, spread = torch.ones(E * K * N, device="cuda"), torch.ones(R, K, device="cuda"), torch.ones(R + 3, K, device="cuda")
-            dg, du = torch.zeros(R, K, device="cuda", dtype=torch.bfloat16), torch.zeros(R, K, device="cuda", dtype=torch.bfloat16)
-
-            def weights(beta=0.0, src=dY): q.gemm_nt(wgrad(G, src, beta), E, K, N, *bf, cur)
-
-            def inputs():
-                if form == "plain": q.gemm_tn(d, s, 128, igrad(dX, dY, 0), E, N, K, *bf, cur)
-                elif form == "added": q.gemm_tn(d, s, 128, igrad(dX, dY, 0, 1.0), E, N, K, *bf, cur)
-                elif form == "continued": q.gemm_tn_pair(d, s, 128, igrad(dX, dY, 0), igrad(dX, dY2, E, 1.0), E, N, K, *bf, cur)
-                elif form == "swiglu": q.gemm_tn_swiglu_bwd(d, s, 128, igrad(gp, dY, 0), E, N, K, gp, up, dg, du, cur)
-                else: q.gemm_tn_pair_scatter(d, s, 128, igrad(idx, dY, 0), igrad(idx, dY2, E), E, N, K, spread, cur)
-            if pair:
-                q.pair_begin(cur)
-            if partner in ("before", "twice"): weights()
-            inputs()
-            if partner == "twice":
-                weights(1.0, dY2)
-                inputs()
-            if partner == "after": weights()
-            if pair and partner != "twice":
-                torch.cuda.synchronize()
-                ran = [bool((t != fresh).any()) for t, fresh in ((G, 1), (dX, 1), (spread, 1), (dg, 0), (du, 0))]
-                assert not ran[0] and any(ran[1:]) == (tall and partner != "before"), (partner, ran)
-            if pair:
-                q.pair_end(cur)
-            torch.cuda.synchronize()
-            outs.append((G, dX, spread, dg, du))
+            for _ in range(3):
+                out, ran = one(pair, partner)
+                if not pair or partner == "twice" or ran == [False, tall and partner != "before"]:
+                    break
+            else:
+                raise AssertionError((partner, ran))
+            outs.append(out)
     for a, b in zip(outs[:4], outs[4:]):
         for x, y in zip(a, b):
             assert torch.equal(x, y)

@@ -141,8 +141,8 @@ def test_every_even_group_up_to_eighty(lib, orc, tail):
         assert used == got.size and np.array_equal(back + f32(0), P + f32(0)), group
 
 
-def test_callers_share_the_threads_and_a_child_has_its_own(lib):
-    """Calls from several threads at once, calls after the threads have gone for want of work, and calls in a child process."""
+def test_callers_share_the_threads(lib):
+    """Calls from several threads at once, and calls after the threads have gone for want of work."""
     import threading
     import time
     rng = np.random.default_rng(9)
@@ -161,13 +161,41 @@ def test_callers_share_the_threads_and_a_child_has_its_own(lib):
         [t.start() for t in ts]
         [t.join() for t in ts]
     assert ok == [40] * len(data)
-    child = os.fork()
-    if child == 0:
-        try:
-            os._exit(0 if np.array_equal(lib.q4n_quantize(data[0], 128)[0], alone[0]) else 1)
-        finally:
-            os._exit(2)
-    assert os.waitstatus_to_exitcode(os.waitpid(child, 0)[1]) == 0
+
+
+def test_a_child_of_fork_has_threads_of_its_own():
+    """Children made while threads of the library sleep, and while other threads are in calls: each writes the same bytes on threads of its own, and ends in time."""
+    code = CREW_CODE + """
+import signal
+want = lib.q4n_quantize(P, 128)[0]
+def child():
+    pid = os.fork()
+    if pid: return pid
+    try:
+        signal.alarm(20)                  # a child that waits for what only its parent has
+        own.update(os.listdir("/proc/self/task"))
+        ok = np.array_equal(lib.q4n_quantize(P, 128)[0], want)
+        os._exit(0 if ok and (crew() or os.cpu_count() == 1) else 1)
+    finally:
+        os._exit(2)
+def finish(pid): assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
+assert crew() or os.cpu_count() == 1
+finish(child())
+stop = []
+def busy():
+    while not stop: call()
+busy_ones = [threading.Thread(target=busy) for _ in range(3)]
+[t.start() for t in busy_ones]
+pids = []
+for i in range(8):
+    time.sleep(0.01)
+    pids.append(child())
+stop.append(1)
+[t.join() for t in busy_ones]
+for pid in pids: finish(pid)
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
 
 
 MODES = ("default", "flush", "up", "down", "zero")
