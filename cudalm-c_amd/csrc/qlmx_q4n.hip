@@ -36,7 +36,8 @@
  * group: with scalar divisions there, as the remainders of 32 had, 40 K values in groups of 24 took 350 us to write, of 16 384, of 56 175; now 66, 91, 42 (with divisions eight at a time
  * 87, 116, 67). All of it in parts by up to eight threads (sixteen were slower). Seven threads take 80 us to start and 15 to wake, so they are kept (Q4nCrew below).
  * 4 M values, a tenth of the groups raw, on the 16 CPUs of a GPU's share, us: write and read by one thread with scalar arithmetic 7900 + 990, divisions and threads started in
- * each call 330-500 + 180, as here 160-200 + 95-125; half the groups raw, groups of 64: 560 + 420 -> 290 + 340. */
+ * each call 350-410 + 230-260, as here 180-190 + 160-170, into memory that has been written before. A caller that takes new memory for each call, as the Python calls do, pays for the first touch
+ * of its pages: 510-540 + 160-170 (reused by the allocator in part; all pages new 850-930 + 3200-3500). */
 #define Q4N_WRITE_PART (48 * 1024)              /* values to a part: several parts a thread, since threads wake one after the other */
 #define Q4N_READ_PART (128 * 1024)
 #define Q4N_MAX_THREADS 8
@@ -54,7 +55,7 @@ static int q4n_parts(size_t n, size_t ngroups, int group, size_t part){ return (
 struct Q4nJob {
     const std::function<void(int)> *phase[2]; int parts;
     const unsigned mode = _mm_getcsr() & ~(unsigned)_MM_EXCEPT_MASK;
-    cpu_set_t cpus; const bool placed = sched_getaffinity(0, sizeof cpus, &cpus) == 0;      /* false: more CPUs than the set has room for */
+    cpu_set_t cpus; bool placed;                           /* not placed: more CPUs than the set has room for */
     std::atomic<int> next[2], done[2];
     int holders; Q4nJob *link;                             /* both under the crew's lock */
     Q4nJob() : parts(0), holders(0), link(nullptr) { for(int i = 0; i < 2; i++){ phase[i] = nullptr; next[i] = 0; done[i] = 0; } }
@@ -115,6 +116,7 @@ struct Q4nCrew {
     }
     bool run(Q4nJob &j, int wanted){                       /* false: not for this caller */
         const Q4nPriority mine;
+        j.placed = sched_getaffinity(0, sizeof j.cpus, &j.cpus) == 0;
         {
             std::lock_guard<std::mutex> l(lock);
             if(threads == 0) theirs = mine;
