@@ -37,7 +37,7 @@
  * 87, 116, 67). All of it in parts by up to eight threads (sixteen were slower). Seven threads take 80 us to start and 15 to wake, so they are kept (Q4nCrew below).
  * 4 M values, a tenth of the groups raw, on the 16 CPUs of a GPU's share, us: write and read by one thread with scalar arithmetic 7900 + 990, divisions and threads started in
  * each call 350-410 + 230-260, as here 180-190 + 160-170, into memory that has been written before. A caller that takes new memory for each call, as the Python calls do, pays for the first touch
- * of its pages: 510-540 + 160-170 (reused by the allocator in part; all pages new 850-930 + 3200-3500). */
+ * of its pages: 510-540 + 160-170 (large pages, in part used ones; all new, of 4 KB, 850-930 + 3200-3500). */
 #define Q4N_WRITE_PART (48 * 1024)              /* values to a part: several parts a thread, since threads wake one after the other */
 #define Q4N_READ_PART (128 * 1024)
 #define Q4N_MAX_THREADS 8

@@ -77,7 +77,8 @@ int         qlmx_side_join(void *stream);
  * hardware queues that the side stream costs at its fork and join. The caller promises what it promises for the
  * side stream: neither of the two reads what the other writes. Everything else keeps its order on the stream:
  * a second launch of a kind already held, a launch of a shape that none of these kernels takes, and any
- * other library call that queues work first issue what is held. One pair at a time; not for use across host
+ * other library call that queues work first issue what is held. An input gradient of few rows whose tiles are
+ * taller on its own is held only for a weight gradient that is held already: queue the weight gradient first. One pair at a time; not for use across host
  * synchronisation (nothing held runs before qlmx_pair_end or one of the calls just named). */
 int         qlmx_pair_begin(void *stream);
 int         qlmx_pair_end(void *stream);
@@ -446,7 +447,8 @@ int qlmx_test_step_wide(int on);
  * (may be NULL) = groups stored raw. dequantize: *used (may be NULL) = bytes consumed.
  * Scratch is a few bytes per group of the values (writer) or per group that len bytes can hold (reader), and one group's digits
  * for each 48 K values (groups longer than 4096: eight times); QLMX_E_LIMIT if it cannot be had.
- * Large calls share up to seven threads of the library with all callers; the threads end after a second without work.
+ * Large calls share up to seven threads of the library with all callers of one scheduling policy and priority; other callers start threads for the
+ * call. A thread works in its caller's floating-point mode and on its caller's CPUs; the kept ones end after a second without work.
  * ===================================================================================== */
 size_t qlmx_q4n_bound(size_t n, int group);
 int qlmx_q4n_quantize(const float *P, size_t n, int group, unsigned char *out, size_t cap, size_t *out_len, size_t *nraw);
