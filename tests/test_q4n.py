@@ -291,6 +291,7 @@ for want, many in ((everywhere, 20), (two, 20)):
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+@pytest.mark.skipif(os.getpriority(os.PRIO_PROCESS, 0) >= 19, reason="needs a priority below its own")
 def test_kept_threads_serve_callers_of_their_own_priority():
     """Threads started by a caller of low priority do nothing for one of ordinary priority, which has threads of its own as long as they are there, and the other
     way round; once they have gone the next caller's are kept."""
@@ -311,7 +312,7 @@ time.sleep(2.5)
 assert not crew()
 call()
 kept = crew()
-assert kept and all(os.getpriority(os.PRIO_PROCESS, t) == 0 for t in kept)
+assert kept and all(os.getpriority(os.PRIO_PROCESS, t) == os.getpriority(os.PRIO_PROCESS, 0) for t in kept)
 before = {t: ran(t) for t in kept}
 threaded(low)
 assert not worked()
